@@ -26,7 +26,7 @@ class Layout(C.Structure):
 def build(ref=True):
     """Compile the oracle (and the reference shim when the reference tree is present)."""
     subprocess.run(["make", "-s", "-C", _HERE], check=True)
-    if ref and os.path.isdir(os.environ.get("PTO_REFERENCE", "/root/reference")):
+    if ref and os.path.isdir(os.path.join(os.environ.get("PTO_REFERENCE", "/root/reference"), "include", "pto")):
         subprocess.run(["make", "-s", "-C", _HERE, "ref"], check=True)
 
 

@@ -76,7 +76,10 @@ def build_host(verbose=True):
             print("built", out)
 
 
+# the reference's tree, "" where it is not mounted (an empty mount point counts as not mounted)
 REFERENCE = os.environ.get("PTO_REFERENCE", "/root/reference")
+if not os.path.isdir(os.path.join(REFERENCE, "include", "pto")):
+    REFERENCE = ""
 # the reference's kernel sources compiled against this library's headers are the thing under test, not the checker: they are
 # kept apart from oracle/_ref (the compiled reference that the oracle is pinned against)
 PORTED_DIR = os.path.join(ROOT, "build", "ported")
