@@ -19,6 +19,8 @@ int pto_gemm_f16f32_variant(void *stream, float *c, const uint16_t *a, const uin
 /* four wavefronts, K-steps of 64, A in a ring per wave: 0 = 256 x 256 tiles, 1 = 256 x 192, 2 = 256 x 128, 3 = 192 x 256,
  * 4 = 192 x 192, 5 = 192 x 128 (csrc/pto_gemm_w4.hip) */
 int pto_gemm_f16f32_w4_variant(void *stream, float *c, const uint16_t *a, const uint16_t *b, int m, int n, int k, int variant);
+/* eight wavefronts, k split over two groups: tile shapes by number (csrc/pto_gemm_ks.hip) */
+int pto_gemm_f16f32_ks_variant(void *stream, float *c, const uint16_t *a, const uint16_t *b, int m, int n, int k, int variant);
 /* MX GEMM: variant 0 .. 3: bit 0 = quarter tiles in the last round, bit 1 = the shallower copy pipeline (csrc/pto_gemm_mx.hip);
  * fp8 formats only: 4 = the four-wave kernel with the width its estimate picks, 5 = its 256 x 192 tiles, 6 = 256 x 128
  * (csrc/pto_gemm_mxw4.hip) */

@@ -71,6 +71,28 @@ def test_gemm_four_wave_tile_widths_exact():
     assert fn(0, p, p, p, 256, 770, 256, 1) == capi.ERR_UNSUPPORTED      # rows of C not a multiple of 16 bytes
 
 
+@pytest.mark.parametrize("variant,bm,bn", [(0, 32, 64), (1, 64, 64), (2, 64, 96), (3, 128, 64), (4, 128, 96), (5, 128, 128), (6, 192, 128),
+                                           (7, 256, 128), (8, 192, 192)])
+def test_gemm_k_split_tile_shapes_exact(variant, bm, bn):
+    """Every tile shape of the kernel that splits k over two groups of wavefronts, integer inputs, the whole matrix exactly:
+    less than a tile, one tile, edges one row / four columns past a tile, several tile rows and columns; one K-step, an odd
+    and an even number of them, a last half step (k % 64 == 32) alone and behind whole ones.  Nothing outside C is written."""
+    import torch
+    from gpu_util import to_dev
+    fn = capi.load_st().pto_gemm_f16f32_ks_variant
+    for m, n, k in ((1, 4, 32), (bm, bn, 64), (bm + 1, bn + 4, 96), (bm - 1, bn - 4, 128), (3 * bm + 5, 2 * bn + 12, 192), (2 * bm, 9 * bn, 352),
+                    (9 * bm - 7, bn, 448)):
+        a, b = datagen.gemm_inputs_integer(m, n, k)
+        want = (a.astype(np.int64) @ b.astype(np.int64).T).astype(np.float32)
+        ta, tb = to_dev(a), to_dev(b)
+        guarded = torch.full((m * n + 512,), -1.0, dtype=torch.float32, device="cuda:0")
+        capi.check(fn(0, guarded.data_ptr() + 1024, ta.data_ptr(), tb.data_ptr(), m, n, k, variant), "k-split GEMM shape %d" % variant)
+        torch.cuda.synchronize()
+        got = guarded.cpu().numpy()
+        assert np.array_equal(got[256:256 + m * n].reshape(m, n), want), (m, n, k)
+        assert (got[:256] == -1.0).all() and (got[256 + m * n:] == -1.0).all(), (m, n, k)
+
+
 def test_gemm_ragged_m_and_n_exact():
     """Extents that the tiles do not divide: the last tile row / column is moved back to end with the matrix.  Integer
     operands, every element exact: each width of the four-wave kernel on small shapes (one tile that is also the moved
