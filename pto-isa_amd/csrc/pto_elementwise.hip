@@ -53,31 +53,61 @@ __global__ __launch_bounds__(kBlockThreads) AICORE void CvtF32(__gm__ D *dst, __
     TSTORE(dstGlobal, dstTile);
 }
 
-// Whole tiles in the default rounding mode take a streaming form of the same conversion below the tile instructions:
-// a lane loads 16 bytes and stores 8, so that every load instruction of a wave covers 1 KiB of consecutive addresses and
-// every store 512 bytes (a Vec tile gives a lane eight consecutive elements, i.e. two loads 32 bytes apart per lane and
-// half-used lines per instruction), all eight loads of a lane are in flight before the first conversion, and there is
-// no barrier; the stores are non-temporal (measured with inputs and outputs that no cache holds: 6.5 against 6.2 TB/s
-// with plain stores).  Same element function as TCVT (detail::convert), so the results are the same bits.
-template <typename D>
-__global__ __launch_bounds__(kBlockThreads) void CvtF32Stream(D *dst, const float *src, size_t firstTile)
+// Buffers aligned to its accesses take a streaming form of the same conversion below the tile instructions: a lane loads
+// 16 bytes and stores 8, so that every load instruction of a wave covers 1 KiB of consecutive addresses and every store
+// 512 bytes (a Vec tile gives a lane eight consecutive elements, i.e. two loads 32 bytes apart per lane and half-used
+// lines per instruction), all loads of a lane are in flight before the first conversion, and there is no barrier; the
+// stores are non-temporal (measured with inputs and outputs that no cache holds: 6.5 against 6.2 TB/s with plain
+// stores).  Same element function as TCVT (detail::convert), so the results are the same bits.  The last workgroup takes
+// what is left behind the whole pieces, element by element past the last four: as a launch of its own that rest took
+// 3.7 us (16 524 000 elements 20.0 -> 16.2 us, 6.1 TB/s; 2^27 - 5 elements 126.6 -> 123.9, 6.5 TB/s).  Four loads per lane
+// rather than eight: 2^26 elements 61.6 -> 61.1 us; two for the modes that round in integer arithmetic, where more waves
+// hide more of it (2^26 elements downwards: tile form 77.4, eight loads 68.7, four 64.3, two 63.5 us).
+template <int MODE>
+constexpr int kCvtPiece = MODE == PTO_CAST_RINT ? 4 * 4 * kBlockThreads : 2 * 4 * kBlockThreads; // elements per workgroup
+template <typename D, int MODE>
+__global__ __launch_bounds__(kBlockThreads) void CvtF32Stream(D *dst, const float *src, size_t n, size_t firstPiece)
 {
     typedef float f32x4 __attribute__((ext_vector_type(4)));
     typedef uint16_t u16x4 __attribute__((ext_vector_type(4)));
-    constexpr int kPerStep = kBlockThreads * 4, kSteps = kCvtTile / kPerStep;
-    static_assert(kCvtTile % kPerStep == 0 && sizeof(D) == 2, "whole steps of 16-bit results");
-    const size_t base = (firstTile + blockIdx.x) * (size_t)kCvtTile + 4 * threadIdx.x;
+    constexpr int kPerStep = kBlockThreads * 4, kSteps = kCvtPiece<MODE> / kPerStep;
+    static_assert(sizeof(D) == 2, "16-bit results");
+    auto cvt = [](float v) { return __builtin_bit_cast(uint16_t, ::pto::detail::convert<D, float>(v, static_cast<RoundMode>(MODE))); };
+    const size_t first = (firstPiece + blockIdx.x) * (size_t)kCvtPiece<MODE>, base = first + 4 * threadIdx.x;
     f32x4 x[kSteps];
+    if (first + kCvtPiece<MODE> <= n) {
 #pragma unroll
-    for (int i = 0; i < kSteps; ++i)
-        x[i] = __builtin_nontemporal_load(reinterpret_cast<const f32x4 *>(src + base + (size_t)i * kPerStep));
+        for (int i = 0; i < kSteps; ++i)
+            x[i] = __builtin_nontemporal_load(reinterpret_cast<const f32x4 *>(src + base + (size_t)i * kPerStep));
+#pragma unroll
+        for (int i = 0; i < kSteps; ++i) {
+            u16x4 y;
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                y[j] = cvt(x[i][j]);
+            __builtin_nontemporal_store(y, reinterpret_cast<u16x4 *>(dst + base + (size_t)i * kPerStep));
+        }
+        return;
+    }
 #pragma unroll
     for (int i = 0; i < kSteps; ++i) {
-        u16x4 y;
+        const size_t at = base + (size_t)i * kPerStep;
+        if (at + 4 <= n)
+            x[i] = __builtin_nontemporal_load(reinterpret_cast<const f32x4 *>(src + at));
+    }
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
-            y[j] = __builtin_bit_cast(uint16_t, ::pto::detail::convert<D, float>(x[i][j], RoundMode::CAST_RINT));
-        __builtin_nontemporal_store(y, reinterpret_cast<u16x4 *>(dst + base + (size_t)i * kPerStep));
+    for (int i = 0; i < kSteps; ++i) {
+        const size_t at = base + (size_t)i * kPerStep;
+        if (at + 4 <= n) {
+            u16x4 y;
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                y[j] = cvt(x[i][j]);
+            __builtin_nontemporal_store(y, reinterpret_cast<u16x4 *>(dst + at));
+        } else {
+            for (size_t e = at; e < n; ++e) // at most three, of one lane
+                dst[e] = __builtin_bit_cast(D, cvt(src[e]));
+        }
     }
 }
 
@@ -150,12 +180,24 @@ int launch_cvt(void *stream, D *dst, const float *src, size_t n, int mode)
     const bool aligned = reinterpret_cast<uintptr_t>(src) % 16 == 0 && reinterpret_cast<uintptr_t>(dst) % 8 == 0;
     // the grid's x extent is limited to 2^31-1 blocks; stay far below it per launch
     constexpr size_t kMaxBlocks = 1u << 30;
+    if (aligned) {
+        using Kernel = void (*)(D *, const float *, size_t, size_t);
+        Kernel kernel = CvtF32Stream<D, PTO_CAST_RINT>;
+        if constexpr (std::is_same_v<D, half>) { // (bf16 has the one mode)
+            static constexpr Kernel kByMode[] = {CvtF32Stream<D, PTO_CAST_RINT>, CvtF32Stream<D, PTO_CAST_ROUND>, CvtF32Stream<D, PTO_CAST_FLOOR>,
+                                                 CvtF32Stream<D, PTO_CAST_CEIL>, CvtF32Stream<D, PTO_CAST_TRUNC>, CvtF32Stream<D, PTO_CAST_ODD>};
+            kernel = kByMode[mode - PTO_CAST_RINT];
+        }
+        const size_t piece = mode == PTO_CAST_RINT ? kCvtPiece<PTO_CAST_RINT> : kCvtPiece<PTO_CAST_ROUND>, pieces = (n + piece - 1) / piece;
+        for (size_t t0 = 0; t0 < pieces; t0 += kMaxBlocks) {
+            const size_t nb = pieces - t0 < kMaxBlocks ? pieces - t0 : kMaxBlocks;
+            kernel<<<dim3((unsigned)nb), dim3(kBlockThreads), 0, st>>>(dst, src, n, t0);
+        }
+        return pto_amd::check_launch();
+    }
     for (size_t t0 = 0; t0 < full; t0 += kMaxBlocks) {
         const size_t nb = full - t0 < kMaxBlocks ? full - t0 : kMaxBlocks;
-        if (mode == PTO_CAST_RINT && aligned)
-            CvtF32Stream<D><<<dim3((unsigned)nb), dim3(kBlockThreads), 0, st>>>(dst, src, t0);
-        else
-            CvtF32<D, false><<<dim3((unsigned)nb), dim3(kBlockThreads), 0, st>>>(dst, src, n, t0, mode);
+        CvtF32<D, false><<<dim3((unsigned)nb), dim3(kBlockThreads), 0, st>>>(dst, src, n, t0, mode);
     }
     if (tail)
         CvtF32<D, true><<<dim3(1), dim3(kBlockThreads), 0, st>>>(dst, src, n, full, mode);

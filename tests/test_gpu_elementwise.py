@@ -72,6 +72,26 @@ def test_tcvt_round_modes(oracle):
         assert np.all(np.abs(h - xf) <= np.maximum(np.abs(xf) * 2.0**-10, 2.0**-24))   # within one fp16 ulp
 
 
+@pytest.mark.parametrize("n", [1, 3, 4, 1023, 2048, 2051, 4096, 4101, 3 * 4096 + 1021])
+def test_tcvt_streaming_and_tile_forms_agree(n):
+    """Buffers aligned to 16 / 8 bytes take the streaming kernel, others the tile form: the same bits in every mode, whole
+    pieces, their edges and the rest behind them; nothing written behind the last element."""
+    from gpu_util import to_dev
+    lib = capi.load()
+    x = datagen.tcvt_input(1, n + 8, inject=0.05).reshape(-1)[:n]
+    src = torch.zeros(n + 1, dtype=torch.float32, device="cuda:0")
+    tx = to_dev(x)
+    src[1:] = tx                                      # 4 bytes off: not aligned
+    for fn, modes in ((lib.pto_tcvt_f32_f16, range(capi.CAST_RINT, capi.CAST_ODD + 1)), (lib.pto_tcvt_f32_bf16, (capi.CAST_RINT,))):
+        for mode in modes:
+            a, b = (torch.full((n + 16,), 0x5a5a, dtype=torch.int16, device="cuda:0") for _ in range(2))
+            capi.check(fn(0, a.data_ptr(), tx.data_ptr(), n, mode), "aligned")
+            capi.check(fn(0, b.data_ptr(), src.data_ptr() + 4, n, mode), "not aligned")
+            torch.cuda.synchronize()
+            assert torch.equal(a, b), (n, mode)
+            assert (a[n:] == 0x5a5a).all() and (b[n:] == 0x5a5a).all(), (n, mode)
+
+
 def test_tcvt_full_size_config(oracle):
     """Config 5 at full size 16384 x 8192 with 0.1% special values: compared in slabs against the oracle."""
     from gpu_util import to_dev, stream
