@@ -111,33 +111,42 @@ __global__ __launch_bounds__(kBlockThreads) void CvtF32Stream(D *dst, const floa
     }
 }
 
-constexpr int kGatherRows = 32, kGatherCols = 256; // one Vec tile: 8192 elements
-
-template <typename T, bool kTailCols>
-__global__ __launch_bounds__(kBlockThreads) AICORE void GatherRows(__gm__ T *out, __gm__ const T *table,
-                                                                   __gm__ const int32_t *idx, int nIdx, int tableRows,
-                                                                   int cols, int colBlocks)
+// Row gather as a stream of 16-byte chunks: out is n_idx rows of cpr chunks, chunk c comes from chunk c % cpr of table row
+// idx[c / cpr] (zeros for an index outside the table).  Consecutive lanes take consecutive chunks, whatever the width of a
+// row, so every store instruction of a wave is 1 KiB of consecutive addresses and every load whole lines of the table's
+// rows; the indices, then all loads of a lane are in flight before its first store; no LDS, no barrier.  The division is
+// a multiplication: for c < 2^31, c / cpr = c magic >> shift with magic = ceil(2^shift / cpr), shift = 31 + ceil(log2 cpr).
+// The row is cut into `parts` (1, 2, 4 or 8) slices of cpr chunks, and workgroup b works on slice (b % 8) % parts: as the
+// workgroups are dealt to the eight XCDs in turn, an XCD's L2 then sees one slice of the table only.
+constexpr int kGatherSteps = 2, kGatherChunks = kBlockThreads * kGatherSteps;
+__global__ __launch_bounds__(kBlockThreads) void GatherChunks(char *out, const char *table, const int32_t *idx, uint32_t chunks, uint32_t cpr,
+                                                              uint32_t magic, int shift, uint32_t tableRows, uint32_t parts)
 {
-    const int rb = (int)(get_block_idx() / colBlocks), cb = (int)(get_block_idx() % colBlocks);
-    const int row0 = rb * kGatherRows, col0 = cb * kGatherCols;
-    const int vRows = nIdx - row0 < kGatherRows ? nIdx - row0 : kGatherRows;
-    const int vCols = cols - col0 < kGatherCols ? cols - col0 : kGatherCols;
-    using IdxTile = Tile<TileType::Vec, int32_t, kGatherRows, 1, BLayout::ColMajor, DYNAMIC, 1>;
-    using DstTile = Tile<TileType::Vec, T, kGatherRows, kGatherCols, BLayout::RowMajor, DYNAMIC, DYNAMIC>;
-    using GIdx = GlobalTensor<int32_t, Shape<1, 1, 1, DYNAMIC, 1>, Stride<1, 1, 1, 1, DYNAMIC>, Layout::DN>;
-    using GTab = GlobalTensor<T, Shape<1, 1, 1, DYNAMIC, DYNAMIC>, Stride<1, 1, 1, DYNAMIC, 1>>;
-    IdxTile idxTile((size_t)vRows);
-    DstTile dstTile((size_t)vRows, (size_t)vCols);
-    GIdx idxGlobal(const_cast<int32_t *>(idx) + row0, Shape<1, 1, 1, DYNAMIC, 1>(vRows), Stride<1, 1, 1, 1, DYNAMIC>(vRows));
-    GTab tableGlobal(const_cast<T *>(table) + col0, Shape<1, 1, 1, DYNAMIC, DYNAMIC>(tableRows, vCols),
-                     Stride<1, 1, 1, DYNAMIC, 1>(cols));
-    GTab outGlobal(out + (int64_t)row0 * cols + col0, Shape<1, 1, 1, DYNAMIC, DYNAMIC>(vRows, vCols),
-                   Stride<1, 1, 1, DYNAMIC, 1>(cols));
-    TLOAD(idxTile, idxGlobal);
-    MGATHER_ROWS(dstTile, tableGlobal, idxTile, tableRows);
-    set_flag(PIPE_V, PIPE_MTE3, EVENT_ID0);
-    wait_flag(PIPE_V, PIPE_MTE3, EVENT_ID0);
-    TSTORE(outGlobal, dstTile);
+    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+    const uint32_t xcd = blockIdx.x % 8, slice = xcd % parts, block = blockIdx.x / 8 * (8 / parts) + xcd / parts;
+    const uint32_t first = block * (uint32_t)kGatherChunks + threadIdx.x, rowChunks = cpr * parts;
+    if (block * (uint32_t)kGatherChunks >= chunks)
+        return;
+    uint32_t row[kGatherSteps], at[kGatherSteps], part[kGatherSteps];
+#pragma unroll
+    for (int i = 0; i < kGatherSteps; ++i) {
+        const uint32_t c = first + i * kBlockThreads < chunks ? first + i * kBlockThreads : chunks - 1;
+        at[i] = (uint32_t)(((uint64_t)c * magic) >> shift);
+        part[i] = slice * cpr + (c - at[i] * cpr);
+        row[i] = (uint32_t)idx[at[i]];
+    }
+    u32x4 v[kGatherSteps];
+#pragma unroll
+    for (int i = 0; i < kGatherSteps; ++i) {
+        const bool inside = row[i] < tableRows; // (a negative index is a large one)
+        v[i] = *reinterpret_cast<const u32x4 *>(table + ((size_t)(inside ? row[i] : 0u) * rowChunks + part[i]) * 16);
+        if (!inside)
+            v[i] = u32x4{0, 0, 0, 0};
+    }
+#pragma unroll
+    for (int i = 0; i < kGatherSteps; ++i)
+        if (first + i * kBlockThreads < chunks)
+            __builtin_nontemporal_store(v[i], reinterpret_cast<u32x4 *>(out + ((size_t)at[i] * rowChunks + part[i]) * 16));
 }
 
 // One-tile TGATHER (index form), the half 16x1024 -> 16x128 case of the reference's tgather test.
@@ -228,17 +237,29 @@ extern "C" int pto_gather_rows(void *stream, void *out, const void *table, const
         return PTO_ERR_BAD_ARG;
     if (cols % 8 || n_idx > 0x7fffffffu || table_rows > 0x7fffffffu || cols > 0x7fffffffu)
         return PTO_ERR_UNSUPPORTED;
-    const size_t rowBlocks = (n_idx + kGatherRows - 1) / kGatherRows, colBlocks = (cols + kGatherCols - 1) / kGatherCols;
-    if (rowBlocks * colBlocks > 0x7fffffffu)
-        return PTO_ERR_UNSUPPORTED;
+    const size_t rowChunks = cols * (size_t)elem_bytes / 16; // cols % 8 == 0: whole chunks; below 2^30
+    uint32_t parts = 1;
+    // Slices of whole 128-byte lines, as few as bring a slice of the table down to 2 MiB of an XCD's 4 MiB of L2, where the
+    // batch reads a row twice or more on average (65536 rows of 2 KiB from a table of 16384: 38.3 us in one slice, 33.1 in
+    // four, 28.2 in eight; a table of 65536 rows, 43.9 in one, 48.5 in eight)
+    if (n_idx >= 2 * table_rows)
+        while (parts < 8 && rowChunks % (16 * parts) == 0 && table_rows * rowChunks * 16 / parts > ((size_t)2 << 20))
+            parts *= 2;
+    const size_t cpr = rowChunks / parts;
+    int shift = 31;
+    while (((size_t)1 << (shift - 31)) < cpr)
+        ++shift;
+    const uint32_t magic = (uint32_t)((((uint64_t)1 << shift) + cpr - 1) / cpr);
     hipStream_t st = static_cast<hipStream_t>(stream);
-    const dim3 grid((unsigned)(rowBlocks * colBlocks)), block(kBlockThreads);
-    if (elem_bytes == 2)
-        GatherRows<uint16_t, true><<<grid, block, 0, st>>>(static_cast<uint16_t *>(out), static_cast<const uint16_t *>(table),
-                                                           idx, (int)n_idx, (int)table_rows, (int)cols, (int)colBlocks);
-    else
-        GatherRows<uint32_t, true><<<grid, block, 0, st>>>(static_cast<uint32_t *>(out), static_cast<const uint32_t *>(table),
-                                                           idx, (int)n_idx, (int)table_rows, (int)cols, (int)colBlocks);
+    // (whole rows per launch, fewer than 2^31 chunks a slice)
+    const size_t rowsPerLaunch = 0x7fffffffu / rowChunks;
+    for (size_t r0 = 0; r0 < n_idx; r0 += rowsPerLaunch) {
+        const size_t chunks = (n_idx - r0 < rowsPerLaunch ? n_idx - r0 : rowsPerLaunch) * cpr, blocks = (chunks + kGatherChunks - 1) / kGatherChunks;
+        const size_t perGroup = 8 / parts, groups = (blocks + perGroup - 1) / perGroup;
+        GatherChunks<<<dim3((unsigned)(groups * 8)), dim3(kBlockThreads), 0, st>>>(
+            static_cast<char *>(out) + r0 * rowChunks * 16, static_cast<const char *>(table), idx + r0, (uint32_t)chunks, (uint32_t)cpr, magic, shift,
+            (uint32_t)table_rows, parts);
+    }
     return pto_amd::check_launch();
 }
 

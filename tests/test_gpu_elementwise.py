@@ -125,6 +125,21 @@ def test_gather_rows_out_of_range_indices_give_zero_rows(oracle):
     assert not got[2].any() and not got[3].any() and np.array_equal(got[4], table[5])
 
 
+@pytest.mark.parametrize("rows,cols,nidx", [(3, 8, 1), (5, 24, 700), (700, 40, 131), (1024, 1024, 2048), (1500, 1032, 3001), (2048, 2048, 4096), (3000, 1024, 6001),
+                                            (9000, 1024, 18001)])
+def test_gather_rows_widths_and_slices(oracle, rows, cols, nidx):
+    """Rows narrower than a wave's accesses and rows that no power of two divides; tables that are cut into 1, 2, 4 and 8
+    slices (read twice or more, larger than 2 / 4 / 8 MiB) with a last workgroup that is partly full, both element sizes."""
+    from gpu_util import gather_rows
+    table, idx = datagen.gather_inputs(rows, cols, nidx)
+    idx = idx.copy()
+    idx[::17] = -1 - idx[::17]
+    idx[5::31] = rows
+    assert np.array_equal(gather_rows(table, idx), oracle.gather_rows(table, idx))
+    t32 = np.random.default_rng(1).integers(0, 2**32, size=(rows, cols), dtype=np.uint64).astype(np.uint32)
+    assert np.array_equal(gather_rows(t32, idx), oracle.gather_rows(t32, idx))
+
+
 def test_gather_rows_full_size_config(oracle):
     """Config 5: 65536 int32 row indices over a 16384 x 1024 fp16 table: bit-exact copy."""
     from gpu_util import gather_rows
