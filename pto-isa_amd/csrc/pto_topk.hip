@@ -7,14 +7,27 @@
 // (include/pto/cpu/TSort32.hpp:32-41: score descending, then index ascending, -0 == +0).
 //
 // The reference builds the order from 32-element hardware sorts and 4-way merges in its unified buffer, re-viewing one
-// buffer through differently shaped tiles.  On a CDNA4 compute unit the natural form is one workgroup (four waves) per
-// row and a bitonic network over 64-bit keys whose unsigned order is the comparator:
-//   key = (order-preserving image of the score) << 32 | low word that decides among equal scores.
-// * Indices that increase with the column (the reference passes 0, 1, 2, ...): low word = ~column, and a thread keeps
-//   its N/256 consecutive keys in registers.  Partners inside a thread are compared in registers, partners inside a
-//   wave are fetched with lane swizzles, and only the two or three strides that cross waves go through LDS.
-// * Any other index vector: low word = ~index, keys and columns in LDS, every stage a pass over LDS; each wave owns a
-//   quarter of the row and the stages whose partners lie inside a quarter need no workgroup barrier.
+// buffer through differently shaped tiles.  On a CDNA4 compute unit the natural form is a bitonic network in registers:
+// one wave per row of up to 1024 columns with 2 .. 16 keys per lane, two or four waves for 2048 and 4096.
+// * Indices that increase with the column (the reference passes 0, 1, 2, ...): the order is that of (score, -column), 32 +
+//   12 bits, which fit the mantissa of a double: key = 1.order(score).(4095 - column).x, always a normal number between 1
+//   and 2.  A compare-exchange of two keys in a lane is then v_max_f64 + v_min_f64, two instructions instead of a 64-bit
+//   compare and four selects (measured, four waves per SIMD: 1.8 ns each on one SIMD, like v_cndmask and v_cmp_u64).
+// * Across lanes the sign does the choosing: before a stage a lane that is to keep the smaller key of a pair negates its
+//   key (one v_xor on the upper word); the pair then holds k and -k', and max(own, -received) is right for both lanes.
+// * The lanes of a row of 16 are numbered so that the partners of the four lowest lane strides are lane ^ 1, ^ 2, ^ 7, ^ 8:
+//   one DPP move for the upper word, and the lower word over the LDS pipe (ds_swizzle), which the network leaves idle
+//   otherwise; partners 16 and 32 lanes away come over the LDS pipe whole (v_permlane*_swap: 3.5 ns a word, 4.2 us of the
+//   kernel's time for three stages of 55); strides across waves go through LDS memory.
+// * topk below the padded row length: once the sorted runs are as long as topk (rounded up to keys per lane times a power of
+//   two), a merge of two runs keeps their larger halves only, in both runs' lanes, and its sort passes no longer cover the
+//   dropped half.
+// * Any other index vector: low word = ~index, keys and columns in LDS, every stage a pass over LDS, four waves on one row
+//   after another; each wave owns a quarter of the row and the stages whose partners lie inside a quarter need no barrier.
+// What bounds it: vector instructions, 2240 per row of 1024 (3850 in the integer network this replaced), behind a phase of
+// loads and before one of stores that all waves share: of 26.9 us (4800 x 1024, top 1000, 58 MB = 9 us at 6.5 TB/s) 12 are
+// launch, loads and stores.  Persistent waves that load the next row while they sort one, and wave priorities that let
+// some run ahead, do not hide them (32 us and no change).
 #include <hip/hip_runtime.h>
 
 #include "common.hpp"
@@ -23,52 +36,8 @@ namespace {
 
 constexpr int kTopkThreads = 256, kTopkWaves = 4;
 
-__device__ inline uint32_t ScoreOrder(uint32_t bits) { return (bits & 0x80000000u) ? ~bits : (bits | 0x80000000u); }
-__device__ inline uint32_t ScoreBits(uint32_t ord) { return (ord & 0x80000000u) ? (ord & 0x7fffffffu) : ~ord; }
-
-// value of lane ^ M of the wave, M a power of two below 64
-template <int M>
-__device__ inline uint32_t LaneXor(uint32_t v, int lane)
-{
-    // (every lane has a source lane in these three patterns, so the destination needs no initial value: mov_dpp, not
-    // update_dpp with a zero that costs a move per call)
-    if constexpr (M == 1)
-        return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0xB1, 0xf, 0xf, true); // quad_perm [1,0,3,2]
-    else if constexpr (M == 2)
-        return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x4E, 0xf, 0xf, true); // quad_perm [2,3,0,1]
-    else if constexpr (M == 8)
-        return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x128, 0xf, 0xf, true); // row_ror:8 (rows of 16 lanes)
-    else if constexpr (M < 32)
-        return (uint32_t)__builtin_amdgcn_ds_swizzle((int)v, (M << 10) | 0x1f); // bit mode: lane ^ M within 32 lanes
-    else
-        return (uint32_t)__builtin_amdgcn_ds_bpermute(((lane ^ 32) << 2), (int)v);
-}
-template <int M>
-__device__ inline uint64_t LaneXor64(uint64_t v, int lane)
-{
-    return ((uint64_t)LaneXor<M>((uint32_t)(v >> 32), lane) << 32) | LaneXor<M>((uint32_t)v, lane);
-}
-
-// Compare and select on wave masks held in scalar register pairs.  (Measured on gfx950: a conditional move that takes its
-// mask from VCC issues at a fifth of the rate of one that takes it from a scalar register pair, so the selects of the
-// network name their masks themselves instead of leaving the choice to the compiler.)  All 64 lanes are active here.
-__device__ inline uint64_t MaskLess(uint64_t a, uint64_t b)
-{
-    uint64_t m;
-    asm("v_cmp_lt_u64_e64 %0, %1, %2" : "=s"(m) : "v"(a), "v"(b));
-    return m;
-}
-__device__ inline uint32_t SelectWord(uint64_t mask, uint32_t ifSet, uint32_t ifClear)
-{
-    uint32_t r;
-    asm("v_cndmask_b32_e64 %0, %1, %2, %3" : "=v"(r) : "v"(ifClear), "v"(ifSet), "s"(mask));
-    return r;
-}
-__device__ inline uint64_t Select(uint64_t mask, uint64_t ifSet, uint64_t ifClear)
-{
-    return ((uint64_t)SelectWord(mask, (uint32_t)(ifSet >> 32), (uint32_t)(ifClear >> 32)) << 32) |
-           SelectWord(mask, (uint32_t)ifSet, (uint32_t)ifClear);
-}
+__device__ inline uint32_t ScoreOrder(uint32_t bits) { return bits ^ ((uint32_t)((int32_t)bits >> 31) | 0x80000000u); }
+__device__ inline uint32_t ScoreBits(uint32_t ord) { return ord ^ ((uint32_t)(~(int32_t)ord >> 31) | 0x80000000u); }
 
 template <int FIRST, int LAST, typename F>
 __device__ inline void StaticFor(F &&f)
@@ -79,67 +48,205 @@ __device__ inline void StaticFor(F &&f)
     }
 }
 
-// Bitonic sort, descending, of the 256 E keys of a workgroup; thread t holds the keys of ranks t E .. t E + E - 1.
-template <int E>
-__device__ inline void SortInRegisters(uint64_t (&k)[E], uint64_t *lds, int tid)
+constexpr uint32_t kSign = 0x80000000u;
+
+__device__ inline uint32_t High(double k) { return (uint32_t)(__builtin_bit_cast(uint64_t, k) >> 32); }
+__device__ inline uint32_t Low(double k) { return (uint32_t)__builtin_bit_cast(uint64_t, k); }
+__device__ inline double Key(uint32_t high, uint32_t low) { return __builtin_bit_cast(double, ((uint64_t)high << 32) | low); }
+
+// (as assembly: the compiler would add instructions that quieten signalling NaNs, and no key is one)
+__device__ inline double Max(double a, double b)
 {
-    constexpr int N = kTopkThreads * E, kLogN = __builtin_ctz(N), kLogE = __builtin_ctz(E);
-    const int lane = tid & 63;
-    // The lane predicates of the network, once: bit s of the key's rank for every run length and partner distance that
-    // spans threads (as lane masks they live in scalar registers; computed per stage they were an eighth of the vector
-    // instructions).
-    uint64_t rankBitClear[kLogN + 1]; // wave masks
-#pragma unroll
-    for (int s = 0; s <= kLogN; ++s)
-        rankBitClear[s] = s < kLogE ? ~0ull : __builtin_amdgcn_ballot_w64(((tid >> (s - kLogE)) & 1) == 0);
-    StaticFor<1, kLogN + 1>([&](auto sizeTag) {
-        constexpr int kk = 1 << decltype(sizeTag)::value; // the network sorts runs of kk keys, alternating direction
-        // lanes whose run is descending (the last stage sorts the whole row downwards)
-        const uint64_t descending = kk == N ? ~0ull : rankBitClear[decltype(sizeTag)::value];
-        StaticFor<0, decltype(sizeTag)::value>([&](auto strideTag) {
-            constexpr int j = kk >> (decltype(strideTag)::value + 1); // distance between partners
-            if constexpr (j < E) {
-#pragma unroll
-                for (int e = 0; e < E; ++e)
-                    if ((e & j) == 0) {
-                        const uint64_t a = k[e], b = k[e | j];
-                        const uint64_t less = MaskLess(a, b);
-                        // descending runs swap where a < b, ascending ones where a >= b (equal keys are the padding:
-                        // swapping them changes nothing).  Run lengths below E: the direction is a property of the
-                        // register, not of the lane.
-                        const uint64_t swap = kk < E ? ((e & kk) == 0 ? less : ~less) : ~(less ^ descending);
-                        k[e] = Select(swap, b, a);
-                        k[e | j] = Select(swap, a, b);
-                    }
-            } else {
-                uint64_t other[E];
-                if constexpr (j < 64 * E) {
-#pragma unroll
-                    for (int e = 0; e < E; ++e)
-                        other[e] = LaneXor64<j / E>(k[e], lane);
-                } else {
-                    // partners are E (j / E) ranks apart: the same register of thread tid ^ (j / E).  Register e of all
-                    // threads is one contiguous run of LDS, so a wave's 64 lanes touch 64 consecutive 8-byte words
-                    __syncthreads(); // everyone is done reading the previous exchange
-#pragma unroll
-                    for (int e = 0; e < E; ++e)
-                        lds[e * kTopkThreads + tid] = k[e];
-                    __syncthreads();
-#pragma unroll
-                    for (int e = 0; e < E; ++e)
-                        other[e] = lds[e * kTopkThreads + (tid ^ (j / E))];
-                }
-                // the lower rank of a pair keeps the larger key where the run is descending
-                const uint64_t keepMax = ~(rankBitClear[__builtin_ctz(j)] ^ descending);
-#pragma unroll
-                for (int e = 0; e < E; ++e) {
-                    const uint64_t otherLarger = MaskLess(k[e], other[e]);
-                    k[e] = Select(~(otherLarger ^ keepMax), other[e], k[e]);
-                }
-            }
-        });
-    });
+    double r;
+    asm("v_max_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
 }
+__device__ inline double Min(double a, double b)
+{
+    double r;
+    asm("v_min_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+__device__ inline double MaxOfNegated(double a, double b) // max(a, -b)
+{
+    double r;
+    asm("v_max_f64 %0, %1, -%2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+// Between instructions written as assembly and lane moves of their results: the compiler does not know that the former
+// are vector instructions, so the wait states that a lane move asks for are placed here.
+__device__ inline void StageEdge()
+{
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("s_nop 1");
+    __builtin_amdgcn_sched_barrier(0);
+}
+
+// A word of the partner at lane stride J (of the numbering by LaneRank: lane ^ 1, ^ 2, ^ 7, ^ 8, ^ 16, ^ 32), moved by the
+// vector pipe or by the LDS pipe
+template <int J>
+__device__ inline uint32_t LaneMove(uint32_t v)
+{
+    static_assert(J < 4, "inside a row of 16 lanes");
+    constexpr int kCtrl = J == 0 ? 0xB1 : J == 1 ? 0x4E : J == 2 ? 0x141 : 0x128; // quad_perm twice, row_half_mirror, row_ror:8
+    return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, kCtrl, 0xf, 0xf, true);
+}
+template <int J>
+__device__ inline uint32_t ThroughLds(uint32_t v)
+{
+    if constexpr (J < 5) {
+        constexpr int kXor = J == 0 ? 1 : J == 1 ? 2 : J == 2 ? 7 : J == 3 ? 8 : 16;
+        return (uint32_t)__builtin_amdgcn_ds_swizzle((int)v, (kXor << 10) | 0x1f);
+    } else {
+        return (uint32_t)__builtin_amdgcn_ds_bpermute((int)((threadIdx.x ^ 32u) << 2), (int)v);
+    }
+}
+// the upper word goes through the LDS pipe only where the vector pipe would need two moves
+template <int J>
+constexpr bool kHighThroughLds = J >= 4;
+
+// lane = c0 ^ 2 c1 ^ 7 c2 ^ 8 c3 ^ 16 c4 ^ 32 c5  ->  c0 + 2 c1 + 4 c2 + ...
+__device__ inline uint32_t LaneRank(uint32_t lane) { return (lane & 4u) ? lane ^ 3u : lane; }
+
+// Sorting of the 64 E W keys of a row, descending; key e of the lane with number q = 64 (wave of the row) + LaneRank(lane) is of
+// rank q E + e in the end.  keepBits: the ranks below E << keepBits are wanted.  A key is kept negated where `form` has its
+// sign bit set.  xchg: E x 64 keys per wave (W > 1).
+template <int E, int W>
+struct RowSort {
+    static constexpr int kLaneBits = 6 + (W == 4 ? 2 : W == 2 ? 1 : 0);
+    double k[E];
+    uint32_t form, q;
+    uint64_t *xchg;
+
+    __device__ inline void SetForm(uint32_t f)
+    {
+        uint32_t d = form ^ f;
+        asm("" : "+v"(d)); // (one xor per key: left to itself the compiler applies both terms to every key)
+#pragma unroll
+        for (int e = 0; e < E; ++e)
+            k[e] = Key(High(k[e]) ^ d, Low(k[e]));
+        form = f;
+    }
+    __device__ inline uint32_t Bit(int b) const { return (q >> b & 1u) ? kSign : 0u; }
+    // compare-exchange inside the lane: the larger key to the lower register
+    __device__ inline void Exchange(double &hi, double &lo)
+    {
+        const double a = Max(hi, lo), b = Min(hi, lo);
+        hi = a;
+        lo = b;
+    }
+    __device__ inline void SortLane() // all E keys, descending in the present form (Batcher's odd-even merge sort: 63 exchanges of 16 keys)
+    {
+#pragma unroll
+        for (int run = 1; run < E; run <<= 1)
+#pragma unroll
+            for (int j = run; j > 0; j >>= 1)
+#pragma unroll
+                for (int e = j % run; e + j < E; e += 2 * j)
+#pragma unroll
+                    for (int i = 0; i < j; ++i)
+                        if (e + i + j < E && (e + i) / (2 * run) == (e + i + j) / (2 * run))
+                            Exchange(k[e + i], k[e + i + j]);
+    }
+    __device__ inline void MergeLane() // a bitonic sequence of E keys
+    {
+#pragma unroll
+        for (int j = E >> 1; j > 0; j >>= 1)
+#pragma unroll
+            for (int e = 0; e < E; ++e)
+                if ((e & j) == 0)
+                    Exchange(k[e], k[e | j]);
+    }
+    // partners at lane stride J: the lane whose bit is clear keeps the larger key where dir is 0.  BOTH: either keeps the larger
+    template <int J, bool BOTH>
+    __device__ inline void Stage(uint32_t dir)
+    {
+        if constexpr (J < 6) {
+            SetForm(BOTH ? 0u : dir ^ Bit(J));
+            StageEdge();
+            uint32_t low[E], high[E];
+#pragma unroll
+            for (int e = 0; e < E; ++e) {
+                low[e] = ThroughLds<J>(Low(k[e]));
+                if constexpr (kHighThroughLds<J>)
+                    high[e] = ThroughLds<J>(High(k[e]));
+            }
+#pragma unroll
+            for (int e = 0; e < E; ++e) {
+                if constexpr (!kHighThroughLds<J>)
+                    high[e] = LaneMove<J>(High(k[e]));
+                const double o = Key(high[e], low[e]);
+                k[e] = BOTH ? Max(k[e], o) : MaxOfNegated(k[e], o);
+            }
+        } else if constexpr (J < kLaneBits) { // another wave of the row
+            SetForm(BOTH ? 0u : dir ^ Bit(J));
+            const uint32_t wave = threadIdx.x / 64, lane = threadIdx.x % 64, other = wave ^ (1u << (J - 6));
+            __syncthreads(); // everyone is done with the exchange before
+#pragma unroll
+            for (int e = 0; e < E; ++e)
+                xchg[(wave * E + e) * 64 + lane] = __builtin_bit_cast(uint64_t, k[e]);
+            __syncthreads();
+#pragma unroll
+            for (int e = 0; e < E; ++e) {
+                const double o = __builtin_bit_cast(double, xchg[(other * E + e) * 64 + lane]);
+                k[e] = BOTH ? Max(k[e], o) : MaxOfNegated(k[e], o);
+            }
+        }
+        StageEdge();
+    }
+    __device__ inline void Sort(int keepBits)
+    {
+        SetForm(Bit(0));
+        StageEdge();
+        SortLane();
+        StageEdge();
+        // (few keys: straight-line code, the branches are most of what they cost; many: one copy of the code for all runs)
+        if constexpr (E <= 4)
+            StaticFor<1, kLaneBits + 1>([&](auto run) { Merge(decltype(run)::value, keepBits); });
+        else
+            for (int run = 1; run <= kLaneBits; ++run)
+                Merge(run, keepBits);
+    }
+    // runs of E << run keys out of two of half the length, descending and ascending in turn (the last: descending)
+    __device__ inline __attribute__((always_inline)) void Merge(int run, int keepBits)
+    {
+        const uint32_t dir = run == kLaneBits ? 0u : Bit(run);
+        int strides = run;
+        if (run > keepBits) {
+            strides = keepBits;
+            switch (run - 1) {
+            case 0: Stage<0, true>(dir); break;
+            case 1: Stage<1, true>(dir); break;
+            case 2: Stage<2, true>(dir); break;
+            case 3: Stage<3, true>(dir); break;
+            case 4: Stage<4, true>(dir); break;
+            case 5: Stage<5, true>(dir); break;
+            case 6: Stage<6, true>(dir); break;
+            default: Stage<7, true>(dir); break;
+            }
+        }
+        if (W > 2 && strides > 7)
+            Stage<7, false>(dir);
+        if (W > 1 && strides > 6)
+            Stage<6, false>(dir);
+        if (strides > 5)
+            Stage<5, false>(dir);
+        if (strides > 4)
+            Stage<4, false>(dir);
+        if (strides > 3)
+            Stage<3, false>(dir);
+        if (strides > 2)
+            Stage<2, false>(dir);
+        if (strides > 1)
+            Stage<1, false>(dir);
+        if (strides > 0)
+            Stage<0, false>(dir);
+        SetForm(dir);
+        StageEdge();
+        MergeLane();
+        StageEdge();
+    }
+};
 
 // Any index vector: keys and columns in LDS, one pass over LDS per stage.
 template <int N>
@@ -173,71 +280,147 @@ __device__ inline void SortInLds(uint64_t *key, uint16_t *pos, int tid)
     __syncthreads();
 }
 
-// E: keys per thread; the row is padded to N = 256 E keys (padding keys are 0, below every real key).
-template <int E>
+// E keys per lane, W waves per row (the row is padded to 64 E W keys; padding keys lie below every real one), 4 / W rows per
+// workgroup.
+template <int E, int W>
 __global__ __launch_bounds__(kTopkThreads) void TopkRows(float *outScore, uint32_t *outIndex, const float *src, const uint32_t *inIdx,
-                                                         int validCols, int ld, int topk)
+                                                         int rows, int validCols, int ld, int topk, int keepBits)
 {
-    constexpr int N = kTopkThreads * E;
-    __shared__ uint64_t key[N];
-    __shared__ uint16_t pos[N];
-    const int tid = threadIdx.x;
-    const float *row = src + (size_t)blockIdx.x * (size_t)ld;
-    float *rowScore = outScore + (size_t)blockIdx.x * (size_t)topk;
-    uint32_t *rowIndex = outIndex + (size_t)blockIdx.x * (size_t)topk;
+    constexpr int N = 64 * E * W, kRows = kTopkWaves / W;
+    constexpr int kStaged = 64 * E + 4 * E; // words of a wave's results, one of padding behind every 16
+    constexpr int kStages = E <= 8 ? 2 : 1;  // scores and columns side by side, or one after the other (LDS for four workgroups more)
+    constexpr size_t kFallback = (size_t)N * 10, kExchange = W > 1 ? (size_t)kTopkWaves * E * 64 * 8 : 0, kStage = (size_t)kTopkWaves * kStaged * 4 * kStages;
+    constexpr size_t kLds = kFallback > kExchange ? (kFallback > kStage ? kFallback : kStage) : (kExchange > kStage ? kExchange : kStage);
+    __shared__ __attribute__((aligned(16))) char lds[kLds];
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / 64), lane = tid % 64;
+    const int waveOfRow = wave % W, row0 = (int)blockIdx.x * kRows, row = row0 + wave / W < rows ? row0 + wave / W : rows - 1;
+    const uint32_t i0 = (uint32_t)(waveOfRow * E * 64 + lane); // this lane's first column; then every 64th
 
-    // do the indices increase with the column?  (then the column decides among equal scores, as the index would)
-    bool increasing = true;
+    // A lane past the last column looks at the last one: loads without branches are all in flight at once (16 of them one
+    // behind the other were half of the kernel's time)
+    auto load = [&](const uint32_t *from, uint32_t (&to)[E]) __attribute__((always_inline)) {
+        if (validCols == N) {
+#pragma unroll
+            for (int e = 0; e < E; ++e)
+                to[e] = from[i0 + e * 64];
+        } else {
+#pragma unroll
+            for (int e = 0; e < E; ++e)
+                to[e] = from[i0 + e * 64 < (uint32_t)validCols ? i0 + e * 64 : (uint32_t)validCols - 1u];
+        }
+    };
+    uint32_t bits[E], ids[E];
+    load(reinterpret_cast<const uint32_t *>(src) + (size_t)row * (size_t)ld, bits);
+    load(inIdx, ids);
+
+    // are the indices first, first + 1, ... or at least increasing with the column?  (then the column decides among equal
+    // scores, as the index would; the same answer in every wave of the workgroup)
+    const uint32_t first = inIdx[0];
+    uint32_t wrong = 0;
 #pragma unroll
     for (int e = 0; e < E; ++e) {
-        const int i = tid * E + e;
-        if (i + 1 < validCols)
-            increasing = increasing && inIdx[i] < inIdx[i + 1];
+        const uint32_t at = i0 + e * 64 < (uint32_t)validCols ? i0 + e * 64 : (uint32_t)validCols - 1u;
+        wrong |= (ids[e] - first) ^ at;
     }
-    bool inRegisters = false;
-    if constexpr (E <= 8)
-        inRegisters = __syncthreads_and(increasing) != 0;
-    if constexpr (E <= 8) if (inRegisters) {
-        uint64_t k[E];
-#pragma unroll
+    auto everyone = [&](bool v) { return W > 1 ? __syncthreads_and(v) != 0 : __builtin_amdgcn_ballot_w64(!v) == 0; };
+    const bool consecutive = everyone(wrong == 0 && first <= 0xffffffffu - (uint32_t)validCols);
+    bool increasing = consecutive;
+    if (!consecutive) {
+        bool ok = true;
         for (int e = 0; e < E; ++e) {
-            const int i = tid * E + e;
-            k[e] = 0;
-            if (i < validCols) {
-                const uint32_t b = __float_as_uint(row[i]);
-                const bool negZero = b == 0x80000000u; // compares equal to +0: same key, remembered below the column bits
-                k[e] = ((uint64_t)ScoreOrder(negZero ? 0u : b) << 32) | ((uint32_t)(4095 - i) << 20) | (negZero ? 1u : 0u);
-            }
+            const int i = (int)i0 + e * 64;
+            if (i + 1 < validCols)
+                ok = ok && inIdx[i] < inIdx[i + 1];
         }
-        SortInRegisters<E>(k, key, tid);
-#pragma unroll
-        for (int e = 0; e < E; ++e) {
-            const int i = tid * E + e;
-            if (i < topk) {
-                const uint32_t low = (uint32_t)k[e];
-                rowScore[i] = __uint_as_float((low & 1u) ? 0x80000000u : ScoreBits((uint32_t)(k[e] >> 32)));
-                rowIndex[i] = inIdx[4095 - (int)(low >> 20)];
+        increasing = everyone(ok);
+    }
+    if (!increasing) {
+        uint64_t *key = reinterpret_cast<uint64_t *>(lds);
+        uint16_t *pos = reinterpret_cast<uint16_t *>(lds + (size_t)N * 8);
+        for (int r = row0; r < row0 + kRows && r < rows; ++r) {
+            const float *scores = src + (size_t)r * (size_t)ld;
+            __syncthreads();
+            for (int i = tid; i < N; i += kTopkThreads) {
+                uint64_t kv = 0;
+                if (i < validCols) {
+                    uint32_t b = __float_as_uint(scores[i]);
+                    if (b == kSign)
+                        b = 0; // -0 and +0 compare equal
+                    kv = ((uint64_t)ScoreOrder(b) << 32) | (uint32_t)~inIdx[i];
+                }
+                key[i] = kv;
+                pos[i] = (uint16_t)i;
+            }
+            __syncthreads();
+            SortInLds<N>(key, pos, tid);
+            for (int i = tid; i < topk; i += kTopkThreads) {
+                const int p = pos[i];
+                outScore[(size_t)r * (size_t)topk + i] = scores[p];
+                outIndex[(size_t)r * (size_t)topk + i] = inIdx[p];
             }
         }
         return;
     }
-    for (int i = tid; i < N; i += kTopkThreads) {
-        uint64_t kv = 0;
-        if (i < validCols) {
-            uint32_t b = __float_as_uint(row[i]);
-            if (b == 0x80000000u)
-                b = 0; // -0 and +0 compare equal
-            kv = ((uint64_t)ScoreOrder(b) << 32) | (uint32_t)~inIdx[i];
-        }
-        key[i] = kv;
-        pos[i] = (uint16_t)i;
+
+    RowSort<E, W> s;
+    s.q = (uint32_t)waveOfRow * 64u + LaneRank((uint32_t)lane);
+    s.xchg = reinterpret_cast<uint64_t *>(lds);
+    const uint32_t columnBits = (4095u - i0) << 8;
+    // the ranks of a wave go in order through its piece of LDS, so that its stores cover consecutive addresses
+    uint32_t *staged = reinterpret_cast<uint32_t *>(lds) + wave * (kStaged * kStages), *stagedColumn = staged + (kStages - 1) * kStaged;
+    const int firstRank = waveOfRow * 64 * E, laneRank = (int)LaneRank((uint32_t)lane) * E, count = topk - firstRank;
+    auto ordered = [] { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); __builtin_amdgcn_wave_barrier(); };
+    s.form = 0;
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+        const bool negZero = bits[e] == kSign; // compares equal to +0: same key, remembered below the column bits
+        const uint32_t order = ScoreOrder(negZero ? 0u : bits[e]);
+        s.k[e] = Key(__builtin_amdgcn_alignbit(0x3ffu, order, 12), (order << 20) | (columnBits - (uint32_t)(e * 64 << 8) + (negZero ? 1u : 0u)));
     }
-    __syncthreads();
-    SortInLds<N>(key, pos, tid);
-    for (int i = tid; i < topk; i += kTopkThreads) {
-        const int p = pos[i];
-        rowScore[i] = row[p];
-        rowIndex[i] = inIdx[p];
+    if (validCols != N) {
+#pragma unroll
+        for (int e = 0; e < E; ++e)
+            if (i0 + e * 64 >= (uint32_t)validCols)
+                s.k[e] = 1.0;
+    }
+    s.Sort(keepBits);
+
+    if (W > 1)
+        __syncthreads(); // (the exchanges are over)
+    if (row0 + wave / W >= rows || count <= 0)
+        return;
+    float *toScore = outScore + (size_t)row * (size_t)topk + firstRank;
+    uint32_t *toIndex = outIndex + (size_t)row * (size_t)topk + firstRank;
+    uint32_t column[E];
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+        const uint32_t low = Low(s.k[e]), order = (High(s.k[e]) << 12) | (low >> 20);
+        column[e] = 4095u - ((low >> 8) & 0xfffu);
+        staged[laneRank + e + (laneRank + e) / 16] = (low & 1u) ? kSign : ScoreBits(order);
+        if (kStages == 2)
+            stagedColumn[laneRank + e + (laneRank + e) / 16] = column[e];
+    }
+    ordered();
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+        const int i = e * 64 + lane;
+        if (i < count)
+            toScore[i] = __uint_as_float(staged[i + i / 16]);
+    }
+    if (kStages == 1) {
+        ordered();
+#pragma unroll
+        for (int e = 0; e < E; ++e)
+            stagedColumn[laneRank + e + (laneRank + e) / 16] = column[e];
+        ordered();
+    }
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+        const int i = e * 64 + lane;
+        if (i < count) {
+            const uint32_t c = stagedColumn[i + i / 16];
+            toIndex[i] = consecutive ? first + c : inIdx[c];
+        }
     }
 }
 
@@ -251,16 +434,46 @@ extern "C" int pto_topk_f32(void *stream, float *out_score, uint32_t *out_index,
     if (ld < valid_cols || topk > valid_cols || valid_cols > 4096)
         return PTO_ERR_UNSUPPORTED;
     hipStream_t st = static_cast<hipStream_t>(stream);
-#define PTO_TOPK_CASE(EE)                                                                                              \
-    if (valid_cols <= kTopkThreads * EE) {                                                                             \
-        TopkRows<EE><<<dim3(rows), dim3(kTopkThreads), 0, st>>>(out_score, out_index, src, in_idx, valid_cols, ld, topk); \
-        return pto_amd::check_launch();                                                                                \
+    // Waves per row.  One wave per row does the least work (1024 columns, top 1000: 4800 rows 29.8 us, with two 32.4, with four
+    // 33.5), more waves per row put more of the chip to work on few rows (1200 rows 14.7 / 12.9 / 12.3 us, 145 rows 12.4 / 9.0 /
+    // 7.0): as many as keep all of them within five on a SIMD, the four of a compute unit's workgroup at most, and none
+    // for rows of up to 256, whose exchanges across waves cost more than they save (1000 rows 4.8 / 5.1 / 6.6).
+    const int most = 5 * 4 * 256 / rows;
+#define PTO_TOPK_CASE(E, W)                                                                                              \
+    {                                                                                                                    \
+        int keepBits = 0;                                                                                                \
+        while ((E << keepBits) < topk)                                                                                   \
+            ++keepBits;                                                                                                  \
+        constexpr int kRows = kTopkWaves / W;                                                                            \
+        TopkRows<E, W><<<dim3((unsigned)(((long long)rows + kRows - 1) / kRows)), dim3(kTopkThreads), 0, st>>>(          \
+            out_score, out_index, src, in_idx, rows, valid_cols, ld, topk, keepBits);                                    \
+        return pto_amd::check_launch();                                                                                  \
     }
-    PTO_TOPK_CASE(1)
-    PTO_TOPK_CASE(2)
-    PTO_TOPK_CASE(4)
-    PTO_TOPK_CASE(8)
-    PTO_TOPK_CASE(16)
+    if (valid_cols <= 64)
+        PTO_TOPK_CASE(1, 1)
+    if (valid_cols <= 128)
+        PTO_TOPK_CASE(2, 1)
+    if (valid_cols <= 256)
+        PTO_TOPK_CASE(4, 1)
+    if (valid_cols <= 512) {
+        if (most >= 4)
+            PTO_TOPK_CASE(2, 4)
+        if (most >= 2)
+            PTO_TOPK_CASE(4, 2)
+        PTO_TOPK_CASE(8, 1)
+    }
+    if (valid_cols <= 1024) {
+        if (most >= 4)
+            PTO_TOPK_CASE(4, 4)
+        if (most >= 2)
+            PTO_TOPK_CASE(8, 2)
+        PTO_TOPK_CASE(16, 1)
+    }
+    if (valid_cols <= 2048) {
+        if (most >= 4)
+            PTO_TOPK_CASE(8, 4)
+        PTO_TOPK_CASE(16, 2)
+    }
+    PTO_TOPK_CASE(16, 4)
 #undef PTO_TOPK_CASE
-    return PTO_ERR_UNSUPPORTED;
 }

@@ -59,6 +59,53 @@ def test_topk_ties_signed_zeros_infinities_and_arbitrary_indices(oracle):
             assert same(topk_gpu(s2, mono, c, c), oracle.topk_f32(s2, mono, c, c))
 
 
+@pytest.mark.parametrize("cols", [1, 63, 64, 65, 128, 129, 250, 256, 257, 512, 513, 1000, 1024, 1025, 2048, 2049, 4095, 4096])
+def test_topk_row_lengths_and_kept_lengths(oracle, cols):
+    """Every number of keys per lane and waves per row at its smallest and largest rows, topk on both sides of every length that
+    the merges stop at (keys per lane times powers of two), row counts that do not fill the last workgroup, many ties and
+    signed zeros; consecutive indices, increasing ones, ones that start near 2^32, and any (the pass through LDS)."""
+    r = np.random.Generator(np.random.Philox(key=cols))
+    keys = next(e for e in (2, 4, 8, 16) if cols <= 64 * e or e == 16)
+    kept = sorted({k for b in range(9) for k in ((keys << b) - 1, keys << b, (keys << b) + 1) if 1 <= k <= cols} | {1, cols})
+    for n, k in enumerate(kept):
+        rows = 1 + n % 6
+        src, idx = datagen.topk_inputs(rows, cols, cols + 8 * (n % 2), distinct=0 if n % 3 else 11)
+        src[0, ::7] = -0.0
+        assert same(topk_gpu(src, idx, cols, k), oracle.topk_f32(src, idx, cols, k)), (k, "consecutive")
+        which = (idx * np.uint32(5) + np.uint32(3), np.uint32(0xFFFFFFFF) - idx[::-1], r.permutation(1 << 16)[:cols].astype(np.uint32))[n % 3]
+        assert same(topk_gpu(src, which, cols, k), oracle.topk_f32(src, which, cols, k)), (k, n % 3)
+
+
+@pytest.mark.parametrize("cols,k", [(500, 500), (500, 9), (1024, 1000), (1024, 70), (1900, 1900), (1900, 200)])
+@pytest.mark.parametrize("rows", [1280, 1281, 2560, 2563])
+def test_topk_waves_per_row(oracle, rows, cols, k):
+    """Both sides of the row counts where the number of waves per row changes, consecutive and other increasing indices."""
+    src, idx = datagen.topk_inputs(rows, cols, cols + 1, distinct=300)
+    for ids in (idx, idx * np.uint32(3)):
+        assert same(topk_gpu(src, ids, cols, k), oracle.topk_f32(src, ids, cols, k))
+
+
+def test_topk_every_kind_of_score():
+    """Infinities, denormals, NaNs of either sign and random bit patterns: ordered by bit pattern as the interface states
+    (the float comparison of the oracle puts NaNs nowhere), equal ones by column, and their bits are kept."""
+    r = np.random.Generator(np.random.Philox(key=5))
+    for cols in (100, 1024, 3000):
+        bits = r.integers(0, 2**32, size=(5, cols), dtype=np.uint64).astype(np.uint32)
+        bits[1, ::3] = 0x7F800000
+        bits[2, ::5] = 0x00000123
+        bits[3, ::4] = 0xFFFFFFFF
+        bits[3, 1::4] = 0x7FFFFFFF
+        bits[4, ::2] = 0x80000000
+        plain = np.where(bits == 0x80000000, 0, bits)
+        order = np.where(plain & 0x80000000, ~plain, plain | 0x80000000).astype(np.int64)
+        idx = np.arange(cols, dtype=np.uint32)
+        want = np.argsort(-order, axis=1, kind="stable")
+        for k in (cols, 17):
+            got = topk_gpu(bits.view(np.float32), idx, cols, k)
+            assert np.array_equal(got[1], want[:, :k]), (cols, k)
+            assert np.array_equal(got[0].view(np.uint32), np.take_along_axis(bits, want[:, :k], axis=1)), (cols, k)
+
+
 def test_topk_reference_config_4800x1024_top1000(oracle):
     """The reference kernel's case: 4800 rows of 1024 valid columns (row stride 1280), top 1000, its generator's data."""
     rows, cols, ld, k = 4800, 1024, 1280, 1000
