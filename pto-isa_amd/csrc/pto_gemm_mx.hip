@@ -24,7 +24,6 @@
 #define PTO_WAVES_N 4
 #include "gemm_kernels.hpp"
 
-#include <algorithm>
 
 PTO_DEVICE_CODE_BEGIN
 
@@ -348,26 +347,74 @@ int gemm_mx_dispatch(hipStream_t st, void *c, const uint8_t *a, const uint8_t *b
 } // namespace
 
 namespace {
-// Two kernels: 256 x 256 tiles on eight wavefronts (this file; quarter tiles in a last partial round) and 256 x 192 /
-// 256 x 128 tiles on four wavefronts (pto_gemm_mxw4.hip: the faster engine, the smaller tile).  Estimated times in
-// microseconds, rounds over the compute units x (K-steps of 128 bytes x step time + fixed time) as measured in one run at
-// 4096^3, 6144^3 and 8192^3 (eight against four wavefronts).  fp8: 6144^3 2240 against 2590 TFLOP/s, 8192^3 2460 against
-// 2545, 4096^3 2150 against 2165.  fp4: 6144^3 3600 against 4020, 8192^3 4030 against 4090, m, k, n = 2040, 8192, 8100
-// (one round of 256 x 256) 3680 against 3910.
-bool mx_four_wave_is_faster(int m, int n, int k, int k_bytes, bool fp4)
+// Three kernels: 256 x 256 tiles on eight wavefronts (this file; quarter tiles in a last partial round), 256 x 192 and 256 x 128
+// tiles on four (pto_gemm_mxw4.hip), and tiles of 64 .. 192 rows with k split over two groups of wavefronts
+// (pto_gemm_mxks.hip).  What a problem takes with one tile shape, in microseconds, launch included: tiles are dealt to the
+// compute units, `more` rounds beyond the first, `share` of the units busy in the last one, steps of 128 bytes,
+//   time = fixed + per_round more + steps (step + step_round more + step_share share) + per_mega (4e-6 m n)
+// Least-squares fits to 240 problems between 256 x 256 x 512 and 6144 x 6144 x 6144, three operand sets in turn, bf16 result
+// (root mean square of the relative error 3 .. 5 %).  The k-split shapes are taken 3 % dearer and the 256 x 256 tiles of fp8
+// 8 % than fitted (against moves on the noise of the fit); so chosen, a problem is 0.3 % (fp8) and 0.4 % (fp4) from its best
+// shape on average, 7 % at worst.  Against the 256-row tiles alone: 256 x 256 x 6144 fp8 34.1 -> 11.0 us, 512 x 512 x 2048 fp4
+// 12.0 -> 4.9, 592 x 736 x 4096 24.7 -> 9.9, 2048^3 17.3 -> 13.3, geometric mean of the 240 problems 1.50 (fp8), 1.67 (fp4).
+struct MxShape {
+    enum Kernel { kBlock, kW4, kKs } kernel;
+    int number, bm, bn;
+    double fixed, perRound, step, stepRound, perMega, stepShare;
+};
+constexpr MxShape kMxShapes[2][9] = {
+    {{MxShape::kBlock, 0, 256, 256, 5.15, 3.00, 1.132, 1.742, 0.112, 0.421},
+     {MxShape::kW4, 0, 256, 192, 8.10, 4.31, 0.680, 1.102, 0.060, 0.259},
+     {MxShape::kW4, 0, 256, 128, 5.89, 3.38, 0.551, 0.784, 0.071, 0.135},
+     {MxShape::kKs, 0, 64, 64, 2.93, 0.75, 0.179, 0.201, 0.125, 0.057},
+     {MxShape::kKs, 1, 64, 128, 3.70, 2.38, 0.235, 0.319, 0.097, 0.142},
+     {MxShape::kKs, 2, 128, 64, 3.61, 2.01, 0.266, 0.312, 0.150, 0.061},
+     {MxShape::kKs, 3, 128, 128, 4.67, 2.62, 0.355, 0.489, 0.159, 0.093},
+     {MxShape::kKs, 4, 128, 192, 5.85, 3.75, 0.496, 0.718, 0.117, 0.159},
+     {MxShape::kKs, 5, 192, 128, 5.90, 3.39, 0.506, 0.716, 0.127, 0.124}}, // fp8
+    {{MxShape::kBlock, 0, 256, 256, 5.15, 12.01, 1.157, 1.296, 0.081, 0.754},
+     {MxShape::kW4, 0, 256, 192, 7.67, 6.75, 0.912, 1.065, 0.073, 0.227},
+     {MxShape::kW4, 0, 256, 128, 5.97, 5.46, 0.657, 0.800, 0.058, 0.246},
+     {MxShape::kKs, 0, 64, 64, 2.93, 0.44, 0.233, 0.216, 0.244, 0.000},
+     {MxShape::kKs, 1, 64, 128, 3.68, 2.13, 0.304, 0.354, 0.157, 0.081},
+     {MxShape::kKs, 2, 128, 64, 3.75, 2.28, 0.307, 0.339, 0.159, 0.057},
+     {MxShape::kKs, 3, 128, 128, 4.88, 3.16, 0.405, 0.545, 0.135, 0.133},
+     {MxShape::kKs, 4, 128, 192, 5.78, 3.34, 0.569, 0.843, 0.140, 0.092},
+     {MxShape::kKs, 5, 192, 128, 5.83, 3.42, 0.568, 0.856, 0.137, 0.103}}, // fp4
+};
+constexpr double kMxStepQuarter[2] = {0.34, 0.25}; // a step of the round of 128 x 128 quarter tiles
+
+int gemm_mx_any(hipStream_t st, void *c, const uint8_t *a, const uint8_t *b, const uint8_t *sa, const uint8_t *sb, int m, int n, int k,
+                int format, int c_fp32)
 {
-    if (m < 256 || n < 128 || n % 4 != 0 || k % (fp4 ? 1024 : 512) != 0)
-        return false;
-    const int cus = compute_units(), steps = k_bytes / 128;
-    const double t4 = std::min(pto_amd::mx_w4_time(m, n, k_bytes, 192, fp4), pto_amd::mx_w4_time(m, n, k_bytes, 128, fp4));
-    double t8 = 1e30;
-    if (n >= 256) {
-        const double step = fp4 ? 1.63 : 1.5, quarter = fp4 ? 0.25 : 0.34;
-        const long long tiles = (long long)((m + 255) / 256) * ((n + 255) / 256), full = tiles / cus, rest = tiles - full * cus;
-        const bool quarters = rest > 0 && full > 0 && rest * 4 <= cus && m % 256 == 0 && n % 256 == 0;
-        t8 = (double)full * (steps * step + 16.0) + (rest == 0 ? 0.0 : (quarters ? steps * quarter + 16.0 : steps * step + 16.0));
+    const bool fp4 = format == 4;
+    const bool block = m >= 256 && n >= 256 && k % 512 == 0, w4 = m >= 256 && n >= 128 && n % 4 == 0 && k % (fp4 ? 1024 : 512) == 0;
+    if (!block && !w4)
+        return PTO_ERR_UNSUPPORTED;
+    const int cus = compute_units(), steps = k / (fp4 ? 256 : 128);
+    const MxShape *best = nullptr;
+    double bestTime = 0.0;
+    for (const MxShape &s : kMxShapes[fp4]) {
+        if ((s.kernel == MxShape::kBlock && !block) || (s.kernel == MxShape::kW4 && (!w4 || n < s.bn)) || (s.kernel == MxShape::kKs && n % 4))
+            continue;
+        const long long tiles = (long long)((m + s.bm - 1) / s.bm) * ((n + s.bn - 1) / s.bn), rest = tiles % cus;
+        double more = (double)((tiles - 1) / cus), share = (double)((tiles - 1) % cus + 1) / cus, quarter = 0.0;
+        if (s.kernel == MxShape::kBlock && rest > 0 && rest * 4 <= cus && tiles > cus && m % 256 == 0 && n % 256 == 0) {
+            more -= 1.0;
+            share = 1.0;
+            quarter = steps * kMxStepQuarter[fp4] + 4.0;
+        }
+        const double time = s.fixed + s.perRound * more + steps * (s.step + s.stepRound * more + s.stepShare * share) + s.perMega * (4e-6 * m * n) + quarter;
+        if (best == nullptr || time < bestTime) {
+            best = &s;
+            bestTime = time;
+        }
     }
-    return t4 < t8;
+    switch (best->kernel) {
+    case MxShape::kW4: return pto_amd::gemm_mx_w4(st, c, a, b, sa, sb, m, n, k, format, c_fp32, best->bn);
+    case MxShape::kKs: return pto_amd::gemm_mx_ks(st, c, a, b, sa, sb, m, n, k, format, c_fp32, best->number);
+    default: return gemm_mx_dispatch(st, c, a, b, sa, sb, m, n, k, format, c_fp32, 1);
+    }
 }
 } // namespace
 
@@ -378,9 +425,7 @@ extern "C" int pto_gemm_mxfp8(void *stream, void *c, const uint8_t *a, const uin
         return PTO_ERR_BAD_ARG;
     if (format < 0 || format > 3)
         return PTO_ERR_UNSUPPORTED;
-    if (mx_four_wave_is_faster(m, n, k, k, false))
-        return pto_amd::gemm_mx_w4(static_cast<hipStream_t>(stream), c, a, b, scale_a, scale_b, m, n, k, format, c_fp32, 0);
-    return gemm_mx_dispatch(static_cast<hipStream_t>(stream), c, a, b, scale_a, scale_b, m, n, k, format, c_fp32, 1);
+    return gemm_mx_any(static_cast<hipStream_t>(stream), c, a, b, scale_a, scale_b, m, n, k, format, c_fp32);
 }
 
 extern "C" int pto_gemm_mxfp4(void *stream, void *c, const uint8_t *a, const uint8_t *b, const uint8_t *scale_a,
@@ -388,9 +433,7 @@ extern "C" int pto_gemm_mxfp4(void *stream, void *c, const uint8_t *a, const uin
 {
     if (!c || !a || !b || !scale_a || !scale_b || m <= 0 || n <= 0 || k <= 0)
         return PTO_ERR_BAD_ARG;
-    if (mx_four_wave_is_faster(m, n, k, k / 2, true))
-        return pto_amd::gemm_mx_w4(static_cast<hipStream_t>(stream), c, a, b, scale_a, scale_b, m, n, k, 4, c_fp32, 0);
-    return gemm_mx_dispatch(static_cast<hipStream_t>(stream), c, a, b, scale_a, scale_b, m, n, k, 4, c_fp32, 1);
+    return gemm_mx_any(static_cast<hipStream_t>(stream), c, a, b, scale_a, scale_b, m, n, k, 4, c_fp32);
 }
 
 #if defined(PTO_ST_HOOKS)
@@ -399,11 +442,14 @@ extern "C" int pto_gemm_mxfp4(void *stream, void *c, const uint8_t *a, const uin
 extern "C" int pto_gemm_mxfp8_variant(void *stream, void *c, const uint8_t *a, const uint8_t *b, const uint8_t *scale_a,
                                       const uint8_t *scale_b, int m, int n, int k, int format, int c_fp32, int variant)
 {
-    if (!c || !a || !b || !scale_a || !scale_b || m <= 0 || n <= 0 || k <= 0 || variant < 0 || variant > 6)
+    if (!c || !a || !b || !scale_a || !scale_b || m <= 0 || n <= 0 || k <= 0 || variant < 0 || variant > 12)
         return PTO_ERR_BAD_ARG;
-    if (variant >= 4) // the four-wave engine: 4 = width by rounds, 5 = 256 x 192 tiles, 6 = 256 x 128
-        return pto_amd::gemm_mx_w4(static_cast<hipStream_t>(stream), c, a, b, scale_a, scale_b, m, n, k, format, c_fp32,
-                                      variant == 4 ? 0 : (variant == 5 ? 192 : 128));
+    if (variant >= 7) // k split over two groups of wavefronts, shape by number
+        return pto_amd::gemm_mx_ks(static_cast<hipStream_t>(stream), c, a, b, scale_a, scale_b, m, n, k, format, c_fp32, variant - 7);
+    if (variant >= 5) // the four-wave engine: 5 = 256 x 192 tiles, 6 = 256 x 128
+        return pto_amd::gemm_mx_w4(static_cast<hipStream_t>(stream), c, a, b, scale_a, scale_b, m, n, k, format, c_fp32, variant == 5 ? 192 : 128);
+    if (variant == 4) // what the public entry points take
+        return gemm_mx_any(static_cast<hipStream_t>(stream), c, a, b, scale_a, scale_b, m, n, k, format, c_fp32);
     return gemm_mx_dispatch(static_cast<hipStream_t>(stream), c, a, b, scale_a, scale_b, m, n, k, format, c_fp32, variant);
 }
 #endif // PTO_ST_HOOKS

@@ -328,3 +328,40 @@ def test_mx_gemm_rejects_bad_arguments():
     assert lib.pto_gemm_mxfp8(0, p, p, p, p, p, 256, 256, 512, 5, 1) == capi.ERR_UNSUPPORTED   # unknown format
     assert lib.pto_gemm_mxfp8(0, p, p, p, 0, p, 256, 256, 512, 0, 1) == capi.ERR_BAD_ARG
     assert lib.pto_gemm_mxfp8(0, p, p, p, p, p, 256, 0, 512, 0, 1) == capi.ERR_BAD_ARG
+
+
+@pytest.mark.parametrize("fmt", [0, 1, 2, 3, 4])
+@pytest.mark.parametrize("shape,bm,bn", [(0, 64, 64), (1, 64, 128), (2, 128, 64), (3, 128, 128), (4, 128, 192), (5, 192, 128)])
+def test_mx_gemm_k_split_tile_shapes_exact(oracle, shape, bm, bn, fmt):
+    """Every tile shape and format of the kernel that splits k over two groups of wavefronts: integer operands under the scales
+    2^0 .. 2^2, every element exactly; less than a tile, one tile, edges one row / four columns past a tile, several tiles; the
+    shortest K, an odd number of 512s (half a period of scales at the end) and several periods; the bf16 result = RNE."""
+    fmt_a, fmt_b = {2: (0, 1), 3: (1, 0)}.get(fmt, (fmt, fmt))
+    for m, n, k in ((1, 4, 512), (bm, bn, 1024), (bm + 1, bn + 4, 1536), (bm - 1, 2 * bn - 4, 2560), (3 * bm + 5, 3 * bn + 12, 4096)):
+        a, _, sa, sb = datagen.mx_inputs(m, n, k, fmt_a, dist="integer")
+        _, b, _, _ = datagen.mx_inputs(m, n, k, fmt_b, dist="integer")
+        rc, got = _mx_variant(a, b, sa, sb, fmt, 7 + shape)
+        capi.check(rc, "k-split MX kernel")
+        assert np.array_equal(got, oracle.mx_gemm(a, b, sa, sb, fmt_a, fmt_b)), (m, n, k)
+        rc, got16 = _mx_variant(a, b, sa, sb, fmt, 7 + shape, c_fp32=False)
+        assert rc == 0 and np.array_equal(got16, bf16_rne(got)), (m, n, k)
+
+
+@pytest.mark.parametrize("fmt", [0, 1, 4])
+def test_mx_gemm_k_split_scale_of_every_block(oracle, fmt):
+    """Operands of ones, scales drawn per block: C[i, j] = 32 sum_b 2^(sa[i, b] + sb[j, b] - 254) exactly (multiples of 2^-3
+    below 2^18); every finite encoding with a wide range of scales to the GEMM tolerance."""
+    m, n, k = 260, 388, 4608
+    one = np.full((m, k), datagen.fp8_encode(np.ones(1), fmt)[0], dtype=np.uint8), np.full((n, k), datagen.fp8_encode(np.ones(1), fmt)[0], dtype=np.uint8)
+    a, b = (datagen.fp4_pack(x) for x in one) if fmt == 4 else one
+    rng = np.random.default_rng(79)
+    sa = rng.integers(125, 131, size=(m, k // 32)).astype(np.uint8)
+    sb = rng.integers(125, 131, size=(n, k // 32)).astype(np.uint8)
+    want = 32.0 * (np.exp2(sa.astype(np.float64) - 127) @ np.exp2(sb.astype(np.float64) - 127).T)
+    ra, rb, rsa, rsb = datagen.mx_inputs(m, n, k, fmt, dist="bytes", scale_lo=110, scale_hi=140)
+    rwant = oracle.mx_gemm(ra, rb, rsa, rsb, fmt)
+    for shape in range(6):
+        rc, got = _mx_variant(a, b, sa, sb, fmt, 7 + shape)
+        assert rc == 0 and np.array_equal(got.astype(np.float64), want), shape
+        rc, got = _mx_variant(ra, rb, rsa, rsb, fmt, 7 + shape)
+        assert rc == 0 and np.all(np.isfinite(got)) and rel_err(got, rwant) <= TOL, shape
