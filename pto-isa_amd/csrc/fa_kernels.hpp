@@ -138,14 +138,23 @@ struct VTReader {
     }
 };
 
-template <int D, bool CAUSAL, bool OUT_F32, int MIN_BLOCKS, int kBKV = kBKVDefault, bool PP = false, int NQ_ = 1>
+// G > 1: the keys of a query block are split over G groups of the workgroup's waves, for launches with too few query blocks
+// to fill the chip (a workgroup then owns kBQ1 / G queries).  Wave w works on query block w % (waves / G) in group
+// w / (waves / G); in round r group g takes key tile G r + g, out of a double buffer of its own that all waves fill
+// together, so the barriers of a round are those of the unsplit kernel.  At the end every wave hands its (max, sum) and
+// the accumulator quads that other groups store over the LDS; group g adds up and stores its own 1 / G of the head
+// dimension.  O = sum_g w_g O_g / sum_g w_g S_g, w_g = exp(s (M_g - M)), M = max_g M_g, all in fp32.
+template <int D, bool CAUSAL, bool OUT_F32, int MIN_BLOCKS, int kBKV = kBKVDefault, bool PP = false, int NQ_ = 1, int G = 1>
 __global__ __launch_bounds__(kBlockThreads, MIN_BLOCKS) AICORE void FlashAttnFwd(__gm__ void *outO, __gm__ float *outLse,
                                                                       __gm__ const half *qAll, __gm__ const half *kAll,
                                                                       __gm__ const half *vAll, int heads, int seqQ,
                                                                       int seqKv, int numBH, int causalOff)
 {
     constexpr int NQ = NQ_;        // 32-query blocks per wave
-    constexpr int kBQ = kBQ1 * NQ; // queries per workgroup
+    constexpr int kBQ = kBQ1 * NQ; // columns of the tile types: 32 NQ per wave
+    constexpr int kBQOwn = kBQ / G; // queries per workgroup
+    constexpr int kQWaves = PTO_WAVES_N / G; // waves of a group
+    static_assert(G == 1 || (NQ == 1 && !PP && PTO_WAVES_N % G == 0), "key groups: one query block per wave");
     constexpr int KB = kBKV / 32;  // 32-key blocks per tile
     constexpr int DB = D / 32;    // 32-wide blocks of the head dimension
     // ---- tiles ----
@@ -164,12 +173,13 @@ __global__ __launch_bounds__(kBlockThreads, MIN_BLOCKS) AICORE void FlashAttnFwd
 
     constexpr uint32_t kTileBytes = kBKV * D * sizeof(half);
     constexpr uint32_t kStageBytes = 2 * kTileBytes;
-    static_assert(D * kBQ * sizeof(half) <= 2 * kStageBytes, "Q^T is staged in the K/V stages");
+    constexpr uint32_t kGroupBytes = 2 * kStageBytes; // the double buffer of one key group
+    static_assert(G > 1 || D * kBQ * sizeof(half) <= 2 * kStageBytes, "Q^T is staged in the K/V stages");
 
     // ---- which (batch*head, query tile) this workgroup owns.  Workgroups are dealt round-robin to
     // the 8 XCDs: keep a head on one XCD so that its K/V stay in that XCD's L2.  Causal: the query
     // tiles with the most keys go first.
-    const int numQT = seqQ / kBQ;
+    const int numQT = seqQ / kBQOwn;
     int bh, qt;
     {
         const int bid = (int)get_block_idx();
@@ -184,7 +194,7 @@ __global__ __launch_bounds__(kBlockThreads, MIN_BLOCKS) AICORE void FlashAttnFwd
         if (CAUSAL)
             qt = numQT - 1 - qt;
     }
-    const int q0 = qt * kBQ;
+    const int q0 = qt * kBQOwn;
     __gm__ half *qBase = const_cast<half *>(qAll) + ((int64_t)bh * seqQ + q0) * D;
     // (the same in every lane: kept in scalar registers, so that the tile addresses of the copies are scalar arithmetic)
     __gm__ half *kBase = reinterpret_cast<half *>(const_cast<char *>(
@@ -194,7 +204,7 @@ __global__ __launch_bounds__(kBlockThreads, MIN_BLOCKS) AICORE void FlashAttnFwd
 
     int numTiles = seqKv / kBKV;
     if (CAUSAL) { // tiles wholly above the diagonal are skipped (fa_performance_kernel.cpp:757-758)
-        const int lastKey = q0 + kBQ - 1 + causalOff;
+        const int lastKey = q0 + kBQOwn - 1 + causalOff;
         const int lim = lastKey / kBKV + 1;
         numTiles = lim < numTiles ? lim : numTiles;
     }
@@ -213,7 +223,8 @@ __global__ __launch_bounds__(kBlockThreads, MIN_BLOCKS) AICORE void FlashAttnFwd
     float runMax[NQ], runSum[NQ]; // per lane and query block; runSum is the half-wave partial
     const int lane = hw::lane();
     // row of Q that this lane's column of query block 0 holds (block nb: + 32 nb)
-    const int myQuery = q0 + hw::wave_n() * (32 * NQ) + (lane & 31);
+    const int group = G == 1 ? 0 : hw::wave_n() / kQWaves;
+    const int myQuery = q0 + (G == 1 ? hw::wave_n() : hw::wave_n() % kQWaves) * (32 * NQ) + (lane & 31);
     const uint32_t hHalf = (uint32_t)lane >> 5;
     // s = 1/sqrt(D) folded with log2(e): exp(s y) = exp2(s log2e y)
     const float sLog2e = (D == 128 ? 0.08838834764831845f : 0.125f) * 1.4426950408889634f;
@@ -222,6 +233,11 @@ __global__ __launch_bounds__(kBlockThreads, MIN_BLOCKS) AICORE void FlashAttnFwd
     // X^T = K Q^T for the key tile in LDS stage st: one MFMA per K fragment, fragments requested kAhead MFMAs ahead
     KReader<D> kr;
     kr.Init();
+    if constexpr (G > 1) {
+#pragma unroll
+        for (int ks = 0; ks < D / 16; ++ks)
+            kr.base[ks] += (uint32_t)group * kGroupBytes;
+    }
     // `between(i)` runs before the MFMA on fragment i (the caller issues its asynchronous copies there).
     // A scheduling barrier after every MFMA keeps the issue order exactly as written.
     // `extraTag`: number of LDS reads that between(kTotal - kAhead) issues itself (they are younger than every K read).
@@ -259,7 +275,7 @@ __global__ __launch_bounds__(kBlockThreads, MIN_BLOCKS) AICORE void FlashAttnFwd
     };
     // streaming softmax on the accumulator fragments of tile t (one query per lane and query block)
     auto softmaxTile = [&](AccS(&sAcc)[KB], int t, RightP &pRight, float(&alpha)[NQ], bool &anyRaise) {
-        const int key0 = t * kBKV;
+        const int key0 = (t * G + group) * kBKV; // t: key tile of this wave's group
         if (CAUSAL && key0 + kBKV - 1 > q0 + causalOff) { // the diagonal crosses this tile
 #pragma unroll
             for (int nb = 0; nb < NQ; ++nb) {
@@ -302,6 +318,8 @@ __global__ __launch_bounds__(kBlockThreads, MIN_BLOCKS) AICORE void FlashAttnFwd
                         for (int v = 0; v < 16; ++v)
                             locMax = fmaxf(locMax, sAcc[kb].st.f[0][nb][v]);
                     locMax = MaxOverHalves(locMax);
+                    if constexpr (G > 1) // a group may hold nothing but scores of -inf; also never a NaN, so that the
+                        locMax = fmaxf(locMax, kMaskValue); // maxima of the groups compare (the NaN is in the sums)
                     const bool raise = t == 0 || (locMax - runMax[nb]) * sLog2e > kSlack;
                     const float newMax = raise ? locMax : runMax[nb];
                     if (t > 0)
@@ -344,6 +362,13 @@ __global__ __launch_bounds__(kBlockThreads, MIN_BLOCKS) AICORE void FlashAttnFwd
     using VT = VTReader<D, kBKV>;
     VT vt;
     vt.template Init<TileMatV>();
+    if constexpr (G > 1) {
+#pragma unroll
+        for (int db = 0; db < DB; ++db)
+#pragma unroll
+            for (int u = 0; u < 2; ++u)
+                vt.base[db][u] += (uint32_t)group * kGroupBytes;
+    }
     // O^T += V^T P^T with the 16-key step as the outer loop: consecutive MFMAs go to different accumulator
     // blocks.  (An MFMA that needs the result of the one before it can only issue in the very cycle that one
     // ends; when another wave of the SIMD issues vector instructions meanwhile, every such issue slips and the
@@ -429,7 +454,32 @@ __global__ __launch_bounds__(kBlockThreads, MIN_BLOCKS) AICORE void FlashAttnFwd
 #pragma unroll
             for (int v = 0; v < 16; ++v)
                 oAcc[db].st.f[0][nb][v] = 0.0f;
-    {
+    // the waves fill stage st of every group with the tiles of round r (K and V apart: they are issued at different times)
+    auto loadGroups = [&](auto stTag, auto isVTag, __gm__ half *base, int r) {
+        StaticFor<0, G>([&](auto gTag) {
+            constexpr uint32_t off = decltype(gTag)::value * kGroupBytes + decltype(stTag)::value * kStageBytes;
+            GlobalKV gm = keyTile(base, r * G + decltype(gTag)::value);
+            if constexpr (decltype(isVTag)::value) {
+                TileMatV dst;
+                TASSIGN(dst, off + kTileBytes);
+                TLOAD(dst, gm);
+            } else {
+                TileMatK dst;
+                TASSIGN(dst, off);
+                TLOAD(dst, gm);
+            }
+        });
+    };
+    if constexpr (G > 1) {
+        // Q^T straight into the operand registers: 16 bytes of the lane's own query per step of 16
+        loadGroups(std::integral_constant<int, 0>(), std::false_type(), kBase, 0);
+        loadGroups(std::integral_constant<int, 0>(), std::true_type(), vBase, 0);
+        const half *qRow = qAll + ((int64_t)bh * seqQ + myQuery) * D + 8 * hHalf;
+#pragma unroll
+        for (int ks = 0; ks < D / 16; ++ks)
+            qRight.st.f[0][ks] = *reinterpret_cast<const f16x8 *>(qRow + 16 * ks);
+        set_flag(PIPE_MTE2, PIPE_MTE1, EVENT_ID0);
+    } else {
         GlobalQT gmQ(qBase);
         TLOAD(qMat, gmQ);
         set_flag(PIPE_MTE2, PIPE_MTE1, EVENT_ID0);
@@ -521,10 +571,13 @@ __global__ __launch_bounds__(kBlockThreads, MIN_BLOCKS) AICORE void FlashAttnFwd
         if (group == 0) // pairs with the barrier that ends the second group's last phase
             phaseEnd();
     } else {
+    const int rounds = (numTiles + G - 1) / G; // a wave whose group has no tile in the last round only takes part in its barrier
     // One key tile in LDS stage st (a compile-time constant: every LDS address is an immediate).
     auto tileStep = [&](auto stageTag, int t) {
         constexpr int st = decltype(stageTag)::value;
         wait_flag(PIPE_MTE2, PIPE_MTE1, EVENT_ID0); // tile t has landed; everyone left tile t-1
+        if (G > 1 && t * G + group >= numTiles)
+            return;
         // The next tile is fetched while this tile's score MFMAs issue: the K copies before the second
         // MFMA, the V copies halfway.  Past the last tile the copies re-fetch it into the free stage,
         // which keeps the loop free of special cases.
@@ -533,12 +586,10 @@ __global__ __launch_bounds__(kBlockThreads, MIN_BLOCKS) AICORE void FlashAttnFwd
         scoreTile(sAcc, stageTag, [&](auto i) {
             constexpr int I = decltype(i)::value;
             if constexpr (I == 1) {
-                GlobalKV gmK = keyTile(kBase, t + 1);
-                TLOAD(kMat[st ^ 1], gmK);
+                loadGroups(std::integral_constant<int, st ^ 1>(), std::false_type(), kBase, t + 1);
             }
             if constexpr (I == kScoreFrags / 2 + 1) {
-                GlobalKV gmV = keyTile(vBase, t + 1);
-                TLOAD(vMat[st ^ 1], gmV);
+                loadGroups(std::integral_constant<int, st ^ 1>(), std::true_type(), vBase, t + 1);
                 set_flag(PIPE_MTE2, PIPE_MTE1, EVENT_ID0);
             }
         }, std::integral_constant<int, 0>());
@@ -550,13 +601,89 @@ __global__ __launch_bounds__(kBlockThreads, MIN_BLOCKS) AICORE void FlashAttnFwd
         softmaxTile(sAcc, t, pRight, alpha, anyRaise);
         outputTileWide(stageTag, vFirst, pRight, alpha, anyRaise);
     };
-    for (int tile = 0; tile < numTiles; tile += 2) {
+    for (int tile = 0; tile < rounds; tile += 2) {
         tileStep(std::integral_constant<int, 0>(), tile);
-        if (tile + 1 < numTiles)
+        if (tile + 1 < rounds)
             tileStep(std::integral_constant<int, 1>(), tile + 1);
     }
     }
     hw::wait_vm0(); // the copy issued by the last tile must not outlive the workgroup's LDS
+    if constexpr (G > 1) {
+        // ---- join the key groups, O /= S, write O (and LSE) ----
+        constexpr int kQuads = DB * 4, kOwn = kQuads / G; // groups of four d that a lane holds; those that its wave stores
+        constexpr uint32_t kWaveBytes = kQuads * 64 * 16, kStats = PTO_WAVES_N * kWaveBytes; // sized in launch_fa
+        char *lds = hw::lds_base();
+        const int wave = hw::wave_n(), qWave = wave % kQWaves;
+        if (group >= numTiles) { // no tile at all
+            runMax[0] = kMaskValue;
+            runSum[0] = 0.0f;
+        }
+        const float ownSum = SumOverHalves(runSum[0]);
+        __syncthreads(); // all reads of the last tiles are over
+        if (hHalf == 0) {
+            float *stats = reinterpret_cast<float *>(lds + kStats) + (wave * 32 + lane) * 2;
+            stats[0] = runMax[0];
+            stats[1] = ownSum;
+        }
+        StaticFor<0, kQuads>([&](auto cTag) {
+            constexpr int c = decltype(cTag)::value;
+            if (c / kOwn != group) {
+                const auto &f = oAcc[c / 4].st.f[0][0];
+                f32x4 v = {f[c % 4 * 4], f[c % 4 * 4 + 1], f[c % 4 * 4 + 2], f[c % 4 * 4 + 3]};
+                *reinterpret_cast<f32x4 *>(lds + (uint32_t)wave * kWaveBytes + (c * 64 + lane) * 16) = v;
+            }
+        });
+        __syncthreads();
+        // A query that sees no key of a group has M_g = kMaskValue and whatever the masked scores gave in S_g and O_g:
+        // left out by selection, not by a weight of zero
+        float weight[G], sum[G], top = kMaskValue;
+        bool seen[G];
+#pragma unroll
+        for (int g = 0; g < G; ++g) {
+            const float *stats = reinterpret_cast<const float *>(lds + kStats) + ((g * kQWaves + qWave) * 32 + (lane & 31)) * 2;
+            seen[g] = g < numTiles && (!CAUSAL || g * kBKV <= myQuery + causalOff);
+            weight[g] = stats[0];
+            sum[g] = stats[1];
+            top = seen[g] ? fmaxf(top, weight[g]) : top;
+        }
+        float total = 0.0f;
+#pragma unroll
+        for (int g = 0; g < G; ++g) {
+            weight[g] = __builtin_amdgcn_exp2f((weight[g] - top) * sLog2e);
+            total += seen[g] ? weight[g] * sum[g] : 0.0f;
+        }
+        const float inv = 1.0f / total;
+        const int64_t row = (int64_t)bh * seqQ + myQuery;
+        StaticFor<0, kQuads>([&](auto cTag) {
+            constexpr int c = decltype(cTag)::value;
+            if (c / kOwn == group) {
+                float o4[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+                for (int g = 0; g < G; ++g) {
+                    const auto &f = oAcc[c / 4].st.f[0][0];
+                    f32x4 part = {f[c % 4 * 4], f[c % 4 * 4 + 1], f[c % 4 * 4 + 2], f[c % 4 * 4 + 3]};
+                    if (g != c / kOwn)
+                        part = *reinterpret_cast<const f32x4 *>(lds + (uint32_t)(g * kQWaves + qWave) * kWaveBytes + (c * 64 + lane) * 16);
+#pragma unroll
+                    for (int r = 0; r < 4; ++r)
+                        o4[r] += seen[g] ? weight[g] * part[r] : 0.0f;
+                }
+                const int d = c * 8 + (int)hHalf * 4;
+                if constexpr (OUT_F32) {
+                    f32x4 v = {o4[0] * inv, o4[1] * inv, o4[2] * inv, o4[3] * inv};
+                    *reinterpret_cast<f32x4 *>(static_cast<float *>(outO) + row * D + d) = v;
+                } else {
+                    f16x4 v = {(half)(o4[0] * inv), (half)(o4[1] * inv), (half)(o4[2] * inv), (half)(o4[3] * inv)};
+                    *reinterpret_cast<f16x4 *>(static_cast<half *>(outO) + row * D + d) = v;
+                }
+            }
+        });
+        if (outLse != nullptr && hHalf == 0 && group == 0) {
+            const float scale = D == 128 ? 0.08838834764831845f : 0.125f;
+            outLse[row] = top * scale + __builtin_logf(total);
+        }
+        return;
+    }
     // ---- finish: O /= S, write O (and LSE) ----
 #pragma unroll
     for (int nb = 0; nb < NQ; ++nb) {
@@ -592,16 +719,19 @@ __global__ __launch_bounds__(kBlockThreads, MIN_BLOCKS) AICORE void FlashAttnFwd
 PTO_DEVICE_CODE_END
 
 namespace {
-template <int D, bool CAUSAL, bool OUT_F32, int MIN_BLOCKS = 1, int kBKV = kBKVDefault, bool PP = false, int NQ = 1>
+template <int D, bool CAUSAL, bool OUT_F32, int MIN_BLOCKS = 1, int kBKV = kBKVDefault, bool PP = false, int NQ = 1, int G = 1>
 int launch_fa(hipStream_t st, void *o, float *lse, const half *q, const half *k, const half *v, int batch, int heads,
               int seqQ, int seqKv, int causalOff)
 {
-    constexpr int kBQ = kBQ1 * NQ;
+    constexpr int kBQ = kBQ1 * NQ / G;
     if (seqQ % kBQ || seqKv % kBKV)
         return PTO_ERR_UNSUPPORTED;
-    static_assert(D * kBQ <= 4 * kBKV * D, "Q^T must fit the K/V stages it is staged in");
-    constexpr int lds = 2 * 2 * kBKV * D * (int)sizeof(half);
-    auto kernel = FlashAttnFwd<D, CAUSAL, OUT_F32, MIN_BLOCKS, kBKV, PP, NQ>;
+    static_assert(G > 1 || D * kBQ <= 4 * kBKV * D, "Q^T must fit the K/V stages it is staged in");
+    // the K / V stages of every key group; what the groups hand over at the end (accumulators, then maxima and sums)
+    constexpr int stages = G * 2 * 2 * kBKV * D * (int)sizeof(half), joined = PTO_WAVES_N * 32 * (D + 2) * (int)sizeof(float);
+    constexpr int lds = G > 1 && joined > stages ? joined : stages;
+    static_assert(lds <= 160 * 1024, "stages fit the LDS");
+    auto kernel = FlashAttnFwd<D, CAUSAL, OUT_F32, MIN_BLOCKS, kBKV, PP, NQ, G>;
     static const int attr = pto_amd::allow_lds(kernel, lds);
     if (attr != PTO_OK)
         return attr;

@@ -25,6 +25,19 @@
 
 #include "fa_kernels.hpp"
 
+namespace {
+// head_dim 64, the keys split over two groups of two waves: 64 queries per workgroup, two workgroups per compute unit
+int launch_split_w4(hipStream_t st, void *o, float *lse, const half *q, const half *k, const half *v, int batch, int heads, int seqQ, int seqKv,
+                    bool causal, bool oFp32, int causalOff)
+{
+    if (causal)
+        return oFp32 ? launch_fa<64, true, true, 2, 64, false, 1, 2>(st, o, lse, q, k, v, batch, heads, seqQ, seqKv, causalOff)
+                     : launch_fa<64, true, false, 2, 64, false, 1, 2>(st, o, lse, q, k, v, batch, heads, seqQ, seqKv, causalOff);
+    return oFp32 ? launch_fa<64, false, true, 2, 64, false, 1, 2>(st, o, lse, q, k, v, batch, heads, seqQ, seqKv, causalOff)
+                 : launch_fa<64, false, false, 2, 64, false, 1, 2>(st, o, lse, q, k, v, batch, heads, seqQ, seqKv, causalOff);
+}
+} // namespace
+
 #if defined(PTO_ST_HOOKS)
 // Tuning hook (not part of the public header).
 extern "C" int pto_fa_fwd_f16_variant(void *stream, void *o, float *lse, const uint16_t *q, const uint16_t *k,
@@ -55,6 +68,10 @@ extern "C" int pto_fa_fwd_f16_variant(void *stream, void *o, float *lse, const u
         return pto_amd::fa_fwd_d128_w8m16(st, o, lse, hq, hk, hv, batch, heads, seq_q, seq_kv, causal != 0, false, causalOff);
     if (variant == 21 && head_dim == 128) // fp32 output and LSE
         return pto_amd::fa_fwd_d128_w8m16(st, o, lse, hq, hk, hv, batch, heads, seq_q, seq_kv, causal != 0, true, causalOff);
+    if (variant == 42 || variant == 44) // keys over two or four groups of waves
+        return pto_amd::fa_fwd_split(st, o, lse, hq, hk, hv, batch, heads, seq_q, seq_kv, head_dim, causal != 0, false, causalOff, variant - 40);
+    if (variant == 32 && head_dim == 64) // over two groups of two waves
+        return launch_split_w4(st, o, lse, hq, hk, hv, batch, heads, seq_q, seq_kv, causal != 0, false, causalOff);
     if (variant == 6 && head_dim == 128 && !causal)
         return launch_fa<128, false, false, 2, 32>(st, o, lse, hq, hk, hv, batch, heads, seq_q, seq_kv, causalOff);
     if (variant == 6 && head_dim == 64 && causal)
@@ -85,16 +102,38 @@ extern "C" int pto_fa_fwd_f16(void *stream, void *o, float *lse, const uint16_t 
     hipStream_t st = static_cast<hipStream_t>(stream);
     const half *hq = reinterpret_cast<const half *>(q), *hk = reinterpret_cast<const half *>(k),
                *hv = reinterpret_cast<const half *>(v);
+    static const int cus = [] {
+        int dev = 0, n = 0;
+        if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0)
+            n = 256;
+        return n;
+    }();
+    // At most one 128-query workgroup of four waves per compute unit: every SIMD has one wave or none, and the launch takes as
+    // long as that wave needs for all keys of its queries.  The keys are split over groups of waves (FlashAttnFwd, G > 1) where
+    // there are enough of them to pay for joining the groups.  With 64-query workgroups one per compute unit (us, 128 of 128
+    // queries, no mask; four waves / two groups of four / four groups of two):
+    //   head_dim 128, keys  128:  6.6 /  8.4 /  7.4   256:  8.8 / 10.0 /  8.7   1024: 21.5 / 19.2 / 15.2   4096: 71.1 / 54.2 / 44.1
+    //   head_dim  64, keys  128:  4.7 /  5.7 /  5.5   512:  8.5 /  8.7 /  7.3   1024: 13.4 / 12.6 /  9.7   4096: 45.2 / 37.2 / 26.4
+    // at head_dim 64 and fewer than 1024 keys workgroups of four waves, two groups of two, are better still (128: 4.6, 512: 6.9).
+    // Between one half and one whole workgroup per compute unit two groups of four waves (us, 192 workgroups, four waves / split):
+    //   head_dim 128, keys 512: 13.3 / 13.5   1024: 21.3 / 19.8   4096: 71.7 / 60.9;   64, 512: 8.7 / 8.8   1024: 13.7 / 13.0   4096: 45.2 / 38.3
+    // and at head_dim 64 with a mask that hides a good part of the keys (up to two keys per query), where the 64-query
+    // workgroups even out: 256: 6.8 / 6.0 (two groups of two), 1024: 15.2 / 10.4, 2048: 26.5 / 19.2.
+    const long long blocks = (long long)batch * heads * (seq_q / 128);
+    const int keys = causal && seq_q < seq_kv - causalOff ? seq_q + causalOff : seq_kv; // that the last query sees
+    int groups = 0; // 1: two groups of two waves
+    if (blocks * 2 <= cus)
+        groups = keys >= (head_dim == 128 ? 256 : 1024) ? 4 : head_dim == 64 ? 1 : 0;
+    else if (blocks <= cus)
+        groups = head_dim == 64 && causal && keys >= 256 && keys / 2 <= seq_q ? 1 : keys >= 1024 ? 2 : 0;
+    if (groups == 1)
+        return launch_split_w4(st, o, lse, hq, hk, hv, batch, heads, seq_q, seq_kv, causal != 0, o_fp32 != 0, causalOff);
+    if (groups > 1)
+        return pto_amd::fa_fwd_split(st, o, lse, hq, hk, hv, batch, heads, seq_q, seq_kv, head_dim, causal != 0, o_fp32 != 0, causalOff, groups);
     // head_dim 128 with enough work to give every compute unit a workgroup of eight wavefronts (256 queries): the
     // K / V tiles are shared by twice the queries and the two waves of a SIMD alternate between MFMA and softmax
     // phases (measured +10-15 % at B1 H16 S4096 over workgroups of four waves)
     if (head_dim == 128 && seq_q % 256 == 0) {
-        static const int cus = [] {
-            int dev = 0, n = 0;
-            if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0)
-                n = 256;
-            return n;
-        }();
         if ((long long)batch * heads * (seq_q / 256) >= cus) {
             // the same schedule on 16 x 16 x 32 MFMAs: +1.5 .. 3.6 % without a mask and for long causal sequences
             // (interleaved runs; B2 H16 S2048 causal is 6 % slower on it and stays on the 32 x 32 x 16 kernel)

@@ -309,3 +309,72 @@ def test_fa_causal_diagonal_from_the_first_key(oracle, D, Sq, Skv):
         assert np.max(np.abs(lse[b, h] - (m + np.log(p.sum(axis=1, keepdims=True))).reshape(-1))) <= 1e-3
         oo, mm, ll = oracle.fa_stream_f16(q[b, h], k[b, h], v[b, h], tile_s1=64, causal=True, q_offset=0, round_away=False)
         assert rel(o[b, h], oo) <= 5e-4
+
+
+def fa_variant(q, k, v, causal, variant):
+    from gpu_util import stream, to_dev
+    B, H, Sq, D = q.shape
+    tq, tk, tv = to_dev(q), to_dev(k), to_dev(v)
+    to = torch.full((B, H, Sq, D), float("nan"), dtype=torch.float16, device="cuda:0")
+    tl = torch.full((B, H, Sq), float("nan"), dtype=torch.float32, device="cuda:0")
+    capi.check(capi.load_st().pto_fa_fwd_f16_variant(stream(), to.data_ptr(), tl.data_ptr(), tq.data_ptr(), tk.data_ptr(), tv.data_ptr(), B, H, Sq,
+                                               k.shape[2], D, int(causal), variant), "pto_fa_fwd_f16_variant")
+    torch.cuda.synchronize()
+    return to.cpu().numpy().astype(np.float32), tl.cpu().numpy()
+
+
+SPLIT = [(64, 32), (64, 42), (64, 44), (128, 42), (128, 44)]  # head_dim, variant: keys over 2 groups of 2, 2 of 4, 4 of 2 waves
+
+
+@pytest.mark.parametrize("D,variant", SPLIT)
+@pytest.mark.parametrize("Sq,Skv,causal", [(128, 64, False), (128, 192, False), (128, 128, True), (256, 576, False), (256, 576, True)])
+def test_fa_keys_split_over_groups(D, variant, Sq, Skv, causal):
+    """Groups without a tile, with one tile fewer than others, and (causal) whose keys are hidden from some of the queries."""
+    rng = np.random.default_rng(Sq + Skv + D)
+    q, k, v = (rng.standard_normal((1, 3, n, D)).astype(np.float16) for n in (Sq, Skv, Skv))
+    o, lse = fa_variant(q, k, v, causal, variant)
+    for h in range(3):
+        want, want_lse = dense_fp64(q[0, h], k[0, h], v[0, h], causal)
+        assert rel(o[0, h], want) <= TOL
+        assert np.max(np.abs(lse[0, h] - want_lse)) <= 1e-4
+
+
+@pytest.mark.parametrize("D,variant", SPLIT)
+def test_fa_keys_split_infinite_and_nan_scores(D, variant):
+    """Scores of -inf for all that one group sees leave the others' result; a NaN in any group's key reaches every query."""
+    rng = np.random.default_rng(D + variant)
+    q, k, v = (rng.standard_normal((1, 1, n, D)).astype(np.float16) for n in (128, 256, 256))
+    q[..., 0] = 1.0
+    k[..., 0] = 0.0
+    keep = np.arange(256) // (32 if (D, variant) == (128, 44) else 64) % (4 if variant == 44 else 2) != 1  # the tiles of group 1
+    k[0, 0, ~keep, 0] = -np.inf
+    o, lse = fa_variant(q, k, v, False, variant)
+    want, want_lse = dense_fp64(q[0, 0], k[0, 0][keep], v[0, 0][keep])
+    assert rel(o[0, 0], want) <= TOL
+    assert np.max(np.abs(lse[0, 0] - want_lse)) <= 1e-4
+    for key in (0, 40, 130, 255):
+        bad = k.copy()
+        bad[0, 0, ~keep, 0] = 0.0
+        bad[0, 0, key, 1] = np.nan
+        assert np.isnan(fa_variant(q, bad, v, False, variant)[0]).all()
+
+
+@pytest.mark.parametrize("B,H,Sq,Skv,D,causal", [(1, 3, 256, 1024, 64, 0), (1, 3, 128, 128, 64, 1), (1, 128, 128, 256, 128, 0), (3, 43, 128, 1024, 128, 1),
+                                                  (2, 64, 256, 256, 64, 2), (1, 2, 512, 256, 128, 2), (1, 256, 128, 1024, 64, 0)])
+@pytest.mark.parametrize("o_fp32", [False, True])
+def test_fa_few_query_blocks(B, H, Sq, Skv, D, causal, o_fp32):
+    """Both sides of the lines at which the keys are split, through the entry point."""
+    rng = np.random.default_rng(B + H + Sq)
+    q, k, v = (rng.standard_normal((B, H, n, D)).astype(np.float16) for n in (Sq, Skv, Skv))
+    o, lse = fa_gpu(q, k, v, causal, o_fp32)
+    for b, h in {(0, 0), (B - 1, H - 1), (B // 2, H // 2)}:
+        if causal == 2 and Skv != Sq:  # the diagonal starts in the first key
+            s = q[b, h].astype(np.float64) @ k[b, h].astype(np.float64).T / np.sqrt(D)
+            s = np.where(np.arange(Skv)[None, :] > np.arange(Sq)[:, None], -np.inf, s)
+            m = s.max(axis=1, keepdims=True)
+            p = np.exp(s - m)
+            want, want_lse = (p / p.sum(axis=1, keepdims=True)) @ v[b, h].astype(np.float64), (m[:, 0] + np.log(p.sum(axis=1)))
+        else:
+            want, want_lse = dense_fp64(q[b, h], k[b, h], v[b, h], causal != 0)
+        assert rel(o[b, h], want) <= TOL, (b, h)
+        assert np.max(np.abs(lse[b, h] - want_lse)) <= 1e-4, (b, h)
