@@ -1,5 +1,5 @@
 // Flash-attention forward kernel template and launcher, shared by the translation units that fix the
-// wave grid (1 x 4 in pto_fa.hip, 1 x 8 in pto_fa_w8.hip).  Include after <pto/pto-inst.hpp>.
+// wave grid (1 x 4 in pto_fa.hip, 1 x 8 in pto_fa_w8.hip and pto_fa_split.hip).  Include after <pto/pto-inst.hpp>.
 #pragma once
 #include "common.hpp"
 #include <cstdlib>
