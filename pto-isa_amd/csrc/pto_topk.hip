@@ -16,8 +16,8 @@
 // * Across lanes the sign does the choosing: before a stage a lane that is to keep the smaller key of a pair negates its
 //   key (one v_xor on the upper word); the pair then holds k and -k', and max(own, -received) is right for both lanes.
 // * The lanes of a row of 16 are numbered so that the partners of the four lowest lane strides are lane ^ 1, ^ 2, ^ 7, ^ 8:
-//   one DPP move for the upper word, and the lower word over the LDS pipe (ds_swizzle), which the network leaves idle
-//   otherwise; partners 16 and 32 lanes away come over the LDS pipe whole (v_permlane*_swap: 3.5 ns a word, 4.2 us of the
+//   one DPP move for the upper word, and for the lower word another, or the LDS pipe (ds_swizzle), which the network leaves idle
+//   otherwise (LOW_DPP, at the dispatch); partners 16 and 32 lanes away come over the LDS pipe whole (v_permlane*_swap: 3.5 ns a word, 4.2 us of the
 //   kernel's time for three stages of 55); strides across waves go through LDS memory.
 // * topk below the padded row length: once the sorted runs are as long as topk (rounded up to keys per lane times a power of
 //   two), a merge of two runs keeps their larger halves only, in both runs' lanes, and its sort passes no longer cover the
@@ -101,9 +101,10 @@ __device__ inline uint32_t ThroughLds(uint32_t v)
         return (uint32_t)__builtin_amdgcn_ds_bpermute((int)((threadIdx.x ^ 32u) << 2), (int)v);
     }
 }
-// the upper word goes through the LDS pipe only where the vector pipe would need two moves
+// the words go through the LDS pipe where the vector pipe would need two moves; else the upper one never, the lower one as the
+// launch has it
 template <int J>
-constexpr bool kHighThroughLds = J >= 4;
+constexpr bool kFarLane = J >= 4;
 
 // lane = c0 ^ 2 c1 ^ 7 c2 ^ 8 c3 ^ 16 c4 ^ 32 c5  ->  c0 + 2 c1 + 4 c2 + ...
 __device__ inline uint32_t LaneRank(uint32_t lane) { return (lane & 4u) ? lane ^ 3u : lane; }
@@ -111,7 +112,7 @@ __device__ inline uint32_t LaneRank(uint32_t lane) { return (lane & 4u) ? lane ^
 // Sorting of the 64 E W keys of a row, descending; key e of the lane with number q = 64 (wave of the row) + LaneRank(lane) is of
 // rank q E + e in the end.  keepBits: the ranks below E << keepBits are wanted.  A key is kept negated where `form` has its
 // sign bit set.  xchg: E x 64 keys per wave (W > 1).
-template <int E, int W>
+template <int E, int W, bool LOW_DPP>
 struct RowSort {
     static constexpr int kLaneBits = 6 + (W == 4 ? 2 : W == 2 ? 1 : 0);
     double k[E];
@@ -167,14 +168,17 @@ struct RowSort {
             uint32_t low[E], high[E];
 #pragma unroll
             for (int e = 0; e < E; ++e) {
-                low[e] = ThroughLds<J>(Low(k[e]));
-                if constexpr (kHighThroughLds<J>)
+                if constexpr (kFarLane<J> || !LOW_DPP)
+                    low[e] = ThroughLds<J>(Low(k[e]));
+                if constexpr (kFarLane<J>)
                     high[e] = ThroughLds<J>(High(k[e]));
             }
 #pragma unroll
             for (int e = 0; e < E; ++e) {
-                if constexpr (!kHighThroughLds<J>)
+                if constexpr (!kFarLane<J>)
                     high[e] = LaneMove<J>(High(k[e]));
+                if constexpr (!kFarLane<J> && LOW_DPP)
+                    low[e] = LaneMove<J>(Low(k[e]));
                 const double o = Key(high[e], low[e]);
                 k[e] = BOTH ? Max(k[e], o) : MaxOfNegated(k[e], o);
             }
@@ -282,7 +286,7 @@ __device__ inline void SortInLds(uint64_t *key, uint16_t *pos, int tid)
 
 // E keys per lane, W waves per row (the row is padded to 64 E W keys; padding keys lie below every real one), 4 / W rows per
 // workgroup.
-template <int E, int W>
+template <int E, int W, bool LOW_DPP>
 __global__ __launch_bounds__(kTopkThreads) void TopkRows(float *outScore, uint32_t *outIndex, const float *src, const uint32_t *inIdx,
                                                          int rows, int validCols, int ld, int topk, int keepBits)
 {
@@ -362,7 +366,7 @@ __global__ __launch_bounds__(kTopkThreads) void TopkRows(float *outScore, uint32
         return;
     }
 
-    RowSort<E, W> s;
+    RowSort<E, W, LOW_DPP> s;
     s.q = (uint32_t)waveOfRow * 64u + LaneRank((uint32_t)lane);
     s.xchg = reinterpret_cast<uint64_t *>(lds);
     const uint32_t columnBits = (4095u - i0) << 8;
@@ -437,7 +441,11 @@ extern "C" int pto_topk_f32(void *stream, float *out_score, uint32_t *out_index,
     // Waves per row.  One wave per row does the least work (1024 columns, top 1000: 4800 rows 29.8 us, with two 32.4, with four
     // 33.5), more waves per row put more of the chip to work on few rows (1200 rows 14.7 / 12.9 / 12.3 us, 145 rows 12.4 / 9.0 /
     // 7.0): as many as keep all of them within five on a SIMD, the four of a compute unit's workgroup at most, and none
-    // for rows of up to 256, whose exchanges across waves cost more than they save (1000 rows 4.8 / 5.1 / 6.6).
+    // for rows of up to 256, whose exchanges across waves cost more than they save (1000 rows 4.6 / 4.6 / 5.0).  512 columns:
+    // four up to 731 rows (600 rows 6.4 / 5.9 with two / four, 1000 rows 6.6 / 6.8).
+    // Lower words between near lanes: with up to four waves on a SIMD the latency of the LDS pipe shows, a DPP move is shorter
+    // (LDS / DPP, whole sorts: 300 x 256 4.53 / 4.28 us, 300 x 512 5.51 / 5.16, 1000 x 2048 18.95 / 18.13, 1000 x 4096 36.6 / 35.1);
+    // with more the moves take issue slots (4800 x 512 14.37 / 14.69).  16 keys per lane cover the latency either way.
     const int most = 5 * 4 * 256 / rows;
 #define PTO_TOPK_CASE(E, W)                                                                                              \
     {                                                                                                                    \
@@ -445,8 +453,11 @@ extern "C" int pto_topk_f32(void *stream, float *out_score, uint32_t *out_index,
         while ((E << keepBits) < topk)                                                                                   \
             ++keepBits;                                                                                                  \
         constexpr int kRows = kTopkWaves / W;                                                                            \
-        TopkRows<E, W><<<dim3((unsigned)(((long long)rows + kRows - 1) / kRows)), dim3(kTopkThreads), 0, st>>>(          \
-            out_score, out_index, src, in_idx, rows, valid_cols, ld, topk, keepBits);                                    \
+        const dim3 grid((unsigned)(((long long)rows + kRows - 1) / kRows)), block(kTopkThreads);                         \
+        if (E == 16 || (long long)rows * W <= 4 * 4 * 256)                                                               \
+            TopkRows<E, W, true><<<grid, block, 0, st>>>(out_score, out_index, src, in_idx, rows, valid_cols, ld, topk, keepBits); \
+        else                                                                                                             \
+            TopkRows<E, W, E == 16><<<grid, block, 0, st>>>(out_score, out_index, src, in_idx, rows, valid_cols, ld, topk, keepBits); \
         return pto_amd::check_launch();                                                                                  \
     }
     if (valid_cols <= 64)
@@ -456,7 +467,7 @@ extern "C" int pto_topk_f32(void *stream, float *out_score, uint32_t *out_index,
     if (valid_cols <= 256)
         PTO_TOPK_CASE(4, 1)
     if (valid_cols <= 512) {
-        if (most >= 4)
+        if (most >= 7)
             PTO_TOPK_CASE(2, 4)
         if (most >= 2)
             PTO_TOPK_CASE(4, 2)

@@ -85,6 +85,15 @@ def test_topk_waves_per_row(oracle, rows, cols, k):
         assert same(topk_gpu(src, ids, cols, k), oracle.topk_f32(src, ids, cols, k))
 
 
+@pytest.mark.parametrize("rows,cols", [(4096, 60), (4097, 60), (4097, 120), (4096, 200), (4097, 200), (731, 500), (732, 500), (2048, 500),
+                                       (2049, 500), (4097, 500)])
+def test_topk_lane_moves(oracle, rows, cols):
+    """Both sides of the row counts where the lower words' way between lanes and the waves per row of 512 columns change."""
+    src, idx = datagen.topk_inputs(rows, cols, cols + 1, distinct=300)
+    for k in (cols, 9):
+        assert same(topk_gpu(src, idx, cols, k), oracle.topk_f32(src, idx, cols, k))
+
+
 def test_topk_every_kind_of_score():
     """Infinities, denormals, NaNs of either sign and random bit patterns: ordered by bit pattern as the interface states
     (the float comparison of the oracle puts NaNs nowhere), equal ones by column, and their bits are kept."""
