@@ -25,7 +25,7 @@
 // * Any other index vector: low word = ~index, keys and columns in LDS, every stage a pass over LDS, four waves on one row
 //   after another; each wave owns a quarter of the row and the stages whose partners lie inside a quarter need no barrier.
 // What bounds it: vector instructions, 2240 per row of 1024 (3850 in the integer network this replaced), behind a phase of
-// loads and before one of stores that all waves share: of 26.9 us (4800 x 1024, top 1000, 58 MB = 9 us at 6.5 TB/s) 12 are
+// loads and before one of stores that all waves share: of 26.4 us (4800 x 1024, top 1000, 58 MB = 9 us at 6.5 TB/s) 12 are
 // launch, loads and stores.  Persistent waves that load the next row while they sort one, and wave priorities that let
 // some run ahead, do not hide them (32 us and no change).
 #include <hip/hip_runtime.h>
@@ -204,12 +204,9 @@ struct RowSort {
         StageEdge();
         SortLane();
         StageEdge();
-        // (few keys: straight-line code, the branches are most of what they cost; many: one copy of the code for all runs)
-        if constexpr (E <= 4)
-            StaticFor<1, kLaneBits + 1>([&](auto run) { Merge(decltype(run)::value, keepBits); });
-        else
-            for (int run = 1; run <= kLaneBits; ++run)
-                Merge(run, keepBits);
+        // (straight-line code: one copy for all runs branches around its stages, 8 to 15 % of the time at 8 and 16 keys per lane
+        // where topk is small, 2 to 6 % of a whole sort)
+        StaticFor<1, kLaneBits + 1>([&](auto run) { Merge(decltype(run)::value, keepBits); });
     }
     // runs of E << run keys out of two of half the length, descending and ascending in turn (the last: descending)
     __device__ inline __attribute__((always_inline)) void Merge(int run, int keepBits)
@@ -438,14 +435,15 @@ extern "C" int pto_topk_f32(void *stream, float *out_score, uint32_t *out_index,
     if (ld < valid_cols || topk > valid_cols || valid_cols > 4096)
         return PTO_ERR_UNSUPPORTED;
     hipStream_t st = static_cast<hipStream_t>(stream);
-    // Waves per row.  One wave per row does the least work (1024 columns, top 1000: 4800 rows 29.8 us, with two 32.4, with four
-    // 33.5), more waves per row put more of the chip to work on few rows (1200 rows 14.7 / 12.9 / 12.3 us, 145 rows 12.4 / 9.0 /
-    // 7.0): as many as keep all of them within five on a SIMD, the four of a compute unit's workgroup at most, and none
-    // for rows of up to 256, whose exchanges across waves cost more than they save (1000 rows 4.6 / 4.6 / 5.0).  512 columns:
-    // four up to 731 rows (600 rows 6.4 / 5.9 with two / four, 1000 rows 6.6 / 6.8).
+    // Waves per row.  One wave per row does the least work, more put more of the chip to work on few rows (one / two / four waves,
+    // whole sorts: 1024 columns, 600 rows 11.2 / 9.7 / 8.8 us, 1000 rows 11.6 / 10.2 / 10.2, 2400 rows 18.8 / 17.2 / 18.6, 4800
+    // rows 26.5 / 28.3; 1000 rows top 256 9.1 / 8.6 / 9.0): at 1024 columns four up to 853 rows, two up to 2560.  512 columns:
+    // four up to 731 rows (600 rows 6.5 / 6.4 / 5.9, 1000 rows 6.8 / 7.0 / 7.2), then one.  2048 columns: four up to 1706 rows (1700
+    // rows with two 27.2, with four 25.7; 2400 rows 32.4, 33.0).  Rows of up to 256: one, the exchanges across waves cost more
+    // than they save (1000 rows 4.6 / 4.6 / 5.0).
     // Lower words between near lanes: with up to four waves on a SIMD the latency of the LDS pipe shows, a DPP move is shorter
-    // (LDS / DPP, whole sorts: 300 x 256 4.53 / 4.28 us, 300 x 512 5.51 / 5.16, 1000 x 2048 18.95 / 18.13, 1000 x 4096 36.6 / 35.1);
-    // with more the moves take issue slots (4800 x 512 14.37 / 14.69).  16 keys per lane cover the latency either way.
+    // (LDS / DPP, whole sorts: 300 x 128 3.48 / 3.26 us, 300 x 256 4.53 / 4.28); with more the moves take issue slots (4800 x 128
+    // 5.09 / 5.23).  8 and 16 keys per lane cover the latency either way and take DPP.
     const int most = 5 * 4 * 256 / rows;
 #define PTO_TOPK_CASE(E, W)                                                                                              \
     {                                                                                                                    \
@@ -454,10 +452,10 @@ extern "C" int pto_topk_f32(void *stream, float *out_score, uint32_t *out_index,
             ++keepBits;                                                                                                  \
         constexpr int kRows = kTopkWaves / W;                                                                            \
         const dim3 grid((unsigned)(((long long)rows + kRows - 1) / kRows)), block(kTopkThreads);                         \
-        if (E == 16 || (long long)rows * W <= 4 * 4 * 256)                                                               \
+        if (E >= 8 || (long long)rows * W <= 4 * 4 * 256)                                                               \
             TopkRows<E, W, true><<<grid, block, 0, st>>>(out_score, out_index, src, in_idx, rows, valid_cols, ld, topk, keepBits); \
         else                                                                                                             \
-            TopkRows<E, W, E == 16><<<grid, block, 0, st>>>(out_score, out_index, src, in_idx, rows, valid_cols, ld, topk, keepBits); \
+            TopkRows<E, W, (E >= 8)><<<grid, block, 0, st>>>(out_score, out_index, src, in_idx, rows, valid_cols, ld, topk, keepBits); \
         return pto_amd::check_launch();                                                                                  \
     }
     if (valid_cols <= 64)
@@ -469,19 +467,17 @@ extern "C" int pto_topk_f32(void *stream, float *out_score, uint32_t *out_index,
     if (valid_cols <= 512) {
         if (most >= 7)
             PTO_TOPK_CASE(2, 4)
-        if (most >= 2)
-            PTO_TOPK_CASE(4, 2)
         PTO_TOPK_CASE(8, 1)
     }
     if (valid_cols <= 1024) {
-        if (most >= 4)
+        if (most >= 6)
             PTO_TOPK_CASE(4, 4)
         if (most >= 2)
             PTO_TOPK_CASE(8, 2)
         PTO_TOPK_CASE(16, 1)
     }
     if (valid_cols <= 2048) {
-        if (most >= 4)
+        if (most >= 3)
             PTO_TOPK_CASE(8, 4)
         PTO_TOPK_CASE(16, 2)
     }

@@ -86,7 +86,7 @@ def test_topk_waves_per_row(oracle, rows, cols, k):
 
 
 @pytest.mark.parametrize("rows,cols", [(4096, 60), (4097, 60), (4097, 120), (4096, 200), (4097, 200), (731, 500), (732, 500), (2048, 500),
-                                       (2049, 500), (4097, 500)])
+                                       (2049, 500), (4097, 500), (853, 1000), (854, 1000), (1706, 1900), (1707, 1900)])
 def test_topk_lane_moves(oracle, rows, cols):
     """Both sides of the row counts where the lower words' way between lanes and the waves per row of 512 columns change."""
     src, idx = datagen.topk_inputs(rows, cols, cols + 1, distinct=300)
