@@ -25,20 +25,24 @@ namespace {
 typedef _Float16 ks_f16x8 __attribute__((ext_vector_type(8)));
 typedef float ks_f32x4 __attribute__((ext_vector_type(4)));
 
-// 16 bytes per lane from the LDS; in flight until a wait that the kernel places itself
+// 16 bytes per lane from the LDS.  A load that the compiler knows: the registers of one in flight may be spilled or moved, behind
+// a wait that it then places (as assembly it stored them with the read still outstanding where a tile had too few registers).
 template <int IMM>
 PTO_DEV ks_f16x8 KsLdsRead16(uint32_t addr)
 {
-    ks_f16x8 r;
-    asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(r) : "v"(addr), "n"(IMM));
-    return r;
+    const auto *p = (const __attribute__((address_space(3))) char *)(uintptr_t)addr;
+    return *(const __attribute__((address_space(3))) ks_f16x8 *)(p + IMM);
 }
 
-// the reads into a set of fragments are over; ties them to their registers, before anything else may touch those
+// lgkmcnt(0), the other counters left alone: the builtin, which the compiler counts with (behind one in assembly it would add
+// a wait of its own for every fragment)
+PTO_DEV void KsWaitLds() { __builtin_amdgcn_s_waitcnt(0xc07f); }
+
+// the reads into a set of fragments are over; keeps them where they were issued, ahead of the MFMAs
 template <int MB, int NB>
 PTO_DEV void KsArrived(ks_f16x8 (&a)[MB], ks_f16x8 (&b)[NB])
 {
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    KsWaitLds();
 #pragma unroll
     for (int i = 0; i < NB; ++i)
         asm volatile("" : "+v"(b[i]));
@@ -124,16 +128,20 @@ __global__ __launch_bounds__(512, MIN_WAVES) AICORE void GemmF16F32Ks(float *out
             copyOne(j, s, s * kStage);
     hw::wait_vm<(S - 1) * kCopies>();
     __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory"); // (the barrier alone does not hold loads back from moving ahead of it)
     readStep(std::integral_constant<int, 0>(), 0u);
     KsArrived(a[0], b[0]);
 
-    auto step = [&](auto setTag, int it) __attribute__((always_inline)) {
+    auto step = [&](auto setTag, auto readTag, int it) __attribute__((always_inline)) {
         constexpr int set = decltype(setTag)::value;
+        constexpr bool read = decltype(readTag)::value; // the fragments of step it + 1
         // this wave has read all of step it, its copies of step it + 1 have landed; behind the barrier that is so of every wave
         hw::wait_vm<(S - 2) * kCopies>();
         __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
         __builtin_amdgcn_sched_barrier(0);
-        readStep(std::integral_constant<int, 1 - set>(), readOff);
+        if constexpr (read)
+            readStep(std::integral_constant<int, 1 - set>(), readOff);
         __builtin_amdgcn_sched_barrier(0);
         const bool mine = !HALF || group == 0 || it < steps - 1;
 #pragma unroll
@@ -150,20 +158,22 @@ __global__ __launch_bounds__(512, MIN_WAVES) AICORE void GemmF16F32Ks(float *out
         copyOff = readOff;
         readOff = readOff + kStage == kRing ? 0u : readOff + kStage;
         __builtin_amdgcn_sched_barrier(0);
-        KsArrived(a[1 - set], b[1 - set]);
+        if constexpr (read)
+            KsArrived(a[1 - set], b[1 - set]);
     };
     int it = 0;
-    for (; it + 2 <= steps; it += 2) {
-        step(std::integral_constant<int, 0>(), it);
-        step(std::integral_constant<int, 1>(), it + 1);
+    for (; it + 2 <= steps; it += 2) { // (past the end it reads fragments that nobody uses)
+        step(std::integral_constant<int, 0>(), std::true_type(), it);
+        step(std::integral_constant<int, 1>(), std::true_type(), it + 1);
     }
     if (it < steps)
-        step(std::integral_constant<int, 0>(), it);
+        step(std::integral_constant<int, 0>(), std::false_type(), it);
 
     // Partial sums: each group keeps half of its wave's blocks, gives the other half to its partner (same rows and
     // columns, other k) and stores the sums of the half it keeps.
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); // the copies past the end
     __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
     constexpr int kHalfBlocks = MB * NB / 2;
     char *sums = hw::lds_base();
     const int pair = wave & 3;

@@ -27,7 +27,7 @@ namespace {
 template <int MB, int NB>
 PTO_DEV void MxKsArrived(ks_f16x8 (&a)[MB][2], ks_f16x8 (&b)[NB][2], ks_f16x8 (&scales)[MB + NB])
 {
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    KsWaitLds();
 #pragma unroll
     for (int i = 0; i < NB; ++i)
         asm volatile("" : "+v"(b[i][0]), "+v"(b[i][1]));
@@ -183,6 +183,7 @@ __global__ __launch_bounds__(512, MIN_WAVES) AICORE
             copyOne(j, s, s * kStage);
     hw::wait_vm<(S - 1) * kCopies>();
     __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory"); // (the barrier alone does not hold loads back from moving ahead of it)
     readStep(std::integral_constant<int, 0>(), 0u);
     readScales(0);
     MxKsArrived(a[0], b[0], scales);
@@ -199,6 +200,7 @@ __global__ __launch_bounds__(512, MIN_WAVES) AICORE
         // (scale copies among the younger ones only make the wait stricter)
         hw::wait_vm<(S - 2) * kCopies>();
         __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
         __builtin_amdgcn_sched_barrier(0);
         readStep(std::integral_constant<int, 1 - set>(), readOff);
         if constexpr (t == Q - 1)
@@ -236,6 +238,7 @@ __global__ __launch_bounds__(512, MIN_WAVES) AICORE
     // columns, other k) and stores the sums of those it keeps.
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); // the copies past the end
     __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
     char *sums = hw::lds_base();
     const int pair = wave & 3;
     // piece 2 idx + u of pair, group: registers 8 g + 4 u .. + 3 of block idx that group g keeps
