@@ -31,7 +31,9 @@ template <int IMM>
 PTO_DEV ks_f16x8 KsLdsRead16(uint32_t addr)
 {
     const auto *p = (const __attribute__((address_space(3))) char *)(uintptr_t)addr;
-    return *(const __attribute__((address_space(3))) ks_f16x8 *)(p + IMM);
+    const ks_f16x8 r = *(const __attribute__((address_space(3))) ks_f16x8 *)(p + IMM);
+    __builtin_amdgcn_sched_barrier(0); // (in the order written)
+    return r;
 }
 
 // lgkmcnt(0), the other counters left alone: the builtin, which the compiler counts with (behind one in assembly it would add
