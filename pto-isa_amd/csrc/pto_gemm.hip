@@ -42,31 +42,33 @@ extern "C" int pto_gemm_f16f32_variant(void *stream, float *c, const uint16_t *a
 namespace {
 // What a problem takes with one tile shape: tiles are dealt to the compute units, `rounds` of them to the busiest one, and
 //   time = fixed + per_round more + (k / 64) (step + step_round more + step_share share) + per_mb (megabytes of C),
-// more = rounds - 1, share of the units busy in the last round, in microseconds, launch included.  The figures are
-// least-squares fits to 330 problems between 128 x 128 x 256 and 6144 x 6144 x 6144, three operand sets in turn (root mean
-// square of the relative error 4 .. 6 %).  The k-split shapes are taken 6 % dearer than fitted: where the two kinds come out
-// even, the four-wave tiles stay (without it 5768 x 500 x 256 ran 8 % and 3 of 330 problems over 2 % longer than on four-wave
-// tiles alone, with it 1 of 330); so chosen, a problem is 0.1 % from its best shape on average.  What the figures say: a small
-// tile's step is cheap and moves more bytes per flop (64 x 64: 0.17 us a step, 128 x 128: 0.34, the four-wave 256 x 192: 0.67),
-// so it wins while it puts more compute units to work -- 512^3 8.9 us on six 192 x 128 tiles, 4.1 on 32 x 64 ones; 1024^3 13.7
-// and 6.8; 128 x 4096 x 4096 68 and 13; 768 x 768 x 6144 48 and 20 -- and the tiles of 192 and 256 rows win from about one
-// whole round of them on (2048^3 24 against 21 on 128 x 128, 4096^3 106 against 142 on 192 x 128).
+// more = rounds - 1, share of the units busy in the last round, in microseconds, launch included; the k-split tiles take 6 %
+// longer where k ends in half a step.  The figures are least-squares fits to 2293 problems (128 x 128 x 128 .. 6144^3 ragged,
+// .. 16384 x 8192 x 8192 in whole tiles, three operand sets in turn) in which those near a shape's best use count most (root
+// mean square of the relative error there 3 .. 6 %).  The k-split shapes are taken 3 %, the 128 x 256 block 2 % dearer than
+// fitted: where they and the four-wave tiles come out even, the latter stay.  So chosen, a problem is 0.15 % from its best
+// shape on average (21 % at worst) and 12 of the 2293 are over 2 % slower than with four-wave tiles (k a multiple of 128)
+// or blocks alone, the worst 7.6 % (with a fit to 330 problems that counted every one alike: 24 of 1893, and 12.4 %).  What the figures say: a
+// small tile's step is cheap and moves more bytes per flop (64 x 64: 0.2 us a step, 128 x 128: 0.45, the four-wave 256 x 192:
+// 1.1), so it wins while it puts more compute units to work -- 512^3 8.9 us on twelve 192 x 128 tiles, 4.0 on 32 x 64 ones;
+// 1024^3 13.7 and 6.8; 128 x 4096 x 4096 68 and 12; 768 x 768 x 6144 48 and 20 -- and the tiles of 192 and 256 rows win from
+// about one whole round of them on (2048^3 22.7 against 21.0 on 128 x 128, 4096^3 104 against 137 on 192 x 128).
 struct TileShape {
     enum Kernel { kW4, kKs, kBlock } kernel;
     int number, bm, bn;
     double fixed, perRound, step, stepRound, perMb, stepShare;
 };
 constexpr TileShape kShapes[] = {
-    {TileShape::kW4, 0, 256, 256, 8.66, 3.98, 0.888, 1.402, 0.112, 0.336}, {TileShape::kW4, 1, 256, 192, 6.82, 2.09, 0.672, 1.070, 0.126, 0.286},
-    {TileShape::kW4, 2, 256, 128, 4.99, 1.25, 0.520, 0.744, 0.171, 0.103}, {TileShape::kW4, 3, 192, 256, 7.05, 2.80, 0.674, 1.078, 0.114, 0.302},
-    {TileShape::kW4, 4, 192, 192, 5.77, 2.47, 0.524, 0.818, 0.135, 0.197}, {TileShape::kW4, 5, 192, 128, 4.04, 0.99, 0.434, 0.611, 0.180, 0.103},
-    {TileShape::kKs, 0, 32, 64, 2.70, 0.69, 0.134, 0.139, 0.194, 0.022},   {TileShape::kKs, 1, 64, 64, 2.67, 0.59, 0.166, 0.169, 0.189, 0.030},
-    {TileShape::kKs, 2, 64, 96, 2.91, 0.52, 0.224, 0.239, 0.207, 0.031},   {TileShape::kKs, 3, 128, 64, 2.63, 0.01, 0.286, 0.259, 0.252, 0.028},
-    {TileShape::kKs, 4, 128, 96, 4.00, 1.67, 0.315, 0.372, 0.202, 0.038},  {TileShape::kKs, 5, 128, 128, 4.38, 1.62, 0.340, 0.441, 0.186, 0.066},
-    {TileShape::kKs, 6, 192, 128, 5.58, 2.65, 0.441, 0.622, 0.159, 0.118}, {TileShape::kKs, 7, 256, 128, 6.25, 2.69, 0.572, 0.788, 0.153, 0.128},
-    {TileShape::kKs, 8, 192, 192, 6.74, 3.26, 0.642, 0.863, 0.144, 0.139},
-    // the 128 x 256 block written with the tile instructions: 2048 x 6144 x 1056 38 us against 44 on 256 x 128
-    {TileShape::kBlock, 0, 128, 256, 3.03, 0.00, 1.000, 0.750, 0.161, 0.000},
+    {TileShape::kW4, 0, 256, 256, 9.263, 7.420, 0.770, 1.429, 0.085, 0.610}, {TileShape::kW4, 1, 256, 192, 8.193, 6.015, 0.543, 1.115, 0.070, 0.533},
+    {TileShape::kW4, 2, 256, 128, 6.567, 3.898, 0.379, 0.817, 0.083, 0.373}, {TileShape::kW4, 3, 192, 256, 7.814, 4.941, 0.581, 1.150, 0.084, 0.490},
+    {TileShape::kW4, 4, 192, 192, 7.134, 4.643, 0.393, 0.916, 0.072, 0.451}, {TileShape::kW4, 5, 192, 128, 4.741, 1.197, 0.337, 0.658, 0.159, 0.242},
+    {TileShape::kKs, 0, 32, 64, 2.670, 0.853, 0.135, 0.136, 0.178, 0.026},   {TileShape::kKs, 1, 64, 64, 2.822, 0.902, 0.152, 0.165, 0.175, 0.044},
+    {TileShape::kKs, 2, 64, 96, 3.214, 0.965, 0.207, 0.240, 0.183, 0.052},   {TileShape::kKs, 3, 128, 64, 3.221, 0.868, 0.249, 0.258, 0.180, 0.080},
+    {TileShape::kKs, 4, 128, 96, 4.595, 2.050, 0.258, 0.411, 0.162, 0.127},  {TileShape::kKs, 5, 128, 128, 5.026, 2.036, 0.293, 0.488, 0.140, 0.156},
+    {TileShape::kKs, 6, 192, 128, 6.565, 2.833, 0.384, 0.682, 0.109, 0.218}, {TileShape::kKs, 7, 256, 128, 7.789, 4.862, 0.468, 0.875, 0.072, 0.314},
+    {TileShape::kKs, 8, 192, 192, 8.656, 5.901, 0.502, 0.952, 0.058, 0.342},
+    // the 128 x 256 block written with the tile instructions: 2048 x 6144 x 1056 37 us against 44 on 256 x 128
+    {TileShape::kBlock, 0, 128, 256, 3.292, 0.364, 0.919, 0.820, 0.114, 0.161},
 };
 } // namespace
 
@@ -88,7 +90,7 @@ extern "C" int pto_gemm_f16f32(void *stream, float *c, const uint16_t *a, const 
         const long long tiles = (long long)((m + s.bm - 1) / s.bm) * ((n + s.bn - 1) / s.bn);
         const double more = (double)((tiles - 1) / cus), share = (double)((tiles - 1) % cus + 1) / cus, steps = (k + 63) / 64;
         const double time = (s.fixed + s.perRound * more + steps * (s.step + s.stepRound * more + s.stepShare * share) + s.perMb * (4e-6 * m * n)) *
-                            (s.kernel == TileShape::kKs ? 1.06 : 1.0);
+                            (s.kernel == TileShape::kW4 ? 1.0 : s.kernel == TileShape::kKs ? 1.03 : 1.02) * (s.kernel == TileShape::kKs && k % 64 ? 1.06 : 1.0);
         if (best == nullptr || time < bestTime) {
             best = &s;
             bestTime = time;

@@ -351,38 +351,43 @@ namespace {
 // tiles on four (pto_gemm_mxw4.hip), and tiles of 64 .. 192 rows with k split over two groups of wavefronts
 // (pto_gemm_mxks.hip).  What a problem takes with one tile shape, in microseconds, launch included: tiles are dealt to the
 // compute units, `more` rounds beyond the first, `share` of the units busy in the last one, steps of 128 bytes,
-//   time = fixed + per_round more + steps (step + step_round more + step_share share) + per_mega (4e-6 m n)
-// Least-squares fits to 240 problems between 256 x 256 x 512 and 6144 x 6144 x 6144, three operand sets in turn, bf16 result
-// (root mean square of the relative error 3 .. 5 %).  The k-split shapes are taken 3 % dearer and the 256 x 256 tiles of fp8
-// 8 % than fitted (against moves on the noise of the fit); so chosen, a problem is 0.3 % (fp8) and 0.4 % (fp4) from its best
-// shape on average, 7 % at worst.  Against the 256-row tiles alone: 256 x 256 x 6144 fp8 34.1 -> 11.0 us, 512 x 512 x 2048 fp4
-// 12.0 -> 4.9, 592 x 736 x 4096 24.7 -> 9.9, 2048^3 17.3 -> 13.3, geometric mean of the 240 problems 1.50 (fp8), 1.67 (fp4).
+//   time = fixed + per_round more + steps (step + step_round more + step_share share) + (per_mega + fp32 result: per_mega_f32) (4e-6 m n);
+// the 256 x 256 tiles take `ragged` longer a step and round where m or n is no multiple of 256 (the last tiles are moved back).
+// Least-squares fits to 1520 problems (256 x 256 x 512 .. 6144^3 ragged, .. 16384 x 8192 x 8192 in whole tiles, both results,
+// three operand sets in turn) in which those near a shape's best use count most (root mean square of the relative error there
+// 2 .. 5 %).  The k-split shapes are taken 2 %, the 256 x 256 tiles 3 % dearer than fitted (against moves on the noise of the
+// fit); so chosen, a problem is 0.4 % (fp8) and 0.3 % (fp4) from its best shape on average, 12 % at worst, and 8 of the 1520
+// are over 2 % slower than on 256-row tiles alone, the worst 10.6 % (with a fit to ragged bf16 problems only: 16, and 24 %).
+// Against the 256-row tiles alone: 256 x 256 x 6144 fp8 34.0 -> 12.0 us, 512 x 512 x 2048 fp4 12.0 -> 4.9, 592 x 736 x 4096
+// 24.6 -> 9.8, 2048^3 17.3 -> 13.5, geometric mean of the problems 1.58 (fp8), 1.66 (fp4).  (128 x 192 with fp8 is the best
+// shape of 9 of 1002 problems, by up to 5 %: 1024 x 4608 x 1536.)
 struct MxShape {
     enum Kernel { kBlock, kW4, kKs } kernel;
     int number, bm, bn;
-    double fixed, perRound, step, stepRound, perMega, stepShare;
+    double fixed, perRound, step, stepRound, perMega, stepShare, perMegaF32;
 };
 constexpr MxShape kMxShapes[2][9] = {
-    {{MxShape::kBlock, 0, 256, 256, 5.15, 3.00, 1.132, 1.742, 0.112, 0.421},
-     {MxShape::kW4, 0, 256, 192, 8.10, 4.31, 0.680, 1.102, 0.060, 0.259},
-     {MxShape::kW4, 0, 256, 128, 5.89, 3.38, 0.551, 0.784, 0.071, 0.135},
-     {MxShape::kKs, 0, 64, 64, 2.93, 0.75, 0.179, 0.201, 0.125, 0.057},
-     {MxShape::kKs, 1, 64, 128, 3.70, 2.38, 0.235, 0.319, 0.097, 0.142},
-     {MxShape::kKs, 2, 128, 64, 3.61, 2.01, 0.266, 0.312, 0.150, 0.061},
-     {MxShape::kKs, 3, 128, 128, 4.67, 2.62, 0.355, 0.489, 0.159, 0.093},
-     {MxShape::kKs, 4, 128, 192, 5.85, 3.75, 0.496, 0.718, 0.117, 0.159},
-     {MxShape::kKs, 5, 192, 128, 5.90, 3.39, 0.506, 0.716, 0.127, 0.124}}, // fp8
-    {{MxShape::kBlock, 0, 256, 256, 5.15, 12.01, 1.157, 1.296, 0.081, 0.754},
-     {MxShape::kW4, 0, 256, 192, 7.67, 6.75, 0.912, 1.065, 0.073, 0.227},
-     {MxShape::kW4, 0, 256, 128, 5.97, 5.46, 0.657, 0.800, 0.058, 0.246},
-     {MxShape::kKs, 0, 64, 64, 2.93, 0.44, 0.233, 0.216, 0.244, 0.000},
-     {MxShape::kKs, 1, 64, 128, 3.68, 2.13, 0.304, 0.354, 0.157, 0.081},
-     {MxShape::kKs, 2, 128, 64, 3.75, 2.28, 0.307, 0.339, 0.159, 0.057},
-     {MxShape::kKs, 3, 128, 128, 4.88, 3.16, 0.405, 0.545, 0.135, 0.133},
-     {MxShape::kKs, 4, 128, 192, 5.78, 3.34, 0.569, 0.843, 0.140, 0.092},
-     {MxShape::kKs, 5, 192, 128, 5.83, 3.42, 0.568, 0.856, 0.137, 0.103}}, // fp4
+    {{MxShape::kBlock, 0, 256, 256, 6.233, 4.744, 0.882, 1.791, 0.025, 0.728, 0.076},
+     {MxShape::kW4, 0, 256, 192, 8.332, 5.596, 0.666, 1.163, 0.062, 0.369, 0.033},
+     {MxShape::kW4, 0, 256, 128, 6.086, 2.935, 0.553, 0.842, 0.093, 0.144, 0.035},
+     {MxShape::kKs, 0, 64, 64, 2.595, 0.634, 0.196, 0.185, 0.191, 0.051, 0.027},
+     {MxShape::kKs, 1, 64, 128, 3.318, 1.592, 0.277, 0.320, 0.188, 0.054, 0.039},
+     {MxShape::kKs, 2, 128, 64, 3.318, 1.545, 0.284, 0.315, 0.201, 0.039, 0.036},
+     {MxShape::kKs, 3, 128, 128, 4.635, 2.138, 0.354, 0.508, 0.146, 0.110, 0.048},
+     {MxShape::kKs, 4, 128, 192, 5.785, 2.957, 0.481, 0.728, 0.124, 0.168, 0.059},
+     {MxShape::kKs, 5, 192, 128, 5.833, 2.802, 0.482, 0.730, 0.129, 0.170, 0.056}}, // fp8
+    {{MxShape::kBlock, 0, 256, 256, 5.763, 3.741, 1.024, 2.102, 0.045, 0.821, 0.085},
+     {MxShape::kW4, 0, 256, 192, 8.060, 6.472, 0.880, 1.293, 0.066, 0.435, 0.026},
+     {MxShape::kW4, 0, 256, 128, 6.084, 3.053, 0.645, 0.951, 0.098, 0.213, 0.036},
+     {MxShape::kKs, 0, 64, 64, 2.952, 0.929, 0.213, 0.209, 0.125, 0.078, 0.033},
+     {MxShape::kKs, 1, 64, 128, 3.633, 2.235, 0.289, 0.363, 0.135, 0.113, 0.039},
+     {MxShape::kKs, 2, 128, 64, 3.647, 2.183, 0.294, 0.356, 0.147, 0.100, 0.038},
+     {MxShape::kKs, 3, 128, 128, 4.723, 2.682, 0.406, 0.591, 0.136, 0.166, 0.045},
+     {MxShape::kKs, 4, 128, 192, 5.718, 3.475, 0.547, 0.827, 0.125, 0.234, 0.054},
+     {MxShape::kKs, 5, 192, 128, 5.765, 3.304, 0.543, 0.883, 0.122, 0.257, 0.056}}, // fp4
 };
-constexpr double kMxStepQuarter[2] = {0.34, 0.25}; // a step of the round of 128 x 128 quarter tiles
+// fp8, fp4: the round of 128 x 128 quarter tiles, fixed and a step; `ragged`
+constexpr double kMxQuarter[2] = {0.000, 4.513}, kMxStepQuarter[2] = {0.830, 0.753}, kMxStepRagged[2] = {0.080, 0.125};
 
 int gemm_mx_any(hipStream_t st, void *c, const uint8_t *a, const uint8_t *b, const uint8_t *sa, const uint8_t *sb, int m, int n, int k,
                 int format, int c_fp32)
@@ -398,13 +403,17 @@ int gemm_mx_any(hipStream_t st, void *c, const uint8_t *a, const uint8_t *b, con
         if ((s.kernel == MxShape::kBlock && !block) || (s.kernel == MxShape::kW4 && (!w4 || n < s.bn)) || (s.kernel == MxShape::kKs && n % 4))
             continue;
         const long long tiles = (long long)((m + s.bm - 1) / s.bm) * ((n + s.bn - 1) / s.bn), rest = tiles % cus;
-        double more = (double)((tiles - 1) / cus), share = (double)((tiles - 1) % cus + 1) / cus, quarter = 0.0;
-        if (s.kernel == MxShape::kBlock && rest > 0 && rest * 4 <= cus && tiles > cus && m % 256 == 0 && n % 256 == 0) {
+        double more = (double)((tiles - 1) / cus), share = (double)((tiles - 1) % cus + 1) / cus, extra = 0.0;
+        if (s.kernel == MxShape::kBlock && !(m % 256 == 0 && n % 256 == 0)) {
+            extra = steps * kMxStepRagged[fp4] * (more + 1.0);
+        } else if (s.kernel == MxShape::kBlock && rest > 0 && rest * 4 <= cus && tiles > cus) {
             more -= 1.0;
             share = 1.0;
-            quarter = steps * kMxStepQuarter[fp4] + 4.0;
+            extra = kMxQuarter[fp4] + steps * kMxStepQuarter[fp4];
         }
-        const double time = s.fixed + s.perRound * more + steps * (s.step + s.stepRound * more + s.stepShare * share) + s.perMega * (4e-6 * m * n) + quarter;
+        const double time = (s.fixed + s.perRound * more + steps * (s.step + s.stepRound * more + s.stepShare * share) +
+                             (s.perMega + (c_fp32 ? s.perMegaF32 : 0.0)) * (4e-6 * m * n) + extra) *
+                            (s.kernel == MxShape::kW4 ? 1.0 : s.kernel == MxShape::kKs ? 1.02 : 1.03);
         if (best == nullptr || time < bestTime) {
             best = &s;
             bestTime = time;

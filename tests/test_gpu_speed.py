@@ -1,0 +1,53 @@
+"""Choices of a kernel that a wrong rule makes slow: the public entry point against a call that bounds it, both timed in turn.
+The margins are several times what repeated timings of one call differ by (about 1 %)."""
+import numpy as np
+import pytest
+import torch
+
+from pto_amd import capi
+
+pytestmark = pytest.mark.gpu
+
+
+def best_us(calls, launches=20, rounds=9):
+    """The shortest time of each call, in microseconds: `launches` of it in a row, the calls in turn."""
+    best = [float("inf")] * len(calls)
+    for _ in range(rounds):
+        for i, call in enumerate(calls):
+            start, end = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            call()
+            start.record()
+            for _ in range(launches):
+                call()
+            end.record()
+            end.synchronize()
+            best[i] = min(best[i], start.elapsed_time(end) * 1000.0 / launches)
+    return best
+
+
+@pytest.mark.parametrize("m,n,k", [(2048, 5888, 800), (1792, 6144, 736)])
+def test_gemm_choice_against_blocks(m, n, k):
+    """Whole 128 x 256 blocks with a k that no multiple of 128 is: no slower than the block kernel that used to take them
+    (it was, by 7 to 11 %)."""
+    lib = capi.load_st()
+    stream = torch.cuda.current_stream().cuda_stream
+    a, b = (torch.rand((r, k), device="cuda:0").half() for r in (m, n))
+    c = torch.empty((m, n), device="cuda:0")
+    args = (stream, c.data_ptr(), a.data_ptr(), b.data_ptr(), m, n, k)
+    public, block = best_us([lambda: capi.check(lib.pto_gemm_f16f32(*args), "entry point"),
+                             lambda: capi.check(lib.pto_gemm_f16f32_variant(*args, 2), "blocks")])
+    assert public <= 1.05 * block, (public, block)
+
+
+@pytest.mark.parametrize("m,n,k,fmt,c_fp32,variant", [(5632, 3328, 6144, 1, 1, 5), (8192, 8192, 8192, 0, 0, 5), (16384, 8192, 8192, 4, 0, 5)])
+def test_mx_gemm_choice_against_four_waves(m, n, k, fmt, c_fp32, variant):
+    """Large products in whole tiles: no slower than on 256 x 192 tiles, which used to take them (they were, by 5 to 24 %)."""
+    lib = capi.load_st()
+    stream = torch.cuda.current_stream().cuda_stream
+    a, b = (torch.randint(0, 120, (r, k // 2 if fmt == 4 else k), dtype=torch.uint8, device="cuda:0") for r in (m, n))
+    sa, sb = (torch.full((r, k // 32), 127, dtype=torch.uint8, device="cuda:0") for r in (m, n))
+    c = torch.empty((m, n), dtype=torch.float32 if c_fp32 else torch.bfloat16, device="cuda:0")
+    args = (stream, c.data_ptr(), a.data_ptr(), b.data_ptr(), sa.data_ptr(), sb.data_ptr(), m, n, k, fmt, c_fp32)
+    public, four = best_us([lambda: capi.check(lib.pto_gemm_mxfp8_variant(*args, 4), "as the entry points choose"),
+                            lambda: capi.check(lib.pto_gemm_mxfp8_variant(*args, variant), "256 x 192")], launches=5)
+    assert public <= 1.035 * four, (public, four)
