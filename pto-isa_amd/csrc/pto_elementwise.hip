@@ -116,13 +116,14 @@ __global__ __launch_bounds__(kBlockThreads) void CvtF32Stream(D *dst, const floa
 // row, so every store instruction of a wave is 1 KiB of consecutive addresses and every load whole lines of the table's
 // rows; the indices, then all loads of a lane are in flight before its first store; no LDS, no barrier.  The division is
 // a multiplication: for c < 2^31, c / cpr = c magic >> shift with magic = ceil(2^shift / cpr), shift = 31 + ceil(log2 cpr).
+// Table and output need their elements' alignment only (the chunks are typed so; the same instructions).
 // The row is cut into `parts` (1, 2, 4 or 8) slices of cpr chunks, and workgroup b works on slice (b % 8) % parts: as the
 // workgroups are dealt to the eight XCDs in turn, an XCD's L2 then sees one slice of the table only.
 constexpr int kGatherSteps = 2, kGatherChunks = kBlockThreads * kGatherSteps;
 __global__ __launch_bounds__(kBlockThreads) void GatherChunks(char *out, const char *table, const int32_t *idx, uint32_t chunks, uint32_t cpr,
                                                               uint32_t magic, int shift, uint32_t tableRows, uint32_t parts)
 {
-    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+    typedef uint32_t u32x4 __attribute__((ext_vector_type(4), aligned(2)));
     const uint32_t xcd = blockIdx.x % 8, slice = xcd % parts, block = blockIdx.x / 8 * (8 / parts) + xcd / parts;
     const uint32_t first = block * (uint32_t)kGatherChunks + threadIdx.x, rowChunks = cpr * parts;
     if (block * (uint32_t)kGatherChunks >= chunks)

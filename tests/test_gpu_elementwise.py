@@ -140,6 +140,21 @@ def test_gather_rows_widths_and_slices(oracle, rows, cols, nidx):
     assert np.array_equal(gather_rows(t32, idx), oracle.gather_rows(t32, idx))
 
 
+@pytest.mark.parametrize("rows,cols,nidx", [(5, 24, 700), (1500, 1032, 3001), (3000, 1024, 6001)])
+@pytest.mark.parametrize("dtype", [torch.int16, torch.int32])
+def test_gather_rows_element_alignment(rows, cols, nidx, dtype):
+    """Table and output one element past a 16-byte boundary, one and several slices: the rows, and nothing around the output."""
+    top = torch.iinfo(dtype).max
+    memory = torch.randint(-top, top, (rows * cols + 1,), dtype=dtype, device="cuda:0")
+    ids = torch.randint(0, rows, (nidx,), dtype=torch.int32, device="cuda:0")
+    out = torch.full((nidx * cols + 64,), 77, dtype=dtype, device="cuda:0")
+    size = memory.element_size()
+    capi.check(capi.load().pto_gather_rows(torch.cuda.current_stream().cuda_stream, out.data_ptr() + size, memory.data_ptr() + size, ids.data_ptr(),
+                                           nidx, rows, cols, size), "pto_gather_rows")
+    assert torch.equal(out[1:1 + nidx * cols].view(nidx, cols), memory[1:].view(rows, cols)[ids.long()])
+    assert out[0] == 77 and (out[1 + nidx * cols:] == 77).all()
+
+
 def test_gather_rows_full_size_config(oracle):
     """Config 5: 65536 int32 row indices over a 16384 x 1024 fp16 table: bit-exact copy."""
     from gpu_util import gather_rows
