@@ -471,13 +471,15 @@ __global__ __launch_bounds__(kBlockThreads, MIN_BLOCKS) AICORE void FlashAttnFwd
         });
     };
     if constexpr (G > 1) {
-        // Q^T straight into the operand registers: 16 bytes of the lane's own query per step of 16
+        // Q^T straight into the operand registers: 16 bytes of the lane's own query per step of 16 (typed with the alignment
+        // of an element, as little as the copies of the unsplit form ask for)
+        typedef half Q8 __attribute__((ext_vector_type(8), aligned(2)));
         loadGroups(std::integral_constant<int, 0>(), std::false_type(), kBase, 0);
         loadGroups(std::integral_constant<int, 0>(), std::true_type(), vBase, 0);
         const half *qRow = qAll + ((int64_t)bh * seqQ + myQuery) * D + 8 * hHalf;
 #pragma unroll
         for (int ks = 0; ks < D / 16; ++ks)
-            qRight.st.f[0][ks] = *reinterpret_cast<const f16x8 *>(qRow + 16 * ks);
+            qRight.st.f[0][ks] = *reinterpret_cast<const Q8 *>(qRow + 16 * ks);
         set_flag(PIPE_MTE2, PIPE_MTE1, EVENT_ID0);
     } else {
         GlobalQT gmQ(qBase);

@@ -24,6 +24,7 @@ namespace {
 
 typedef _Float16 ks_f16x8 __attribute__((ext_vector_type(8)));
 typedef float ks_f32x4 __attribute__((ext_vector_type(4)));
+typedef float ks_c4 __attribute__((ext_vector_type(4), aligned(4))); // four elements of C, whose rows need no more alignment than these
 
 // 16 bytes per lane from the LDS.  A load that the compiler knows: the registers of one in flight may be spilled or moved, behind
 // a wait that it then places (as assembly it stored them with the read still outstanding where a tile had too few registers).
@@ -192,7 +193,7 @@ __global__ __launch_bounds__(512, MIN_WAVES) AICORE void GemmF16F32Ks(float *out
             const ks_f32x4 v = acc[i][j] + *reinterpret_cast<const ks_f32x4 *>(sums + ((uint32_t)(pair * MB * NB + idx) * 64u + lane) * 16u);
             const int row = rowLane + 16 * i, col = colLane + 16 * j;
             if (row < m && col < n) // n % 4 == 0: four columns are inside together
-                *reinterpret_cast<ks_f32x4 *>(out + (int64_t)row * n + col) = v;
+                *reinterpret_cast<ks_c4 *>(out + (int64_t)row * n + col) = v;
         }
     });
 }

@@ -269,11 +269,11 @@ __global__ __launch_bounds__(512, MIN_WAVES) AICORE
                 if (row < m && col < n) { // n % 4 == 0: four columns are inside together
                     OutT *dst = out + (int64_t)row * n + col;
                     if constexpr (std::is_same_v<OutT, float>) {
-                        *reinterpret_cast<ks_f32x4 *>(dst) = v;
+                        *reinterpret_cast<ks_c4 *>(dst) = v;
                     } else {
                         const uint32_t lo = (uint32_t)detail::f32_to_bf16_bits_rne(v.x) | ((uint32_t)detail::f32_to_bf16_bits_rne(v.y) << 16);
                         const uint32_t hi = (uint32_t)detail::f32_to_bf16_bits_rne(v.z) | ((uint32_t)detail::f32_to_bf16_bits_rne(v.w) << 16);
-                        typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+                        typedef uint32_t u32x2 __attribute__((ext_vector_type(2), aligned(2)));
                         *reinterpret_cast<u32x2 *>(dst) = u32x2{lo, hi};
                     }
                 }

@@ -340,6 +340,22 @@ def test_fa_keys_split_over_groups(D, variant, Sq, Skv, causal):
 
 
 @pytest.mark.parametrize("D,variant", SPLIT)
+def test_fa_keys_split_query_alignment(D, variant):
+    """Queries one element past a 16-byte boundary: the same bits as on it."""
+    rng = np.random.default_rng(D)
+    q, k, v = (torch.from_numpy(rng.standard_normal((1, 2, n, D)).astype(np.float16)).to("cuda:0") for n in (128, 256, 256))
+    shifted = torch.empty(q.numel() + 1, dtype=torch.float16, device="cuda:0")
+    shifted[1:] = q.reshape(-1)
+    out = []
+    for pointer in (q.data_ptr(), shifted.data_ptr() + 2):
+        o, lse = torch.full(q.shape, float("nan"), dtype=torch.float16, device="cuda:0"), torch.full(q.shape[:3], float("nan"), device="cuda:0")
+        capi.check(capi.load_st().pto_fa_fwd_f16_variant(torch.cuda.current_stream().cuda_stream, o.data_ptr(), lse.data_ptr(), pointer, k.data_ptr(),
+                                                         v.data_ptr(), 1, 2, 128, 256, D, 0, variant), "pto_fa_fwd_f16_variant")
+        out.append((o, lse))
+    assert torch.equal(out[0][0], out[1][0]) and torch.equal(out[0][1], out[1][1]) and torch.isfinite(out[0][1]).all()
+
+
+@pytest.mark.parametrize("D,variant", SPLIT)
 def test_fa_keys_split_infinite_and_nan_scores(D, variant):
     """Scores of -inf for all that one group sees leave the others' result; a NaN in any group's key reaches every query."""
     rng = np.random.default_rng(D + variant)

@@ -93,6 +93,25 @@ def test_gemm_k_split_tile_shapes_exact(variant, bm, bn):
         assert (got[:256] == -1.0).all() and (got[256 + m * n:] == -1.0).all(), (m, n, k)
 
 
+def test_gemm_k_split_element_alignment():
+    """C one element past a 16-byte boundary, every shape of the k-split kernel and the entry point."""
+    import torch
+    from gpu_util import to_dev
+    m, n, k = 256, 512, 96
+    a, b = datagen.gemm_inputs_integer(m, n, k)
+    want = (a.astype(np.int64) @ b.astype(np.int64).T).astype(np.float32)
+    ta, tb = to_dev(a), to_dev(b)
+    lib = capi.load_st()
+    for variant in range(-1, 9):
+        guarded = torch.full((m * n + 64,), -1.0, dtype=torch.float32, device="cuda:0")
+        args = (0, guarded.data_ptr() + 4, ta.data_ptr(), tb.data_ptr(), m, n, k)
+        capi.check(lib.pto_gemm_f16f32(*args) if variant < 0 else lib.pto_gemm_f16f32_ks_variant(*args, variant), "shape %d" % variant)
+        torch.cuda.synchronize()
+        got = guarded.cpu().numpy()
+        assert np.array_equal(got[1:1 + m * n].reshape(m, n), want), variant
+        assert got[0] == -1.0 and (got[1 + m * n:] == -1.0).all(), variant
+
+
 def test_gemm_ragged_m_and_n_exact():
     """Extents that the tiles do not divide: the last tile row / column is moved back to end with the matrix.  Integer
     operands, every element exact: each width of the four-wave kernel on small shapes (one tile that is also the moved

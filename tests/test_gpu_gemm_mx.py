@@ -347,6 +347,26 @@ def test_mx_gemm_k_split_tile_shapes_exact(oracle, shape, bm, bn, fmt):
         assert rc == 0 and np.array_equal(got16, bf16_rne(got)), (m, n, k)
 
 
+@pytest.mark.parametrize("c_fp32", [True, False])
+def test_mx_gemm_k_split_element_alignment(oracle, c_fp32):
+    """C one element past a 16-byte boundary: every shape of the k-split kernel, nothing written around it."""
+    import torch
+    from gpu_util import to_dev
+    m, n, k = 200, 260, 512
+    a, b, sa, sb = datagen.mx_inputs(m, n, k, 0, dist="integer")
+    want = oracle.mx_gemm(a, b, sa, sb, 0, 0)
+    want = want if c_fp32 else bf16_rne(want).view(np.int16)
+    ta, tb, tsa, tsb = (to_dev(x) for x in (a, b, sa, sb))
+    for shape in range(6):
+        guarded = torch.full((m * n + 64,), -1, dtype=torch.float32 if c_fp32 else torch.int16, device="cuda:0")
+        capi.check(capi.load_st().pto_gemm_mxfp8_variant(0, guarded.data_ptr() + guarded.element_size(), ta.data_ptr(), tb.data_ptr(), tsa.data_ptr(),
+                                                         tsb.data_ptr(), m, n, k, 0, int(c_fp32), 7 + shape), "shape %d" % shape)
+        torch.cuda.synchronize()
+        got = guarded.cpu().numpy()
+        assert np.array_equal(got[1:1 + m * n].reshape(m, n), want), shape
+        assert got[0] == -1 and (got[1 + m * n:] == -1).all(), shape
+
+
 @pytest.mark.parametrize("fmt", [0, 1, 4])
 def test_mx_gemm_k_split_scale_of_every_block(oracle, fmt):
     """Operands of ones, scales drawn per block: C[i, j] = 32 sum_b 2^(sa[i, b] + sb[j, b] - 254) exactly (multiples of 2^-3
