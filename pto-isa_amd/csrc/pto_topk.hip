@@ -22,8 +22,9 @@
 // * topk below the padded row length: once the sorted runs are as long as topk (rounded up to keys per lane times a power of
 //   two), a merge of two runs keeps their larger halves only, in both runs' lanes, and its sort passes no longer cover the
 //   dropped half.
-// * Any other index vector: low word = ~index, keys and columns in LDS, every stage a pass over LDS, four waves on one row
-//   after another; each wave owns a quarter of the row and the stages whose partners lie inside a quarter need no barrier.
+// * Any other index vector: the same network sorts the (index, column) pairs first, once per workgroup (the rows share their
+//   indices); the rank of a column in that order then stands in the scores' keys for the column.  4800 x 1024 whole: 42 us (127
+//   with keys in the LDS and a pass over it per stage); 1000 x 256: 6.6 (15).
 // What bounds it: vector instructions, 2240 per row of 1024 (3850 in the integer network this replaced), behind a phase of
 // loads and before one of stores that all waves share: of 26.4 us (4800 x 1024, top 1000, 58 MB = 9 us at 6.5 TB/s) 12 are
 // launch, loads and stores.  Persistent waves that load the next row while they sort one, and wave priorities that let
@@ -198,7 +199,7 @@ struct RowSort {
         }
         StageEdge();
     }
-    __device__ inline void Sort(int keepBits)
+    __device__ inline __attribute__((always_inline)) void Sort(int keepBits)
     {
         SetForm(Bit(0));
         StageEdge();
@@ -249,38 +250,6 @@ struct RowSort {
     }
 };
 
-// Any index vector: keys and columns in LDS, one pass over LDS per stage.
-template <int N>
-__device__ inline void SortInLds(uint64_t *key, uint16_t *pos, int tid)
-{
-    const int wave = tid / 64, lane = tid % 64;
-    constexpr int kChunk = N / kTopkWaves, kPairsPerWave = kChunk / 2;
-    for (int k = 2; k <= N; k <<= 1)
-        for (int j = k >> 1; j > 0; j >>= 1) {
-            const bool crossWave = j >= kChunk;
-            if (crossWave)
-                __syncthreads();
-            for (int u = lane; u < kPairsPerWave; u += 64) {
-                const int t = wave * kPairsPerWave + u;
-                const int i = ((t & ~(j - 1)) << 1) | (t & (j - 1)), l = i | j;
-                const uint64_t a = key[i], b = key[l];
-                const bool descending = (i & k) == 0;
-                if (descending ? a < b : a > b) {
-                    key[i] = b;
-                    key[l] = a;
-                    const uint16_t pa = pos[i], pb = pos[l];
-                    pos[i] = pb;
-                    pos[l] = pa;
-                }
-            }
-            if (crossWave)
-                __syncthreads();
-            else
-                asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); // this wave's exchanges are done before its next stage reads them
-        }
-    __syncthreads();
-}
-
 // E keys per lane, W waves per row (the row is padded to 64 E W keys; padding keys lie below every real one), 4 / W rows per
 // workgroup.
 template <int E, int W, bool LOW_DPP>
@@ -290,12 +259,15 @@ __global__ __launch_bounds__(kTopkThreads) void TopkRows(float *outScore, uint32
     constexpr int N = 64 * E * W, kRows = kTopkWaves / W;
     constexpr int kStaged = 64 * E + 4 * E; // words of a wave's results, one of padding behind every 16
     constexpr int kStages = E <= 8 ? 2 : 1;  // scores and columns side by side, or one after the other (LDS for four workgroups more)
-    constexpr size_t kFallback = (size_t)N * 10, kExchange = W > 1 ? (size_t)kTopkWaves * E * 64 * 8 : 0, kStage = (size_t)kTopkWaves * kStaged * 4 * kStages;
-    constexpr size_t kLds = kFallback > kExchange ? (kFallback > kStage ? kFallback : kStage) : (kExchange > kStage ? kExchange : kStage);
-    __shared__ __attribute__((aligned(16))) char lds[kLds];
+    // exchanges, then results (or, between two sorts, the ranks of the columns); behind them the columns in the order of their indices
+    constexpr size_t kExchange = W > 1 ? (size_t)kTopkWaves * E * 64 * 8 : 0, kStage = (size_t)kTopkWaves * kStaged * 4 * kStages;
+    constexpr size_t kWork = kExchange > kStage ? kExchange : kStage;
+    static_assert(kWork >= (size_t)N * 2, "the ranks fit");
+    __shared__ __attribute__((aligned(16))) char lds[kWork + (size_t)N * 2];
+    uint16_t *rankOf = reinterpret_cast<uint16_t *>(lds), *columnOf = reinterpret_cast<uint16_t *>(lds + kWork);
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / 64), lane = tid % 64;
     const int waveOfRow = wave % W, row0 = (int)blockIdx.x * kRows, row = row0 + wave / W < rows ? row0 + wave / W : rows - 1;
-    const uint32_t i0 = (uint32_t)(waveOfRow * E * 64 + lane); // this lane's first column; then every 64th
+    uint32_t i0 = (uint32_t)(waveOfRow * E * 64 + lane); // this lane's first column; then every 64th
 
     // A lane past the last column looks at the last one: loads without branches are all in flight at once (16 of them one
     // behind the other were half of the kernel's time)
@@ -311,7 +283,8 @@ __global__ __launch_bounds__(kTopkThreads) void TopkRows(float *outScore, uint32
         }
     };
     uint32_t bits[E], ids[E];
-    load(reinterpret_cast<const uint32_t *>(src) + (size_t)row * (size_t)ld, bits);
+    const uint32_t *scores = reinterpret_cast<const uint32_t *>(src) + (size_t)row * (size_t)ld;
+    load(scores, bits);
     load(inIdx, ids);
 
     // are the indices first, first + 1, ... or at least increasing with the column?  (then the column decides among equal
@@ -326,7 +299,7 @@ __global__ __launch_bounds__(kTopkThreads) void TopkRows(float *outScore, uint32
     auto everyone = [&](bool v) { return W > 1 ? __syncthreads_and(v) != 0 : __builtin_amdgcn_ballot_w64(!v) == 0; };
     const bool consecutive = everyone(wrong == 0 && first <= 0xffffffffu - (uint32_t)validCols);
     bool increasing = consecutive;
-    if (!consecutive) {
+    if (__builtin_expect(!consecutive, 0)) {
         bool ok = true;
         for (int e = 0; e < E; ++e) {
             const int i = (int)i0 + e * 64;
@@ -335,48 +308,52 @@ __global__ __launch_bounds__(kTopkThreads) void TopkRows(float *outScore, uint32
         }
         increasing = everyone(ok);
     }
-    if (!increasing) {
-        uint64_t *key = reinterpret_cast<uint64_t *>(lds);
-        uint16_t *pos = reinterpret_cast<uint16_t *>(lds + (size_t)N * 8);
-        for (int r = row0; r < row0 + kRows && r < rows; ++r) {
-            const float *scores = src + (size_t)r * (size_t)ld;
-            __syncthreads();
-            for (int i = tid; i < N; i += kTopkThreads) {
-                uint64_t kv = 0;
-                if (i < validCols) {
-                    uint32_t b = __float_as_uint(scores[i]);
-                    if (b == kSign)
-                        b = 0; // -0 and +0 compare equal
-                    kv = ((uint64_t)ScoreOrder(b) << 32) | (uint32_t)~inIdx[i];
-                }
-                key[i] = kv;
-                pos[i] = (uint16_t)i;
-            }
-            __syncthreads();
-            SortInLds<N>(key, pos, tid);
-            for (int i = tid; i < topk; i += kTopkThreads) {
-                const int p = pos[i];
-                outScore[(size_t)r * (size_t)topk + i] = scores[p];
-                outIndex[(size_t)r * (size_t)topk + i] = inIdx[p];
-            }
-        }
-        return;
-    }
-
     RowSort<E, W, LOW_DPP> s;
     s.q = (uint32_t)waveOfRow * 64u + LaneRank((uint32_t)lane);
     s.xchg = reinterpret_cast<uint64_t *>(lds);
-    const uint32_t columnBits = (4095u - i0) << 8;
     // the ranks of a wave go in order through its piece of LDS, so that its stores cover consecutive addresses
     uint32_t *staged = reinterpret_cast<uint32_t *>(lds) + wave * (kStaged * kStages), *stagedColumn = staged + (kStages - 1) * kStaged;
     const int firstRank = waveOfRow * 64 * E, laneRank = (int)LaneRank((uint32_t)lane) * E, count = topk - firstRank;
     auto ordered = [] { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); __builtin_amdgcn_wave_barrier(); };
+    const uint32_t columnBits = (4095u - i0) << 8;
+    if (__builtin_expect(!increasing, 0)) { // the columns in the order of their indices; rows of one wave: the first wave does it for all four
+        if (W > 1 || wave == 0) {
+            s.form = 0;
+#pragma unroll
+            for (int e = 0; e < E; ++e) {
+                const uint32_t order = ~ids[e];
+                s.k[e] = Key(__builtin_amdgcn_alignbit(0x3ffu, order, 12), (order << 20) | (columnBits - (uint32_t)(e * 64 << 8)));
+                if (i0 + e * 64 >= (uint32_t)validCols)
+                    s.k[e] = 1.0;
+            }
+            s.Sort(31);
+            asm volatile("" : "+v"(i0), "+v"(s.q)); // (nothing that depends on them is kept in registers across the sort)
+            if (W > 1)
+                __syncthreads(); // (the exchanges are over)
+#pragma unroll
+            for (int e = 0; e < E; ++e) {
+                const uint32_t rank = s.q * E + e, column = 4095u - ((Low(s.k[e]) >> 8) & 0xfffu);
+                if (wave < W && rank < (uint32_t)validCols) {
+                    rankOf[column] = (uint16_t)rank;
+                    columnOf[rank] = (uint16_t)column;
+                }
+            }
+        }
+        load(scores, bits);
+    }
     s.form = 0;
 #pragma unroll
     for (int e = 0; e < E; ++e) {
         const bool negZero = bits[e] == kSign; // compares equal to +0: same key, remembered below the column bits
         const uint32_t order = ScoreOrder(negZero ? 0u : bits[e]);
         s.k[e] = Key(__builtin_amdgcn_alignbit(0x3ffu, order, 12), (order << 20) | (columnBits - (uint32_t)(e * 64 << 8) + (negZero ? 1u : 0u)));
+    }
+    if (__builtin_expect(!increasing, 0)) {
+        __syncthreads(); // the ranks are there
+#pragma unroll
+        for (int e = 0; e < E; ++e)
+            s.k[e] = Key(High(s.k[e]), (Low(s.k[e]) & 0xfff000ffu) | (4095u - rankOf[i0 + e * 64]) << 8); // (past the row's end: overwritten below)
+        __syncthreads(); // and read, before their memory is used for something else
     }
     if (validCols != N) {
 #pragma unroll
@@ -415,13 +392,22 @@ __global__ __launch_bounds__(kTopkThreads) void TopkRows(float *outScore, uint32
             stagedColumn[laneRank + e + (laneRank + e) / 16] = column[e];
         ordered();
     }
+    if (__builtin_expect(!consecutive, 0)) { // (staged: the column, or its rank)
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+            const int i = e * 64 + lane;
+            if (i < count) {
+                const uint32_t c = stagedColumn[i + i / 16];
+                toIndex[i] = inIdx[increasing ? c : columnOf[c]];
+            }
+        }
+        return;
+    }
 #pragma unroll
     for (int e = 0; e < E; ++e) {
         const int i = e * 64 + lane;
-        if (i < count) {
-            const uint32_t c = stagedColumn[i + i / 16];
-            toIndex[i] = consecutive ? first + c : inIdx[c];
-        }
+        if (i < count)
+            toIndex[i] = first + stagedColumn[i + i / 16];
     }
 }
 

@@ -51,3 +51,20 @@ def test_mx_gemm_choice_against_four_waves(m, n, k, fmt, c_fp32, variant):
     public, four = best_us([lambda: capi.check(lib.pto_gemm_mxfp8_variant(*args, 4), "as the entry points choose"),
                             lambda: capi.check(lib.pto_gemm_mxfp8_variant(*args, variant), "256 x 192")], launches=5)
     assert public <= 1.035 * four, (public, four)
+
+
+@pytest.mark.parametrize("rows,cols", [(128, 256), (1000, 256), (1000, 512), (4800, 1024)])
+def test_topk_index_order(rows, cols):
+    """An index vector in any order costs one more sort of a row, not one for each, nor passes over the LDS (3 to 9 times)."""
+    lib = capi.load()
+    src = torch.randn((rows, cols), device="cuda:0")
+    ids = torch.arange(cols, dtype=torch.int32, device="cuda:0")
+    mixed = torch.randperm(cols, device="cuda:0").to(torch.int32)
+    score, index = torch.empty((rows, cols), device="cuda:0"), torch.empty((rows, cols), dtype=torch.int32, device="cuda:0")
+    stream = torch.cuda.current_stream().cuda_stream
+
+    def call(which):
+        return lambda: capi.check(lib.pto_topk_f32(stream, score.data_ptr(), index.data_ptr(), src.data_ptr(), which.data_ptr(), rows, cols, cols, cols),
+                                  "pto_topk_f32")
+    increasing, any_order = best_us([call(ids), call(mixed)])
+    assert any_order <= 2.5 * increasing, (any_order, increasing)

@@ -85,6 +85,24 @@ def test_topk_waves_per_row(oracle, rows, cols, k):
         assert same(topk_gpu(src, ids, cols, k), oracle.topk_f32(src, ids, cols, k))
 
 
+@pytest.mark.parametrize("rows,cols", [(300, 60), (501, 128), (1000, 250), (130, 512), (800, 500), (500, 1000), (1001, 1024), (2700, 1000), (500, 1900), (1800, 2048),
+                                       (150, 4096)])
+def test_topk_index_vectors_in_any_order(oracle, rows, cols):
+    """Many rows under a permutation, a descending vector, one with repeated values and one that holds both ends of the range and
+    its middle (as signed and as unsigned numbers), every number of waves per row; few distinct scores, signed zeros."""
+    r = np.random.Generator(np.random.Philox(key=rows))
+    src, idx = datagen.topk_inputs(rows, cols, cols + 1, distinct=9)
+    mixed = r.permutation(1 << 16)[:cols].astype(np.uint32)
+    mixed[:5] = (0xFFFFFFFF, 0x80000000, 0, 0x7FFFFFFF, 0x80000001)
+    for ids in (r.permutation(cols).astype(np.uint32), idx[::-1] + np.uint32(0xFFFF0000), mixed):
+        src[::7, ::5], src[::7, 1::5] = -0.0, 0.0
+        for k in (cols, max(1, cols // 9)):
+            assert same(topk_gpu(src, ids, cols, k), oracle.topk_f32(src, ids, cols, k)), k
+    src[src == 0] = 1.5                                                  # (equal pairs would differ in the zeros' signs alone)
+    ids = (idx // np.uint32(3)).astype(np.uint32)[r.permutation(cols)]
+    assert same(topk_gpu(src, ids, cols, cols), oracle.topk_f32(src, ids, cols, cols))
+
+
 @pytest.mark.parametrize("rows,cols", [(4096, 60), (4097, 60), (4097, 120), (4096, 200), (4097, 200), (731, 500), (732, 500), (2048, 500),
                                        (2049, 500), (4097, 500), (853, 1000), (854, 1000), (1706, 1900), (1707, 1900)])
 def test_topk_lane_moves(oracle, rows, cols):
