@@ -199,6 +199,8 @@ struct RowSort {
         }
         StageEdge();
     }
+    // MOST: the largest keepBits there is; kLaneBits for a whole sort, whose code then holds no branch
+    template <int MOST>
     __device__ inline __attribute__((always_inline)) void Sort(int keepBits)
     {
         SetForm(Bit(0));
@@ -207,42 +209,23 @@ struct RowSort {
         StageEdge();
         // (straight-line code: one copy for all runs branches around its stages, 8 to 15 % of the time at 8 and 16 keys per lane
         // where topk is small, 2 to 6 % of a whole sort)
-        StaticFor<1, kLaneBits + 1>([&](auto run) { Merge(decltype(run)::value, keepBits); });
+        StaticFor<1, kLaneBits + 1>([&](auto run) { Merge<decltype(run)::value, MOST>(MOST == kLaneBits ? kLaneBits : keepBits); });
     }
-    // runs of E << run keys out of two of half the length, descending and ascending in turn (the last: descending)
-    __device__ inline __attribute__((always_inline)) void Merge(int run, int keepBits)
+    // runs of E << RUN keys out of two of half the length, descending and ascending in turn (the last: descending)
+    template <int RUN, int MOST>
+    __device__ inline __attribute__((always_inline)) void Merge(int keepBits)
     {
-        const uint32_t dir = run == kLaneBits ? 0u : Bit(run);
-        int strides = run;
-        if (run > keepBits) {
+        const uint32_t dir = RUN == kLaneBits ? 0u : Bit(RUN);
+        int strides = RUN;
+        if (RUN > MOST || RUN > keepBits) {
             strides = keepBits;
-            switch (run - 1) {
-            case 0: Stage<0, true>(dir); break;
-            case 1: Stage<1, true>(dir); break;
-            case 2: Stage<2, true>(dir); break;
-            case 3: Stage<3, true>(dir); break;
-            case 4: Stage<4, true>(dir); break;
-            case 5: Stage<5, true>(dir); break;
-            case 6: Stage<6, true>(dir); break;
-            default: Stage<7, true>(dir); break;
-            }
+            Stage<RUN - 1, true>(dir);
         }
-        if (W > 2 && strides > 7)
-            Stage<7, false>(dir);
-        if (W > 1 && strides > 6)
-            Stage<6, false>(dir);
-        if (strides > 5)
-            Stage<5, false>(dir);
-        if (strides > 4)
-            Stage<4, false>(dir);
-        if (strides > 3)
-            Stage<3, false>(dir);
-        if (strides > 2)
-            Stage<2, false>(dir);
-        if (strides > 1)
-            Stage<1, false>(dir);
-        if (strides > 0)
-            Stage<0, false>(dir);
+        StaticFor<0, RUN>([&](auto below) {
+            constexpr int j = RUN - 1 - decltype(below)::value;
+            if (j < MOST && strides > j)
+                Stage<j, false>(dir);
+        });
         SetForm(dir);
         StageEdge();
         MergeLane();
@@ -251,12 +234,18 @@ struct RowSort {
 };
 
 // E keys per lane, W waves per row (the row is padded to 64 E W keys; padding keys lie below every real one), 4 / W rows per
-// workgroup.
-template <int E, int W, bool LOW_DPP>
+// workgroup.  WHOLE: a whole sort, otherwise keepBits is below the row's by more than kWholeBits.  Where more than an eighth of
+// the row is wanted the merges save less than their branches cost (cut to keepBits / whole sort: 1024 columns, 600 rows, top 256
+// 7.4 / 7.2 us, 4800 rows 21.6 / 21.6; 128 x 256, top 64 3.7 / 3.3, top 256 4.0 / 3.6; 4800 x 1024, top 1024 26.0 / 25.5).
+constexpr int kWholeBits = 2;
+// one key per lane and four waves per row: for few rows of which more than 16 are wanted, where the whole sort is the shorter one
+template <int E, int W>
+constexpr bool kOnlyWhole = E == 1 && W == 4;
+template <int E, int W, bool LOW_DPP, bool WHOLE>
 __global__ __launch_bounds__(kTopkThreads) void TopkRows(float *outScore, uint32_t *outIndex, const float *src, const uint32_t *inIdx,
                                                          int rows, int validCols, int ld, int topk, int keepBits)
 {
-    constexpr int N = 64 * E * W, kRows = kTopkWaves / W;
+    constexpr int N = 64 * E * W, kRows = kTopkWaves / W, kBits = RowSort<E, W, LOW_DPP>::kLaneBits;
     constexpr int kStaged = 64 * E + 4 * E; // words of a wave's results, one of padding behind every 16
     constexpr int kStages = E <= 8 ? 2 : 1;  // scores and columns side by side, or one after the other (LDS for four workgroups more)
     // exchanges, then results (or, between two sorts, the ranks of the columns); behind them the columns in the order of their indices
@@ -270,9 +259,11 @@ __global__ __launch_bounds__(kTopkThreads) void TopkRows(float *outScore, uint32
     uint32_t i0 = (uint32_t)(waveOfRow * E * 64 + lane); // this lane's first column; then every 64th
 
     // A lane past the last column looks at the last one: loads without branches are all in flight at once (16 of them one
-    // behind the other were half of the kernel's time)
+    // behind the other were half of the kernel's time).  Up to four keys and few waves: always so, the branch around
+    // it takes longer (1 x 200, top 16: 3.29 / 3.18 us; with many waves 8192 x 256, top 8: 6.4 / 6.7)
+    constexpr bool kClamp = E <= 4 && LOW_DPP;
     auto load = [&](const uint32_t *from, uint32_t (&to)[E]) __attribute__((always_inline)) {
-        if (validCols == N) {
+        if (!kClamp && validCols == N) {
 #pragma unroll
             for (int e = 0; e < E; ++e)
                 to[e] = from[i0 + e * 64];
@@ -326,7 +317,7 @@ __global__ __launch_bounds__(kTopkThreads) void TopkRows(float *outScore, uint32
                 if (i0 + e * 64 >= (uint32_t)validCols)
                     s.k[e] = 1.0;
             }
-            s.Sort(31);
+            s.template Sort<kBits>(kBits);
             asm volatile("" : "+v"(i0), "+v"(s.q)); // (nothing that depends on them is kept in registers across the sort)
             if (W > 1)
                 __syncthreads(); // (the exchanges are over)
@@ -355,13 +346,13 @@ __global__ __launch_bounds__(kTopkThreads) void TopkRows(float *outScore, uint32
             s.k[e] = Key(High(s.k[e]), (Low(s.k[e]) & 0xfff000ffu) | (4095u - rankOf[i0 + e * 64]) << 8); // (past the row's end: overwritten below)
         __syncthreads(); // and read, before their memory is used for something else
     }
-    if (validCols != N) {
+    if (kClamp || validCols != N) {
 #pragma unroll
         for (int e = 0; e < E; ++e)
             if (i0 + e * 64 >= (uint32_t)validCols)
                 s.k[e] = 1.0;
     }
-    s.Sort(keepBits);
+    s.template Sort<WHOLE ? kBits : kBits - kWholeBits - 1>(keepBits);
 
     if (W > 1)
         __syncthreads(); // (the exchanges are over)
@@ -411,6 +402,27 @@ __global__ __launch_bounds__(kTopkThreads) void TopkRows(float *outScore, uint32
     }
 }
 
+template <int E, int W>
+int launch_topk(hipStream_t st, float *out_score, uint32_t *out_index, const float *src, const uint32_t *in_idx, int rows, int valid_cols, int ld,
+                int topk)
+{
+    int keepBits = 0;
+    while ((E << keepBits) < topk)
+        ++keepBits;
+    const bool whole = kOnlyWhole<E, W> || keepBits + kWholeBits >= RowSort<E, W, true>::kLaneBits;
+    // Lower words between near lanes: with up to four waves on a SIMD the latency of the LDS pipe shows, a DPP move is shorter
+    // (LDS / DPP, whole sorts: 300 x 128 3.48 / 3.26 us, 300 x 256 4.53 / 4.28); with more the moves take issue slots (4800 x 128
+    // 5.09 / 5.23).  8 and 16 keys per lane cover the latency either way and take DPP.
+    const bool dpp = E >= 8 || (long long)rows * W <= 4 * 4 * 256;
+    constexpr bool kCut = kOnlyWhole<E, W>, kDpp = E >= 8 || kOnlyWhole<E, W>; // (names the one form that there is)
+    auto kernel = dpp ? (whole ? TopkRows<E, W, true, true> : TopkRows<E, W, true, kCut>) :
+                        (whole ? TopkRows<E, W, kDpp, true> : TopkRows<E, W, kDpp, kCut>);
+    constexpr int kRows = kTopkWaves / W;
+    kernel<<<dim3((unsigned)(((long long)rows + kRows - 1) / kRows)), dim3(kTopkThreads), 0, st>>>(out_score, out_index, src, in_idx, rows, valid_cols,
+                                                                                                   ld, topk, keepBits);
+    return pto_amd::check_launch();
+}
+
 } // namespace
 
 extern "C" int pto_topk_f32(void *stream, float *out_score, uint32_t *out_index, const float *src, const uint32_t *in_idx, int rows,
@@ -427,29 +439,17 @@ extern "C" int pto_topk_f32(void *stream, float *out_score, uint32_t *out_index,
     // four up to 731 rows (600 rows 6.5 / 6.4 / 5.9, 1000 rows 6.8 / 7.0 / 7.2), then one.  2048 columns: four up to 1706 rows (1700
     // rows with two 27.2, with four 25.7; 2400 rows 32.4, 33.0).  Rows of up to 256: one, the exchanges across waves cost more
     // than they save (1000 rows 4.6 / 4.6 / 5.0).
-    // Lower words between near lanes: with up to four waves on a SIMD the latency of the LDS pipe shows, a DPP move is shorter
-    // (LDS / DPP, whole sorts: 300 x 128 3.48 / 3.26 us, 300 x 256 4.53 / 4.28); with more the moves take issue slots (4800 x 128
-    // 5.09 / 5.23).  8 and 16 keys per lane cover the latency either way and take DPP.
     const int most = 5 * 4 * 256 / rows;
-#define PTO_TOPK_CASE(E, W)                                                                                              \
-    {                                                                                                                    \
-        int keepBits = 0;                                                                                                \
-        while ((E << keepBits) < topk)                                                                                   \
-            ++keepBits;                                                                                                  \
-        constexpr int kRows = kTopkWaves / W;                                                                            \
-        const dim3 grid((unsigned)(((long long)rows + kRows - 1) / kRows)), block(kTopkThreads);                         \
-        if (E >= 8 || (long long)rows * W <= 4 * 4 * 256)                                                               \
-            TopkRows<E, W, true><<<grid, block, 0, st>>>(out_score, out_index, src, in_idx, rows, valid_cols, ld, topk, keepBits); \
-        else                                                                                                             \
-            TopkRows<E, W, (E >= 8)><<<grid, block, 0, st>>>(out_score, out_index, src, in_idx, rows, valid_cols, ld, topk, keepBits); \
-        return pto_amd::check_launch();                                                                                  \
-    }
+#define PTO_TOPK_CASE(E, W) return launch_topk<E, W>(st, out_score, out_index, src, in_idx, rows, valid_cols, ld, topk);
     if (valid_cols <= 64)
         PTO_TOPK_CASE(1, 1)
     if (valid_cols <= 128)
         PTO_TOPK_CASE(2, 1)
-    if (valid_cols <= 256)
+    if (valid_cols <= 256) {
+        if (most >= 14 && topk > 16)
+            PTO_TOPK_CASE(1, 4)
         PTO_TOPK_CASE(4, 1)
+    }
     if (valid_cols <= 512) {
         if (most >= 7)
             PTO_TOPK_CASE(2, 4)

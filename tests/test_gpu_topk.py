@@ -85,6 +85,22 @@ def test_topk_waves_per_row(oracle, rows, cols, k):
         assert same(topk_gpu(src, ids, cols, k), oracle.topk_f32(src, ids, cols, k))
 
 
+@pytest.mark.parametrize("rows", [1, 365, 366])
+@pytest.mark.parametrize("cols", [60, 129, 256, 500, 1000, 2000, 4000])
+def test_topk_whole_and_cut_sorts(oracle, rows, cols):
+    """topk on both sides of 16 (256 columns in four waves) and of an eighth of the padded row (whole sorts), rows on both sides
+    of where 256 columns change their waves; indices in order and in any order."""
+    if rows * cols > 1 << 20:
+        rows = rows // 366 * 128 + 1
+    r = np.random.Generator(np.random.Philox(key=rows + cols))
+    src, idx = datagen.topk_inputs(rows, cols, cols + 3, distinct=200)
+    src[0, ::7] = -0.0
+    eighth = max(64, 1 << (cols - 1).bit_length()) // 8
+    for k in sorted({k for k in (16, 17, eighth, eighth + 1, cols) if k <= cols}):
+        for ids in (idx, r.permutation(cols).astype(np.uint32)):
+            assert same(topk_gpu(src, ids, cols, k), oracle.topk_f32(src, ids, cols, k)), k
+
+
 @pytest.mark.parametrize("rows,cols", [(300, 60), (501, 128), (1000, 250), (130, 512), (800, 500), (500, 1000), (1001, 1024), (2700, 1000), (500, 1900), (1800, 2048),
                                        (150, 4096)])
 def test_topk_index_vectors_in_any_order(oracle, rows, cols):
