@@ -20,6 +20,18 @@ inline int check_launch()
     return PTO_OK;
 }
 
+// compute units of the device that is current at the first call
+inline int compute_units()
+{
+    static const int cus = [] {
+        int dev = 0, n = 0;
+        if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0)
+            n = 256;
+        return n;
+    }();
+    return cus;
+}
+
 // Dynamic LDS above 64 KiB has to be opted into per kernel.
 template <typename K>
 inline int allow_lds(K kernel, int bytes)

@@ -164,18 +164,3 @@ int launch_gemm(hipStream_t st, float *c, const half *a, const half *b, int m, i
     return pto_amd::check_launch();
 }
 } // namespace
-
-namespace {
-// compute units of the device that is current at the first call
-inline int compute_units()
-{
-    static const int cus = [] {
-        int dev = 0, n = 0;
-        if (hipGetDevice(&dev) != hipSuccess ||
-            hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0)
-            n = 256;
-        return n;
-    }();
-    return cus;
-}
-} // namespace

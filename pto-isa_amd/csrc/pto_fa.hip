@@ -102,12 +102,7 @@ extern "C" int pto_fa_fwd_f16(void *stream, void *o, float *lse, const uint16_t 
     hipStream_t st = static_cast<hipStream_t>(stream);
     const half *hq = reinterpret_cast<const half *>(q), *hk = reinterpret_cast<const half *>(k),
                *hv = reinterpret_cast<const half *>(v);
-    static const int cus = [] {
-        int dev = 0, n = 0;
-        if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0)
-            n = 256;
-        return n;
-    }();
+    const int cus = pto_amd::compute_units();
     // At most one 128-query workgroup of four waves per compute unit: every SIMD has one wave or none, and the launch takes as
     // long as that wave needs for all keys of its queries.  The keys are split over groups of waves (FlashAttnFwd, G > 1) where
     // there are enough of them to pay for joining the groups.  With 64-query workgroups one per compute unit (us, 128 of 128

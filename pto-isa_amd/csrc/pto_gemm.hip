@@ -81,7 +81,7 @@ extern "C" int pto_gemm_f16f32(void *stream, float *c, const uint16_t *a, const 
         return PTO_ERR_UNSUPPORTED;
     hipStream_t st = static_cast<hipStream_t>(stream);
     const half *ha = reinterpret_cast<const half *>(a), *hb = reinterpret_cast<const half *>(b);
-    const int cus = compute_units();
+    const int cus = pto_amd::compute_units();
     const TileShape *best = nullptr;
     double bestTime = 0.0;
     for (const TileShape &s : kShapes) {

@@ -303,7 +303,7 @@ int launch_gemm_mx(hipStream_t st, void *c, const uint8_t *a, const uint8_t *b, 
     static const int attr = pto_amd::allow_lds(kernel, lds);
     if (attr != PTO_OK)
         return attr;
-    const int tiles = ((m + BM - 1) / BM) * ((n + BN - 1) / BN), cus = compute_units();
+    const int tiles = ((m + BM - 1) / BM) * ((n + BN - 1) / BN), cus = pto_amd::compute_units();
     int full = tiles / cus * cus;
     // quarter tiles move twice the operand bytes per flop: only when they fit one round
     if (tailMode == 0 || full == 0 || (tiles - full) * 4 > cus || m % BM || n % BN)
@@ -396,7 +396,7 @@ int gemm_mx_any(hipStream_t st, void *c, const uint8_t *a, const uint8_t *b, con
     const bool block = m >= 256 && n >= 256 && k % 512 == 0, w4 = m >= 256 && n >= 128 && n % 4 == 0 && k % (fp4 ? 1024 : 512) == 0;
     if (!block && !w4)
         return PTO_ERR_UNSUPPORTED;
-    const int cus = compute_units(), steps = k / (fp4 ? 256 : 128);
+    const int cus = pto_amd::compute_units(), steps = k / (fp4 ? 256 : 128);
     const MxShape *best = nullptr;
     double bestTime = 0.0;
     for (const MxShape &s : kMxShapes[fp4]) {

@@ -413,7 +413,7 @@ int launch_topk(hipStream_t st, float *out_score, uint32_t *out_index, const flo
     // Lower words between near lanes: with up to four waves on a SIMD the latency of the LDS pipe shows, a DPP move is shorter
     // (LDS / DPP, whole sorts: 300 x 128 3.48 / 3.26 us, 300 x 256 4.53 / 4.28); with more the moves take issue slots (4800 x 128
     // 5.09 / 5.23).  8 and 16 keys per lane cover the latency either way and take DPP.
-    const bool dpp = E >= 8 || (long long)rows * W <= 4 * 4 * 256;
+    const bool dpp = E >= 8 || (long long)rows * W <= 4 * 4 * pto_amd::compute_units();
     constexpr bool kCut = kOnlyWhole<E, W>, kDpp = E >= 8 || kOnlyWhole<E, W>; // (names the one form that there is)
     auto kernel = dpp ? (whole ? TopkRows<E, W, true, true> : TopkRows<E, W, true, kCut>) :
                         (whole ? TopkRows<E, W, kDpp, true> : TopkRows<E, W, kDpp, kCut>);
@@ -434,12 +434,12 @@ extern "C" int pto_topk_f32(void *stream, float *out_score, uint32_t *out_index,
         return PTO_ERR_UNSUPPORTED;
     hipStream_t st = static_cast<hipStream_t>(stream);
     // Waves per row.  One wave per row does the least work, more put more of the chip to work on few rows (one / two / four waves,
-    // whole sorts: 1024 columns, 600 rows 11.2 / 9.7 / 8.8 us, 1000 rows 11.6 / 10.2 / 10.2, 2400 rows 18.8 / 17.2 / 18.6, 4800
-    // rows 26.5 / 28.3; 1000 rows top 256 9.1 / 8.6 / 9.0): at 1024 columns four up to 853 rows, two up to 2560.  512 columns:
-    // four up to 731 rows (600 rows 6.5 / 6.4 / 5.9, 1000 rows 6.8 / 7.0 / 7.2), then one.  2048 columns: four up to 1706 rows (1700
-    // rows with two 27.2, with four 25.7; 2400 rows 32.4, 33.0).  Rows of up to 256: one, the exchanges across waves cost more
-    // than they save (1000 rows 4.6 / 4.6 / 5.0).
-    const int most = 5 * 4 * 256 / rows;
+    // whole sorts: 1024 columns, 600 rows 9.8 / 8.8 / 7.7 us, 1000 rows 10.3 / 9.3 / 9.2, 2400 rows 17.5 / 16.2 / 17.9, 4800
+    // rows 25.3 / 26.9 / 28.8; 1000 rows top 256 8.7 / 8.1 / 8.2): on 256 units four up to 853 rows, two up to 2560.  512 columns:
+    // four up to 731 rows (600 rows 5.7 / 5.4 / 5.1, 853 rows 5.8 / 5.5 / 5.6, top 15 4.5 / 4.6 / 5.1), then one.  2048 columns: four
+    // up to 1706 rows (1700 rows with two 25.6, with four 24.5; 2000 rows 26.2, 26.9).  129 to 256 columns: four up to 365 rows where
+    // more than 16 are wanted (one / four: 128 rows 3.6 / 3.3, 300 rows 3.6 / 3.4, 600 rows 3.7 / 3.7; top 7 of 128 rows 3.2 / 3.6).
+    const int most = 5 * 4 * pto_amd::compute_units() / rows; // waves per row for five on every SIMD
 #define PTO_TOPK_CASE(E, W) return launch_topk<E, W>(st, out_score, out_index, src, in_idx, rows, valid_cols, ld, topk);
     if (valid_cols <= 64)
         PTO_TOPK_CASE(1, 1)
