@@ -147,7 +147,7 @@ struct VTReader {
 template <int D, bool CAUSAL, bool OUT_F32, int MIN_BLOCKS, int kBKV = kBKVDefault, bool PP = false, int NQ_ = 1, int G = 1>
 __global__ __launch_bounds__(kBlockThreads, MIN_BLOCKS) AICORE void FlashAttnFwd(__gm__ void *outO, __gm__ float *outLse,
                                                                       __gm__ const half *qAll, __gm__ const half *kAll,
-                                                                      __gm__ const half *vAll, int heads, int seqQ,
+                                                                      __gm__ const half *vAll, [[maybe_unused]] int perXcd, int seqQ,
                                                                       int seqKv, int numBH, int causalOff)
 {
     constexpr int NQ = NQ_;        // 32-query blocks per wave
@@ -183,10 +183,19 @@ __global__ __launch_bounds__(kBlockThreads, MIN_BLOCKS) AICORE void FlashAttnFwd
     int bh, qt;
     {
         const int bid = (int)get_block_idx();
-        if (numBH % 8 == 0) {
-            const int xcd = bid % 8, slot = bid / 8, perXcd = numBH / 8;
-            bh = xcd + 8 * (slot % perXcd);
-            qt = slot / perXcd;
+        if constexpr (G > 1) { // one division; perXcd heads on an XCD, 0: not dealt so
+            const unsigned x = perXcd ? (unsigned)bid / 8u : (unsigned)bid, n = (unsigned)(perXcd ? perXcd : numBH);
+            qt = (int)(x / n);
+            bh = (int)(x - (unsigned)qt * n);
+            if (perXcd) {
+                bh = bid % 8 + 8 * bh;
+                if (bh >= numBH) // the launch has workgroups for a whole number of heads per XCD
+                    return;
+            }
+        } else if (numBH % 8 == 0) {
+            const int xcd = bid % 8, slot = bid / 8, share = numBH / 8;
+            bh = xcd + 8 * (slot % share);
+            qt = slot / share;
         } else {
             bh = bid % numBH;
             qt = bid / numBH;
@@ -738,10 +747,21 @@ int launch_fa(hipStream_t st, void *o, float *lse, const half *q, const half *k,
     if (attr != PTO_OK)
         return attr;
     const int numBH = batch * heads;
-    const long long blocks = (long long)numBH * (seqQ / kBQ);
+    long long blocks = (long long)numBH * (seqQ / kBQ);
     if (blocks > 0x7fffffffLL)
         return PTO_ERR_UNSUPPORTED;
-    kernel<<<dim3((unsigned)blocks), dim3(kBlockThreads), lds, st>>>(o, lse, q, k, v, heads, seqQ, seqKv, numBH, causalOff);
+    // Key groups: one XCD reads the keys of a head, also where 8 does not divide the heads; the launch then has workgroups for
+    // heads that are not there, if all run at once (100 heads x 128 x 448 x 128: 12.5 us with a head's two workgroups on different
+    // XCDs, 10.1 so)
+    int perXcd = 0;
+    if (G > 1) {
+        const long long padded = (numBH + 7ll) / 8 * 8 * (seqQ / kBQ);
+        if (numBH % 8 == 0 || padded <= (long long)MIN_BLOCKS * pto_amd::compute_units()) {
+            perXcd = (numBH + 7) / 8;
+            blocks = padded;
+        }
+    }
+    kernel<<<dim3((unsigned)blocks), dim3(kBlockThreads), lds, st>>>(o, lse, q, k, v, perXcd, seqQ, seqKv, numBH, causalOff);
     return pto_amd::check_launch();
 }
 } // namespace

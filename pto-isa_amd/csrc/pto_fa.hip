@@ -114,13 +114,16 @@ extern "C" int pto_fa_fwd_f16(void *stream, void *o, float *lse, const uint16_t 
     //   head_dim 128, keys 512: 13.3 / 13.5   1024: 21.3 / 19.8   4096: 71.7 / 60.9;   64, 512: 8.7 / 8.8   1024: 13.7 / 13.0   4096: 45.2 / 38.3
     // and at head_dim 64 with a mask that hides a good part of the keys (up to two keys per query), where the 64-query
     // workgroups even out: 256: 6.8 / 6.0 (two groups of two), 1024: 15.2 / 10.4, 2048: 26.5 / 19.2.
+    // Nearly one workgroup per compute unit and one to a head at head_dim 128: K and V come from memory once and bound the launch, from
+    // 2048 keys (256 heads x 128 queries, four waves / split, keys 1024: 24.9 / 27.8   1536: 34.5 / 36.6   2048: 53.4 / 47.2).
     const long long blocks = (long long)batch * heads * (seq_q / 128);
+    const bool fromMemory = head_dim == 128 && seq_q == 128 && blocks * 8 > cus * 7ll;
     const int keys = causal && seq_q < seq_kv - causalOff ? seq_q + causalOff : seq_kv; // that the last query sees
     int groups = 0; // 1: two groups of two waves
     if (blocks * 2 <= cus)
         groups = keys >= (head_dim == 128 ? 256 : 1024) ? 4 : head_dim == 64 ? 1 : 0;
     else if (blocks <= cus)
-        groups = head_dim == 64 && causal && keys >= 256 && keys / 2 <= seq_q ? 1 : keys >= 1024 ? 2 : 0;
+        groups = head_dim == 64 && causal && keys >= 256 && keys / 2 <= seq_q ? 1 : keys >= (fromMemory ? 2048 : 1024) ? 2 : 0;
     if (groups == 1)
         return launch_split_w4(st, o, lse, hq, hk, hv, batch, heads, seq_q, seq_kv, causal != 0, o_fp32 != 0, causalOff);
     if (groups > 1)

@@ -394,3 +394,24 @@ def test_fa_few_query_blocks(B, H, Sq, Skv, D, causal, o_fp32):
             want, want_lse = dense_fp64(q[b, h], k[b, h], v[b, h], causal != 0)
         assert rel(o[b, h], want) <= TOL, (b, h)
         assert np.max(np.abs(lse[b, h] - want_lse)) <= 1e-4, (b, h)
+
+
+@pytest.mark.parametrize("B,H,Sq,Skv,D,causal", [(1, 9, 128, 448, 128, 0), (3, 17, 256, 320, 64, 1), (1, 100, 128, 448, 128, 1), (1, 51, 512, 1024, 64, 1),
+                                                  (1, 180, 128, 1024, 128, 0), (1, 3, 512, 2048, 128, 1), (1, 230, 128, 1024, 128, 0)])
+def test_fa_heads_that_eight_does_not_divide(B, H, Sq, Skv, D, causal):
+    """The same heads alone and as part of a multiple of eight of them: the same bits in every head, nothing behind the last."""
+    rng = np.random.default_rng(H)
+    more = (B * H + 7) // 8 * 8
+    q, k, v = (torch.from_numpy(rng.standard_normal((1, more, n, D)).astype(np.float16)).to("cuda:0") for n in (Sq, Skv, Skv))
+    out = []
+    for batch, heads in ((B, H), (1, more)):
+        o, lse = torch.full((1, more, Sq, D), 7.0, dtype=torch.float16, device="cuda:0"), torch.full((1, more, Sq), 7.0, device="cuda:0")
+        capi.check(capi.load().pto_fa_fwd_f16(torch.cuda.current_stream().cuda_stream, o.data_ptr(), lse.data_ptr(), q.data_ptr(), k.data_ptr(),
+                                              v.data_ptr(), batch, heads, Sq, Skv, D, causal, 0), "pto_fa_fwd_f16")
+        out.append((o, lse))
+    n = B * H
+    for alone, among in zip(*out):
+        assert torch.equal(alone[:, :n], among[:, :n]) and (alone[:, n:] == 7.0).all()
+    want, want_lse = dense_fp64(q[0, n - 1].cpu().numpy(), k[0, n - 1].cpu().numpy(), v[0, n - 1].cpu().numpy(), causal != 0)
+    assert rel(out[0][0][0, n - 1].float().cpu().numpy(), want) <= TOL
+    assert np.max(np.abs(out[0][1][0, n - 1].cpu().numpy() - want_lse)) <= 1e-4
