@@ -118,14 +118,16 @@ __global__ __launch_bounds__(kBlockThreads) void CvtF32Stream(D *dst, const floa
 // a multiplication: for c < 2^31, c / cpr = c magic >> shift with magic = ceil(2^shift / cpr), shift = 31 + ceil(log2 cpr).
 // Table and output need their elements' alignment only (the chunks are typed so; the same instructions).
 // The row is cut into `parts` (1, 2, 4 or 8) slices of cpr chunks, and workgroup b works on slice (b % 8) % parts: as the
-// workgroups are dealt to the eight XCDs in turn, an XCD's L2 then sees one slice of the table only.
+// workgroups are dealt to the eight XCDs in turn, an XCD's L2 then sees one slice of the table only.  SHORT: the last slice has
+// fewer chunks, the lanes past its end idle (a kernel of its own: the test costs the others 2 to 3 %).
 constexpr int kGatherSteps = 2, kGatherChunks = kBlockThreads * kGatherSteps;
-__global__ __launch_bounds__(kBlockThreads) void GatherChunks(char *out, const char *table, const int32_t *idx, uint32_t chunks, uint32_t cpr,
-                                                              uint32_t magic, int shift, uint32_t tableRows, uint32_t parts)
+template <bool SHORT>
+__global__ __launch_bounds__(kBlockThreads) void GatherChunks(char *out, const char *table, const int32_t *idx, uint32_t chunks, uint32_t rowChunks,
+                                                              uint32_t cpr, uint32_t magic, int shift, uint32_t tableRows, uint32_t parts)
 {
     typedef uint32_t u32x4 __attribute__((ext_vector_type(4), aligned(2)));
     const uint32_t xcd = blockIdx.x % 8, slice = xcd % parts, block = blockIdx.x / 8 * (8 / parts) + xcd / parts;
-    const uint32_t first = block * (uint32_t)kGatherChunks + threadIdx.x, rowChunks = cpr * parts;
+    const uint32_t first = block * (uint32_t)kGatherChunks + threadIdx.x;
     if (block * (uint32_t)kGatherChunks >= chunks)
         return;
     uint32_t row[kGatherSteps], at[kGatherSteps], part[kGatherSteps];
@@ -140,13 +142,14 @@ __global__ __launch_bounds__(kBlockThreads) void GatherChunks(char *out, const c
 #pragma unroll
     for (int i = 0; i < kGatherSteps; ++i) {
         const bool inside = row[i] < tableRows; // (a negative index is a large one)
-        v[i] = *reinterpret_cast<const u32x4 *>(table + ((size_t)(inside ? row[i] : 0u) * rowChunks + part[i]) * 16);
+        const uint32_t from = !SHORT || part[i] < rowChunks ? part[i] : rowChunks - 1;
+        v[i] = *reinterpret_cast<const u32x4 *>(table + ((size_t)(inside ? row[i] : 0u) * rowChunks + from) * 16);
         if (!inside)
             v[i] = u32x4{0, 0, 0, 0};
     }
 #pragma unroll
     for (int i = 0; i < kGatherSteps; ++i)
-        if (first + i * kBlockThreads < chunks)
+        if (first + i * kBlockThreads < chunks && (!SHORT || part[i] < rowChunks))
             __builtin_nontemporal_store(v[i], reinterpret_cast<u32x4 *>(out + ((size_t)at[i] * rowChunks + part[i]) * 16));
 }
 
@@ -240,26 +243,36 @@ extern "C" int pto_gather_rows(void *stream, void *out, const void *table, const
         return PTO_ERR_UNSUPPORTED;
     const size_t rowChunks = cols * (size_t)elem_bytes / 16; // cols % 8 == 0: whole chunks; below 2^30
     uint32_t parts = 1;
-    // Slices of whole 128-byte lines, as few as bring a slice of the table down to 2 MiB of an XCD's 4 MiB of L2, where the
-    // batch reads a row twice or more on average (65536 rows of 2 KiB from a table of 16384: 38.3 us in one slice, 33.1 in
-    // four, 28.2 in eight; a table of 65536 rows, 43.9 in one, 48.5 in eight)
-    if (n_idx >= 2 * table_rows)
-        while (parts < 8 && rowChunks % (16 * parts) == 0 && table_rows * rowChunks * 16 / parts > ((size_t)2 << 20))
-            parts *= 2;
-    const size_t cpr = rowChunks / parts;
+    size_t cpr = rowChunks;
+    // Slices, as few as bring a slice of the table down to 1 MiB of an XCD's 4 MiB of L2, where the batch reads a row twice or more
+    // on average (65536 rows of 2 KiB from a table of 16384: 38.3 us in one slice, 33.1 in four, 28.2 in eight; a table of 65536
+    // rows, 43.9 in one, 48.5 in eight; slices of 2 MiB take 6 % longer with tables of 5 and 6 MiB).  Of whole 128-byte lines where
+    // the rows are; else of six and more half lines where the rows are whole numbers of those (16639 rows of 5696 bytes out of
+    // 1972: 24.6 us whole, 17.5 in eight); at most an eighth of the lanes idle past a shorter last slice (32768 rows of 3840 bytes
+    // out of 8192: 33.7 whole, 25.9 in eight).  Lines cut by a slice are written twice, in part: slices of other rows (20000 of
+    // 2064 bytes 12.0 us, cut 14.1) and into an output off the 16 bytes (the first of these 58.6, whole 38.6) lose more than they win.
+    if (n_idx >= 2 * table_rows && rowChunks % 4 == 0 && reinterpret_cast<uintptr_t>(out) % 16 == 0)
+        for (const size_t unit = rowChunks % 8 == 0 ? 8 : 4, least = rowChunks % 8 == 0 ? 8 : 24;
+             parts < 8 && table_rows * rowChunks * 16 / parts > ((size_t)1 << 20); parts *= 2) {
+            const size_t next = (rowChunks + 2 * parts * unit - 1) / (2 * parts * unit) * unit;
+            if (next < least || next * 2 * parts * 7 > rowChunks * 8)
+                break;
+            cpr = next;
+        }
     int shift = 31;
     while (((size_t)1 << (shift - 31)) < cpr)
         ++shift;
     const uint32_t magic = (uint32_t)((((uint64_t)1 << shift) + cpr - 1) / cpr);
     hipStream_t st = static_cast<hipStream_t>(stream);
+    const auto kernel = cpr * parts == rowChunks ? GatherChunks<false> : GatherChunks<true>;
     // (whole rows per launch, fewer than 2^31 chunks a slice)
     const size_t rowsPerLaunch = 0x7fffffffu / rowChunks;
     for (size_t r0 = 0; r0 < n_idx; r0 += rowsPerLaunch) {
         const size_t chunks = (n_idx - r0 < rowsPerLaunch ? n_idx - r0 : rowsPerLaunch) * cpr, blocks = (chunks + kGatherChunks - 1) / kGatherChunks;
         const size_t perGroup = 8 / parts, groups = (blocks + perGroup - 1) / perGroup;
-        GatherChunks<<<dim3((unsigned)(groups * 8)), dim3(kBlockThreads), 0, st>>>(
-            static_cast<char *>(out) + r0 * rowChunks * 16, static_cast<const char *>(table), idx + r0, (uint32_t)chunks, (uint32_t)cpr, magic, shift,
-            (uint32_t)table_rows, parts);
+        kernel<<<dim3((unsigned)(groups * 8)), dim3(kBlockThreads), 0, st>>>(
+            static_cast<char *>(out) + r0 * rowChunks * 16, static_cast<const char *>(table), idx + r0, (uint32_t)chunks, (uint32_t)rowChunks,
+            (uint32_t)cpr, magic, shift, (uint32_t)table_rows, parts);
     }
     return pto_amd::check_launch();
 }

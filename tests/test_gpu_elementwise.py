@@ -140,6 +140,20 @@ def test_gather_rows_widths_and_slices(oracle, rows, cols, nidx):
     assert np.array_equal(gather_rows(t32, idx), oracle.gather_rows(t32, idx))
 
 
+@pytest.mark.parametrize("rows,cols,nidx", [(600, 2848, 1201), (1972, 2848, 4001), (1100, 1920, 2300), (4096, 448, 9000), (2300, 864, 5001), (8192, 64, 17000),
+                                            (700, 8000, 1401)])
+def test_gather_rows_unequal_slices(oracle, rows, cols, nidx):
+    """Rows of whole lines or half lines that the slices do not divide: a last slice with fewer chunks, two to eight slices."""
+    from gpu_util import gather_rows
+    table, idx = datagen.gather_inputs(rows, cols, nidx)
+    idx = idx.copy()
+    idx[::19] = -5
+    idx[7::41] = rows + 3
+    assert np.array_equal(gather_rows(table, idx), oracle.gather_rows(table, idx))
+    t32 = np.random.default_rng(2).integers(0, 2**32, size=(rows, cols // 2), dtype=np.uint64).astype(np.uint32)
+    assert np.array_equal(gather_rows(t32, idx), oracle.gather_rows(t32, idx))
+
+
 @pytest.mark.parametrize("rows,cols,nidx", [(5, 24, 700), (1500, 1032, 3001), (3000, 1024, 6001)])
 @pytest.mark.parametrize("dtype", [torch.int16, torch.int32])
 def test_gather_rows_element_alignment(rows, cols, nidx, dtype):
