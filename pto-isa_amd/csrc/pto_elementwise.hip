@@ -60,22 +60,23 @@ __global__ __launch_bounds__(kBlockThreads) AICORE void CvtF32(__gm__ D *dst, __
 // stores are non-temporal (measured with inputs and outputs that no cache holds: 6.5 against 6.2 TB/s with plain
 // stores).  Same element function as TCVT (detail::convert), so the results are the same bits.  The last workgroup takes
 // what is left behind the whole pieces, element by element past the last four: as a launch of its own that rest took
-// 3.7 us (16 524 000 elements 20.0 -> 16.2 us, 6.1 TB/s; 2^27 - 5 elements 126.6 -> 123.9, 6.5 TB/s).  Four loads per lane
-// rather than eight: 2^26 elements 61.6 -> 61.1 us; two for the modes that round in integer arithmetic, where more waves
-// hide more of it (2^26 elements downwards: tile form 77.4, eight loads 68.7, four 64.3, two 63.5 us).
-template <int MODE>
-constexpr int kCvtPiece = MODE == PTO_CAST_RINT ? 4 * 4 * kBlockThreads : 2 * 4 * kBlockThreads; // elements per workgroup
-template <typename D, int MODE>
+// 3.7 us (16 524 000 elements 20.0 -> 16.2 us, 6.1 TB/s; 2^27 - 5 elements 126.6 -> 123.9, 6.5 TB/s).  LOADS: 16-byte loads of a
+// lane: four; two for the modes that round in integer arithmetic, where more waves hide more of it (2^26 elements downwards: tile
+// form 77.4, eight loads 68.7, four 64.3, two 63.5 us), and for fp16 from 2^24 elements on (2^24, 2^25, 2^27 elements: two 17.1, 31.9,
+// 123.1 us, four 17.8, 32.9, 126.4, eight 17.5, 33.0, 125.2; below, which is faster depends on where the buffers lie).
+template <int LOADS>
+constexpr int kCvtPiece = LOADS * 4 * kBlockThreads; // elements per workgroup
+template <typename D, int MODE, int LOADS>
 __global__ __launch_bounds__(kBlockThreads) void CvtF32Stream(D *dst, const float *src, size_t n, size_t firstPiece)
 {
     typedef float f32x4 __attribute__((ext_vector_type(4)));
     typedef uint16_t u16x4 __attribute__((ext_vector_type(4)));
-    constexpr int kPerStep = kBlockThreads * 4, kSteps = kCvtPiece<MODE> / kPerStep;
+    constexpr int kPerStep = kBlockThreads * 4, kSteps = LOADS, kPiece = kCvtPiece<LOADS>;
     static_assert(sizeof(D) == 2, "16-bit results");
     auto cvt = [](float v) { return __builtin_bit_cast(uint16_t, ::pto::detail::convert<D, float>(v, static_cast<RoundMode>(MODE))); };
-    const size_t first = (firstPiece + blockIdx.x) * (size_t)kCvtPiece<MODE>, base = first + 4 * threadIdx.x;
+    const size_t first = (firstPiece + blockIdx.x) * (size_t)kPiece, base = first + 4 * threadIdx.x;
     f32x4 x[kSteps];
-    if (first + kCvtPiece<MODE> <= n) {
+    if (first + kPiece <= n) {
 #pragma unroll
         for (int i = 0; i < kSteps; ++i)
             x[i] = __builtin_nontemporal_load(reinterpret_cast<const f32x4 *>(src + base + (size_t)i * kPerStep));
@@ -195,13 +196,17 @@ int launch_cvt(void *stream, D *dst, const float *src, size_t n, int mode)
     constexpr size_t kMaxBlocks = 1u << 30;
     if (aligned) {
         using Kernel = void (*)(D *, const float *, size_t, size_t);
-        Kernel kernel = CvtF32Stream<D, PTO_CAST_RINT>;
+        Kernel kernel = CvtF32Stream<D, PTO_CAST_RINT, 4>;
+        size_t piece = kCvtPiece<4>;
         if constexpr (std::is_same_v<D, half>) { // (bf16 has the one mode)
-            static constexpr Kernel kByMode[] = {CvtF32Stream<D, PTO_CAST_RINT>, CvtF32Stream<D, PTO_CAST_ROUND>, CvtF32Stream<D, PTO_CAST_FLOOR>,
-                                                 CvtF32Stream<D, PTO_CAST_CEIL>, CvtF32Stream<D, PTO_CAST_TRUNC>, CvtF32Stream<D, PTO_CAST_ODD>};
-            kernel = kByMode[mode - PTO_CAST_RINT];
+            static constexpr Kernel kByMode[] = {CvtF32Stream<D, PTO_CAST_RINT, 2>, CvtF32Stream<D, PTO_CAST_ROUND, 2>, CvtF32Stream<D, PTO_CAST_FLOOR, 2>,
+                                                 CvtF32Stream<D, PTO_CAST_CEIL, 2>, CvtF32Stream<D, PTO_CAST_TRUNC, 2>, CvtF32Stream<D, PTO_CAST_ODD, 2>};
+            if (mode != PTO_CAST_RINT || n >= (size_t)1 << 24) {
+                kernel = kByMode[mode - PTO_CAST_RINT];
+                piece = kCvtPiece<2>;
+            }
         }
-        const size_t piece = mode == PTO_CAST_RINT ? kCvtPiece<PTO_CAST_RINT> : kCvtPiece<PTO_CAST_ROUND>, pieces = (n + piece - 1) / piece;
+        const size_t pieces = (n + piece - 1) / piece;
         for (size_t t0 = 0; t0 < pieces; t0 += kMaxBlocks) {
             const size_t nb = pieces - t0 < kMaxBlocks ? pieces - t0 : kMaxBlocks;
             kernel<<<dim3((unsigned)nb), dim3(kBlockThreads), 0, st>>>(dst, src, n, t0);

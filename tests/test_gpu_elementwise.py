@@ -92,6 +92,21 @@ def test_tcvt_streaming_and_tile_forms_agree(n):
             assert (a[n:] == 0x5a5a).all() and (b[n:] == 0x5a5a).all(), (n, mode)
 
 
+@pytest.mark.parametrize("n", [(1 << 24) - 1, 1 << 24, (1 << 24) + 2047, (1 << 24) + 2051])
+def test_tcvt_f16_loads_per_lane(n):
+    """Both sides of the size from which a lane has two loads in flight, whole and partial last pieces: the bits of the tile
+    form, nothing written behind the last element."""
+    lib = capi.load()
+    memory = torch.empty(n + 1, device="cuda:0").normal_()
+    memory[::1001] = float("nan")
+    x = memory[1:].clone()
+    a, b = (torch.full((n + 16,), 0x5a5a, dtype=torch.int16, device="cuda:0") for _ in range(2))
+    capi.check(lib.pto_tcvt_f32_f16(0, a.data_ptr(), x.data_ptr(), n, capi.CAST_RINT), "aligned")
+    capi.check(lib.pto_tcvt_f32_f16(0, b.data_ptr(), memory.data_ptr() + 4, n, capi.CAST_RINT), "tile form")
+    torch.cuda.synchronize()
+    assert torch.equal(a, b) and (a[n:] == 0x5a5a).all()
+
+
 def test_tcvt_full_size_config(oracle):
     """Config 5 at full size 16384 x 8192 with 0.1% special values: compared in slabs against the oracle."""
     from gpu_util import to_dev, stream
