@@ -54,6 +54,10 @@ int pto_st_tri_mask_f32_64x128(void *stream, float *out, const float *x, int dia
 int pto_st_tgather_mask_b16_16x64(void *stream, uint16_t *out, const uint16_t *src, int pattern);
 /* MGATHER element form: out[8,128] = gm[idx[8,128]] (tests/cpu/st/testcase/mgather). */
 int pto_st_mgather_b16_8x128(void *stream, uint16_t *out, const uint16_t *gm, const int32_t *idx, int gm_elems);
+/* MGATHER_ROWS: out[rows,cols] = table[idx[rows], :cols], table rows ld elements apart, through a 32 x 64 tile; rows of zeros for
+ * indices outside [0, table_rows).  rows <= 32, cols <= 64, cols % 8 == 0, elem_bytes 2 or 4. */
+int pto_st_mgather_rows_32x64(void *stream, void *out, const void *table, const int32_t *idx, int rows, int cols, int table_rows, int ld,
+                              int elem_bytes);
 /* TLOAD of a [10,20] fp32 region into a [16,32] tile with PadValue::Max; the whole tile image comes back
  * (tload/main.cpp:138-183, PADMAX case). */
 int pto_st_tload_pad_f32_16x32(void *stream, float *image, const float *gm);

@@ -179,6 +179,27 @@ __global__ __launch_bounds__(kBlockThreads) AICORE void GatherMask(__gm__ uint16
     }
 }
 
+// ---- row-form MGATHER: dst[i,:] = table[rowIdx[i],:], valid rows x cols of a 32 x 64 tile, rows outside the table zero ----
+template <typename T>
+__global__ __launch_bounds__(kBlockThreads) AICORE void MGatherRowsTile(__gm__ T *out, __gm__ const T *table, __gm__ const int32_t *idx, int rows,
+                                                                        int cols, int tableRows, int ld)
+{
+    using Dst = Tile<TileType::Vec, T, 32, 64, BLayout::RowMajor, DYNAMIC, DYNAMIC>;
+    using Idx = Tile<TileType::Vec, int32_t, 32, 1, BLayout::ColMajor, DYNAMIC, 1>;
+    Dst d((size_t)rows, (size_t)cols);
+    Idx ti((size_t)rows);
+    GlobalTensor<int32_t, Shape<1, 1, 1, DYNAMIC, 1>, Stride<1, 1, 1, 1, DYNAMIC>, Layout::DN> gi(
+        const_cast<int32_t *>(idx), Shape<1, 1, 1, DYNAMIC, 1>(rows), Stride<1, 1, 1, 1, DYNAMIC>(rows));
+    using G = GlobalTensor<T, Shape<1, 1, 1, DYNAMIC, DYNAMIC>, Stride<1, 1, 1, DYNAMIC, 1>>;
+    G gt(const_cast<T *>(table), Shape<1, 1, 1, DYNAMIC, DYNAMIC>(tableRows, cols), Stride<1, 1, 1, DYNAMIC, 1>(ld));
+    G go(out, Shape<1, 1, 1, DYNAMIC, DYNAMIC>(rows, cols), Stride<1, 1, 1, DYNAMIC, 1>(cols));
+    TLOAD(ti, gi);
+    MGATHER_ROWS(d, gt, ti, tableRows);
+    set_flag(PIPE_V, PIPE_MTE3, EVENT_ID0);
+    wait_flag(PIPE_V, PIPE_MTE3, EVENT_ID0);
+    TSTORE(go, d);
+}
+
 // ---- element-form MGATHER: dst[8,128] = gm[idx[8,128]] ----
 __global__ __launch_bounds__(kBlockThreads) AICORE void MGatherElems(__gm__ uint16_t *out, __gm__ const uint16_t *gm,
                                                                      __gm__ const int32_t *idx, int gmElems)
@@ -757,6 +778,22 @@ extern "C" int pto_st_mgather_b16_8x128(void *stream, uint16_t *out, const uint1
 {
     PTO_ST_NONNULL(out, gm, idx);
     MGatherElems<<<dim3(1), dim3(kBlockThreads), 0, static_cast<hipStream_t>(stream)>>>(out, gm, idx, gm_elems);
+    return pto_amd::check_launch();
+}
+
+extern "C" int pto_st_mgather_rows_32x64(void *stream, void *out, const void *table, const int32_t *idx, int rows, int cols, int table_rows, int ld,
+                                         int elem_bytes)
+{
+    PTO_ST_NONNULL(out, table, idx);
+    if (rows < 1 || rows > 32 || cols < 8 || cols > 64 || cols % 8 || table_rows < 1 || ld < cols || (elem_bytes != 2 && elem_bytes != 4))
+        return PTO_ERR_BAD_ARG;
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    if (elem_bytes == 2)
+        MGatherRowsTile<uint16_t><<<dim3(1), dim3(kBlockThreads), 0, st>>>(static_cast<uint16_t *>(out), static_cast<const uint16_t *>(table), idx, rows,
+                                                                          cols, table_rows, ld);
+    else
+        MGatherRowsTile<uint32_t><<<dim3(1), dim3(kBlockThreads), 0, st>>>(static_cast<uint32_t *>(out), static_cast<const uint32_t *>(table), idx, rows,
+                                                                          cols, table_rows, ld);
     return pto_amd::check_launch();
 }
 

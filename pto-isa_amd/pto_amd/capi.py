@@ -45,6 +45,7 @@ ST_SYMBOLS = {
     "pto_st_tri_mask_f32_64x128": (C.c_int, [C.c_void_p] * 3 + [C.c_int, C.c_float, C.c_int]),
     "pto_st_tgather_mask_b16_16x64": (C.c_int, [C.c_void_p] * 3 + [C.c_int]),
     "pto_st_mgather_b16_8x128": (C.c_int, [C.c_void_p] * 4 + [C.c_int]),
+    "pto_st_mgather_rows_32x64": (C.c_int, [C.c_void_p] * 4 + [C.c_int] * 5),
     "pto_st_tload_pad_f32_16x32": (C.c_int, [C.c_void_p] * 3),
     "pto_st_tload_5d_f32": (C.c_int, [C.c_void_p] * 4),
     "pto_st_mat_view_walk": (C.c_int, [C.c_void_p, C.c_void_p, C.c_int]),

@@ -133,6 +133,23 @@ def test_mgather_elements(oracle):
     assert np.array_equal(out.cpu().numpy().view(np.uint16), gm[idx])
 
 
+@pytest.mark.parametrize("rows,cols,ld,dtype", [(32, 64, 64, np.uint16), (32, 64, 96, np.uint32), (7, 40, 40, np.uint16), (1, 8, 24, np.uint32), (31, 56, 57, np.uint16)])
+def test_mgather_rows(rows, cols, ld, dtype):
+    """The row form, whole and partly valid tiles, strided tables whose rows need no alignment, indices outside the table."""
+    rng = np.random.default_rng(rows + cols)
+    table = rng.integers(1, np.iinfo(dtype).max, size=(50, ld), dtype=dtype)
+    idx = rng.integers(0, 50, size=rows).astype(np.int32)
+    idx[::5] = (-1, 50, 2**31 - 1, -2**31)[rows % 4]
+    out = torch.full((rows * cols + 8,), -1, dtype=torch.int16 if dtype == np.uint16 else torch.int32, device=DEV)
+    tt, ti = dev(table), dev(idx)
+    capi.check(capi.load_st().pto_st_mgather_rows_32x64(st(), out.data_ptr(), tt.data_ptr(), ti.data_ptr(), rows, cols, 50, ld, dtype().itemsize), "rows")
+    torch.cuda.synchronize()
+    got = out.cpu().numpy().view(dtype)
+    inside = (idx >= 0) & (idx < 50)
+    want = np.where(inside[:, None], table[np.where(inside, idx, 0), :cols], 0)
+    assert np.array_equal(got[:rows * cols].reshape(rows, cols), want) and (got[rows * cols:] == np.iinfo(dtype).max).all()
+
+
 def test_tload_pad_and_valid_region(oracle):
     lib = capi.load_st()
     x = np.arange(200, dtype=np.float32)
