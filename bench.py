@@ -24,8 +24,8 @@ PEAK_FP8_TFLOPS = 5033.2    # dense fp8 matrix peak (published)
 PEAK_FP4_TFLOPS = 10066.3   # dense fp4 matrix peak (published)
 PEAK_HBM_GBS = 8000.0       # MI355X HBM3E peak (published)
 # row gather, 65536 x 1024 fp16 from a 32 MiB table: bytes per launch at the L2 <-> fabric boundary (FETCH_SIZE + WRITE_SIZE
-# runs summarised in profiles/cvt_f32_16384x8192_and_gather_rows_65536x1024.md)
-GATHER_HBM_SIDE_BYTES = 85.0e6 + 134.3e6
+# runs summarised in profiles/kernel_durations_small_ragged_large.md)
+GATHER_HBM_SIDE_BYTES = 44.8e6 + 134.2e6
 
 # HBM-side traffic of one 6144^3 GEMM launch, from two rocprofv3 --pmc runs of this script
 # (FETCH_SIZE, then WRITE_SIZE; KiB per dispatch of the GEMM kernel), each scaled by what the same
@@ -365,7 +365,7 @@ def main():
                                                "frac_hbm_peak_hbm_side": hbm_side / (r["ms"] * 1e-3) / 1e9 / PEAK_HBM_GBS,
                                                "note": "cache-resident figure, not an HBM roofline number: gbs_algorithmic counts rows read + "
                                                        "rows written + indices (268.7 MB), but the 32 MiB table is served from cache; the "
-                                                       "FETCH_SIZE / WRITE_SIZE counters (profiles/) read 85.0 MB + 134.3 MB per launch at the "
+                                                       "FETCH_SIZE / WRITE_SIZE counters (profiles/) read 44.8 MB + 134.2 MB per launch at the "
                                                        "L2 <-> fabric boundary, which gbs_hbm_side is computed from"}
 
     if only in ("", "gemm") and args.size == 6144:

@@ -56,8 +56,8 @@ int pto_last_hip_error(void);
 
 /* C[m,n] fp32 row-major = A[m,k] fp16 row-major x B, where B is stored [n,k] fp16 (a column-major
  * k x n operand), fp32 accumulation.  Accepted extents: m % 128 == 0, n % 256 == 0, k % 32 == 0 (multiples of the
- * 128 x 256 block of the reference kernel), or any m >= 192 and n >= 128 with n % 4 == 0 and k % 128 == 0 (256- or 192-row
- * tiles whose last row / column of tiles is moved back to end with the matrix).  Anything else: PTO_ERR_UNSUPPORTED. */
+ * 128 x 256 block of the reference kernel), or any m >= 192 and n >= 128 with n % 4 == 0 and k % 128 == 0.  Anything else:
+ * PTO_ERR_UNSUPPORTED.  Tiles of 32 x 64 to 256 x 256, chosen by the extents; the sums are added in their order. */
 int pto_gemm_f16f32(void *stream, float *c, const uint16_t *a, const uint16_t *b, int m, int n, int k);
 
 /* MXFP8 GEMM: C[m,n] row-major = (A .* 2^(scale_a - 127)) x (B .* 2^(scale_b - 127)) with fp32 accumulation.
@@ -129,7 +129,7 @@ int pto_tcvt_f32_f16(void *stream, uint16_t *dst, const float *src, size_t n, in
 int pto_tcvt_f32_bf16(void *stream, uint16_t *dst, const float *src, size_t n, int round_mode);
 
 /* out[i, :] = table[idx[i], :] for i < n_idx; rows whose index is outside [0, table_rows) are zero.
- * elem_bytes in {2, 4}; cols % 8 == 0.  table [table_rows, cols] and out [n_idx, cols] contiguous. */
+ * elem_bytes in {2, 4}; cols % 8 == 0.  table [table_rows, cols] and out [n_idx, cols] contiguous, aligned to their elements. */
 int pto_gather_rows(void *stream, void *out, const void *table, const int32_t *idx, size_t n_idx,
                     size_t table_rows, size_t cols, int elem_bytes);
 

@@ -12,8 +12,9 @@
 // them loading), so the (BM + BN) 128 bytes of a 128 x 128 step are 620 clocks against 512 of its MFMAs; with one part
 // taken out a step of 0.46 us (1024 x 3072 x 8192) runs 0.43 without the fragment reads, 0.36 with copies alone and 0.33
 // with MFMAs alone.  The place of the copies in the step, raised wave priority and deeper rings changed nothing (1 %).
-// Small tiles lose there what they win in compute units at work: 512^3 8.96 -> 4.0 us, 1000 x 3000 x 2048 21.1 -> 17.0,
-// 128 x 4096 x 4096 68 -> 13.
+// (1000 x 3000 x 2048 on 128 x 96 tiles runs 0.4 us a step: 28 KiB of copies, from beyond the L2.)
+// Small tiles lose there what they win in compute units at work: 512^3 8.96 -> 3.9 us, 1000 x 3000 x 2048 21.1 -> 18.0,
+// 128 x 4096 x 4096 68 -> 12.
 //
 // Rows past m and columns past n repeat the last one on the way in (their memory may not exist) and are not stored.
 #pragma once

@@ -12,8 +12,8 @@
 // apart meet in four of the 32 banks that a 4-byte read sees; 128 x 128 tiles 25 % slower.)
 //
 // What bounds a step: the copies, as in the fp16 kernel.  One 64 x 64 tile takes 0.16 us a step, 64 x 128 0.24, 128 x 128 0.37,
-// 128 x 192 0.52: 85 to 100 bytes per ns and compute unit, where its MFMAs take 0.05, 0.11, 0.21, 0.32.
-// 512 x 512 x 512 fp8 9.1 -> 4.0 us, 256 x 256 x 6144 34.1 -> 11.0, 2048^3 17.3 -> 13.3; 3072^3 stays on 256 x 192 tiles (31
+// 128 x 192 0.52: 79 to 102 bytes per ns and compute unit, where its MFMAs take 0.05, 0.11, 0.21, 0.32.
+// 512 x 512 x 512 fp8 9.1 -> 3.8 us, 256 x 256 x 6144 34.0 -> 11.9, 2048^3 17.3 -> 13.5; 3072^3 stays on 256 x 192 tiles (31
 // against 40).
 #pragma once
 #include "gemm_kernels_ks.hpp"

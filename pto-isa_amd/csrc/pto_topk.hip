@@ -19,14 +19,14 @@
 //   one DPP move for the upper word, and for the lower word another, or the LDS pipe (ds_swizzle), which the network leaves idle
 //   otherwise (LOW_DPP, at the dispatch); partners 16 and 32 lanes away come over the LDS pipe whole (v_permlane*_swap: 3.5 ns a word, 4.2 us of the
 //   kernel's time for three stages of 55); strides across waves go through LDS memory.
-// * topk below the padded row length: once the sorted runs are as long as topk (rounded up to keys per lane times a power of
+// * topk of an eighth of the padded row length or less: once the sorted runs are as long as topk (rounded up to keys per lane times a power of
 //   two), a merge of two runs keeps their larger halves only, in both runs' lanes, and its sort passes no longer cover the
 //   dropped half.
 // * Any other index vector: the same network sorts the (index, column) pairs first, once per workgroup (the rows share their
 //   indices); the rank of a column in that order then stands in the scores' keys for the column.  4800 x 1024 whole: 42 us (127
 //   with keys in the LDS and a pass over it per stage); 1000 x 256: 6.6 (15).
-// What bounds it: vector instructions, 2240 per row of 1024 (3850 in the integer network this replaced), behind a phase of
-// loads and before one of stores that all waves share: of 26.4 us (4800 x 1024, top 1000, 58 MB = 9 us at 6.5 TB/s) 12 are
+// What bounds it: vector instructions, 2520 per row of 1024 (3850 in the integer network this replaced), behind a phase of
+// loads and before one of stores that all waves share: of 25.0 us (4800 x 1024, top 1000, 58 MB = 9 us at 6.5 TB/s) 12 are
 // launch, loads and stores.  Persistent waves that load the next row while they sort one, and wave priorities that let
 // some run ahead, do not hide them (32 us and no change).
 #include <hip/hip_runtime.h>

@@ -47,7 +47,7 @@ def test_topk_ties_signed_zeros_infinities_and_arbitrary_indices(oracle):
     idx[0] = 0xFFFFFFFF
     for k in (1, 100, cols):
         assert same(topk_gpu(src, idx, cols, k), oracle.topk_f32(src, idx, cols, k))
-    # indices that increase with the column (the register-resident network; the rows above went through LDS)
+    # indices that increase with the column
     for mono in (np.arange(cols, dtype=np.uint32), (np.arange(cols, dtype=np.uint32) * 3 + 7) ** 2):
         for k in (1, 100, cols):
             assert same(topk_gpu(src, mono, cols, k), oracle.topk_f32(src, mono, cols, k))
@@ -63,7 +63,7 @@ def test_topk_ties_signed_zeros_infinities_and_arbitrary_indices(oracle):
 def test_topk_row_lengths_and_kept_lengths(oracle, cols):
     """Every number of keys per lane and waves per row at its smallest and largest rows, topk on both sides of every length that
     the merges stop at (keys per lane times powers of two), row counts that do not fill the last workgroup, many ties and
-    signed zeros; consecutive indices, increasing ones, ones that start near 2^32, and any (the pass through LDS)."""
+    signed zeros; consecutive indices, increasing ones, ones that start near 2^32, and any."""
     r = np.random.Generator(np.random.Philox(key=cols))
     keys = next(e for e in (2, 4, 8, 16) if cols <= 64 * e or e == 16)
     kept = sorted({k for b in range(9) for k in ((keys << b) - 1, keys << b, (keys << b) + 1) if 1 <= k <= cols} | {1, cols})
@@ -79,7 +79,8 @@ def test_topk_row_lengths_and_kept_lengths(oracle, cols):
 @pytest.mark.parametrize("cols,k", [(500, 500), (500, 9), (1024, 1000), (1024, 70), (1900, 1900), (1900, 200)])
 @pytest.mark.parametrize("rows", [1280, 1281, 2560, 2563])
 def test_topk_waves_per_row(oracle, rows, cols, k):
-    """Both sides of the row counts where the number of waves per row changes, consecutive and other increasing indices."""
+    """Around 256 units times five and ten waves (1024 columns change from two waves per row to one behind 2560), and a last workgroup
+    that is not full; consecutive and other increasing indices."""
     src, idx = datagen.topk_inputs(rows, cols, cols + 1, distinct=300)
     for ids in (idx, idx * np.uint32(3)):
         assert same(topk_gpu(src, ids, cols, k), oracle.topk_f32(src, ids, cols, k))
