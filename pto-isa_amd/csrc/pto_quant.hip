@@ -69,7 +69,14 @@ __device__ inline uint32_t QuantFour(f32x4 x, uint8_t &scaleByte)
 
 // Four loads per lane (16384 x 8192: 109.4 us with eight, 108.2 with four) and the last, partial piece in the same launch
 // (333 x 4128: 7.2 -> 4.3 us; 4096 x 6144 21.7 -> 20.7).
+// STREAM: elements stored past the caches.  The usual next reader is a GEMM, which finds what is stored the ordinary way in the
+// memory-side cache (256 MB): 1000 x 4096 and the product with 6144 columns behind it 39.7 -> 34.4 us, 4096 x 4096 and 2048
+// columns 52.8 -> 48.1, 8192 x 8192 and 512 columns 99 -> 90; the quantiser alone within 3 % up to 64 Mi elements (1000 x 4096
+// 5.4 and 5.0 us, 8192 x 8192 53.7 and 52.0).  Above that its input and output no longer fit there together and the ordinary stores cost
+// the quantiser 6 % (16384 x 8192: 106 and 113 us).
 // (n is a multiple of 32, so groups and lanes are whole; the last workgroup's steps past n load and store nothing)
+constexpr size_t kQuantStreamFrom = ((size_t)1 << 26) + 1;
+template <bool STREAM>
 __global__ __launch_bounds__(kQuantThreads) void QuantMxFp8(uint8_t *q, uint8_t *e8m0, const float *src, size_t n, size_t firstTile)
 {
     const size_t base = (firstTile + blockIdx.x) * (size_t)kQuantTile + 4 * threadIdx.x;
@@ -88,7 +95,10 @@ __global__ __launch_bounds__(kQuantThreads) void QuantMxFp8(uint8_t *q, uint8_t 
         uint8_t scaleByte;
         const uint32_t four = QuantFour(x[i], scaleByte); // every lane takes part in the lane moves
         if (at < n) {
-            __builtin_nontemporal_store(four, reinterpret_cast<uint32_t *>(q + at));
+            if constexpr (STREAM)
+                __builtin_nontemporal_store(four, reinterpret_cast<uint32_t *>(q + at));
+            else
+                *reinterpret_cast<uint32_t *>(q + at) = four;
             if ((threadIdx.x & 7) == 0)
                 e8m0[at >> 5] = scaleByte;
         }
@@ -112,7 +122,7 @@ extern "C" int pto_quant_mxfp8_f32(void *stream, uint8_t *q, uint8_t *scale, con
     constexpr size_t kMaxBlocks = 1u << 30;
     for (size_t t0 = 0; t0 < tiles; t0 += kMaxBlocks) {
         const size_t nb = tiles - t0 < kMaxBlocks ? tiles - t0 : kMaxBlocks;
-        QuantMxFp8<<<dim3((unsigned)nb), dim3(kQuantThreads), 0, st>>>(q, scale, src, n, t0);
+        (n >= kQuantStreamFrom ? QuantMxFp8<true> : QuantMxFp8<false>)<<<dim3((unsigned)nb), dim3(kQuantThreads), 0, st>>>(q, scale, src, n, t0);
     }
     return pto_amd::check_launch();
 }

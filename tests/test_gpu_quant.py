@@ -134,3 +134,17 @@ def test_quant_mxfp8_refuses_pointers_below_the_alignment_of_its_accesses():
     assert lib.pto_quant_mxfp8_f32(None, o.data_ptr() + 2, o.data_ptr(), d.data_ptr(), 1, 64) == capi.ERR_UNSUPPORTED
     assert lib.pto_quant_mxfp8_f32(None, o.data_ptr(), o.data_ptr() + 1, d.data_ptr(), 1, 64) == capi.OK
     torch.cuda.synchronize()
+
+
+def test_quant_mxfp8_both_sides_of_the_streaming_size():
+    """2^26 elements are stored the ordinary way, more past the caches: the same bytes for the rows that both have."""
+    rows, cols = 1 << 16, 1 << 10
+    x = torch.randn((rows + 1, cols), device="cuda:0", generator=torch.Generator("cuda:0").manual_seed(1))
+    out = []
+    for r in (rows, rows + 1):
+        q, s = torch.zeros((r, cols), dtype=torch.uint8, device="cuda:0"), torch.zeros((r, cols // 32), dtype=torch.uint8, device="cuda:0")
+        capi.check(capi.load().pto_quant_mxfp8_f32(torch.cuda.current_stream().cuda_stream, q.data_ptr(), s.data_ptr(), x.data_ptr(), r, cols),
+                   "pto_quant_mxfp8_f32")
+        out.append((q, s))
+    for whole, more in zip(*out):
+        assert torch.equal(whole, more[:rows]) and more[rows].any()
