@@ -63,7 +63,7 @@ int gemm_mx_ks(hipStream_t st, void *c, const uint8_t *a, const uint8_t *b, cons
 // opposite MFMA / softmax phases)
 int fa_fwd_d128_w8(hipStream_t st, void *o, float *lse, const _Float16 *q, const _Float16 *k, const _Float16 *v, int batch, int heads,
                    int seqQ, int seqKv, bool causal, bool oFp32, int causalOff);
-// defined in pto_fa_split.hip: the keys of a query block split over two or four groups of a workgroup's eight wavefronts
+// defined in pto_fa_split.hip: the keys of a query block split over two, four or eight groups of a workgroup's eight wavefronts
 int fa_fwd_split(hipStream_t st, void *o, float *lse, const _Float16 *q, const _Float16 *k, const _Float16 *v, int batch, int heads,
                  int seqQ, int seqKv, int headDim, bool causal, bool oFp32, int causalOff, int groups);
 // defined in pto_fa_w8m16.hip: the schedule of fa_fwd_d128_w8 on v_mfma_f32_16x16x32_f16

@@ -144,6 +144,9 @@ struct VTReader {
 // together, so the barriers of a round are those of the unsplit kernel.  At the end every wave hands its (max, sum) and
 // the accumulator quads that other groups store over the LDS; group g adds up and stores its own 1 / G of the head
 // dimension.  O = sum_g w_g O_g / sum_g w_g S_g, w_g = exp(s (M_g - M)), M = max_g M_g, all in fp32.
+// As many groups as waves: nobody else reads a wave's tiles, so it copies them itself into one K and one V buffer of its own
+// and waits for its own copies only; no barrier until the groups join, so the MFMAs, the softmax and the copies of different waves
+// overlap as they fall.
 template <int D, bool CAUSAL, bool OUT_F32, int MIN_BLOCKS, int kBKV = kBKVDefault, bool PP = false, int NQ_ = 1, int G = 1>
 __global__ __launch_bounds__(kBlockThreads, MIN_BLOCKS) AICORE void FlashAttnFwd(__gm__ void *outO, __gm__ float *outLse,
                                                                       __gm__ const half *qAll, __gm__ const half *kAll,
@@ -155,6 +158,7 @@ __global__ __launch_bounds__(kBlockThreads, MIN_BLOCKS) AICORE void FlashAttnFwd
     constexpr int kBQOwn = kBQ / G; // queries per workgroup
     constexpr int kQWaves = PTO_WAVES_N / G; // waves of a group
     static_assert(G == 1 || (NQ == 1 && !PP && PTO_WAVES_N % G == 0), "key groups: one query block per wave");
+    constexpr bool kOwnKeys = G > 1 && kQWaves == 1; // groups of one wave
     constexpr int KB = kBKV / 32;  // 32-key blocks per tile
     constexpr int DB = D / 32;    // 32-wide blocks of the head dimension
     // ---- tiles ----
@@ -173,7 +177,7 @@ __global__ __launch_bounds__(kBlockThreads, MIN_BLOCKS) AICORE void FlashAttnFwd
 
     constexpr uint32_t kTileBytes = kBKV * D * sizeof(half);
     constexpr uint32_t kStageBytes = 2 * kTileBytes;
-    constexpr uint32_t kGroupBytes = 2 * kStageBytes; // the double buffer of one key group
+    constexpr uint32_t kGroupBytes = (kOwnKeys ? 1 : 2) * kStageBytes; // the (double) buffer of one key group
     static_assert(G > 1 || D * kBQ * sizeof(half) <= 2 * kStageBytes, "Q^T is staged in the K/V stages");
 
     // ---- which (batch*head, query tile) this workgroup owns.  Workgroups are dealt round-robin to
@@ -479,16 +483,48 @@ __global__ __launch_bounds__(kBlockThreads, MIN_BLOCKS) AICORE void FlashAttnFwd
             }
         });
     };
-    if constexpr (G > 1) {
-        // Q^T straight into the operand registers: 16 bytes of the lane's own query per step of 16 (typed with the alignment
-        // of an element, as little as the copies of the unsplit form ask for)
+    // Groups of one wave: instruction i of a tile covers its bytes 1024 i .. + 1023, whole rows of the image (the tile is
+    // contiguous in memory); the swizzle depends on the row modulo 16.
+    constexpr int kOwnCopies = (int)kTileBytes / 1024, kRowsPerCopy = 1024 / (2 * D), kOwnOffs = kOwnKeys ? 16 / kRowsPerCopy : 1;
+    [[maybe_unused]] uint32_t ownOff[kOwnOffs];
+    if constexpr (kOwnKeys) {
+        constexpr uint32_t kChunks = 2 * D / 16; // of a row
+#pragma unroll
+        for (int i = 0; i < kOwnOffs; ++i)
+            ownOff[i] = (uint32_t)(lane * 16) ^ (detail::mat_swz<2 * D>((uint32_t)(kRowsPerCopy * i) + (uint32_t)lane / kChunks) * 16u);
+    }
+    // instruction i of tile t of K or V, into this wave's buffer
+    auto copyOwn = [&](auto isVTag, __gm__ half *base, int t, auto iTag) {
+        constexpr uint32_t at = decltype(iTag)::value * 1024u;
+        const char *from = reinterpret_cast<const char *>(base) + (int64_t)t * kTileBytes + at;
+        char *to = hw::lds_base() + (uint32_t)group * kGroupBytes + (decltype(isVTag)::value ? kTileBytes : 0u) + at;
+        __builtin_amdgcn_global_load_lds(PTO_GLOBAL_PTR(detail::uniform_ptr(from) + ownOff[decltype(iTag)::value % kOwnOffs]), PTO_LDS_PTR(to), 16, 0, 0);
+        asm volatile("" ::: "memory");
+    };
+    auto copyOwnTile = [&](auto isVTag, __gm__ half *base, int t) {
+        __builtin_amdgcn_sched_barrier(0);
+        StaticFor<0, kOwnCopies>([&](auto iTag) { copyOwn(isVTag, base, t, iTag); });
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    // Q^T straight into the operand registers: 16 bytes of the lane's own query per step of 16 (typed with the alignment
+    // of an element, as little as the copies of the unsplit form ask for)
+    [[maybe_unused]] auto loadQuery = [&]() {
         typedef half Q8 __attribute__((ext_vector_type(8), aligned(2)));
-        loadGroups(std::integral_constant<int, 0>(), std::false_type(), kBase, 0);
-        loadGroups(std::integral_constant<int, 0>(), std::true_type(), vBase, 0);
         const half *qRow = qAll + ((int64_t)bh * seqQ + myQuery) * D + 8 * hHalf;
 #pragma unroll
         for (int ks = 0; ks < D / 16; ++ks)
             qRight.st.f[0][ks] = *reinterpret_cast<const Q8 *>(qRow + 16 * ks);
+    };
+    if constexpr (kOwnKeys) {
+        if (group < numTiles)
+            copyOwnTile(std::false_type(), kBase, group);
+        loadQuery();
+        if (group < numTiles)
+            copyOwnTile(std::true_type(), vBase, group);
+    } else if constexpr (G > 1) {
+        loadGroups(std::integral_constant<int, 0>(), std::false_type(), kBase, 0);
+        loadGroups(std::integral_constant<int, 0>(), std::true_type(), vBase, 0);
+        loadQuery();
         set_flag(PIPE_MTE2, PIPE_MTE1, EVENT_ID0);
     } else {
         GlobalQT gmQ(qBase);
@@ -581,6 +617,47 @@ __global__ __launch_bounds__(kBlockThreads, MIN_BLOCKS) AICORE void FlashAttnFwd
         }
         if (group == 0) // pairs with the barrier that ends the second group's last phase
             phaseEnd();
+    } else if constexpr (kOwnKeys) {
+        // ---- every wave by itself: its own tiles through its own buffer, no barrier ----
+        // K of the next tile is copied once the last fragment of this one has been read, V of this tile between the score
+        // MFMAs (the tile before is done with the buffer): a copy instruction holds its wave until the address unit takes it,
+        // and takes nothing from MFMAs that are queued already.
+        using Zero = std::integral_constant<int, 0>;
+        static_assert(kOwnCopies <= kScoreFrags, "a V copy per score MFMA");
+        for (int r = 0; r * G + group < numTiles; ++r) {
+            const int t = r * G + group;
+            const bool more = t + G < numTiles;
+            if (r == 0)
+                hw::wait_vm<kOwnCopies>(); // K has landed, and Q (V, issued after them, need not have)
+            else
+                hw::wait_vm0(); // K has landed (issued last)
+            __builtin_amdgcn_sched_barrier(0);
+            AccS sAcc[KB];
+            __builtin_amdgcn_s_setprio(2); // (the other wave of the SIMD in its softmax leaves slots for these MFMAs)
+            scoreTile(sAcc, Zero(), [&](auto i) {
+                if constexpr (decltype(i)::value < kOwnCopies)
+                    if (r > 0)
+                        copyOwn(std::true_type(), vBase, t, i);
+            }, Zero());
+            __builtin_amdgcn_s_setprio(0);
+            if (more)
+                copyOwnTile(std::false_type(), kBase, t + G);
+            RightP pRight;
+            float alpha[NQ];
+            bool anyRaise;
+            softmaxTile(sAcc, r, pRight, alpha, anyRaise);
+            __builtin_amdgcn_sched_barrier(0);
+            if (more)
+                hw::wait_vm<kOwnCopies>(); // V has landed (K of the next tile was issued after it)
+            else
+                hw::wait_vm0();
+            __builtin_amdgcn_sched_barrier(0);
+            VStep vFirst;
+            issueVStep(std::integral_constant<uint32_t, kTileBytes>(), Zero(), vFirst);
+            __builtin_amdgcn_s_setprio(2);
+            outputTileWide(Zero(), vFirst, pRight, alpha, anyRaise);
+            __builtin_amdgcn_s_setprio(0);
+        }
     } else {
     const int rounds = (numTiles + G - 1) / G; // a wave whose group has no tile in the last round only takes part in its barrier
     // One key tile in LDS stage st (a compile-time constant: every LDS address is an immediate).
@@ -739,7 +816,7 @@ int launch_fa(hipStream_t st, void *o, float *lse, const half *q, const half *k,
         return PTO_ERR_UNSUPPORTED;
     static_assert(G > 1 || D * kBQ <= 4 * kBKV * D, "Q^T must fit the K/V stages it is staged in");
     // the K / V stages of every key group; what the groups hand over at the end (accumulators, then maxima and sums)
-    constexpr int stages = G * 2 * 2 * kBKV * D * (int)sizeof(half), joined = PTO_WAVES_N * 32 * (D + 2) * (int)sizeof(float);
+    constexpr int stages = G * (G == PTO_WAVES_N && G > 1 ? 1 : 2) * 2 * kBKV * D * (int)sizeof(half), joined = PTO_WAVES_N * 32 * (D + 2) * (int)sizeof(float);
     constexpr int lds = G > 1 && joined > stages ? joined : stages;
     static_assert(lds <= 160 * 1024, "stages fit the LDS");
     auto kernel = FlashAttnFwd<D, CAUSAL, OUT_F32, MIN_BLOCKS, kBKV, PP, NQ, G>;

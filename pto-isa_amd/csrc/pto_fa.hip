@@ -68,7 +68,7 @@ extern "C" int pto_fa_fwd_f16_variant(void *stream, void *o, float *lse, const u
         return pto_amd::fa_fwd_d128_w8m16(st, o, lse, hq, hk, hv, batch, heads, seq_q, seq_kv, causal != 0, false, causalOff);
     if (variant == 21 && head_dim == 128) // fp32 output and LSE
         return pto_amd::fa_fwd_d128_w8m16(st, o, lse, hq, hk, hv, batch, heads, seq_q, seq_kv, causal != 0, true, causalOff);
-    if (variant == 42 || variant == 44) // keys over two or four groups of waves
+    if (variant == 42 || variant == 44 || variant == 48) // keys over two, four or eight groups of waves
         return pto_amd::fa_fwd_split(st, o, lse, hq, hk, hv, batch, heads, seq_q, seq_kv, head_dim, causal != 0, false, causalOff, variant - 40);
     if (variant == 32 && head_dim == 64) // over two groups of two waves
         return launch_split_w4(st, o, lse, hq, hk, hv, batch, heads, seq_q, seq_kv, causal != 0, false, causalOff);
@@ -120,7 +120,14 @@ extern "C" int pto_fa_fwd_f16(void *stream, void *o, float *lse, const uint16_t 
     const bool fromMemory = head_dim == 128 && seq_q == 128 && blocks * 8 > cus * 7ll;
     const int keys = causal && seq_q < seq_kv - causalOff ? seq_q + causalOff : seq_kv; // that the last query sees
     int groups = 0; // 1: two groups of two waves
-    if (blocks * 2 <= cus)
+    // Four 32-query workgroups per 128 queries and still no more than one for a compute unit: eight groups of one wave, each
+    // streaming its own keys without a barrier (us, form taken before / eight groups, 128 queries, no mask):
+    //   64 heads,  128 keys: 6.5 /  6.0   320: 9.1 / 7.9   768: 12.5 / 10.6   1536: 18.8 / 15.2, at head_dim  64: 4.25 / 4.40, 5.7 / 5.2, 8.4 / 7.0, 11.8 / 9.6
+    //    4 heads,  128 keys: 6.2 /  5.4   320: 8.2 / 7.0   768: 11.0 /  8.9   1536: 16.3 / 12.4, at head_dim  64: 4.11 / 4.10, 5.5 / 4.8, 7.6 / 6.0, 10.9 / 8.0
+    // With more of them a second round comes in that costs as much as the first (80 heads, 1024 keys: 15.3 / 22.0).
+    if (blocks * 4 <= cus && (head_dim == 128 || keys > 128))
+        groups = 8;
+    else if (blocks * 2 <= cus)
         groups = keys >= (head_dim == 128 ? 256 : 1024) ? 4 : head_dim == 64 ? 1 : 0;
     else if (blocks <= cus)
         groups = head_dim == 64 && causal && keys >= 256 && keys / 2 <= seq_q ? 1 : keys >= (fromMemory ? 2048 : 1024) ? 2 : 0;

@@ -415,3 +415,41 @@ def test_fa_heads_that_eight_does_not_divide(B, H, Sq, Skv, D, causal):
     want, want_lse = dense_fp64(q[0, n - 1].cpu().numpy(), k[0, n - 1].cpu().numpy(), v[0, n - 1].cpu().numpy(), causal != 0)
     assert rel(out[0][0][0, n - 1].float().cpu().numpy(), want) <= TOL
     assert np.max(np.abs(out[0][1][0, n - 1].cpu().numpy() - want_lse)) <= 1e-4
+
+
+OWN = [(64, 48), (128, 48)]  # eight groups of one wave, each with its own buffer and no barrier between tiles
+
+
+@pytest.mark.parametrize("D,variant", OWN)
+@pytest.mark.parametrize("Sq,Skv,causal", [(128, 64, False), (128, 256, False), (128, 320, False), (128, 128, True), (256, 576, True), (384, 1280, True)])
+def test_fa_keys_split_over_single_waves(D, variant, Sq, Skv, causal):
+    """Waves without a tile, with one, with one fewer than others, and whose keys are hidden from some or all of the queries."""
+    test_fa_keys_split_over_groups(D, variant, Sq, Skv, causal)
+
+
+@pytest.mark.parametrize("D,variant", OWN)
+def test_fa_keys_split_over_single_waves_special_values(D, variant):
+    """Unaligned queries; scores of -inf in all tiles of one wave and a NaN in any key; a running max that rises along the keys."""
+    test_fa_keys_split_query_alignment(D, variant)
+    rng = np.random.default_rng(D)
+    q, k, v = (rng.standard_normal((1, 1, n, D)).astype(np.float16) for n in (128, 1024, 1024))
+    q[..., 0] = 1.0
+    k[..., 0] = 0.0
+    keep = np.arange(1024) // (32 if D == 128 else 64) % 8 != 3  # the tiles of wave 3
+    k[0, 0, ~keep, 0] = -np.inf
+    o, lse = fa_variant(q, k, v, False, variant)
+    want, want_lse = dense_fp64(q[0, 0], k[0, 0][keep], v[0, 0][keep])
+    assert rel(o[0, 0], want) <= TOL
+    assert np.max(np.abs(lse[0, 0] - want_lse)) <= 1e-4
+    k[0, 0, ~keep, 0] = 0.0
+    for key in (0, 100, 500, 1023):
+        bad = k.copy()
+        bad[0, 0, key, 1] = np.nan
+        assert np.isnan(fa_variant(q, bad, v, False, variant)[0]).all()
+    k = (np.abs(k.astype(np.float32)) * (1.0 + np.arange(1024) / 128)[None, None, :, None]).astype(np.float16)
+    q = np.abs(q)
+    q[:, :, 1::2] *= 0.02
+    o, lse = fa_variant(q, k, v, True, variant)
+    want, want_lse = dense_fp64(q[0, 0], k[0, 0], v[0, 0], True)
+    assert rel(o[0, 0], want) <= TOL
+    assert np.max(np.abs(lse[0, 0] - want_lse)) <= 1e-3
