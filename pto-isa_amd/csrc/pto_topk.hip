@@ -26,8 +26,8 @@
 //   indices); the rank of a column in that order then stands in the scores' keys for the column.  4800 x 1024 whole: 42 us (127
 //   with keys in the LDS and a pass over it per stage); 1000 x 256: 6.6 (15).
 // What bounds it: vector instructions, 2520 per row of 1024 (3850 in the integer network this replaced), behind a phase of
-// loads and before one of stores that all waves share: of 25.0 us (4800 x 1024, top 1000, 58 MB = 9 us at 6.5 TB/s) 12 are
-// launch, loads and stores.  Persistent waves that load the next row while they sort one, and wave priorities that let
+// loads and before one of stores that all waves share: of 23.2 us (4800 x 1024, top 1000, 58 MB = 9 us at 6.5 TB/s) 10 are
+// launch, loads and stores (five waves on a SIMD instead of four, at 96 registers of 106: 28.0 and 28.2 us on one card).  Persistent waves that load the next row while they sort one, and wave priorities that let
 // some run ahead, do not hide them (32 us and no change).
 #include <hip/hip_runtime.h>
 
@@ -243,7 +243,7 @@ template <int E, int W>
 constexpr bool kOnlyWhole = E == 1 && W == 4;
 template <int E, int W, bool LOW_DPP, bool WHOLE>
 __global__ __launch_bounds__(kTopkThreads) void TopkRows(float *outScore, uint32_t *outIndex, const float *src, const uint32_t *inIdx,
-                                                         int rows, int validCols, int ld, int topk, int keepBits)
+                                                         int rows, int validCols, int ld, int topk, int keepBits, int through)
 {
     constexpr int N = 64 * E * W, kRows = kTopkWaves / W, kBits = RowSort<E, W, LOW_DPP>::kLaneBits;
     constexpr int kStaged = 64 * E + 4 * E; // words of a wave's results, one of padding behind every 16
@@ -358,8 +358,26 @@ __global__ __launch_bounds__(kTopkThreads) void TopkRows(float *outScore, uint32
         __syncthreads(); // (the exchanges are over)
     if (row0 + wave / W >= rows || count <= 0)
         return;
-    float *toScore = outScore + (size_t)row * (size_t)topk + firstRank;
+    uint32_t *toScore = reinterpret_cast<uint32_t *>(outScore) + (size_t)row * (size_t)topk + firstRank;
     uint32_t *toIndex = outIndex + (size_t)row * (size_t)topk + firstRank;
+    // lane by lane consecutive words; through: past the L2 (launch_topk)
+    auto store = [&](uint32_t *to, auto &&word) __attribute__((always_inline)) {
+        if (through) {
+#pragma unroll
+            for (int e = 0; e < E; ++e) {
+                const int i = e * 64 + lane;
+                if (i < count)
+                    __hip_atomic_store(to + i, word(i), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+            }
+        } else {
+#pragma unroll
+            for (int e = 0; e < E; ++e) {
+                const int i = e * 64 + lane;
+                if (i < count)
+                    to[i] = word(i);
+            }
+        }
+    };
     uint32_t column[E];
 #pragma unroll
     for (int e = 0; e < E; ++e) {
@@ -370,12 +388,7 @@ __global__ __launch_bounds__(kTopkThreads) void TopkRows(float *outScore, uint32
             stagedColumn[laneRank + e + (laneRank + e) / 16] = column[e];
     }
     ordered();
-#pragma unroll
-    for (int e = 0; e < E; ++e) {
-        const int i = e * 64 + lane;
-        if (i < count)
-            toScore[i] = __uint_as_float(staged[i + i / 16]);
-    }
+    store(toScore, [&](int i) { return staged[i + i / 16]; });
     if (kStages == 1) {
         ordered();
 #pragma unroll
@@ -394,12 +407,7 @@ __global__ __launch_bounds__(kTopkThreads) void TopkRows(float *outScore, uint32
         }
         return;
     }
-#pragma unroll
-    for (int e = 0; e < E; ++e) {
-        const int i = e * 64 + lane;
-        if (i < count)
-            toIndex[i] = first + stagedColumn[i + i / 16];
-    }
+    store(toIndex, [&](int i) { return first + stagedColumn[i + i / 16]; });
 }
 
 template <int E, int W>
@@ -417,9 +425,14 @@ int launch_topk(hipStream_t st, float *out_score, uint32_t *out_index, const flo
     constexpr bool kCut = kOnlyWhole<E, W>, kDpp = E >= 8 || kOnlyWhole<E, W>; // (names the one form that there is)
     auto kernel = dpp ? (whole ? TopkRows<E, W, true, true> : TopkRows<E, W, true, kCut>) :
                         (whole ? TopkRows<E, W, kDpp, true> : TopkRows<E, W, kDpp, kCut>);
+    // Results past the L2: a kernel ends with every L2 writing back what is dirty in it, 3 us for the 38 MB of 4800 x 1000 (25.4 ->
+    // 23.3 us; 8192 x 500, top 333 19.2 -> 17.0; 300 x 128 whole 2.69 -> 2.67).  Not where a row's results are less than a store
+    // instruction's 256 bytes (8192 x 64, top 1 3.2 / 3.7, 131072 x 64, top 33 32.6 / 34.1), nor where they are much more than the L2s'
+    // 32 MB, which then are written back while others sort (30000 x 2048, top 1500 261 / 268).
+    const int through = topk >= 64 && 8ll * rows * topk <= 1ll << 26;
     constexpr int kRows = kTopkWaves / W;
     kernel<<<dim3((unsigned)(((long long)rows + kRows - 1) / kRows)), dim3(kTopkThreads), 0, st>>>(out_score, out_index, src, in_idx, rows, valid_cols,
-                                                                                                   ld, topk, keepBits);
+                                                                                                   ld, topk, keepBits, through);
     return pto_amd::check_launch();
 }
 

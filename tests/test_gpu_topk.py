@@ -172,3 +172,19 @@ def test_topk_rejects_bad_arguments():
     assert lib.pto_topk_f32(0, p, p, p, p, 4, 100, 128, 101) == capi.ERR_UNSUPPORTED     # k above the valid columns
     assert lib.pto_topk_f32(0, p, 0, p, p, 4, 100, 128, 10) == capi.ERR_BAD_ARG
     assert lib.pto_topk_f32(0, p, p, p, p, 0, 100, 128, 10) == capi.ERR_BAD_ARG
+
+
+@pytest.mark.parametrize("rows,cols,topk", [(100, 128, 63), (100, 128, 64), (7, 130, 65), (9, 1024, 127), (33, 2048, 2047), (16384, 1024, 512), (16385, 1024, 512)])
+def test_topk_results_past_the_l2(rows, cols, topk):
+    """Both sides of the lines at which results are stored past the L2, rows that are no whole store instruction long: torch's stable sort."""
+    lib = capi.load()
+    g = torch.Generator(device="cuda:0").manual_seed(rows + topk)
+    src = torch.randint(-1000, 1000, (rows, cols), generator=g, device="cuda:0").float()
+    ids = torch.arange(cols, dtype=torch.int32, device="cuda:0")
+    guard = torch.full((rows * topk + 64,), 7.0, device="cuda:0")
+    index = torch.full((rows * topk + 64,), -7, dtype=torch.int32, device="cuda:0")
+    capi.check(lib.pto_topk_f32(torch.cuda.current_stream().cuda_stream, guard.data_ptr(), index.data_ptr(), src.data_ptr(), ids.data_ptr(), rows, cols,
+                                cols, topk), "pto_topk_f32")
+    score, order = torch.sort(src, dim=1, descending=True, stable=True)
+    assert torch.equal(guard[:rows * topk].view(rows, topk), score[:, :topk]) and torch.equal(index[:rows * topk].view(rows, topk), order[:, :topk].int())
+    assert (guard[rows * topk:] == 7.0).all() and (index[rows * topk:] == -7).all()
