@@ -1,6 +1,7 @@
 // Shared host-side helpers of the C ABI translation units.
 #pragma once
 #include <hip/hip_runtime.h>
+#include <stdint.h>
 
 #include "pto_amd.h"
 #if defined(PTO_ST_HOOKS)
@@ -30,6 +31,18 @@ inline int compute_units()
         return n;
     }();
     return cus;
+}
+
+// Are the results of a launch to be stored past the L2 (write-through, system scope)?  A kernel ends with every L2 writing back what
+// is dirty in it, after the last store and before the next kernel: 1.3 us behind 1 MB, 1.8 behind 4, 3.3 behind 12, 5.4 behind 33.
+// Stored through, whole 64-byte pieces (what the kernels that ask write per row and instruction) are on their way at once:
+// GEMM 256 x 3072 x 1024 6.12 -> 5.61 us, 1024 x 3072 x 1024 13.3 -> 11.9, 6144 x 3072 x 512 37.7 -> 31.7, 3072^3 50.6 -> 49.2.
+// Pieces that straddle the 64 bytes are written by parts, which costs more (6144 x 3068 x 512 38.5 -> 50.6), and of a result much
+// larger than the L2s (32 MB) most is written back while other tiles run (4096 x 6144 x 4096, 101 MB: 160.5 -> 157.9, 6144 x 6144 x 2048,
+// 151 MB: 133 and 135).
+inline bool store_through(const void *out, uint64_t rowBytes, uint64_t bytes)
+{
+    return (rowBytes | (uint64_t)(uintptr_t)out) % 64 == 0 && bytes <= (uint64_t)96 << 20;
 }
 
 // Dynamic LDS above 64 KiB has to be opted into per kernel.

@@ -51,6 +51,18 @@ AICORE inline void TileOfBlock(int block, int tilesM, int tilesN, int &tm, int &
     TileOfId<GROUP_M>(RegroupXcd(block, tilesM * tilesN), tilesM, tilesN, tm, tn);
 }
 
+// Four elements of C, past the L2 or into it (pto_amd::store_through), at the alignment of an element.
+// (the wait state: a store of more than 8 bytes may read its registers in the cycle behind it)
+typedef float Four __attribute__((ext_vector_type(4)));
+AICORE inline __attribute__((always_inline)) void StoreFour(float *p, Four v, int through)
+{
+    typedef float C4 __attribute__((ext_vector_type(4), aligned(4)));
+    if (through)
+        asm volatile("global_store_dwordx4 %0, %1, off sc0 sc1\n\ts_nop 0" ::"v"(p), "v"(v) : "memory");
+    else
+        *reinterpret_cast<C4 *>(p) = v;
+}
+
 template <int BM, int BN, int BK, int STAGES, int MIN_BLOCKS, int GROUP_M>
 __global__ __launch_bounds__(kBlockThreads, MIN_BLOCKS) AICORE
     void GemmF16F32(__gm__ float *out, __gm__ const half *src0, __gm__ const half *src1, int m, int n, int k)

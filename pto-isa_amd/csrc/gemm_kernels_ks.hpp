@@ -14,7 +14,7 @@
 // with MFMAs alone.  The place of the copies in the step, raised wave priority and deeper rings changed nothing (1 %).
 // (1000 x 3000 x 2048 on 128 x 96 tiles runs 0.4 us a step: 28 KiB of copies, from beyond the L2.)
 // Small tiles lose there what they win in compute units at work: 512^3 8.96 -> 3.9 us, 1000 x 3000 x 2048 21.1 -> 18.0,
-// 128 x 4096 x 4096 68 -> 12.
+// 128 x 4096 x 4096 68 -> 12.  C past the L2 where that pays (store_through): 1000 x 3072 x 2048 18.5 -> 17.0.
 //
 // Rows past m and columns past n repeat the last one on the way in (their memory may not exist) and are not stored.
 #pragma once
@@ -64,7 +64,7 @@ constexpr int KsLdsBytes() // S stages of 128-byte rows; the partial sums of hal
 
 // HALF: k % 64 == 32, the last step is one of 32 (group 1 has no part in it)
 template <int BM, int BN, int S, int MIN_WAVES, bool HALF, int GROUP_M>
-__global__ __launch_bounds__(512, MIN_WAVES) AICORE void GemmF16F32Ks(float *out, const half *src0, const half *src1, int m, int n, int k)
+__global__ __launch_bounds__(512, MIN_WAVES) AICORE void GemmF16F32Ks(float *out, const half *src0, const half *src1, int m, int n, int k, int through)
 {
     constexpr int MB = BM / 32, NB = BN / 32;                  // 16 x 16 blocks of a wave
     constexpr int kInst = (BM + BN) / 8, kCopies = (kInst + 7) / 8; // copy instructions of 8 rows a step; per wave
@@ -194,7 +194,7 @@ __global__ __launch_bounds__(512, MIN_WAVES) AICORE void GemmF16F32Ks(float *out
             const ks_f32x4 v = acc[i][j] + *reinterpret_cast<const ks_f32x4 *>(sums + ((uint32_t)(pair * MB * NB + idx) * 64u + lane) * 16u);
             const int row = rowLane + 16 * i, col = colLane + 16 * j;
             if (row < m && col < n) // n % 4 == 0: four columns are inside together
-                *reinterpret_cast<ks_c4 *>(out + (int64_t)row * n + col) = v;
+                StoreFour(out + (int64_t)row * n + col, v, through);
         }
     });
 }
@@ -218,7 +218,11 @@ int launch_gemm_ks(hipStream_t st, float *c, const half *a, const half *b, int m
     const long long tiles = (long long)((m + BM - 1) / BM) * ((n + BN - 1) / BN);
     if (tiles > 0x7fffffffll)
         return PTO_ERR_UNSUPPORTED;
-    (k % 64 ? half64 : whole)<<<dim3((unsigned)tiles), dim3(512), lds, st>>>(c, a, b, m, n, k);
+    // (half pieces past the L2 cost no more than they save while C is small: 1000 x 3000 x 2048 18.4 -> 17.9 us, 1024 x 3064 x 1024 13.0 and 13.1,
+    // 1024 x 6136 x 1024 18.8 and 19.8)
+    const uint64_t bytes = 4ull * m * n;
+    const int through = pto_amd::store_through(c, 4ull * n, bytes) || (bytes <= 12u << 20 && (n * 4ull | (uintptr_t)c) % 32 == 0);
+    (k % 64 ? half64 : whole)<<<dim3((unsigned)tiles), dim3(512), lds, st>>>(c, a, b, m, n, k, through);
     return pto_amd::check_launch();
 }
 } // namespace

@@ -344,14 +344,14 @@ AICORE inline __attribute__((always_inline)) void W4TileCompute(__gm__ const hal
 
 // this wave's accumulator blocks to C (row-major, n floats between rows)
 template <int BN, int NMB>
-AICORE inline __attribute__((always_inline)) void W4StoreTile(float *out, int64_t n, int row0, int col0)
+AICORE inline __attribute__((always_inline)) void W4StoreTile(float *out, int64_t n, int row0, int col0, int through)
 {
     constexpr int NNB = BN / 16;
     const uint32_t lane = (uint32_t)hw::lane();
     float *cWave = out + ((int64_t)row0 + 16 * NMB * hw::wave() + lane % 16) * n + col0 + 4 * (lane / 16);
     W4For<0, NMB * NNB>([&](auto idxTag) __attribute__((always_inline)) {
         constexpr int idx = decltype(idxTag)::value, mb = idx / NNB, nb = idx % NNB;
-        *reinterpret_cast<detail::AccFrag *>(cWave + (int64_t)(16 * mb) * n + 16 * nb) = W4ReadAcc<idx>();
+        StoreFour(cWave + (int64_t)(16 * mb) * n + 16 * nb, W4ReadAcc<idx>(), through);
     });
 }
 
@@ -360,7 +360,7 @@ AICORE inline __attribute__((always_inline)) void W4StoreTile(float *out, int64_
 // time and stores the same values.
 template <int BN, int GROUP_M, int NMB>
 __global__ __launch_bounds__(kBlockThreads, 1) AICORE
-    void GemmF16F32W4(__gm__ float *out, __gm__ const half *src0, __gm__ const half *src1, int m, int n, int k)
+    void GemmF16F32W4(__gm__ float *out, __gm__ const half *src0, __gm__ const half *src1, int m, int n, int k, int through)
 {
     constexpr int TM = 64 * NMB;
     const int tilesM = (m + TM - 1) / TM, tilesN = (n + BN - 1) / BN;
@@ -370,7 +370,7 @@ __global__ __launch_bounds__(kBlockThreads, 1) AICORE
     const int row0 = __builtin_amdgcn_readfirstlane(r + TM <= m ? r : m - TM);
     const int col0 = __builtin_amdgcn_readfirstlane(c + BN <= n ? c : n - BN);
     W4TileCompute<BN, NMB>(src0, src1, k, row0, col0);
-    W4StoreTile<BN, NMB>(out, n, row0, col0);
+    W4StoreTile<BN, NMB>(out, n, row0, col0, through);
 }
 
 } // namespace
@@ -391,7 +391,7 @@ int launch_gemm_w4(hipStream_t st, float *c, const half *a, const half *b, int m
     if (attr != PTO_OK)
         return attr;
     const int tiles = ((m + TM - 1) / TM) * ((n + BN - 1) / BN);
-    kernel<<<dim3((unsigned)tiles), dim3(kBlockThreads), lds, st>>>(c, a, b, m, n, k);
+    kernel<<<dim3((unsigned)tiles), dim3(kBlockThreads), lds, st>>>(c, a, b, m, n, k, pto_amd::store_through(c, 4ull * n, 4ull * m * n));
     return pto_amd::check_launch();
 }
 } // namespace

@@ -4,6 +4,7 @@ Bar: max |gpu - ref| <= 2e-3 * max|ref| against an fp32-accumulated reference (t
 restates the reference's CPU-simulation arithmetic); integer-valued inputs must match exactly."""
 import numpy as np
 import pytest
+import torch
 
 from pto_amd import capi, datagen
 
@@ -225,3 +226,20 @@ def test_gemm_rejects_bad_shapes():
     assert lib.pto_gemm_f16f32(0, p, p, p, 128, 256, 16) == capi.ERR_UNSUPPORTED
     assert lib.pto_gemm_f16f32(0, 0, p, p, 128, 256, 64) == capi.ERR_BAD_ARG
     assert lib.pto_gemm_f16f32(0, p, p, p, 0, 256, 64) == capi.ERR_BAD_ARG
+
+
+@pytest.mark.parametrize("m,n,k,shift", [(256, 512, 256, 0), (256, 512, 256, 4), (256, 520, 256, 0), (256, 520, 256, 4), (250, 516, 256, 0), (1024, 3072, 128, 0),
+                                         (1024, 3072, 128, 1), (1024, 3080, 128, 0), (6144, 4096, 128, 0), (6145, 4096, 128, 0)])
+def test_gemm_results_past_the_l2(m, n, k, shift):
+    """Whole and half 64-byte pieces of C, a C that begins `shift` elements past them, and both sides of the largest C that goes
+    past the L2: whole numbers, exact; nothing outside C is written."""
+    lib = capi.load()
+    g = torch.Generator(device="cuda:0").manual_seed(m + n)
+    a, b = (torch.randint(-4, 5, (r, k), generator=g, device="cuda:0").half() for r in (m, n))
+    c = torch.full((m * n + 64,), 7.0, device="cuda:0")
+    for _ in range(2):
+        capi.check(lib.pto_gemm_f16f32(torch.cuda.current_stream().cuda_stream, c.data_ptr() + 4 * shift, a.data_ptr(), b.data_ptr(), m, n, k),
+                   "pto_gemm_f16f32")
+    want = a.float() @ b.float().t()
+    assert torch.equal(c[shift:shift + m * n].view(m, n), want)
+    assert (c[:shift] == 7.0).all() and (c[shift + m * n:] == 7.0).all()
