@@ -89,6 +89,14 @@ PTO_DEV uint16_t f32_to_bf16_bits_rne(float x)
     const uint32_t r = (u + 0x7fffu + ((u >> 16) & 1u)) >> 16;
     return (uint16_t)(((u & 0x7fffffffu) > 0x7f800000u) ? ((u >> 16) | 0x0040u) : r);
 }
+// Two elements with the hardware conversion: for each of the 2^32 inputs the bits of the closed form, one instruction instead of
+// fourteen.  (For results in registers.  The streaming conversion is 4 % slower with it: 2^27 elements 125.5 and 129.7 us.)
+PTO_DEV uint32_t f32x2_to_bf16_bits_rne(float lo, float hi)
+{
+    typedef float F2 __attribute__((ext_vector_type(2)));
+    typedef __bf16 B2 __attribute__((ext_vector_type(2)));
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector((F2{lo, hi}), B2));
+}
 
 PTO_DEV float round_integral(float v, RoundMode mode)
 { // cpu/TCvt.hpp:28-63

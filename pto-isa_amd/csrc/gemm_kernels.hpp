@@ -63,6 +63,34 @@ AICORE inline __attribute__((always_inline)) void StoreFour(float *p, Four v, in
         *reinterpret_cast<C4 *>(p) = v;
 }
 
+typedef uint32_t Words4 __attribute__((ext_vector_type(4)));
+// Eight bf16 elements likewise; the second four only where `both`
+AICORE inline __attribute__((always_inline)) void StoreEight(bfloat16_t *p, Words4 v, bool both, int through)
+{
+    typedef uint32_t C4 __attribute__((ext_vector_type(4), aligned(2)));
+    typedef uint32_t C2 __attribute__((ext_vector_type(2), aligned(2)));
+    if (through) // (whole 64-byte pieces of a row: both)
+        asm volatile("global_store_dwordx4 %0, %1, off sc0 sc1\n\ts_nop 0" ::"v"(p), "v"(v) : "memory");
+    else if (both)
+        *reinterpret_cast<C4 *>(p) = v;
+    else
+        *reinterpret_cast<C2 *>(p) = C2{v[0], v[1]};
+}
+AICORE inline uint32_t Bf16Pair(float lo, float hi) { return ::pto::detail::f32x2_to_bf16_bits_rne(lo, hi); }
+// The lanes 16 .. 31 (48 .. 63) of a against the lanes 0 .. 15 (32 .. 47) of b; the upper half of a against the lower half of b
+AICORE inline __attribute__((always_inline)) void SwapRows(uint32_t &a, uint32_t &b)
+{
+    const auto r = __builtin_amdgcn_permlane16_swap(a, b, false, false);
+    a = r[0];
+    b = r[1];
+}
+AICORE inline __attribute__((always_inline)) void SwapHalves(uint32_t &a, uint32_t &b)
+{
+    const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+    a = r[0];
+    b = r[1];
+}
+
 template <int BM, int BN, int BK, int STAGES, int MIN_BLOCKS, int GROUP_M>
 __global__ __launch_bounds__(kBlockThreads, MIN_BLOCKS) AICORE
     void GemmF16F32(__gm__ float *out, __gm__ const half *src0, __gm__ const half *src1, int m, int n, int k)

@@ -13,8 +13,12 @@
 //
 // What bounds a step: the copies, as in the fp16 kernel.  One 64 x 64 tile takes 0.16 us a step, 64 x 128 0.24, 128 x 128 0.37,
 // 128 x 192 0.52: 79 to 102 bytes per ns and compute unit, where its MFMAs take 0.05, 0.11, 0.21, 0.32.
-// 512 x 512 x 512 fp8 9.1 -> 3.8 us, 256 x 256 x 6144 34.0 -> 11.9, 2048^3 17.3 -> 13.5; 3072^3 stays on 256 x 192 tiles (31
+// 512 x 512 x 512 fp8 9.1 -> 3.6 us, 256 x 256 x 6144 34.0 -> 11.9, 2048^3 17.3 -> 12.8; 3072^3 stays on 256 x 192 tiles (31
 // against 40).
+//
+// The way out: bf16 by the hardware conversion (the integer form was 7 instructions an element), 16 bytes a lane, 64 bytes of a row to a
+// store instruction, past the L2 where that pays (store_through): 2048 x 2048 x 1024 to bf16 11.1 -> 8.6 us in fp8, 9.1 -> 6.7 in
+// fp4, to fp32 11.8 -> 9.6 and 9.9 -> 7.7.
 #pragma once
 #include "gemm_kernels_ks.hpp"
 
@@ -50,7 +54,7 @@ constexpr int MxKsLdsBytes() // S stages of 128-byte rows, two buffers of 32 sca
 template <int FMT_A, int FMT_B, typename OutT, int BM, int BN, int S, int MIN_WAVES, int GROUP_M>
 __global__ __launch_bounds__(512, MIN_WAVES) AICORE
     void GemmMxKs(__gm__ OutT *out, __gm__ const uint8_t *src0, __gm__ const uint8_t *src1, __gm__ const uint8_t *scale0,
-                  __gm__ const uint8_t *scale1, int m, int n, uint32_t ld, uint32_t ldScale)
+                  __gm__ const uint8_t *scale1, int m, int n, uint32_t ld, uint32_t ldScale, int through)
 {
     constexpr bool FP4 = FMT_A == 4;
     static_assert((FMT_A == 4) == (FMT_B == 4), "fp4 with fp4");
@@ -234,50 +238,105 @@ __global__ __launch_bounds__(512, MIN_WAVES) AICORE
     for (int it = 0; it < steps; it += Q)
         StaticFor<0, Q>([&](auto tTag) __attribute__((always_inline)) { step(tTag, it + decltype(tTag)::value); });
 
-    // Partial sums: of every block group g keeps registers 8 g .. 8 g + 7, gives the others to its partner (same rows and
-    // columns, other k) and stores the sums of those it keeps.
+    // Partial sums: a group keeps half of its wave's blocks (of a single block half its registers), gives the rest to its partner
+    // (same rows and columns, other k) and stores the sums of what it keeps.  In quads of four registers: quad u of block
+    // half h is columns 8 u + 4 h .. + 3 of row r32.
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); // the copies past the end
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
     char *sums = hw::lds_base();
     const int pair = wave & 3;
-    // piece 2 idx + u of pair, group: registers 8 g + 4 u .. + 3 of block idx that group g keeps
-    auto piece = [&](int g, int idx, int u) __attribute__((always_inline)) {
-        return reinterpret_cast<ks_f32x4 *>(sums + ((uint32_t)(((pair * 2 + g) * MB * NB + idx) * 2 + u) * 64u + lane) * 16u);
+    constexpr int kQuads = MB * NB * 4, kKept = kQuads / 2;
+    auto quad = [&](auto qTag) __attribute__((always_inline)) {
+        constexpr int idx = decltype(qTag)::value / 4, r = 4 * (decltype(qTag)::value % 4);
+        const f32x16_ks &v = acc[idx / NB][idx % NB];
+        return ks_f32x4{v[r], v[r + 1], v[r + 2], v[r + 3]};
     };
     StaticFor<0, 2>([&](auto gTag) __attribute__((always_inline)) {
         constexpr int g = decltype(gTag)::value;
         if (group != g) {
-            StaticFor<0, MB * NB * 2>([&](auto tag) __attribute__((always_inline)) {
-                constexpr int idx = decltype(tag)::value / 2, u = decltype(tag)::value % 2, r = 8 * g + 4 * u;
-                const f32x16_ks &v = acc[idx / NB][idx % NB];
-                *piece(g, idx, u) = ks_f32x4{v[r], v[r + 1], v[r + 2], v[r + 3]};
+            StaticFor<g * kKept, (g + 1) * kKept>([&](auto qTag) __attribute__((always_inline)) {
+                *reinterpret_cast<ks_f32x4 *>(sums + ((uint32_t)(pair * kQuads + decltype(qTag)::value) * 64u + lane) * 16u) = quad(qTag);
             });
         }
     });
     __syncthreads();
-    // accumulator register v of half h: column 8 (v / 4) + 4 h + v % 4, row r32 of the block
-    const int rowLane = row0 + wm * (BM / 2) + (int)r32, colLane = col0 + wn * (BN / 2) + 4 * (int)h;
+    auto summed = [&](auto qTag) __attribute__((always_inline)) {
+        return quad(qTag) + *reinterpret_cast<const ks_f32x4 *>(sums + ((uint32_t)(pair * kQuads + decltype(qTag)::value) * 64u + lane) * 16u);
+    };
+    // Two quads side by side change lanes: then a store instruction writes 64 bytes of fp32 of each of 16 rows, or 32 of bf16 (eight columns
+    // a lane) of 32 rows, and with the block's other two quads 64 of bf16 of 16 rows.
+    const int rowLane = row0 + wm * (BM / 2), colLane = col0 + wn * (BN / 2);
+    auto words = [](const ks_f32x4 &v) __attribute__((always_inline)) { return __builtin_bit_cast(Words4, v); };
     StaticFor<0, 2>([&](auto gTag) __attribute__((always_inline)) {
         constexpr int g = decltype(gTag)::value;
-        if (group == g) {
-            StaticFor<0, MB * NB * 2>([&](auto tag) __attribute__((always_inline)) {
-                constexpr int idx = decltype(tag)::value / 2, u = decltype(tag)::value % 2, r = 8 * g + 4 * u;
-                const f32x16_ks &w = acc[idx / NB][idx % NB];
-                const ks_f32x4 v = ks_f32x4{w[r], w[r + 1], w[r + 2], w[r + 3]} + *piece(g, idx, u);
-                const int row = rowLane + 32 * (idx / NB), col = colLane + 32 * (idx % NB) + 8 * (r / 4);
-                if (row < m && col < n) { // n % 4 == 0: four columns are inside together
-                    OutT *dst = out + (int64_t)row * n + col;
-                    if constexpr (std::is_same_v<OutT, float>) {
-                        *reinterpret_cast<ks_c4 *>(dst) = v;
-                    } else {
-                        const uint32_t lo = (uint32_t)detail::f32_to_bf16_bits_rne(v.x) | ((uint32_t)detail::f32_to_bf16_bits_rne(v.y) << 16);
-                        const uint32_t hi = (uint32_t)detail::f32_to_bf16_bits_rne(v.z) | ((uint32_t)detail::f32_to_bf16_bits_rne(v.w) << 16);
-                        typedef uint32_t u32x2 __attribute__((ext_vector_type(2), aligned(2)));
-                        *reinterpret_cast<u32x2 *>(dst) = u32x2{lo, hi};
-                    }
+        if (group != g)
+            return;
+        if constexpr (std::is_same_v<OutT, float>) {
+            // (one block, past no cache: quads as they lie, 32 bytes of a row; 256 x 256 x 6144 12.2 us, 12.3 with the exchange.  Larger tiles:
+            // 2048 x 2044 x 1024 in fp8 12.2 as they lie, 11.6 with it)
+            if (kKept == 2 && !through) {
+                StaticFor<g * kKept, (g + 1) * kKept>([&](auto qTag) __attribute__((always_inline)) {
+                    constexpr int q = decltype(qTag)::value, idx = q / 4;
+                    const ks_f32x4 v = summed(qTag);
+                    const int row = rowLane + 32 * (idx / NB) + (int)r32, col = colLane + 32 * (idx % NB) + 8 * (q % 4) + 4 * (int)h;
+                    if (row < m && col < n) // n % 4 == 0: four columns are inside together
+                        StoreFour(out + (int64_t)row * n + col, v, 0);
+                });
+                return;
+            }
+            StaticFor<0, kKept / 2>([&](auto tag) __attribute__((always_inline)) {
+                constexpr int q = g * kKept + 2 * decltype(tag)::value, idx = q / 4;
+                Words4 x = words(summed(std::integral_constant<int, q>())), y = words(summed(std::integral_constant<int, q + 1>()));
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    uint32_t xi = x[i], yi = y[i];
+                    SwapRows(xi, yi);
+                    x[i] = xi;
+                    y[i] = yi;
+                }
+                const int row = rowLane + 32 * (idx / NB) + (int)(lane % 16), col = colLane + 32 * (idx % NB) + 8 * (q % 4 + (int)(lane / 16 % 2)) + 4 * (int)h;
+                if (col < n) {
+                    if (row < m)
+                        StoreFour(out + (int64_t)row * n + col, __builtin_bit_cast(Four, x), through);
+                    if (row + 16 < m)
+                        StoreFour(out + (int64_t)(row + 16) * n + col, __builtin_bit_cast(Four, y), through);
                 }
             });
+        } else {
+            auto eight = [&](auto qTag) __attribute__((always_inline)) { // columns 8 (q + h) .. + 7 of the block
+                const ks_f32x4 x = summed(qTag), y = summed(std::integral_constant<int, decltype(qTag)::value + 1>());
+                uint32_t x0 = Bf16Pair(x[0], x[1]), x1 = Bf16Pair(x[2], x[3]), y0 = Bf16Pair(y[0], y[1]), y1 = Bf16Pair(y[2], y[3]);
+                SwapHalves(x0, y0);
+                SwapHalves(x1, y1);
+                return Words4{x0, x1, y0, y1};
+            };
+            if constexpr (kKept % 4 == 0) {
+                StaticFor<0, kKept / 4>([&](auto tag) __attribute__((always_inline)) {
+                    constexpr int q = g * kKept + 4 * decltype(tag)::value, idx = q / 4;
+                    Words4 x = eight(std::integral_constant<int, q>()), y = eight(std::integral_constant<int, q + 2>());
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        uint32_t xi = x[i], yi = y[i];
+                        SwapRows(xi, yi);
+                        x[i] = xi;
+                        y[i] = yi;
+                    }
+                    const int row = rowLane + 32 * (idx / NB) + (int)(lane % 16), col = colLane + 32 * (idx % NB) + 16 * (int)(lane / 16 % 2) + 8 * (int)h;
+                    if (col < n) {
+                        if (row < m)
+                            StoreEight(out + (int64_t)row * n + col, x, col + 4 < n, through);
+                        if (row + 16 < m)
+                            StoreEight(out + (int64_t)(row + 16) * n + col, y, col + 4 < n, through);
+                    }
+                });
+            } else {
+                constexpr int q = g * kKept; // half a block
+                const Words4 x = eight(std::integral_constant<int, q>());
+                const int row = rowLane + (int)r32, col = colLane + 8 * (q + (int)h);
+                if (row < m && col < n)
+                    StoreEight(out + (int64_t)row * n + col, x, col + 4 < n, 0);
+            }
         }
     });
 }
@@ -301,7 +360,7 @@ int launch_gemm_mxks(hipStream_t st, void *c, const uint8_t *a, const uint8_t *b
     if (tiles > 0x7fffffffll)
         return PTO_ERR_UNSUPPORTED;
     kernel<<<dim3((unsigned)tiles), dim3(512), lds, st>>>(reinterpret_cast<OutT *>(c), a, b, sa, sb, m, n, (uint32_t)(FMT_A == 4 ? k / 2 : k),
-                                                          (uint32_t)(k / 32));
+                                                          (uint32_t)(k / 32), pto_amd::store_through(c, sizeof(OutT) * (uint64_t)n, sizeof(OutT) * (uint64_t)m * n));
     return pto_amd::check_launch();
 }
 } // namespace

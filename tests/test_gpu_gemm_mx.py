@@ -385,3 +385,26 @@ def test_mx_gemm_k_split_scale_of_every_block(oracle, fmt):
         assert rc == 0 and np.array_equal(got.astype(np.float64), want), shape
         rc, got = _mx_variant(ra, rb, rsa, rsb, fmt, 7 + shape)
         assert rc == 0 and np.all(np.isfinite(got)) and rel_err(got, rwant) <= TOL, shape
+
+
+@pytest.mark.parametrize("c_fp32", [True, False])
+@pytest.mark.parametrize("variant", [5, 6, 7, 8, 9, 10, 11, 12])
+@pytest.mark.parametrize("m,n,shift", [(256, 256, 0), (256, 256, 1), (300, 288, 0), (257, 260, 0), (289, 332, 0), (270, 264, 2)])
+def test_mx_gemm_results_in_pieces_of_64_bytes(variant, m, n, shift, c_fp32):
+    """C in whole pieces of 64 bytes, in parts of them, beginning `shift` elements past one, with four columns behind the last whole eight, on
+    every tile shape: whole numbers, exact (below 2^8 in bf16), and nothing outside C is written."""
+    import torch
+    k, dtype = 1024, torch.float32 if c_fp32 else torch.bfloat16
+    rng = np.random.default_rng(m + n)
+    codes = datagen.fp8_encode(np.array([-1.0, 0.0, 1.0]), 0).astype(np.uint8)
+    pick = [rng.choice(3, size=(rows, k), p=(0.05, 0.9, 0.05)) for rows in (m, n)]
+    want = (pick[0] - 1) @ (pick[1] - 1).T
+    assert np.abs(want).max() < 256
+    a, b = (torch.from_numpy(codes[p]).to("cuda:0") for p in pick)
+    sa, sb = (torch.full((rows, k // 32), 127, dtype=torch.uint8, device="cuda:0") for rows in (m, n))
+    c = torch.full((m * n + 64,), 7.0, dtype=dtype, device="cuda:0")
+    at = c.data_ptr() + shift * c.element_size()
+    capi.check(capi.load_st().pto_gemm_mxfp8_variant(torch.cuda.current_stream().cuda_stream, at, a.data_ptr(), b.data_ptr(), sa.data_ptr(), sb.data_ptr(),
+                                                     m, n, k, 0, int(c_fp32), variant), "pto_gemm_mxfp8_variant")
+    assert np.array_equal(c[shift:shift + m * n].view(m, n).float().cpu().numpy(), want.astype(np.float32))
+    assert (c[:shift] == 7.0).all() and (c[shift + m * n:] == 7.0).all()
