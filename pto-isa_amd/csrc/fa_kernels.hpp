@@ -2,6 +2,7 @@
 // wave grid (1 x 4 in pto_fa.hip, 1 x 8 in pto_fa_w8.hip and pto_fa_split.hip).  Include after <pto/pto-inst.hpp>.
 #pragma once
 #include "common.hpp"
+#include "stores.hpp"
 #include <cstdlib>
 
 using namespace pto;
@@ -151,7 +152,7 @@ template <int D, bool CAUSAL, bool OUT_F32, int MIN_BLOCKS, int kBKV = kBKVDefau
 __global__ __launch_bounds__(kBlockThreads, MIN_BLOCKS) AICORE void FlashAttnFwd(__gm__ void *outO, __gm__ float *outLse,
                                                                       __gm__ const half *qAll, __gm__ const half *kAll,
                                                                       __gm__ const half *vAll, [[maybe_unused]] int perXcd, int seqQ,
-                                                                      int seqKv, int numBH, int causalOff)
+                                                                      int seqKv, int numBH, int causalOff, [[maybe_unused]] int through)
 {
     constexpr int NQ = NQ_;        // 32-query blocks per wave
     constexpr int kBQ = kBQ1 * NQ; // columns of the tile types: 32 NQ per wave
@@ -778,23 +779,44 @@ __global__ __launch_bounds__(kBlockThreads, MIN_BLOCKS) AICORE void FlashAttnFwd
         const float total = SumOverHalves(runSum[nb]);
         const float inv = 1.0f / total;
         const int64_t row = (int64_t)bh * seqQ + myQuery + 32 * nb;
+        // A lane has four of every eight columns of its query; the lanes change places so that a store instruction writes 64 bytes
+        // of each of 16 queries: quads side by side for fp32, for fp16 first halves (eight columns to a lane), then rows of 16 lanes
+        const int64_t row16 = row - (lane & 31) + (lane & 15);
 #pragma unroll
-        for (int db = 0; db < DB; ++db)
+        for (int db = 0; db < DB; ++db) {
+            const auto &o = oAcc[db].st.f[0][nb];
+            if constexpr (OUT_F32) {
+                float *to = static_cast<float *>(outO) + row16 * D + db * 32 + 8 * (lane / 16 % 2) + 4 * (int)hHalf;
 #pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                const int d = db * 32 + g * 8 + (int)hHalf * 4;
-                float o4[4];
+                for (int g = 0; g < 4; g += 2) {
+                    Four x, y;
 #pragma unroll
-                for (int r = 0; r < 4; ++r)
-                    o4[r] = oAcc[db].st.f[0][nb][g * 4 + r] * inv;
-                if constexpr (OUT_F32) {
-                    f32x4 v = {o4[0], o4[1], o4[2], o4[3]};
-                    *reinterpret_cast<f32x4 *>(static_cast<float *>(outO) + row * D + d) = v;
-                } else {
-                    f16x4 v = {(half)o4[0], (half)o4[1], (half)o4[2], (half)o4[3]};
-                    *reinterpret_cast<f16x4 *>(static_cast<half *>(outO) + row * D + d) = v;
+                    for (int r = 0; r < 4; ++r) {
+                        uint32_t a = __builtin_bit_cast(uint32_t, o[4 * g + r] * inv), b = __builtin_bit_cast(uint32_t, o[4 * g + 4 + r] * inv);
+                        SwapRows(a, b);
+                        x[r] = __builtin_bit_cast(float, a);
+                        y[r] = __builtin_bit_cast(float, b);
+                    }
+                    StoreFour(to + 8 * g, x, through);
+                    StoreFour(to + 8 * g + 16 * D, y, through);
                 }
+            } else {
+                half *to = static_cast<half *>(outO) + row16 * D + db * 32 + 16 * (lane / 16 % 2) + 8 * (int)hHalf;
+                uint32_t w[8]; // quad g: words 2 g and 2 g + 1
+#pragma unroll
+                for (int i = 0; i < 8; ++i)
+                    w[i] = HalfPair(o[2 * i] * inv, o[2 * i + 1] * inv);
+                SwapHalves(w[0], w[2]);
+                SwapHalves(w[1], w[3]);
+                SwapHalves(w[4], w[6]);
+                SwapHalves(w[5], w[7]);
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    SwapRows(w[i], w[4 + i]);
+                StoreEight(to, Words4{w[0], w[1], w[2], w[3]}, true, through);
+                StoreEight(to + 16 * D, Words4{w[4], w[5], w[6], w[7]}, true, through);
             }
+        }
         if (outLse != nullptr && hHalf == 0) {
             const float scale = D == 128 ? 0.08838834764831845f : 0.125f;
             outLse[row] = runMax[nb] * scale + __builtin_logf(total);
@@ -838,7 +860,8 @@ int launch_fa(hipStream_t st, void *o, float *lse, const half *q, const half *k,
             blocks = padded;
         }
     }
-    kernel<<<dim3((unsigned)blocks), dim3(kBlockThreads), lds, st>>>(o, lse, q, k, v, perXcd, seqQ, seqKv, numBH, causalOff);
+    kernel<<<dim3((unsigned)blocks), dim3(kBlockThreads), lds, st>>>(o, lse, q, k, v, perXcd, seqQ, seqKv, numBH, causalOff,
+                                                               fa_through(o, D, OUT_F32, numBH, seqQ));
     return pto_amd::check_launch();
 }
 } // namespace

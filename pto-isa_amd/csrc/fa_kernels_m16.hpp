@@ -6,6 +6,7 @@
 // Include after <pto/pto-inst.hpp> with PTO_MFMA_M 16, PTO_WAVES_M 1, PTO_WAVES_N 8.
 #pragma once
 #include "common.hpp"
+#include "stores.hpp"
 #include <cstdlib>
 
 using namespace pto;
@@ -106,7 +107,7 @@ AICORE inline s16x4 DsReadTr16b(uint32_t addr)
 template <int D, bool CAUSAL, bool OUT_F32>
 __global__ __launch_bounds__(kBlockThreads, 1) AICORE void FlashAttnFwdM16(__gm__ void *outO, __gm__ float *outLse, __gm__ const half *qAll,
                                                                            __gm__ const half *kAll, __gm__ const half *vAll, int heads,
-                                                                           int seqQ, int seqKv, int numBH, int causalOff)
+                                                                           int seqQ, int seqKv, int numBH, int causalOff, int through)
 {
     constexpr int kBQ = kBQ16, kBKV = kBKV16;
     constexpr int NQ = 2;          // 16-query column blocks per wave
@@ -452,19 +453,21 @@ __global__ __launch_bounds__(kBlockThreads, 1) AICORE void FlashAttnFwdM16(__gm_
         const float total = SumOverRowGroups(runSum[nq]);
         const float inv = 1.0f / total;
         const int64_t row = (int64_t)bh * seqQ + myQuery + 16 * nq;
+        if constexpr (OUT_F32) {
 #pragma unroll
-        for (int db = 0; db < DB; ++db) {
-            const int d = db * 16 + (int)g * 4;
-            float o4[4];
+            for (int db = 0; db < DB; ++db) {
+                const auto &o = oAcc[db][nq];
+                StoreFour(static_cast<float *>(outO) + row * D + db * 16 + (int)g * 4, Four{o[0] * inv, o[1] * inv, o[2] * inv, o[3] * inv}, through);
+            }
+        } else { // two blocks side by side change lanes: eight columns of one of them to a lane (groups 0 .. 3: columns 0, 16, 8, 24 onwards)
 #pragma unroll
-            for (int r = 0; r < 4; ++r)
-                o4[r] = oAcc[db][nq][r] * inv;
-            if constexpr (OUT_F32) {
-                f32x4 v = {o4[0], o4[1], o4[2], o4[3]};
-                *reinterpret_cast<f32x4 *>(static_cast<float *>(outO) + row * D + d) = v;
-            } else {
-                f16x4 v = {(half)o4[0], (half)o4[1], (half)o4[2], (half)o4[3]};
-                *reinterpret_cast<f16x4 *>(static_cast<half *>(outO) + row * D + d) = v;
+            for (int db = 0; db < DB; db += 2) {
+                const auto &x = oAcc[db][nq], &y = oAcc[db + 1][nq];
+                uint32_t x0 = HalfPair(x[0] * inv, x[1] * inv), x1 = HalfPair(x[2] * inv, x[3] * inv);
+                uint32_t y0 = HalfPair(y[0] * inv, y[1] * inv), y1 = HalfPair(y[2] * inv, y[3] * inv);
+                SwapRows(x0, y0);
+                SwapRows(x1, y1);
+                StoreEight(static_cast<half *>(outO) + row * D + db * 16 + 16 * ((int)g % 2) + 8 * ((int)g / 2), Words4{x0, x1, y0, y1}, true, through);
             }
         }
         if (outLse != nullptr && g == 0)
@@ -491,7 +494,8 @@ int launch_fa_m16(hipStream_t st, void *o, float *lse, const half *q, const half
     const long long blocks = (long long)numBH * (seqQ / kBQ16);
     if (blocks > 0x7fffffffLL)
         return PTO_ERR_UNSUPPORTED;
-    kernel<<<dim3((unsigned)blocks), dim3(kBlockThreads), lds, st>>>(o, lse, q, k, v, heads, seqQ, seqKv, numBH, causalOff);
+    kernel<<<dim3((unsigned)blocks), dim3(kBlockThreads), lds, st>>>(o, lse, q, k, v, heads, seqQ, seqKv, numBH, causalOff,
+                                                               fa_through(o, D, OUT_F32, numBH, seqQ));
     return pto_amd::check_launch();
 }
 } // namespace

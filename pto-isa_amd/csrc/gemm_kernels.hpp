@@ -4,6 +4,7 @@
 #include <pto/pto-inst.hpp>
 
 #include "common.hpp"
+#include "stores.hpp"
 
 using namespace pto;
 
@@ -49,46 +50,6 @@ template <int GROUP_M>
 AICORE inline void TileOfBlock(int block, int tilesM, int tilesN, int &tm, int &tn)
 {
     TileOfId<GROUP_M>(RegroupXcd(block, tilesM * tilesN), tilesM, tilesN, tm, tn);
-}
-
-// Four elements of C, past the L2 or into it (pto_amd::store_through), at the alignment of an element.
-// (the wait state: a store of more than 8 bytes may read its registers in the cycle behind it)
-typedef float Four __attribute__((ext_vector_type(4)));
-AICORE inline __attribute__((always_inline)) void StoreFour(float *p, Four v, int through)
-{
-    typedef float C4 __attribute__((ext_vector_type(4), aligned(4)));
-    if (through)
-        asm volatile("global_store_dwordx4 %0, %1, off sc0 sc1\n\ts_nop 0" ::"v"(p), "v"(v) : "memory");
-    else
-        *reinterpret_cast<C4 *>(p) = v;
-}
-
-typedef uint32_t Words4 __attribute__((ext_vector_type(4)));
-// Eight bf16 elements likewise; the second four only where `both`
-AICORE inline __attribute__((always_inline)) void StoreEight(bfloat16_t *p, Words4 v, bool both, int through)
-{
-    typedef uint32_t C4 __attribute__((ext_vector_type(4), aligned(2)));
-    typedef uint32_t C2 __attribute__((ext_vector_type(2), aligned(2)));
-    if (through) // (whole 64-byte pieces of a row: both)
-        asm volatile("global_store_dwordx4 %0, %1, off sc0 sc1\n\ts_nop 0" ::"v"(p), "v"(v) : "memory");
-    else if (both)
-        *reinterpret_cast<C4 *>(p) = v;
-    else
-        *reinterpret_cast<C2 *>(p) = C2{v[0], v[1]};
-}
-AICORE inline uint32_t Bf16Pair(float lo, float hi) { return ::pto::detail::f32x2_to_bf16_bits_rne(lo, hi); }
-// The lanes 16 .. 31 (48 .. 63) of a against the lanes 0 .. 15 (32 .. 47) of b; the upper half of a against the lower half of b
-AICORE inline __attribute__((always_inline)) void SwapRows(uint32_t &a, uint32_t &b)
-{
-    const auto r = __builtin_amdgcn_permlane16_swap(a, b, false, false);
-    a = r[0];
-    b = r[1];
-}
-AICORE inline __attribute__((always_inline)) void SwapHalves(uint32_t &a, uint32_t &b)
-{
-    const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
-    a = r[0];
-    b = r[1];
 }
 
 template <int BM, int BN, int BK, int STAGES, int MIN_BLOCKS, int GROUP_M>

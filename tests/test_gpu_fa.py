@@ -453,3 +453,21 @@ def test_fa_keys_split_over_single_waves_special_values(D, variant):
     want, want_lse = dense_fp64(q[0, 0], k[0, 0], v[0, 0], True)
     assert rel(o[0, 0], want) <= TOL
     assert np.max(np.abs(lse[0, 0] - want_lse)) <= 1e-3
+
+
+@pytest.mark.parametrize("B,H,S,D,causal", [(2, 16, 2048, 128, 0), (2, 16, 2048, 128, 1), (1, 16, 4096, 128, 1), (16, 16, 128, 128, 0), (3, 100, 128, 64, 1), (16, 16, 256, 64, 0)])
+@pytest.mark.parametrize("o_fp32", [False, True])
+def test_fa_output_at_any_element(B, H, S, D, causal, o_fp32):
+    """The kernels without key groups store O in 64-byte pieces, past the L2 where O begins at one: the same bits from any element on, nothing
+    around O is written, and rows of every head against float64."""
+    g = torch.Generator(device="cuda:0").manual_seed(S + D)
+    q, k, v = (torch.randn((B, H, S, D), generator=g, device="cuda:0").half() for _ in range(3))
+    dtype, size, out = torch.float32 if o_fp32 else torch.float16, B * H * S * D, []
+    for shift in (0, 32, 8, 1):
+        o, lse = torch.full((size + 128,), 7.0, dtype=dtype, device="cuda:0"), torch.full((B, H, S), float("nan"), device="cuda:0")
+        capi.check(capi.load().pto_fa_fwd_f16(torch.cuda.current_stream().cuda_stream, o.data_ptr() + shift * o.element_size(), lse.data_ptr(), q.data_ptr(),
+                                              k.data_ptr(), v.data_ptr(), B, H, S, S, D, causal, int(o_fp32)), "pto_fa_fwd_f16")
+        assert (o[:shift] == 7.0).all() and (o[shift + size:] == 7.0).all()
+        out.append(o[shift:shift + size].clone())
+        assert torch.equal(out[0], out[-1])
+    check_sampled_rows_of_every_head(*(t.cpu().numpy() for t in (q, k, v, out[0].view(B, H, S, D).float(), lse)), causal != 0, seed=5)
