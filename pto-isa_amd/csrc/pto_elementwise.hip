@@ -58,8 +58,10 @@ __global__ __launch_bounds__(kBlockThreads) AICORE void CvtF32(__gm__ D *dst, __
 // 16 bytes and stores 8, so that every load instruction of a wave covers 1 KiB of consecutive addresses and every store
 // 512 bytes (a Vec tile gives a lane eight consecutive elements, i.e. two loads 32 bytes apart per lane and half-used
 // lines per instruction), all loads of a lane are in flight before the first conversion, and there is no barrier; the
-// stores are non-temporal (measured with inputs and outputs that no cache holds: 6.5 against 6.2 TB/s with plain
-// stores).  Same element function as TCVT (detail::convert), so the results are the same bits.  The last workgroup takes
+// stores go through the L2 to memory (system scope): plain stores leave 32 MB dirty there, which are written back behind the last one (2^27
+// elements to fp16: plain 6.2 TB/s, non-temporal 124.1 us = 6.49, through 121.3 = 6.64; 33 M 31.1 and 29.3 us, 16.5 M to bf16 16.0 and
+// 15.7, 2 M 2.70 and 2.18; geometric mean of 60 sizes 1.023).  What is not whole pieces stays non-temporal: a part of 64 bytes written through
+// holds up the end of the kernel (700001 elements 2.7 and 3.0 us).  Same element function as TCVT (detail::convert), so the results are the same bits.  The last workgroup takes
 // what is left behind the whole pieces, element by element past the last four: as a launch of its own that rest took
 // 3.7 us (16 524 000 elements 20.0 -> 16.2 us, 6.1 TB/s; 2^27 - 5 elements 126.6 -> 123.9, 6.5 TB/s).  LOADS: 16-byte loads of a
 // lane: four; two for the modes that round in integer arithmetic, where more waves hide more of it (2^26 elements downwards: tile
@@ -87,7 +89,7 @@ __global__ __launch_bounds__(kBlockThreads) void CvtF32Stream(D *dst, const floa
 #pragma unroll
             for (int j = 0; j < 4; ++j)
                 y[j] = cvt(x[i][j]);
-            __builtin_nontemporal_store(y, reinterpret_cast<u16x4 *>(dst + base + (size_t)i * kPerStep));
+            __hip_atomic_store(reinterpret_cast<uint64_t *>(dst + base + (size_t)i * kPerStep), __builtin_bit_cast(uint64_t, y), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
         }
         return;
     }
