@@ -22,6 +22,13 @@
 // * topk of an eighth of the padded row length or less: once the sorted runs are as long as topk (rounded up to keys per lane times a power of
 //   two), a merge of two runs keeps their larger halves only, in both runs' lanes, and its sort passes no longer cover the
 //   dropped half.
+// * Few of many (topk of an eighth of the padded row or less, 257 columns or more): a threshold first, then only the keys that reach it are sorted.  The
+//   topk-th largest of the maxima of disjoint groups of keys (64 to 256 groups a wave) is no larger than the topk-th largest key, and not much more
+//   than topk keys reach it (of 1024, 256 groups: 68 for topk 60).  It is found by halving an interval of the scores' order, the groups that reach
+//   the middle counted by ballots; those keys go into a list in the LDS and through the network of 64, 128, 256 or 512 keys in one wave.
+//   Where too many keys equal the threshold (masked rows), as many of them as are wanted are taken in the order of their columns; where that does
+//   not do either, or the indices do not increase, the row is sorted as before.  4800 x 1024, top 40 19.7 -> 8.3 us; 1200 x 4096, top 50 25.1 -> 13.9;
+//   1584 x 2960, top 60 35.8 -> 17.6; 128 x 4096, top 50 10.2 -> 6.5; all equal but 2 %: 4800 x 1024, top 40 20.6 -> 11.0.
 // * Any other index vector: the same network sorts the (index, column) pairs first, once per workgroup (the rows share their
 //   indices); the rank of a column in that order then stands in the scores' keys for the column.  4800 x 1024 whole: 42 us (127
 //   with keys in the LDS and a pass over it per stage); 1000 x 256: 6.6 (15).
@@ -241,16 +248,45 @@ constexpr int kWholeBits = 2;
 // one key per lane and four waves per row: for few rows of which more than 16 are wanted, where the whole sort is the shorter one
 template <int E, int W>
 constexpr bool kOnlyWhole = E == 1 && W == 4;
-template <int E, int W, bool LOW_DPP, bool WHOLE>
-__global__ __launch_bounds__(kTopkThreads) void TopkRows(float *outScore, uint32_t *outIndex, const float *src, const uint32_t *inIdx,
-                                                         int rows, int validCols, int ld, int topk, int keepBits, int through)
+// kCut: merges that keep what topk asks for; kSelect: by a threshold, kCut where that fails.  What bounds kSelect: 5.5 us of 8.3 (4800 x 1024, top 40) are
+// launch and the 20 MB of the rows; the rest is scalar and vector instructions in equal parts.  Four places of the interval at a time instead
+// of one took 2.2 us more (scalar instructions), positions in the list by ballots instead of one scan over the lanes 1.2.
+constexpr int kMostSelected = 8; // times 64 keys
+enum Mode { kCut, kWhole, kSelect };
+// the largest value of the wave, the same in every lane's scalar registers; the sum up to and with this lane
+__device__ inline uint32_t WaveMax(uint32_t v)
+{
+    auto with = [&](uint32_t o) { v = o > v ? o : v; };
+    with(LaneMove<0>(v));
+    with(LaneMove<1>(v));
+    with(LaneMove<2>(v));
+    with(LaneMove<3>(v));
+    with((uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xa, 0xf, false)); // row_bcast:15
+    with((uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xc, 0xf, false)); // row_bcast:31
+    return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
+}
+__device__ inline uint32_t WaveScan(uint32_t v)
+{
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xf, 0xf, false); // row_shr:1, 2, 4, 8
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xf, 0xf, false);
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xf, 0xf, false);
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xf, 0xf, false);
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xa, 0xf, false);
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xc, 0xf, false);
+    return v;
+}
+template <int E, int W, bool LOW_DPP, Mode MODE>
+__global__ __launch_bounds__(kTopkThreads, MODE == kSelect && E == 16 ? 4 : 1) void TopkRows(float *outScore, uint32_t *outIndex, const float *src, const uint32_t *inIdx,
+                                                         int rows, int validCols, int ld, int topk, int keepBits, int through,
+                                                         [[maybe_unused]] int share)
 {
     constexpr int N = 64 * E * W, kRows = kTopkWaves / W, kBits = RowSort<E, W, LOW_DPP>::kLaneBits;
     constexpr int kStaged = 64 * E + 4 * E; // words of a wave's results, one of padding behind every 16
     constexpr int kStages = E <= 8 ? 2 : 1;  // scores and columns side by side, or one after the other (LDS for four workgroups more)
     // exchanges, then results (or, between two sorts, the ranks of the columns); behind them the columns in the order of their indices
     constexpr size_t kExchange = W > 1 ? (size_t)kTopkWaves * E * 64 * 8 : 0, kStage = (size_t)kTopkWaves * kStaged * 4 * kStages;
-    constexpr size_t kWork = kExchange > kStage ? kExchange : kStage;
+    constexpr size_t kSelected = MODE == kSelect ? 128 + (size_t)kRows * 68 * kMostSelected * 8 : 0, kSort = kExchange > kStage ? kExchange : kStage;
+    constexpr size_t kWork = kSort > kSelected ? kSort : kSelected;
     static_assert(kWork >= (size_t)N * 2, "the ranks fit");
     __shared__ __attribute__((aligned(16))) char lds[kWork + (size_t)N * 2];
     uint16_t *rankOf = reinterpret_cast<uint16_t *>(lds), *columnOf = reinterpret_cast<uint16_t *>(lds + kWork);
@@ -273,21 +309,32 @@ __global__ __launch_bounds__(kTopkThreads) void TopkRows(float *outScore, uint32
                 to[e] = from[i0 + e * 64 < (uint32_t)validCols ? i0 + e * 64 : (uint32_t)validCols - 1u];
         }
     };
-    uint32_t bits[E], ids[E];
+    uint32_t bits[E];
     const uint32_t *scores = reinterpret_cast<const uint32_t *>(src) + (size_t)row * (size_t)ld;
     load(scores, bits);
-    load(inIdx, ids);
 
     // are the indices first, first + 1, ... or at least increasing with the column?  (then the column decides among equal
-    // scores, as the index would; the same answer in every wave of the workgroup)
+    // scores, as the index would; the same answer in every wave of the workgroup.)  Where a threshold selects, the four waves look at
+    // a quarter each
+    constexpr bool kQuarters = MODE == kSelect && W < 4;
+    constexpr int kIds = kQuarters ? E * W / 4 : E;
+    uint32_t ids[kIds];
+    const uint32_t id0 = kQuarters ? (uint32_t)(wave * kIds * 64 + lane) : i0;
+    if constexpr (kQuarters) {
+#pragma unroll
+        for (int e = 0; e < kIds; ++e)
+            ids[e] = inIdx[id0 + e * 64 < (uint32_t)validCols ? id0 + e * 64 : (uint32_t)validCols - 1u];
+    } else {
+        load(inIdx, ids);
+    }
     const uint32_t first = inIdx[0];
     uint32_t wrong = 0;
 #pragma unroll
-    for (int e = 0; e < E; ++e) {
-        const uint32_t at = i0 + e * 64 < (uint32_t)validCols ? i0 + e * 64 : (uint32_t)validCols - 1u;
+    for (int e = 0; e < kIds; ++e) {
+        const uint32_t at = id0 + e * 64 < (uint32_t)validCols ? id0 + e * 64 : (uint32_t)validCols - 1u;
         wrong |= (ids[e] - first) ^ at;
     }
-    auto everyone = [&](bool v) { return W > 1 ? __syncthreads_and(v) != 0 : __builtin_amdgcn_ballot_w64(!v) == 0; };
+    auto everyone = [&](bool v) { return W > 1 || kQuarters ? __syncthreads_and(v) != 0 : __builtin_amdgcn_ballot_w64(!v) == 0; };
     const bool consecutive = everyone(wrong == 0 && first <= 0xffffffffu - (uint32_t)validCols);
     bool increasing = consecutive;
     if (__builtin_expect(!consecutive, 0)) {
@@ -306,13 +353,220 @@ __global__ __launch_bounds__(kTopkThreads) void TopkRows(float *outScore, uint32
     uint32_t *staged = reinterpret_cast<uint32_t *>(lds) + wave * (kStaged * kStages), *stagedColumn = staged + (kStages - 1) * kStaged;
     const int firstRank = waveOfRow * 64 * E, laneRank = (int)LaneRank((uint32_t)lane) * E, count = topk - firstRank;
     auto ordered = [] { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); __builtin_amdgcn_wave_barrier(); };
+    // lane by lane consecutive words; through: past the L2 (launch_topk)
+    constexpr bool kThrough = MODE != kCut || N > 512; // (below, topk is 64 at most: 1000 x 300, top 30 5.2 us with the branch, 5.1 without)
+    constexpr auto eTag = std::integral_constant<int, E>();
+    auto store = [&](auto keys, uint32_t *to, int n, auto &&word) __attribute__((always_inline)) {
+        if (kThrough && through) {
+#pragma unroll
+            for (int e = 0; e < decltype(keys)::value; ++e) {
+                const int i = e * 64 + lane;
+                if (i < n)
+                    __hip_atomic_store(to + i, word(i), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+            }
+        } else {
+#pragma unroll
+            for (int e = 0; e < decltype(keys)::value; ++e) {
+                const int i = e * 64 + lane;
+                if (i < n)
+                    to[i] = word(i);
+            }
+        }
+    };
+    if constexpr (MODE == kSelect) {
+        if (increasing) {
+            constexpr int kList = 68 * kMostSelected; // (twice as many words: a list, or its results with their padding)
+            uint32_t *const perWave = reinterpret_cast<uint32_t *>(lds); // T, then 16 words on how many a wave has
+            uint32_t *const list = perWave + 32 + wave / W * (kList * 2);
+            uint32_t order[E], most[4]; // (padding: 0)
+#pragma unroll
+            for (int e = 0; e < E; ++e) {
+                order[e] = ScoreOrder(bits[e]);
+                if ((kClamp || validCols != N) && i0 + e * 64 >= (uint32_t)validCols)
+                    order[e] = 0;
+                most[e % 4] = e < 4 || order[e] > most[e % 4] ? order[e] : most[e % 4];
+            }
+            // T of this wave: `wanted` of its groups' maxima, and few more, are T or larger; a group: the keys of a lane, or every second or
+            // fourth of them
+            const int whole = validCols / (64 * E), left = topk - whole * share; // waves without padding; for the one behind them
+            const int wanted = waveOfRow < whole ? share : waveOfRow == whole && left > 0 ? left : 0;
+            uint32_t t = 0xffffffffu;
+            if (wanted > 0) {
+                constexpr int kMost = E < 4 ? E : 4;
+                uint32_t most2[2] = {most[0], kMost > 1 ? most[1] : 0u};
+                if constexpr (kMost == 4) {
+                    most2[0] = most[0] > most[2] ? most[0] : most[2];
+                    most2[1] = most[1] > most[3] ? most[1] : most[3];
+                }
+                const uint32_t most1[1] = {most2[0] > most2[1] ? most2[0] : most2[1]};
+                uint32_t above = WaveMax(most1[0]);
+                above += above != 0xffffffffu ? 1u : 0u;
+                t = wanted <= 64 ? ~WaveMax(~most1[0]) : 0u;
+                auto search = [&](auto groups, const uint32_t *max) __attribute__((always_inline)) {
+                    // (the first look is right above the smallest: the end already where most are equal)
+                    for (uint32_t mid = t + 1u; above - t > 1u; mid = t + (above - t) / 2u) {
+                        int n = 0;
+#pragma unroll
+                        for (int g = 0; g < decltype(groups)::value; ++g)
+                            n += __builtin_popcountll(__builtin_amdgcn_ballot_w64(max[g] >= mid));
+                        if (n < wanted) {
+                            above = mid;
+                        } else {
+                            t = mid;
+                            if (n <= wanted + wanted / 8)
+                                break;
+                        }
+                    }
+                };
+                if (wanted <= 24)
+                    search(std::integral_constant<int, 1>(), most1);
+                else if (wanted <= 48 || kMost < 4)
+                    search(std::integral_constant<int, 2>(), most2);
+                else
+                    search(std::integral_constant<int, kMost>(), most);
+            }
+            if constexpr (W > 1) {
+                if (lane == 0)
+                    perWave[wave] = t;
+                __syncthreads();
+#pragma unroll
+                for (int w = 0; w < W; ++w) {
+                    const uint32_t other = (uint32_t)__builtin_amdgcn_readfirstlane((int)perWave[wave / W * W + w]);
+                    t = other < t ? other : t;
+                }
+            }
+            // larger than T, and as large (-0 compares equal to +0)
+            const bool zero = t == kSign || t == kSign - 1u;
+            const uint32_t tLow = zero ? kSign - 1u : t, tHigh = zero ? kSign : t;
+            uint32_t mine = 0;
+#pragma unroll
+            for (int e = 0; e < E; ++e)
+                mine += order[e] >= tLow ? 1u : 0u;
+            uint32_t at = WaveScan(mine); // up to this lane
+            int total = __builtin_amdgcn_readlane((int)at, 63);
+            at -= mine;
+            bool fits = total <= 64 * kMostSelected && tLow != 0u;
+            if constexpr (W > 1) {
+                if (lane == 0)
+                    perWave[16 + wave] = (uint32_t)total;
+                __syncthreads();
+                total = 0;
+#pragma unroll
+                for (int w = 0; w < W; ++w) {
+                    const int n = __builtin_amdgcn_readfirstlane((int)perWave[16 + wave / W * W + w]);
+                    at += w < waveOfRow ? (uint32_t)n : 0u;
+                    total += n;
+                }
+                fits = __syncthreads_and(total <= 64 * kMostSelected && tLow != 0u) != 0; // (the other ways have barriers of the whole workgroup)
+            }
+            if (__builtin_expect(fits, 1)) {
+#pragma unroll
+                for (int e = 0; e < E; ++e)
+                    if (order[e] >= tLow)
+                        reinterpret_cast<uint64_t *>(list)[at++] = (uint64_t)(i0 + e * 64) << 32 | order[e];
+            } else {
+                // too many equal ones: as many of them, by their columns, as are wanted
+                int larger = 0, equal = 0, largerBefore = 0, equalBefore = 0;
+#pragma unroll
+                for (int e = 0; e < E; ++e) {
+                    larger += __builtin_popcountll(__builtin_amdgcn_ballot_w64(order[e] > tHigh));
+                    equal += __builtin_popcountll(__builtin_amdgcn_ballot_w64(order[e] >= tLow));
+                }
+                equal -= larger;
+                if constexpr (W > 1) {
+                    if (lane == 0)
+                        perWave[16 + wave] = (uint32_t)larger << 16 | (uint32_t)equal;
+                    __syncthreads();
+                    larger = equal = 0;
+#pragma unroll
+                    for (int w = 0; w < W; ++w) {
+                        const uint32_t n = (uint32_t)__builtin_amdgcn_readfirstlane((int)perWave[16 + wave / W * W + w]);
+                        largerBefore += w < waveOfRow ? (int)(n >> 16) : 0;
+                        equalBefore += w < waveOfRow ? (int)(n & 0xffffu) : 0;
+                        larger += (int)(n >> 16);
+                        equal += (int)(n & 0xffffu);
+                    }
+                }
+                const int taken = larger + equal <= 64 * kMostSelected ? equal : larger < topk ? topk - larger : 0;
+                total = larger + taken;
+                fits = total <= 64 * kMostSelected && tLow != 0u;
+                if constexpr (W > 1)
+                    fits = __syncthreads_and(fits) != 0;
+                if (fits) {
+                    int before = largerBefore + (equalBefore < taken ? equalBefore : taken);
+#pragma unroll
+                    for (int e = 0; e < E; ++e) {
+                        const uint64_t same = __builtin_amdgcn_ballot_w64(order[e] >= tLow && order[e] <= tHigh);
+                        const int nth = equalBefore + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(same >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)same, 0u));
+                        const bool choose = order[e] > tHigh || (order[e] >= tLow && nth < taken);
+                        const uint64_t chosen = __builtin_amdgcn_ballot_w64(choose);
+                        if (choose)
+                            reinterpret_cast<uint64_t *>(list)[(uint32_t)before + __builtin_amdgcn_mbcnt_hi((uint32_t)(chosen >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)chosen, 0u))] =
+                                (uint64_t)(i0 + e * 64) << 32 | order[e];
+                        equalBefore += __builtin_popcountll(same);
+                        before += __builtin_popcountll(chosen);
+                    }
+                }
+            }
+            if (fits) {
+                if constexpr (W > 1)
+                    __syncthreads();
+                else
+                    ordered();
+                if (waveOfRow != 0 || row0 + wave / W >= rows)
+                    return;
+                uint32_t *toScore = reinterpret_cast<uint32_t *>(outScore) + (size_t)row * (size_t)topk, *toIndex = outIndex + (size_t)row * (size_t)topk;
+                auto finish = [&](auto keys) __attribute__((always_inline)) {
+                    constexpr int S = decltype(keys)::value;
+                    RowSort<S, 1, LOW_DPP> few;
+                    few.q = LaneRank((uint32_t)lane);
+                    few.xchg = nullptr;
+                    few.form = 0;
+#pragma unroll
+                    for (int e = 0; e < S; ++e) {
+                        const uint64_t one = reinterpret_cast<const uint64_t *>(list)[e * 64 + lane];
+                        const uint32_t c = 4095u - (uint32_t)(one >> 32), negZero = (uint32_t)one == kSign - 1u ? 1u : 0u, o = (uint32_t)one + negZero;
+                        few.k[e] = e * 64 + lane < total ? Key(__builtin_amdgcn_alignbit(0x3ffu, o, 12), (o << 20) | (c << 8) | negZero) : 1.0;
+                    }
+                    few.template Sort<6>(6);
+                    ordered();
+                    uint32_t *score = list, *at = list + 68 * S;
+                    const int rank0 = (int)LaneRank((uint32_t)lane) * S;
+#pragma unroll
+                    for (int e = 0; e < S; ++e) {
+                        const uint32_t low = Low(few.k[e]), i = (uint32_t)(rank0 + e) + (uint32_t)(rank0 + e) / 16u;
+                        score[i] = (low & 1u) ? kSign : ScoreBits((High(few.k[e]) << 12) | (low >> 20));
+                        at[i] = 4095u - ((low >> 8) & 0xfffu);
+                    }
+                    ordered();
+                    store(keys, toScore, topk, [&](int i) { return score[i + i / 16]; });
+                    if (consecutive)
+                        store(keys, toIndex, topk, [&](int i) { return first + at[i + i / 16]; });
+                    else
+                        store(keys, toIndex, topk, [&](int i) { return inIdx[at[i + i / 16]]; });
+                };
+                if (total <= 64)
+                    finish(std::integral_constant<int, 1>());
+                else if (total <= 128)
+                    finish(std::integral_constant<int, 2>());
+                else if (total <= 256)
+                    finish(std::integral_constant<int, 4>());
+                else
+                    finish(std::integral_constant<int, kMostSelected>());
+                return;
+            }
+            load(scores, bits); // (not kept in registers so far)
+        }
+    }
     const uint32_t columnBits = (4095u - i0) << 8;
     if (__builtin_expect(!increasing, 0)) { // the columns in the order of their indices; rows of one wave: the first wave does it for all four
         if (W > 1 || wave == 0) {
             s.form = 0;
+            uint32_t all[E];
+            load(inIdx, all);
 #pragma unroll
             for (int e = 0; e < E; ++e) {
-                const uint32_t order = ~ids[e];
+                const uint32_t order = ~all[e];
                 s.k[e] = Key(__builtin_amdgcn_alignbit(0x3ffu, order, 12), (order << 20) | (columnBits - (uint32_t)(e * 64 << 8)));
                 if (i0 + e * 64 >= (uint32_t)validCols)
                     s.k[e] = 1.0;
@@ -352,7 +606,7 @@ __global__ __launch_bounds__(kTopkThreads) void TopkRows(float *outScore, uint32
             if (i0 + e * 64 >= (uint32_t)validCols)
                 s.k[e] = 1.0;
     }
-    s.template Sort<WHOLE ? kBits : kBits - kWholeBits - 1>(keepBits);
+    s.template Sort<MODE == kWhole ? kBits : kBits - kWholeBits - 1>(keepBits);
 
     if (W > 1)
         __syncthreads(); // (the exchanges are over)
@@ -360,24 +614,6 @@ __global__ __launch_bounds__(kTopkThreads) void TopkRows(float *outScore, uint32
         return;
     uint32_t *toScore = reinterpret_cast<uint32_t *>(outScore) + (size_t)row * (size_t)topk + firstRank;
     uint32_t *toIndex = outIndex + (size_t)row * (size_t)topk + firstRank;
-    // lane by lane consecutive words; through: past the L2 (launch_topk)
-    auto store = [&](uint32_t *to, auto &&word) __attribute__((always_inline)) {
-        if (through) {
-#pragma unroll
-            for (int e = 0; e < E; ++e) {
-                const int i = e * 64 + lane;
-                if (i < count)
-                    __hip_atomic_store(to + i, word(i), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-            }
-        } else {
-#pragma unroll
-            for (int e = 0; e < E; ++e) {
-                const int i = e * 64 + lane;
-                if (i < count)
-                    to[i] = word(i);
-            }
-        }
-    };
     uint32_t column[E];
 #pragma unroll
     for (int e = 0; e < E; ++e) {
@@ -388,7 +624,7 @@ __global__ __launch_bounds__(kTopkThreads) void TopkRows(float *outScore, uint32
             stagedColumn[laneRank + e + (laneRank + e) / 16] = column[e];
     }
     ordered();
-    store(toScore, [&](int i) { return staged[i + i / 16]; });
+    store(eTag, toScore, count, [&](int i) { return staged[i + i / 16]; });
     if (kStages == 1) {
         ordered();
 #pragma unroll
@@ -407,12 +643,12 @@ __global__ __launch_bounds__(kTopkThreads) void TopkRows(float *outScore, uint32
         }
         return;
     }
-    store(toIndex, [&](int i) { return first + stagedColumn[i + i / 16]; });
+    store(eTag, toIndex, count, [&](int i) { return first + stagedColumn[i + i / 16]; });
 }
 
 template <int E, int W>
 int launch_topk(hipStream_t st, float *out_score, uint32_t *out_index, const float *src, const uint32_t *in_idx, int rows, int valid_cols, int ld,
-                int topk)
+                int topk, [[maybe_unused]] bool select = false)
 {
     int keepBits = 0;
     while ((E << keepBits) < topk)
@@ -422,17 +658,22 @@ int launch_topk(hipStream_t st, float *out_score, uint32_t *out_index, const flo
     // (LDS / DPP, whole sorts: 300 x 128 3.48 / 3.26 us, 300 x 256 4.53 / 4.28); with more the moves take issue slots (4800 x 128
     // 5.09 / 5.23).  8 and 16 keys per lane cover the latency either way and take DPP.
     const bool dpp = E >= 8 || (long long)rows * W <= 4 * 4 * pto_amd::compute_units();
-    constexpr bool kCut = kOnlyWhole<E, W>, kDpp = E >= 8 || kOnlyWhole<E, W>; // (names the one form that there is)
-    auto kernel = dpp ? (whole ? TopkRows<E, W, true, true> : TopkRows<E, W, true, kCut>) :
-                        (whole ? TopkRows<E, W, kDpp, true> : TopkRows<E, W, kDpp, kCut>);
+    constexpr Mode kFew = kOnlyWhole<E, W> ? kWhole : kCut;
+    constexpr bool kDpp = E >= 8 || kOnlyWhole<E, W>; // (names the one form that there is)
+    auto kernel = dpp ? (whole ? TopkRows<E, W, true, kWhole> : TopkRows<E, W, true, kFew>) :
+                        (whole ? TopkRows<E, W, kDpp, kWhole> : TopkRows<E, W, kDpp, kFew>);
+    if constexpr (E == 16 || (E == 8 && W == 1))
+        if (select)
+            kernel = TopkRows<E, W, true, kSelect>;
     // Results past the L2: a kernel ends with every L2 writing back what is dirty in it, 3 us for the 38 MB of 4800 x 1000 (25.4 ->
     // 23.3 us; 8192 x 500, top 333 19.2 -> 17.0; 300 x 128 whole 2.69 -> 2.67).  Not where a row's results are less than a store
     // instruction's 256 bytes (8192 x 64, top 1 3.2 / 3.7, 131072 x 64, top 33 32.6 / 34.1), nor where they are much more than the L2s'
     // 32 MB, which then are written back while others sort (30000 x 2048, top 1500 261 / 268).
     const int through = topk >= 64 && 8ll * rows * topk <= 1ll << 26;
+    const int share = (int)((64ll * E * topk + valid_cols - 1) / valid_cols); // of topk, for a wave without padding
     constexpr int kRows = kTopkWaves / W;
     kernel<<<dim3((unsigned)(((long long)rows + kRows - 1) / kRows)), dim3(kTopkThreads), 0, st>>>(out_score, out_index, src, in_idx, rows, valid_cols,
-                                                                                                   ld, topk, keepBits, through);
+                                                                                                   ld, topk, keepBits, through, share);
     return pto_amd::check_launch();
 }
 
@@ -453,6 +694,26 @@ extern "C" int pto_topk_f32(void *stream, float *out_score, uint32_t *out_index,
     // up to 1706 rows (1700 rows with two 25.6, with four 24.5; 2000 rows 26.2, 26.9).  129 to 256 columns: four up to 365 rows where
     // more than 16 are wanted (one / four: 128 rows 3.6 / 3.3, 300 rows 3.6 / 3.4, 600 rows 3.7 / 3.7; top 7 of 128 rows 3.2 / 3.6).
     const int most = 5 * 4 * pto_amd::compute_units() / rows; // waves per row for five on every SIMD
+    // A threshold, then a sort of what reaches it (us, merges that keep topk / threshold):
+    //   4096 columns:    1 row,  top   1 8.0 / 5.8    128 rows, top 50 10.2 / 6.5   1200 rows, top 300 31.7 / 22.6
+    //   2048 columns:    8 rows, top  10 6.0 / 5.3    900 rows, top 30 11.0 / 6.2   2400 rows, top 256 26.2 / 17.3; few rows and many keys: 8 rows, top 200 7.6 / 8.7
+    //   1024 columns:  600 rows, top 128 7.1 / 6.6   1500 rows, top 16  7.7 / 5.3   4800 rows, top 128 21.2 / 11.4; 128 rows, top 16 4.8 / 4.9, top 128 5.4 / 6.6, 700 rows, top 4 5.1 / 5.3
+    //    512 columns: 4000 rows, top  16 7.9 / 6.1   8000 rows, top 60 16.6 / 12.6; 1000 rows, top 16 4.7 / 4.7, top 60 5.2 / 5.5
+    // One wave per row of 1024 and two per row of 2048 where without the threshold there are four (1500 rows, top 16: 5.2 with one, 6.1 with four).
+    // Few distinct scores take longer (fewer than 64 of them, top 30: 512 x 1024 5.6 / 6.6, 1500 x 1024 8.5 / 7.5), so the line lies where that is even.
+    const int padded = valid_cols <= 512 ? 512 : valid_cols <= 1024 ? 1024 : valid_cols <= 2048 ? 2048 : 4096;
+    if (valid_cols > 256 && topk <= padded / 8 && topk <= (valid_cols > 2048 || most < 10 ? 40 : 20) * kMostSelected) {
+#define PTO_TOPK_SELECT(E, W) return launch_topk<E, W>(st, out_score, out_index, src, in_idx, rows, valid_cols, ld, topk, true);
+        if (valid_cols > 2048)
+            PTO_TOPK_SELECT(16, 4)
+        if (valid_cols > 1024)
+            PTO_TOPK_SELECT(16, 2)
+        if (valid_cols > 512 && most <= (topk > 16 ? 8 : 6))
+            PTO_TOPK_SELECT(16, 1)
+        if (valid_cols <= 512 && most <= 1)
+            PTO_TOPK_SELECT(8, 1)
+#undef PTO_TOPK_SELECT
+    }
 #define PTO_TOPK_CASE(E, W) return launch_topk<E, W>(st, out_score, out_index, src, in_idx, rows, valid_cols, ld, topk);
     if (valid_cols <= 64)
         PTO_TOPK_CASE(1, 1)

@@ -188,3 +188,43 @@ def test_topk_results_past_the_l2(rows, cols, topk):
     score, order = torch.sort(src, dim=1, descending=True, stable=True)
     assert torch.equal(guard[:rows * topk].view(rows, topk), score[:, :topk]) and torch.equal(index[:rows * topk].view(rows, topk), order[:, :topk].int())
     assert (guard[rows * topk:] == 7.0).all() and (index[rows * topk:] == -7).all()
+
+
+@pytest.mark.parametrize("rows,cols", [(2561, 257), (2565, 512), (641, 513), (1026, 1024), (5, 1025), (5, 1100), (515, 1500), (9, 2048), (4, 2049), (7, 3248), (3, 4096)])
+def test_topk_by_threshold(oracle, rows, cols):
+    """topk of an eighth of the padded row and less, on both sides of the numbers of groups that the threshold is taken over (24, 48, 64) and of the
+    lengths that the lists are sorted by (64, 128, 256, 512): continuous scores; all equal; two values; most of a row masked; zeros of both signs as
+    the threshold; ascending and descending rows; the largest scores side by side, in one lane, in one wave."""
+    r = np.random.Generator(np.random.Philox(key=cols))
+    padded = max(512, 1 << (cols - 1).bit_length())
+    src = r.standard_normal((rows, cols + 3)).astype(np.float32)
+    kinds = 10
+    for kind in range(kinds):
+        row = src[kind % rows::kinds] if rows >= kinds else src[kind % rows:kind % rows + 1]
+        if kind == 1:
+            row[:] = 2.5
+        elif kind == 2:
+            row[:] = np.where(row > 0.3, np.float32(1.0), np.float32(-1.0))
+        elif kind == 3:
+            row[:] = np.where(np.arange(cols + 3) % 37 == 5, row, -np.inf)
+        elif kind == 4:
+            row[:] = np.where(np.arange(cols + 3) % 97 == 5, np.abs(row), np.where(row > 0, np.float32(0.0), np.float32(-0.0)))
+        elif kind == 5:
+            row[:] = np.arange(cols + 3, dtype=np.float32)
+        elif kind == 6:
+            row[:] = -np.arange(cols + 3, dtype=np.float32)
+        elif kind == 7:
+            row[:, 100:228] += 50.0
+        elif kind == 8:
+            row[:, 17::64] += 50.0
+        elif kind == 9:
+            row[:] = np.where(row > 1.0, np.float32(np.inf), np.round(row * 3.0))
+    idx = np.arange(cols, dtype=np.uint32)
+    few = [k for k in (1, 2, 23, 24, 25, 48, 49, 63, 64, 65, 97, 128, 160, 161, 255, 256, 320, 321) if k <= min(cols, padded // 8 + 1)]
+    if rows * cols > 1 << 20:
+        few = few[::3] + few[-1:]
+    for n, k in enumerate(few):
+        assert same(topk_gpu(src, idx, cols, k), oracle.topk_f32(src, idx, cols, k)), (k, "consecutive")
+        if n % 3 == 0:
+            ids = (idx * np.uint32(3) + np.uint32(5), np.uint32(0xFFFFFFFF) - idx)[n // 3 % 2]
+            assert same(topk_gpu(src, ids, cols, k), oracle.topk_f32(src, ids, cols, k)), (k, "other indices")
