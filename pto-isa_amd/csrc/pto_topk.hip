@@ -377,7 +377,8 @@ __global__ __launch_bounds__(kTopkThreads, MODE == kSelect && E == 16 ? 4 : 1) v
         if (increasing) {
             constexpr int kList = 68 * kMostSelected; // (twice as many words: a list, or its results with their padding)
             uint32_t *const perWave = reinterpret_cast<uint32_t *>(lds); // T, then 16 words on how many a wave has
-            uint32_t *const list = perWave + 32 + wave / W * (kList * 2);
+            static_assert(W > 1 || kList * 2 == kStaged * kStages, "a wave that sorts the whole row stays in its list's memory");
+            uint32_t *const list = W == 1 ? staged : perWave + 32 + wave / W * (kList * 2);
             uint32_t order[E], most[4]; // (padding: 0)
 #pragma unroll
             for (int e = 0; e < E; ++e) {

@@ -228,3 +228,16 @@ def test_topk_by_threshold(oracle, rows, cols):
         if n % 3 == 0:
             ids = (idx * np.uint32(3) + np.uint32(5), np.uint32(0xFFFFFFFF) - idx)[n // 3 % 2]
             assert same(topk_gpu(src, ids, cols, k), oracle.topk_f32(src, ids, cols, k)), (k, "other indices")
+
+
+@pytest.mark.parametrize("rows,cols,topk", [(740, 1024, 120), (2564, 512, 60)])
+def test_topk_threshold_fails_next_to_a_long_list(oracle, rows, cols, topk):
+    """Rows of one workgroup in turn: keys of the longest list, and so many in so few groups (every fourth block of 64 columns of a lane) that the
+    row is sorted whole; a wave's list and its neighbour's sort do not share memory."""
+    r = np.random.Generator(np.random.Philox(key=rows))
+    src, idx = datagen.topk_inputs(rows, cols, cols)
+    src[:] = r.standard_normal(src.shape)
+    block, lane = np.arange(cols) // 64, np.arange(cols) % 64
+    src[0::2, (block % 4 == 0)] += 100.0
+    src[1::2, (block % 4 == 0) | (block % 4 == 1) | ((block % 4 == 2) & (lane < 6))] += 100.0
+    assert same(topk_gpu(src, idx, cols, topk), oracle.topk_f32(src, idx, cols, topk))
