@@ -139,7 +139,21 @@ extern "C" int pto_fa_fwd_f16(void *stream, void *o, float *lse, const uint16_t 
     // K / V tiles are shared by twice the queries and the two waves of a SIMD alternate between MFMA and softmax
     // phases (measured +10-15 % at B1 H16 S4096 over workgroups of four waves)
     if (head_dim == 128 && seq_q % 256 == 0) {
-        if ((long long)batch * heads * (seq_q / 256) >= cus) {
+        const long long pairs = (long long)batch * heads, perPair = seq_q / 256;
+        // Workgroups beyond the last whole round take as long as that round.  Up to half a round of them, whole heads, go into a launch
+        // of their own, on the form that is best for so few (us, one launch / two; a round and 1/32, 1/8, 1/4, 1/2 of one):
+        //   1024 keys: 61 / 46   61 / 47   62 / 52   64 / 62      2048: 109 / 76   108 / 77   108 / 85   111 / 102      8192: 406 / 280   405 / 307   417 / 337   431 / 381
+        // (256 keys: 25 / 23, 25 / 23, 26 / 25, 27 / 28.  With a mask the workgroups differ in length and the last round fills by itself.)
+        const long long whole = pairs * perPair / cus * cus / perPair, rest = pairs - whole;
+        if (!causal && whole > 0 && rest > 0 && rest * perPair * 2 <= cus && seq_kv >= 512 && pairs <= 0x7fffffffLL) {
+            const int r = pto_amd::fa_fwd_d128_w8m16(st, o, lse, hq, hk, hv, 1, (int)whole, seq_q, seq_kv, false, o_fp32 != 0, causalOff);
+            if (r != PTO_OK)
+                return r;
+            const long long rows = whole * seq_q, keyRows = whole * seq_kv;
+            return pto_fa_fwd_f16(stream, static_cast<char *>(o) + rows * head_dim * (o_fp32 ? 4 : 2), lse ? lse + rows : nullptr, q + rows * head_dim,
+                                  k + keyRows * head_dim, v + keyRows * head_dim, 1, (int)rest, seq_q, seq_kv, head_dim, causal, o_fp32);
+        }
+        if (pairs * perPair >= cus) {
             // the same schedule on 16 x 16 x 32 MFMAs: +1.5 .. 3.6 % without a mask and for long causal sequences
             // (interleaved runs; B2 H16 S2048 causal is 6 % slower on it and stays on the 32 x 32 x 16 kernel)
             if (!causal || seq_kv >= 4096)

@@ -471,3 +471,16 @@ def test_fa_output_at_any_element(B, H, S, D, causal, o_fp32):
         out.append(o[shift:shift + size].clone())
         assert torch.equal(out[0], out[-1])
     check_sampled_rows_of_every_head(*(t.cpu().numpy() for t in (q, k, v, out[0].view(B, H, S, D).float(), lse)), causal != 0, seed=5)
+
+
+@pytest.mark.parametrize("B,H,Sq,Skv", [(5, 13, 1024, 512), (1, 259, 256, 576), (8, 10, 1024, 512), (2, 48, 1024, 1024), (2, 10, 3584, 512), (3, 43, 1024, 512)])
+@pytest.mark.parametrize("o_fp32", [False, True])
+def test_fa_heads_beyond_whole_rounds(B, H, Sq, Skv, o_fp32):
+    """A little more than one or two rounds of 256-query workgroups: 1/64 to half a round of whole heads in a launch of their own (on 256 units with eight, four and
+    two key groups), also where a round is no whole number of heads; with and without the log-sum-exp."""
+    rng = np.random.default_rng(H)
+    q, k, v = (rng.standard_normal((B, H, n, 128), dtype=np.float32).astype(np.float16) for n in (Sq, Skv, Skv))
+    o, lse = fa_gpu(q, k, v, False, o_fp32)
+    check_sampled_rows_of_every_head(q, k, v, o, lse, False, seed=7)
+    if o_fp32:
+        assert np.array_equal(fa_gpu(q, k, v, False, o_fp32, want_lse=False)[0], o)
