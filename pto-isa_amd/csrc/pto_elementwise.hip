@@ -157,6 +157,48 @@ __global__ __launch_bounds__(kBlockThreads) void GatherChunks(char *out, const c
             __builtin_nontemporal_store(v[i], reinterpret_cast<u32x4 *>(out + ((size_t)at[i] * rowChunks + part[i]) * 16));
 }
 
+// The same for rows of any number of chunks, in slices that no 64 bytes of the output are cut by: what is dealt out is the pieces of four chunks
+// (64 bytes) of the whole output, a piece to the slice that the column of its first chunk lies in; its last chunks may belong to the
+// slice, or the row, behind.  Lane by lane `slots` chunks per row and slice, as many as a row can have there; a lane without one idles.
+__global__ __launch_bounds__(kBlockThreads) void GatherPieces(char *out, const char *table, const int32_t *idx, uint32_t chunks, uint32_t rowChunks,
+                                                              uint32_t slots, uint32_t units, uint32_t magic, int shift, uint32_t tableRows, uint32_t parts)
+{
+    typedef uint32_t u32x4 __attribute__((ext_vector_type(4), aligned(2)));
+    const uint32_t xcd = blockIdx.x % 8, slice = xcd % parts, block = blockIdx.x / 8 * (8 / parts) + xcd / parts;
+    const uint32_t first = block * (uint32_t)kGatherChunks + threadIdx.x;
+    if (block * (uint32_t)kGatherChunks >= units)
+        return;
+    const uint32_t low = slice * rowChunks / parts, high = (slice + 1) * rowChunks / parts;
+    uint32_t row[kGatherSteps], chunk[kGatherSteps], part[kGatherSteps];
+    bool mine[kGatherSteps];
+#pragma unroll
+    for (int i = 0; i < kGatherSteps; ++i) {
+        const uint32_t u = first + i * kBlockThreads < units ? first + i * kBlockThreads : units - 1;
+        uint32_t at = (uint32_t)(((uint64_t)u * magic) >> shift);
+        const uint32_t j = u - at * slots, begin = at * rowChunks, start = (begin + low + 3) & ~3u;
+        chunk[i] = start + j;
+        mine[i] = first + i * kBlockThreads < units && start + (j & ~3u) < begin + high && chunk[i] < chunks;
+        part[i] = mine[i] ? chunk[i] - begin : low;
+        if (part[i] >= rowChunks) {
+            part[i] -= rowChunks;
+            ++at;
+        }
+        row[i] = (uint32_t)idx[at];
+    }
+    u32x4 v[kGatherSteps];
+#pragma unroll
+    for (int i = 0; i < kGatherSteps; ++i) {
+        const bool inside = row[i] < tableRows;
+        v[i] = *reinterpret_cast<const u32x4 *>(table + ((size_t)(inside ? row[i] : 0u) * rowChunks + part[i]) * 16);
+        if (!inside)
+            v[i] = u32x4{0, 0, 0, 0};
+    }
+#pragma unroll
+    for (int i = 0; i < kGatherSteps; ++i)
+        if (mine[i])
+            __builtin_nontemporal_store(v[i], reinterpret_cast<u32x4 *>(out + (size_t)chunk[i] * 16));
+}
+
 // One-tile TGATHER (index form), the half 16x1024 -> 16x128 case of the reference's tgather test.
 __global__ __launch_bounds__(kBlockThreads) AICORE void TGatherIndex16x1024(__gm__ half *dst, __gm__ const half *src0,
                                                                             __gm__ const int32_t *idx)
@@ -258,7 +300,7 @@ extern "C" int pto_gather_rows(void *stream, void *out, const void *table, const
     // the rows are; else of six and more half lines where the rows are whole numbers of those (16639 rows of 5696 bytes out of
     // 1972: 24.6 us whole, 17.5 in eight); at most an eighth of the lanes idle past a shorter last slice (32768 rows of 3840 bytes
     // out of 8192: 33.7 whole, 25.9 in eight).  Lines cut by a slice are written twice, in part: slices of other rows (20000 of
-    // 2064 bytes 12.0 us, cut 14.1) and into an output off the 16 bytes (the first of these 58.6, whole 38.6) lose more than they win.
+    // 2064 bytes 12.0 us, so cut 14.1) and into an output off the 16 bytes (the first of these 58.6, whole 38.6) lose more than they win.
     if (n_idx >= 2 * table_rows && rowChunks % 4 == 0 && reinterpret_cast<uintptr_t>(out) % 16 == 0)
         for (const size_t unit = rowChunks % 8 == 0 ? 8 : 4, least = rowChunks % 8 == 0 ? 8 : 24;
              parts < 8 && table_rows * rowChunks * 16 / parts > ((size_t)1 << 20); parts *= 2) {
@@ -267,6 +309,23 @@ extern "C" int pto_gather_rows(void *stream, void *out, const void *table, const
                 break;
             cpr = next;
         }
+    // Rows that this leaves whole, of no whole number of 64 bytes: slices of the output's 64-byte pieces (GatherPieces), as few as bring a slice of the table
+    // down to 1 MiB, of nine chunks and more, where the batch reads a row four times or more on average (us, whole / slices):
+    //   79891 rows of 1680 bytes out of 4950 32.5 / 22.5   110141 of 1168 out of 8421 32.7 / 26.5   16000 of 8016 out of 4000 35.6 / 27.5
+    //   6000 of 16032 out of 1500 26.7 / 18.9   20000 of 2064 out of 2000 10.7 / 8.3   60000 of 2000 out of 30000 35.0 / 39.3
+    // A narrow slice reads lines that it uses in part: not where those fill an XCD's L2 (200000 rows of 656 out of 20000 35.7 / 39.2, 60000 of
+    // 1200 out of 15000 20.9 / 21.6); from 15 chunks on a slice pays all the same (60000 of 2000 out of 15000 34.2 / 32.0).  Nor for
+    // a few MiB (1100 of 4016 out of 275 3.9 / 4.2).
+    const size_t tableBytes = table_rows * rowChunks * 16;
+    uint32_t pieces = 1;
+    if (parts == 1 && n_idx >= 4 * table_rows && rowChunks >= 32 && n_idx * rowChunks >= (size_t)1 << 19 && reinterpret_cast<uintptr_t>(out) % 64 == 0) {
+        while (pieces < 8 && tableBytes / pieces > ((size_t)1 << 20) && rowChunks >= 17 * pieces)
+            pieces *= 2;
+        if (rowChunks < 15 * pieces && tableBytes / pieces + table_rows * 128 > ((size_t)15 << 18))
+            pieces = 1;
+    }
+    if (pieces > 1)
+        cpr = ((rowChunks + pieces - 1) / pieces + 3) / 4 * 4; // (chunks of a row whose number is a multiple of four, with the three behind: no more)
     int shift = 31;
     while (((size_t)1 << (shift - 31)) < cpr)
         ++shift;
@@ -274,6 +333,17 @@ extern "C" int pto_gather_rows(void *stream, void *out, const void *table, const
     hipStream_t st = static_cast<hipStream_t>(stream);
     const auto kernel = cpr * parts == rowChunks ? GatherChunks<false> : GatherChunks<true>;
     // (whole rows per launch, fewer than 2^31 chunks a slice)
+    if (pieces > 1) { // (whole pieces per launch)
+        const size_t most = 0x7fffffffu / rowChunks / 4 * 4;
+        for (size_t r0 = 0; r0 < n_idx; r0 += most) {
+            const size_t rows = n_idx - r0 < most ? n_idx - r0 : most, units = rows * cpr, blocks = (units + kGatherChunks - 1) / kGatherChunks;
+            const size_t perGroup = 8 / pieces, groups = (blocks + perGroup - 1) / perGroup;
+            GatherPieces<<<dim3((unsigned)(groups * 8)), dim3(kBlockThreads), 0, st>>>(
+                static_cast<char *>(out) + r0 * rowChunks * 16, static_cast<const char *>(table), idx + r0, (uint32_t)(rows * rowChunks), (uint32_t)rowChunks,
+                (uint32_t)cpr, (uint32_t)units, magic, shift, (uint32_t)table_rows, pieces);
+        }
+        return pto_amd::check_launch();
+    }
     const size_t rowsPerLaunch = 0x7fffffffu / rowChunks;
     for (size_t r0 = 0; r0 < n_idx; r0 += rowsPerLaunch) {
         const size_t chunks = (n_idx - r0 < rowsPerLaunch ? n_idx - r0 : rowsPerLaunch) * cpr, blocks = (chunks + kGatherChunks - 1) / kGatherChunks;

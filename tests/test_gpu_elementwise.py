@@ -169,6 +169,31 @@ def test_gather_rows_unequal_slices(oracle, rows, cols, nidx):
     assert np.array_equal(gather_rows(t32, idx), oracle.gather_rows(t32, idx))
 
 
+@pytest.mark.parametrize("rows,cols,nidx", [(2048, 264, 16384), (4200, 328, 17001), (2000, 536, 8203), (1600, 584, 7333), (900, 1032, 4099), (900, 1048, 4101), (300, 4008, 1203),
+                                            (77, 8184, 523)])
+def test_gather_rows_in_pieces_of_the_output(oracle, rows, cols, nidx):
+    """Rows of no whole number of 64 bytes, read four times and more: two to eight slices, with one, two or three chunks past a piece; widths on both sides of
+    where the number of slices changes; indices outside the table; and into an output that begins in the middle of a piece, which stays whole."""
+    from gpu_util import gather_rows
+    for name, dtype, width in (("half", np.uint16, cols), ("float", np.uint32, cols - 8 * (cols > 264))):
+        r = np.random.default_rng(cols)
+        table = r.integers(0, np.iinfo(dtype).max, size=(rows, width), dtype=dtype)
+        idx = r.integers(0, rows, size=nidx).astype(np.int32)
+        idx[::17] = -1 - idx[::17]
+        idx[5::31] = rows
+        want = oracle.gather_rows(table, idx)
+        assert np.array_equal(gather_rows(table, idx), want), name
+        view = {2: np.int16, 4: np.int32}[table.itemsize]
+        tt, ti = torch.from_numpy(table.view(view)).to("cuda:0"), torch.from_numpy(idx).to("cuda:0")
+        for shift in (0, 32 // table.itemsize):
+            out = torch.full((nidx * width + 128,), 77, dtype=tt.dtype, device="cuda:0")
+            capi.check(capi.load().pto_gather_rows(torch.cuda.current_stream().cuda_stream, out.data_ptr() + shift * table.itemsize, tt.data_ptr(), ti.data_ptr(),
+                                                   nidx, rows, width, table.itemsize), "pto_gather_rows")
+            got = out.cpu().numpy()
+            assert np.array_equal(got[shift:shift + nidx * width].view(dtype).reshape(nidx, width), want), (name, shift)
+            assert (got[:shift] == 77).all() and (got[shift + nidx * width:] == 77).all()
+
+
 @pytest.mark.parametrize("rows,cols,nidx", [(5, 24, 700), (1500, 1032, 3001), (3000, 1024, 6001)])
 @pytest.mark.parametrize("dtype", [torch.int16, torch.int32])
 def test_gather_rows_element_alignment(rows, cols, nidx, dtype):
