@@ -219,9 +219,9 @@ int launch_gemm_ks(hipStream_t st, float *c, const half *a, const half *b, int m
     if (tiles > 0x7fffffffll)
         return PTO_ERR_UNSUPPORTED;
     // (half pieces past the L2 cost no more than they save while C is small: 1000 x 3000 x 2048 18.4 -> 17.9 us, 1024 x 3064 x 1024 13.0 and 13.1,
-    // 1024 x 6136 x 1024 18.8 and 19.8)
+    // 1024 x 6136 x 1024 18.8 and 19.8; and operands and C together: 503 x 6088 x 3072, 52 MB, 25.0 -> 24.5, x 6016, 91 MB, 51.2 -> 54.0)
     const uint64_t bytes = 4ull * m * n;
-    const int through = pto_amd::store_through(c, 4ull * n, bytes) || (bytes <= 12u << 20 && (n * 4ull | (uintptr_t)c) % 32 == 0);
+    const int through = pto_amd::store_through(c, 4ull * n, bytes) || (bytes <= 12u << 20 && bytes + 2ull * ((uint64_t)m + n) * k <= 64u << 20 && (n * 4ull | (uintptr_t)c) % 32 == 0);
     (k % 64 ? half64 : whole)<<<dim3((unsigned)tiles), dim3(512), lds, st>>>(c, a, b, m, n, k, through);
     return pto_amd::check_launch();
 }
