@@ -10,13 +10,13 @@ PTO_DEVICE_CODE_BEGIN
 namespace {
 
 // Four results, past the L2 or into it (pto_amd::store_through), at the alignment of an element.
-// (the wait state: a store of more than 8 bytes may read its registers in the cycle behind it)
+// (s_nop 1: a store of more than 8 bytes reads its registers up to two wait states behind it, and the compiler does not see that this is one)
 typedef float Four __attribute__((ext_vector_type(4)));
 AICORE inline __attribute__((always_inline)) void StoreFour(float *p, Four v, int through)
 {
     typedef float C4 __attribute__((ext_vector_type(4), aligned(4)));
     if (through)
-        asm volatile("global_store_dwordx4 %0, %1, off sc0 sc1\n\ts_nop 0" ::"v"(p), "v"(v) : "memory");
+        asm volatile("global_store_dwordx4 %0, %1, off sc0 sc1\n\ts_nop 1" ::"v"(p), "v"(v) : "memory");
     else
         *reinterpret_cast<C4 *>(p) = v;
 }
@@ -30,7 +30,7 @@ AICORE inline __attribute__((always_inline)) void StoreEight(T *p, Words4 v, boo
     typedef uint32_t C4 __attribute__((ext_vector_type(4), aligned(2)));
     typedef uint32_t C2 __attribute__((ext_vector_type(2), aligned(2)));
     if (through) // (whole 64-byte pieces of a row: both)
-        asm volatile("global_store_dwordx4 %0, %1, off sc0 sc1\n\ts_nop 0" ::"v"(p), "v"(v) : "memory");
+        asm volatile("global_store_dwordx4 %0, %1, off sc0 sc1\n\ts_nop 1" ::"v"(p), "v"(v) : "memory");
     else if (both)
         *reinterpret_cast<C4 *>(p) = v;
     else

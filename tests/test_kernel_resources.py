@@ -1,4 +1,5 @@
 """What the compiler says of the product's kernels (the metadata in the code objects of libpto_amd.so)."""
+import importlib.util
 import os
 import re
 import shutil
@@ -33,3 +34,37 @@ def test_no_kernel_spills(kernels):
     themselves: where such a read is assembly, the compiler would store its registers before they hold anything."""
     assert len(kernels) > 150 and any("GemmF16F32Ks" in k[0] for k in kernels)
     assert [k for k in kernels if k[1] or k[2]] == []
+
+
+def test_write_through_stores_leave_their_registers_alone(tmp_path):
+    """A store of 16 bytes reads its data registers up to two wait states after it (gfx940 and later).  The compiler, which does not
+    look into assembly, may overwrite them in the very next instruction, so the assembly itself has to hold both."""
+    build = importlib.util.module_from_spec(importlib.util.spec_from_file_location("pto_amd_build", os.path.join(os.path.dirname(capi.LIB_PATH), "build.py")))
+    build.__spec__.loader.exec_module(build)
+    source, listing = tmp_path / "stores.hip", tmp_path / "listing"
+    source.write_text("""#include <pto/pto-inst.hpp>
+#include "stores.hpp"
+__global__ void Fours(float *p, Four v)
+{
+    for (int i = 0; i < 4; ++i, p += 1024, v *= 2.0f)
+        StoreFour(p + 4 * threadIdx.x, v + (float)threadIdx.x, 1);
+}
+__global__ void Eights(_Float16 *p, Words4 v)
+{
+    for (int i = 0; i < 4; ++i, p += 1024, v *= 3u)
+        StoreEight(p + 8 * threadIdx.x, v + threadIdx.x, true, 1);
+}
+""")
+    r = subprocess.run([build.HIPCC] + build.FLAGS + ["--cuda-device-only", "-S", str(source), "-o", str(listing)], capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr
+    code = [l.split(";")[0].split() for l in listing.read_text().split("\n")]
+    code = [w for w in code if w and not w[0].startswith(".") and not w[0].endswith(":")]
+    stores = [i for i, w in enumerate(code) if w[0] == "global_store_dwordx4" and "sc1" in w]
+    assert len(stores) == 8
+    for i in stores:
+        waited = 0
+        for w in code[i + 1:]:
+            if w[0].startswith("v_") or waited >= 2:
+                break
+            waited += int(w[1]) + 1 if w[0] == "s_nop" else 1
+        assert waited >= 2, code[i:i + 4]
