@@ -27,8 +27,8 @@
 //   than topk keys reach it (of 1024, 256 groups: 68 for topk 60).  It is found by halving an interval of the scores' order, the groups that reach
 //   the middle counted by ballots; those keys go into a list in the LDS and through the network of 64, 128, 256 or 512 keys in one wave.
 //   Where too many keys equal the threshold (masked rows), as many of them as are wanted are taken in the order of their columns; where that does
-//   not do either, or the indices do not increase, the row is sorted as before.  4800 x 1024, top 40 19.7 -> 8.3 us; 1200 x 4096, top 50 25.1 -> 13.9;
-//   1584 x 2960, top 60 35.8 -> 17.6; 128 x 4096, top 50 10.2 -> 6.5; all equal but 2 %: 4800 x 1024, top 40 20.6 -> 11.0.
+//   not do either, or the indices do not increase, the row is sorted as before.  4800 x 1024, top 40 18.7 -> 6.9 us (all equal but 2 % 18.5 -> 7.9);
+//   600 x 2048, top 100 10.8 -> 7.1 (ascending 5.9, masked from the middle on 7.4); 600 x 4096, top 100 18.3 -> 7.9.
 // * Any other index vector: the same network sorts the (index, column) pairs first, once per workgroup (the rows share their
 //   indices); the rank of a column in that order then stands in the scores' keys for the column.  4800 x 1024 whole: 42 us (127
 //   with keys in the LDS and a pass over it per stage); 1000 x 256: 6.6 (15).
@@ -277,22 +277,25 @@ __device__ inline uint32_t WaveScan(uint32_t v)
 }
 template <int E, int W, bool LOW_DPP, Mode MODE>
 __global__ __launch_bounds__(kTopkThreads, MODE == kSelect && E == 16 ? 4 : 1) void TopkRows(float *outScore, uint32_t *outIndex, const float *src, const uint32_t *inIdx,
-                                                         int rows, int validCols, int ld, int topk, int keepBits, int through,
-                                                         [[maybe_unused]] int share)
+                                                         int rows, int validCols, int ld, int topk, int keepBits, int through)
 {
     constexpr int N = 64 * E * W, kRows = kTopkWaves / W, kBits = RowSort<E, W, LOW_DPP>::kLaneBits;
     constexpr int kStaged = 64 * E + 4 * E; // words of a wave's results, one of padding behind every 16
     constexpr int kStages = E <= 8 ? 2 : 1;  // scores and columns side by side, or one after the other (LDS for four workgroups more)
     // exchanges, then results (or, between two sorts, the ranks of the columns); behind them the columns in the order of their indices
     constexpr size_t kExchange = W > 1 ? (size_t)kTopkWaves * E * 64 * 8 : 0, kStage = (size_t)kTopkWaves * kStaged * 4 * kStages;
-    constexpr size_t kSelected = MODE == kSelect ? 128 + (size_t)kRows * 68 * kMostSelected * 8 : 0, kSort = kExchange > kStage ? kExchange : kStage;
+    constexpr size_t kSelected = MODE == kSelect ? 384 + (size_t)kRows * 68 * kMostSelected * 8 : 0, kSort = kExchange > kStage ? kExchange : kStage;
     constexpr size_t kWork = kSort > kSelected ? kSort : kSelected;
     static_assert(kWork >= (size_t)N * 2, "the ranks fit");
     __shared__ __attribute__((aligned(16))) char lds[kWork + (size_t)N * 2];
     uint16_t *rankOf = reinterpret_cast<uint16_t *>(lds), *columnOf = reinterpret_cast<uint16_t *>(lds + kWork);
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / 64), lane = tid % 64;
     const int waveOfRow = wave % W, row0 = (int)blockIdx.x * kRows, row = row0 + wave / W < rows ? row0 + wave / W : rows - 1;
-    uint32_t i0 = (uint32_t)(waveOfRow * E * 64 + lane); // this lane's first column; then every 64th
+    // this lane's first column; then every kStep-th.  Where a threshold selects, the waves of a row take blocks of 64 columns in turn, so that each
+    // sees the whole row: the lowest of their thresholds counts, and with adjoining columns to a wave the poorest one set it wherever the
+    // level of the scores changes along the row (600 x 2048, top 100, ascending 15.6 us, more than the 10.5 without a threshold)
+    constexpr uint32_t kStep = MODE == kSelect ? 64 * W : 64;
+    uint32_t i0 = (uint32_t)(waveOfRow * (MODE == kSelect ? 1 : E) * 64 + lane);
 
     // A lane past the last column looks at the last one: loads without branches are all in flight at once (16 of them one
     // behind the other were half of the kernel's time).  Up to four keys and few waves: always so, the branch around
@@ -302,11 +305,11 @@ __global__ __launch_bounds__(kTopkThreads, MODE == kSelect && E == 16 ? 4 : 1) v
         if (!kClamp && validCols == N) {
 #pragma unroll
             for (int e = 0; e < E; ++e)
-                to[e] = from[i0 + e * 64];
+                to[e] = from[i0 + e * kStep];
         } else {
 #pragma unroll
             for (int e = 0; e < E; ++e)
-                to[e] = from[i0 + e * 64 < (uint32_t)validCols ? i0 + e * 64 : (uint32_t)validCols - 1u];
+                to[e] = from[i0 + e * kStep < (uint32_t)validCols ? i0 + e * kStep : (uint32_t)validCols - 1u];
         }
     };
     uint32_t bits[E];
@@ -318,12 +321,13 @@ __global__ __launch_bounds__(kTopkThreads, MODE == kSelect && E == 16 ? 4 : 1) v
     // a quarter each
     constexpr bool kQuarters = MODE == kSelect && W < 4;
     constexpr int kIds = kQuarters ? E * W / 4 : E;
+    constexpr uint32_t kIdStep = kQuarters ? 64 : kStep;
     uint32_t ids[kIds];
     const uint32_t id0 = kQuarters ? (uint32_t)(wave * kIds * 64 + lane) : i0;
     if constexpr (kQuarters) {
 #pragma unroll
         for (int e = 0; e < kIds; ++e)
-            ids[e] = inIdx[id0 + e * 64 < (uint32_t)validCols ? id0 + e * 64 : (uint32_t)validCols - 1u];
+            ids[e] = inIdx[id0 + e * kIdStep < (uint32_t)validCols ? id0 + e * kIdStep : (uint32_t)validCols - 1u];
     } else {
         load(inIdx, ids);
     }
@@ -331,7 +335,7 @@ __global__ __launch_bounds__(kTopkThreads, MODE == kSelect && E == 16 ? 4 : 1) v
     uint32_t wrong = 0;
 #pragma unroll
     for (int e = 0; e < kIds; ++e) {
-        const uint32_t at = id0 + e * 64 < (uint32_t)validCols ? id0 + e * 64 : (uint32_t)validCols - 1u;
+        const uint32_t at = id0 + e * kIdStep < (uint32_t)validCols ? id0 + e * kIdStep : (uint32_t)validCols - 1u;
         wrong |= (ids[e] - first) ^ at;
     }
     auto everyone = [&](bool v) { return W > 1 || kQuarters ? __syncthreads_and(v) != 0 : __builtin_amdgcn_ballot_w64(!v) == 0; };
@@ -340,7 +344,7 @@ __global__ __launch_bounds__(kTopkThreads, MODE == kSelect && E == 16 ? 4 : 1) v
     if (__builtin_expect(!consecutive, 0)) {
         bool ok = true;
         for (int e = 0; e < E; ++e) {
-            const int i = (int)i0 + e * 64;
+            const int i = (int)(i0 + e * kStep);
             if (i + 1 < validCols)
                 ok = ok && inIdx[i] < inIdx[i + 1];
         }
@@ -376,56 +380,65 @@ __global__ __launch_bounds__(kTopkThreads, MODE == kSelect && E == 16 ? 4 : 1) v
     if constexpr (MODE == kSelect) {
         if (increasing) {
             constexpr int kList = 68 * kMostSelected; // (twice as many words: a list, or its results with their padding)
-            uint32_t *const perWave = reinterpret_cast<uint32_t *>(lds); // T, then 16 words on how many a wave has
+            uint32_t *const perWave = reinterpret_cast<uint32_t *>(lds); // T, 16 words on how many a wave has, and E W per row on each block of 64 columns
             static_assert(W > 1 || kList * 2 == kStaged * kStages, "a wave that sorts the whole row stays in its list's memory");
-            uint32_t *const list = W == 1 ? staged : perWave + 32 + wave / W * (kList * 2);
+            uint32_t *const list = W == 1 ? staged : perWave + 96 + wave / W * (kList * 2);
             uint32_t order[E], most[4]; // (padding: 0)
 #pragma unroll
             for (int e = 0; e < E; ++e) {
                 order[e] = ScoreOrder(bits[e]);
-                if ((kClamp || validCols != N) && i0 + e * 64 >= (uint32_t)validCols)
+                if ((kClamp || validCols != N) && i0 + e * kStep >= (uint32_t)validCols)
                     order[e] = 0;
                 most[e % 4] = e < 4 || order[e] > most[e % 4] ? order[e] : most[e % 4];
             }
             // T of this wave: `wanted` of its groups' maxima, and few more, are T or larger; a group: the keys of a lane, or every second or
             // fourth of them
-            const int whole = validCols / (64 * E), left = topk - whole * share; // waves without padding; for the one behind them
-            const int wanted = waveOfRow < whole ? share : waveOfRow == whole && left > 0 ? left : 0;
-            uint32_t t = 0xffffffffu;
-            if (wanted > 0) {
-                constexpr int kMost = E < 4 ? E : 4;
-                uint32_t most2[2] = {most[0], kMost > 1 ? most[1] : 0u};
-                if constexpr (kMost == 4) {
-                    most2[0] = most[0] > most[2] ? most[0] : most[2];
-                    most2[1] = most[1] > most[3] ? most[1] : most[3];
-                }
-                const uint32_t most1[1] = {most2[0] > most2[1] ? most2[0] : most2[1]};
-                uint32_t above = WaveMax(most1[0]);
-                above += above != 0xffffffffu ? 1u : 0u;
-                t = wanted <= 64 ? ~WaveMax(~most1[0]) : 0u;
-                auto search = [&](auto groups, const uint32_t *max) __attribute__((always_inline)) {
-                    // (the first look is right above the smallest: the end already where most are equal)
-                    for (uint32_t mid = t + 1u; above - t > 1u; mid = t + (above - t) / 2u) {
-                        int n = 0;
-#pragma unroll
-                        for (int g = 0; g < decltype(groups)::value; ++g)
-                            n += __builtin_popcountll(__builtin_amdgcn_ballot_w64(max[g] >= mid));
-                        if (n < wanted) {
-                            above = mid;
-                        } else {
-                            t = mid;
-                            if (n <= wanted + wanted / 8)
-                                break;
-                        }
-                    }
-                };
-                if (wanted <= 24)
-                    search(std::integral_constant<int, 1>(), most1);
-                else if (wanted <= 48 || kMost < 4)
-                    search(std::integral_constant<int, 2>(), most2);
-                else
-                    search(std::integral_constant<int, kMost>(), most);
+            const int wanted = (topk + W - 1) / W; // (the waves' numbers of columns differ by 64 at most)
+            constexpr int kMost = E < 4 ? E : 4;
+            uint32_t most2[2] = {most[0], kMost > 1 ? most[1] : 0u};
+            if constexpr (kMost == 4) {
+                most2[0] = most[0] > most[2] ? most[0] : most[2];
+                most2[1] = most[1] > most[3] ? most[1] : most[3];
             }
+            const uint32_t most1[1] = {most2[0] > most2[1] ? most2[0] : most2[1]};
+            uint32_t above = WaveMax(most1[0]);
+            above += above != 0xffffffffu ? 1u : 0u;
+            // (all groups reach the smallest of the maxima; 64 lanes the smallest of the lanes')
+            uint32_t least = most1[0];
+            if (kMost == 4 && wanted > 64) {
+                const uint32_t low0 = most[0] < most[2] ? most[0] : most[2], low1 = most[1] < most[3] ? most[1] : most[3];
+                least = low0 < low1 ? low0 : low1;
+            }
+            uint32_t t = ~WaveMax(~least);
+            // (groups more than wanted; with four waves and more than 64 groups of each, more than a sixteenth would come close to the longest list)
+            const int close = W == 4 && wanted > 64 ? wanted / 16 : wanted / 8;
+            const int loose = wanted > 64 ? (W == 1 || (W == 2 && wanted <= 96) ? 32 : close) : wanted / 2 + 4 < 16 ? wanted / 2 + 4 : 16;
+            // (the first look is right above the smallest: the end already where most are equal.  Few distinct scores may have no place for a tight
+            // threshold: from the eighth look on as many groups more will do as no longer a sort pays for; 4800 x 1024, top 40 of 60 distinct 10.2 -> 8.4 us)
+            auto search = [&](auto groups, const uint32_t *max) __attribute__((always_inline)) {
+                int limit = wanted + close, looks = 0;
+                for (uint32_t mid = t + 1u; above - t > 1u; mid = t + (above - t) / 2u) {
+                    int n = 0;
+#pragma unroll
+                    for (int g = 0; g < decltype(groups)::value; ++g)
+                        n += __builtin_popcountll(__builtin_amdgcn_ballot_w64(max[g] >= mid));
+                    if (++looks == 8)
+                        limit = wanted + loose;
+                    if (n < wanted) {
+                        above = mid;
+                    } else {
+                        t = mid;
+                        if (n <= limit)
+                            break;
+                    }
+                }
+            };
+            if (wanted <= 24)
+                search(std::integral_constant<int, 1>(), most1);
+            else if (wanted <= 48 || kMost < 4)
+                search(std::integral_constant<int, 2>(), most2);
+            else
+                search(std::integral_constant<int, kMost>(), most);
             if constexpr (W > 1) {
                 if (lane == 0)
                     perWave[wave] = t;
@@ -437,79 +450,78 @@ __global__ __launch_bounds__(kTopkThreads, MODE == kSelect && E == 16 ? 4 : 1) v
                 }
             }
             // larger than T, and as large (-0 compares equal to +0)
+            t = (uint32_t)__builtin_amdgcn_readfirstlane((int)t);
             const bool zero = t == kSign || t == kSign - 1u;
-            const uint32_t tLow = zero ? kSign - 1u : t, tHigh = zero ? kSign : t;
-            uint32_t mine = 0;
+            uint32_t tLow = zero ? kSign - 1u : t, tHigh = zero ? kSign : t;
+            // Who reaches T, and where in the list; where that are many more than are wanted, for instance as many equal ones (masked rows), once more with
+            // as many of those that equal T, by their columns, as are wanted behind the larger ones.  (Many: more than random scores bring, and than the
+            // shortest sort takes.  Each block of 64 columns ranked by ballots of its own took 2 us more.)
+            int total;
+            uint32_t at;
+            bool fits;
+            for (bool again = false;; again = true) {
+                uint32_t mine = 0;
 #pragma unroll
-            for (int e = 0; e < E; ++e)
-                mine += order[e] >= tLow ? 1u : 0u;
-            uint32_t at = WaveScan(mine); // up to this lane
-            int total = __builtin_amdgcn_readlane((int)at, 63);
-            at -= mine;
-            bool fits = total <= 64 * kMostSelected && tLow != 0u;
-            if constexpr (W > 1) {
-                if (lane == 0)
-                    perWave[16 + wave] = (uint32_t)total;
-                __syncthreads();
-                total = 0;
+                for (int e = 0; e < E; ++e)
+                    mine += order[e] >= tLow ? 1u : 0u;
+                at = WaveScan(mine); // up to this lane
+                total = __builtin_amdgcn_readlane((int)at, 63);
+                at -= mine;
+                if constexpr (W > 1) {
+                    if (lane == 0)
+                        perWave[16 + wave] = (uint32_t)total;
+                    __syncthreads();
+                    total = 0;
 #pragma unroll
-                for (int w = 0; w < W; ++w) {
-                    const int n = __builtin_amdgcn_readfirstlane((int)perWave[16 + wave / W * W + w]);
-                    at += w < waveOfRow ? (uint32_t)n : 0u;
-                    total += n;
+                    for (int w = 0; w < W; ++w) {
+                        const int n = __builtin_amdgcn_readfirstlane((int)perWave[16 + wave / W * W + w]);
+                        at += w < waveOfRow ? (uint32_t)n : 0u;
+                        total += n;
+                    }
                 }
-                fits = __syncthreads_and(total <= 64 * kMostSelected && tLow != 0u) != 0; // (the other ways have barriers of the whole workgroup)
+                fits = total <= 64 * kMostSelected && tLow != 0u;
+                if (!again)
+                    fits = fits && total <= 2 * topk + 64;
+                if constexpr (W > 1)
+                    fits = __syncthreads_and(fits) != 0; // (the other ways have barriers of the whole workgroup)
+                // (who reaches T is compared again below: E answers take two scalar registers each, more than there are)
+                asm("" : "+s"(tLow), "+s"(tHigh));
+                if (again || __builtin_expect(fits, 1))
+                    break;
+                uint32_t equal = 0; // in the lane's block of 64 columns, of this wave's E, then of the row's E W
+#pragma unroll
+                for (int e = 0; e < E; ++e) {
+                    const uint64_t same = __builtin_amdgcn_ballot_w64(order[e] - tLow <= tHigh - tLow);
+                    equal = lane == e ? (uint32_t)__builtin_popcountll(same) : equal;
+                }
+                if constexpr (W > 1) {
+                    uint32_t *const blocks = perWave + 32 + wave / W * (E * W);
+                    if (lane < E)
+                        blocks[lane * W + waveOfRow] = equal;
+                    __syncthreads();
+                    equal = lane < E * W ? blocks[lane] : 0u;
+                }
+                const uint32_t upTo = WaveScan(equal);
+                // (as many there are: topk keys and more reach T)
+                const int taken = tLow == 0u ? 0 : topk - (total - __builtin_amdgcn_readlane((int)upTo, 63));
+                uint32_t last = 0xffffffffu; // the column of the last one
+                if (taken > 0) {
+                    const int block = __builtin_ctzll(__builtin_amdgcn_ballot_w64((int)upTo >= taken));
+                    const int nth = taken - __builtin_amdgcn_readlane((int)(upTo - equal), block);
+                    const uint32_t column = (uint32_t)(block * 64 + lane), one = ScoreOrder(scores[column < (uint32_t)validCols ? column : 0u]);
+                    const uint64_t same = __builtin_amdgcn_ballot_w64(column < (uint32_t)validCols && one - tLow <= tHigh - tLow);
+                    const int rank = (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(same >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)same, 0u));
+                    last = (uint32_t)(block * 64 + __builtin_ctzll(__builtin_amdgcn_ballot_w64(rank == nth - 1) & same));
+                }
+#pragma unroll
+                for (int e = 0; e < E; ++e)
+                    order[e] = order[e] - tLow <= tHigh - tLow && (int)(i0 + e * kStep) > (int)last ? 0u : order[e];
             }
             if (__builtin_expect(fits, 1)) {
 #pragma unroll
                 for (int e = 0; e < E; ++e)
                     if (order[e] >= tLow)
-                        reinterpret_cast<uint64_t *>(list)[at++] = (uint64_t)(i0 + e * 64) << 32 | order[e];
-            } else {
-                // too many equal ones: as many of them, by their columns, as are wanted
-                int larger = 0, equal = 0, largerBefore = 0, equalBefore = 0;
-#pragma unroll
-                for (int e = 0; e < E; ++e) {
-                    larger += __builtin_popcountll(__builtin_amdgcn_ballot_w64(order[e] > tHigh));
-                    equal += __builtin_popcountll(__builtin_amdgcn_ballot_w64(order[e] >= tLow));
-                }
-                equal -= larger;
-                if constexpr (W > 1) {
-                    if (lane == 0)
-                        perWave[16 + wave] = (uint32_t)larger << 16 | (uint32_t)equal;
-                    __syncthreads();
-                    larger = equal = 0;
-#pragma unroll
-                    for (int w = 0; w < W; ++w) {
-                        const uint32_t n = (uint32_t)__builtin_amdgcn_readfirstlane((int)perWave[16 + wave / W * W + w]);
-                        largerBefore += w < waveOfRow ? (int)(n >> 16) : 0;
-                        equalBefore += w < waveOfRow ? (int)(n & 0xffffu) : 0;
-                        larger += (int)(n >> 16);
-                        equal += (int)(n & 0xffffu);
-                    }
-                }
-                const int taken = larger + equal <= 64 * kMostSelected ? equal : larger < topk ? topk - larger : 0;
-                total = larger + taken;
-                fits = total <= 64 * kMostSelected && tLow != 0u;
-                if constexpr (W > 1)
-                    fits = __syncthreads_and(fits) != 0;
-                if (fits) {
-                    int before = largerBefore + (equalBefore < taken ? equalBefore : taken);
-#pragma unroll
-                    for (int e = 0; e < E; ++e) {
-                        const uint64_t same = __builtin_amdgcn_ballot_w64(order[e] >= tLow && order[e] <= tHigh);
-                        const int nth = equalBefore + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(same >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)same, 0u));
-                        const bool choose = order[e] > tHigh || (order[e] >= tLow && nth < taken);
-                        const uint64_t chosen = __builtin_amdgcn_ballot_w64(choose);
-                        if (choose)
-                            reinterpret_cast<uint64_t *>(list)[(uint32_t)before + __builtin_amdgcn_mbcnt_hi((uint32_t)(chosen >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)chosen, 0u))] =
-                                (uint64_t)(i0 + e * 64) << 32 | order[e];
-                        equalBefore += __builtin_popcountll(same);
-                        before += __builtin_popcountll(chosen);
-                    }
-                }
-            }
-            if (fits) {
+                        reinterpret_cast<uint64_t *>(list)[at++] = (uint64_t)(i0 + e * kStep) << 32 | order[e];
                 if constexpr (W > 1)
                     __syncthreads();
                 else
@@ -556,7 +568,8 @@ __global__ __launch_bounds__(kTopkThreads, MODE == kSelect && E == 16 ? 4 : 1) v
                     finish(std::integral_constant<int, kMostSelected>());
                 return;
             }
-            load(scores, bits); // (not kept in registers so far)
+            asm volatile("" : "+v"(i0)); // (nothing that depends on it is kept so far either)
+            load(scores, bits);
         }
     }
     const uint32_t columnBits = (4095u - i0) << 8;
@@ -568,8 +581,8 @@ __global__ __launch_bounds__(kTopkThreads, MODE == kSelect && E == 16 ? 4 : 1) v
 #pragma unroll
             for (int e = 0; e < E; ++e) {
                 const uint32_t order = ~all[e];
-                s.k[e] = Key(__builtin_amdgcn_alignbit(0x3ffu, order, 12), (order << 20) | (columnBits - (uint32_t)(e * 64 << 8)));
-                if (i0 + e * 64 >= (uint32_t)validCols)
+                s.k[e] = Key(__builtin_amdgcn_alignbit(0x3ffu, order, 12), (order << 20) | (columnBits - (e * kStep << 8)));
+                if (i0 + e * kStep >= (uint32_t)validCols)
                     s.k[e] = 1.0;
             }
             s.template Sort<kBits>(kBits);
@@ -592,19 +605,19 @@ __global__ __launch_bounds__(kTopkThreads, MODE == kSelect && E == 16 ? 4 : 1) v
     for (int e = 0; e < E; ++e) {
         const bool negZero = bits[e] == kSign; // compares equal to +0: same key, remembered below the column bits
         const uint32_t order = ScoreOrder(negZero ? 0u : bits[e]);
-        s.k[e] = Key(__builtin_amdgcn_alignbit(0x3ffu, order, 12), (order << 20) | (columnBits - (uint32_t)(e * 64 << 8) + (negZero ? 1u : 0u)));
+        s.k[e] = Key(__builtin_amdgcn_alignbit(0x3ffu, order, 12), (order << 20) | (columnBits - (e * kStep << 8) + (negZero ? 1u : 0u)));
     }
     if (__builtin_expect(!increasing, 0)) {
         __syncthreads(); // the ranks are there
 #pragma unroll
         for (int e = 0; e < E; ++e)
-            s.k[e] = Key(High(s.k[e]), (Low(s.k[e]) & 0xfff000ffu) | (4095u - rankOf[i0 + e * 64]) << 8); // (past the row's end: overwritten below)
+            s.k[e] = Key(High(s.k[e]), (Low(s.k[e]) & 0xfff000ffu) | (4095u - rankOf[i0 + e * kStep]) << 8); // (past the row's end: overwritten below)
         __syncthreads(); // and read, before their memory is used for something else
     }
     if (kClamp || validCols != N) {
 #pragma unroll
         for (int e = 0; e < E; ++e)
-            if (i0 + e * 64 >= (uint32_t)validCols)
+            if (i0 + e * kStep >= (uint32_t)validCols)
                 s.k[e] = 1.0;
     }
     s.template Sort<MODE == kWhole ? kBits : kBits - kWholeBits - 1>(keepBits);
@@ -671,10 +684,9 @@ int launch_topk(hipStream_t st, float *out_score, uint32_t *out_index, const flo
     // instruction's 256 bytes (8192 x 64, top 1 3.2 / 3.7, 131072 x 64, top 33 32.6 / 34.1), nor where they are much more than the L2s'
     // 32 MB, which then are written back while others sort (30000 x 2048, top 1500 261 / 268).
     const int through = topk >= 64 && 8ll * rows * topk <= 1ll << 26;
-    const int share = (int)((64ll * E * topk + valid_cols - 1) / valid_cols); // of topk, for a wave without padding
     constexpr int kRows = kTopkWaves / W;
     kernel<<<dim3((unsigned)(((long long)rows + kRows - 1) / kRows)), dim3(kTopkThreads), 0, st>>>(out_score, out_index, src, in_idx, rows, valid_cols,
-                                                                                                   ld, topk, keepBits, through, share);
+                                                                                                   ld, topk, keepBits, through);
     return pto_amd::check_launch();
 }
 
@@ -701,7 +713,9 @@ extern "C" int pto_topk_f32(void *stream, float *out_score, uint32_t *out_index,
     //   1024 columns:  600 rows, top 128 7.1 / 6.6   1500 rows, top 16  7.7 / 5.3   4800 rows, top 128 21.2 / 11.4; 128 rows, top 16 4.8 / 4.9, top 128 5.4 / 6.6, 700 rows, top 4 5.1 / 5.3
     //    512 columns: 4000 rows, top  16 7.9 / 6.1   8000 rows, top 60 16.6 / 12.6; 1000 rows, top 16 4.7 / 4.7, top 60 5.2 / 5.5
     // One wave per row of 1024 and two per row of 2048 where without the threshold there are four (1500 rows, top 16: 5.2 with one, 6.1 with four).
-    // Few distinct scores take longer (fewer than 64 of them, top 30: 512 x 1024 5.6 / 6.6, 1500 x 1024 8.5 / 7.5), so the line lies where that is even.
+    // (these with random scores.)  Near the line no kind of row measured is slower by more than 3 % than without, but for 8 x 2048, top 150, masked from the
+    // middle on 7.5 / 8.1.  600 x 1024, top 100: random 7.2 / 6.6, sixty distinct scores 7.2 / 6.6, all equal but 2 % 7.2 / 5.7; 8 x 2048, top 30, all
+    // equal but 2 %: 6.4 / 6.6.  Just past 1024 and 2048 columns the waves' thresholds lie lower for the short rows (1600 x 2049, top 100: 37.3 / 20.3).
     const int padded = valid_cols <= 512 ? 512 : valid_cols <= 1024 ? 1024 : valid_cols <= 2048 ? 2048 : 4096;
     if (valid_cols > 256 && topk <= padded / 8 && topk <= (valid_cols > 2048 || most < 10 ? 40 : 20) * kMostSelected) {
 #define PTO_TOPK_SELECT(E, W) return launch_topk<E, W>(st, out_score, out_index, src, in_idx, rows, valid_cols, ld, topk, true);

@@ -68,3 +68,22 @@ def test_topk_index_order(rows, cols):
                                   "pto_topk_f32")
     increasing, any_order = best_us([call(ids), call(mixed)])
     assert any_order <= 2.5 * increasing, (any_order, increasing)
+
+
+@pytest.mark.parametrize("rows,cols,topk", [(600, 1025, 256), (600, 2048, 100), (1600, 4096, 100), (5200, 512, 30)])
+def test_topk_threshold_and_the_rows(rows, cols, topk):
+    """Few of many by a threshold: whatever the rows look like, no slower than more keys of the same rows through the sort alone (ascending rows,
+    rows masked from the middle on or almost everywhere, and 1025 columns of any kind used to be, by 20 to 50 %)."""
+    lib = capi.load()
+    stream = torch.cuda.current_stream().cuda_stream
+    most = max(512, 1 << (cols - 1).bit_length()) // 8 + 1  # one more than the threshold takes
+    column = torch.arange(cols, device="cuda:0")
+    random = torch.randn((rows, cols), device="cuda:0")
+    ids = column.to(torch.int32)
+    score, index = torch.empty((rows, most), device="cuda:0"), torch.empty((rows, most), dtype=torch.int32, device="cuda:0")
+    for name, src in (("random", random), ("ascending", column.float().expand(rows, cols).contiguous()), ("masked", random.masked_fill(column > cols // 2, -torch.inf)),
+                      ("almost all masked", random.masked_fill(torch.rand_like(random) < 0.98, -torch.inf))):
+        def call(k):
+            return lambda: capi.check(lib.pto_topk_f32(stream, score.data_ptr(), index.data_ptr(), src.data_ptr(), ids.data_ptr(), rows, cols, cols, k), "pto_topk_f32")
+        threshold, sort = best_us([call(topk), call(most)])
+        assert threshold <= 1.05 * sort, (name, threshold, sort)

@@ -241,3 +241,23 @@ def test_topk_threshold_fails_next_to_a_long_list(oracle, rows, cols, topk):
     src[0::2, (block % 4 == 0)] += 100.0
     src[1::2, (block % 4 == 0) | (block % 4 == 1) | ((block % 4 == 2) & (lane < 6))] += 100.0
     assert same(topk_gpu(src, idx, cols, topk), oracle.topk_f32(src, idx, cols, topk))
+
+
+@pytest.mark.parametrize("rows,cols,topks", [(515, 1025, (20, 228, 244, 256)), (515, 1100, (37, 228, 256)), (517, 2048, (100, 256)), (130, 2049, (33, 256, 320)),
+                                             (130, 4096, (97, 320)), (900, 1024, (9, 60, 128)), (5200, 512, (16, 64))])
+def test_topk_threshold_and_the_columns(oracle, rows, cols, topks):
+    """Rows whose level changes along the columns, which the waves of a row share out among them, next to random ones in the same workgroup, and rows of
+    which far more keys equal the threshold than are wanted, in all blocks of 64 columns: those with the lowest columns, behind the larger ones, and
+    zeros of either sign among them."""
+    r = np.random.Generator(np.random.Philox(key=cols))
+    src, c = r.standard_normal((rows, cols)).astype(np.float32), np.arange(cols, dtype=np.float32)
+    kinds = (src[0::7], src[1::7], src[2::7], src[3::7], src[4::7], src[5::7])
+    kinds[0][:] = c
+    kinds[1][:] += 8 * c / cols
+    kinds[2][:, cols // 2:] = -np.inf
+    kinds[3][:] = np.where(r.random(kinds[3].shape) < 0.98, -np.inf, kinds[3])
+    kinds[4][:] = np.where(r.random(kinds[4].shape) < 0.02, np.abs(kinds[4]), np.where(r.random(kinds[4].shape) < 0.5, np.float32(0.0), np.float32(-0.0)))
+    kinds[5][:] = np.round(kinds[5] * 4)
+    idx = np.arange(cols, dtype=np.uint32)
+    for k in topks:
+        assert same(topk_gpu(src, idx, cols, k), oracle.topk_f32(src, idx, cols, k)), k
