@@ -357,24 +357,25 @@ __global__ __launch_bounds__(kTopkThreads, MODE == kSelect && E == 16 ? 4 : 1) v
     uint32_t *staged = reinterpret_cast<uint32_t *>(lds) + wave * (kStaged * kStages), *stagedColumn = staged + (kStages - 1) * kStaged;
     const int firstRank = waveOfRow * 64 * E, laneRank = (int)LaneRank((uint32_t)lane) * E, count = topk - firstRank;
     auto ordered = [] { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); __builtin_amdgcn_wave_barrier(); };
-    // lane by lane consecutive words; through: past the L2 (launch_topk)
+    // lane by lane consecutive words, all read before the first is stored; through: past the L2 (launch_topk)
     constexpr bool kThrough = MODE != kCut || N > 512; // (below, topk is 64 at most: 1000 x 300, top 30 5.2 us with the branch, 5.1 without)
-    constexpr auto eTag = std::integral_constant<int, E>();
+    constexpr int kStored = MODE == kWhole ? E : E * W > 8 ? E * W / 8 : 1; // times 64: of a row that is not sorted whole, an eighth and less
+    constexpr auto stored = std::integral_constant<int, kStored>();
     auto store = [&](auto keys, uint32_t *to, int n, auto &&word) __attribute__((always_inline)) {
+        uint32_t w[decltype(keys)::value];
+#pragma unroll
+        for (int e = 0; e < decltype(keys)::value; ++e)
+            w[e] = word(e * 64 + lane);
         if (kThrough && through) {
 #pragma unroll
-            for (int e = 0; e < decltype(keys)::value; ++e) {
-                const int i = e * 64 + lane;
-                if (i < n)
-                    __hip_atomic_store(to + i, word(i), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-            }
+            for (int e = 0; e < decltype(keys)::value; ++e)
+                if (e * 64 + lane < n)
+                    __hip_atomic_store(to + e * 64 + lane, w[e], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
         } else {
 #pragma unroll
-            for (int e = 0; e < decltype(keys)::value; ++e) {
-                const int i = e * 64 + lane;
-                if (i < n)
-                    to[i] = word(i);
-            }
+            for (int e = 0; e < decltype(keys)::value; ++e)
+                if (e * 64 + lane < n)
+                    to[e * 64 + lane] = w[e];
         }
     };
     if constexpr (MODE == kSelect) {
@@ -556,7 +557,7 @@ __global__ __launch_bounds__(kTopkThreads, MODE == kSelect && E == 16 ? 4 : 1) v
                     if (consecutive)
                         store(keys, toIndex, topk, [&](int i) { return first + at[i + i / 16]; });
                     else
-                        store(keys, toIndex, topk, [&](int i) { return inIdx[at[i + i / 16]]; });
+                        store(keys, toIndex, topk, [&](int i) { return inIdx[i < topk ? at[i + i / 16] : 0u]; }); // (behind topk may stand a column that is none)
                 };
                 if (total <= 64)
                     finish(std::integral_constant<int, 1>());
@@ -638,7 +639,7 @@ __global__ __launch_bounds__(kTopkThreads, MODE == kSelect && E == 16 ? 4 : 1) v
             stagedColumn[laneRank + e + (laneRank + e) / 16] = column[e];
     }
     ordered();
-    store(eTag, toScore, count, [&](int i) { return staged[i + i / 16]; });
+    store(stored, toScore, count, [&](int i) { return staged[i + i / 16]; });
     if (kStages == 1) {
         ordered();
 #pragma unroll
@@ -648,7 +649,7 @@ __global__ __launch_bounds__(kTopkThreads, MODE == kSelect && E == 16 ? 4 : 1) v
     }
     if (__builtin_expect(!consecutive, 0)) { // (staged: the column, or its rank)
 #pragma unroll
-        for (int e = 0; e < E; ++e) {
+        for (int e = 0; e < kStored; ++e) {
             const int i = e * 64 + lane;
             if (i < count) {
                 const uint32_t c = stagedColumn[i + i / 16];
@@ -657,7 +658,7 @@ __global__ __launch_bounds__(kTopkThreads, MODE == kSelect && E == 16 ? 4 : 1) v
         }
         return;
     }
-    store(eTag, toIndex, count, [&](int i) { return first + stagedColumn[i + i / 16]; });
+    store(stored, toIndex, count, [&](int i) { return first + stagedColumn[i + i / 16]; });
 }
 
 template <int E, int W>
