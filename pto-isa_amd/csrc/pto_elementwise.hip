@@ -309,19 +309,24 @@ extern "C" int pto_gather_rows(void *stream, void *out, const void *table, const
                 break;
             cpr = next;
         }
-    // Rows that this leaves whole, of no whole number of 64 bytes: slices of the output's 64-byte pieces (GatherPieces), as few as bring a slice of the table
-    // down to 1 MiB, of nine chunks and more, where the batch reads a row four times or more on average (us, whole / slices):
-    //   79891 rows of 1680 bytes out of 4950 32.5 / 22.5   110141 of 1168 out of 8421 32.7 / 26.5   16000 of 8016 out of 4000 35.6 / 27.5
-    //   6000 of 16032 out of 1500 26.7 / 18.9   20000 of 2064 out of 2000 10.7 / 8.3   60000 of 2000 out of 30000 35.0 / 39.3
-    // A narrow slice reads lines that it uses in part: not where those fill an XCD's L2 (200000 rows of 656 out of 20000 35.7 / 39.2, 60000 of
-    // 1200 out of 15000 20.9 / 21.6); from 15 chunks on a slice pays all the same (60000 of 2000 out of 15000 34.2 / 32.0).  Nor for
-    // a few MiB (1100 of 4016 out of 275 3.9 / 4.2).
+    // Rows that this leaves whole, most of them of no whole number of 64 bytes: slices of the output's 64-byte pieces (GatherPieces), as few as bring a slice of
+    // the table down to 1 MiB (us, whole / slices: a table in the memory-side cache; then one that is in no cache):
+    //   8 MiB, 16 times:  rows of 105 chunks 32.7 / 24.5, 33.4 / 28.7   129 chunks 32.8 / 24.2, 33.2 / 28.2      4.25 MiB, 16 times: 129 chunks 16.1 / 13.5, 16.0 / 15.8
+    //   8 MiB,  8 times:  rows of 253 chunks 17.6 / 14.1, 18.6 / 17.3   501 chunks 17.4 / 12.4, 18.4 / 16.7      24 MiB, 5 times: 501 chunks 34.5 / 24.5, 37.6 / 36.1
+    // A slice reads lines at its edges that it uses in part, and those come from memory again where no cache has them.  Where the batch reads a row sixteen
+    // times or more on average a slice of 24 chunks and more pays (of nine: 4.25 MiB read so 16.0 / 17.9; rows of 49 chunks in two 16.2 / 17.0); where it
+    // reads it less often, four of 32 and more and eight of 56 and more (8 MiB read eight times, 129 chunks in four 17.8 / 14.4, 18.7 / 19.5; 73 in eight 17.9 / 14.7,
+    // 19.1 / 23.0; 257 in eight 17.6 / 12.7, 18.6 / 18.8, in four 14.3, 18.0).  Nor where the L2 holds the whole table (88560 rows of 592 bytes out of
+    // 4428 9.2 / 10.6), nor slices of short rows that it does not hold (57 chunks in two, 24 MiB read five times 36.3 / 39.5), nor for less than 28 MiB of
+    // output (1100 of 4016 out of 275 3.9 / 4.2).
     const size_t tableBytes = table_rows * rowChunks * 16;
+    const bool often = n_idx >= 16 * table_rows;
     uint32_t pieces = 1;
-    if (parts == 1 && n_idx >= 4 * table_rows && rowChunks >= 32 && n_idx * rowChunks >= (size_t)1 << 19 && reinterpret_cast<uintptr_t>(out) % 64 == 0) {
-        while (pieces < 8 && tableBytes / pieces > ((size_t)1 << 20) && rowChunks >= 17 * pieces)
+    if (parts == 1 && n_idx >= 4 * table_rows && rowChunks >= (often ? 64 : 128) && n_idx * rowChunks >= (size_t)7 << 18 && tableBytes > ((size_t)15 << 18) &&
+        reinterpret_cast<uintptr_t>(out) % 64 == 0) {
+        while (pieces < 8 && tableBytes / pieces > ((size_t)1 << 20) && rowChunks >= (often ? 48 : pieces < 4 ? 64 : 112) * pieces)
             pieces *= 2;
-        if (rowChunks < 15 * pieces && tableBytes / pieces + table_rows * 128 > ((size_t)15 << 18))
+        if (rowChunks < 240 && tableBytes / pieces > ((size_t)1 << 22))
             pieces = 1;
     }
     if (pieces > 1)

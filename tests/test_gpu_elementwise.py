@@ -194,6 +194,27 @@ def test_gather_rows_in_pieces_of_the_output(oracle, rows, cols, nidx):
             assert (got[:shift] == 77).all() and (got[shift + nidx * width:] == 77).all()
 
 
+@pytest.mark.parametrize("rows,cols,nidx", [(3850, 520, 61601), (2560, 760, 40961), (2530, 776, 40481), (1290, 1544, 20641), (1290, 1544, 20639), (2100, 1032, 14501), (2100, 1016, 14701), (1020, 1928, 7621),
+                                            (1100, 2056, 7142), (600, 3592, 4101), (270, 8008, 1841)])
+def test_gather_rows_in_pieces_of_large_tables(oracle, rows, cols, nidx):
+    """Tables that no XCD's L2 holds, read sixteen times and more (two, four and eight slices of 24 chunks and more) or less (four of 32 and more, eight of 56 and more), widths on both
+    sides of where the number of slices changes; indices outside the table; nothing around the output, which begins at a piece or in one."""
+    r = np.random.default_rng(cols)
+    table = r.integers(0, 1 << 16, size=(rows, cols), dtype=np.uint16)
+    idx = r.integers(0, rows, size=nidx).astype(np.int32)
+    idx[::17] = -1 - idx[::17]
+    idx[5::31] = rows
+    want = oracle.gather_rows(table, idx)
+    tt, ti = torch.from_numpy(table.view(np.int16)).to("cuda:0"), torch.from_numpy(idx).to("cuda:0")
+    for shift in (0, 32, 8):
+        out = torch.full((nidx * cols + 128,), 77, dtype=tt.dtype, device="cuda:0")
+        capi.check(capi.load().pto_gather_rows(torch.cuda.current_stream().cuda_stream, out.data_ptr() + shift * 2, tt.data_ptr(), ti.data_ptr(), nidx, rows, cols, 2),
+                   "pto_gather_rows")
+        got = out.cpu().numpy()
+        assert np.array_equal(got[shift:shift + nidx * cols].view(np.uint16).reshape(nidx, cols), want), shift
+        assert (got[:shift] == 77).all() and (got[shift + nidx * cols:] == 77).all()
+
+
 @pytest.mark.parametrize("rows,cols,nidx", [(5, 24, 700), (1500, 1032, 3001), (3000, 1024, 6001)])
 @pytest.mark.parametrize("dtype", [torch.int16, torch.int32])
 def test_gather_rows_element_alignment(rows, cols, nidx, dtype):

@@ -87,3 +87,19 @@ def test_topk_threshold_and_the_rows(rows, cols, topk):
             return lambda: capi.check(lib.pto_topk_f32(stream, score.data_ptr(), index.data_ptr(), src.data_ptr(), ids.data_ptr(), rows, cols, cols, k), "pto_topk_f32")
         threshold, sort = best_us([call(topk), call(most)])
         assert threshold <= 1.05 * sort, (name, threshold, sort)
+
+
+def test_gather_of_odd_rows_against_whole_lines():
+    """A table that an XCD's L2 holds is read whole whatever its rows: 592 bytes to a row no slower than 512 (8 to 15 % slower when cut into slices)."""
+    lib = capi.load()
+    stream = torch.cuda.current_stream().cuda_stream
+    calls = []
+    for cols in (296, 256):
+        rows = (5 << 18) // cols
+        table = torch.randint(0, 30000, (rows, cols), dtype=torch.int16, device="cuda:0")
+        idx = torch.randint(0, rows, (20 * rows,), dtype=torch.int32, device="cuda:0")
+        out = torch.empty((20 * rows, cols), dtype=torch.int16, device="cuda:0")
+        calls.append(lambda t=table, i=idx, o=out: capi.check(lib.pto_gather_rows(stream, o.data_ptr(), t.data_ptr(), i.data_ptr(), i.numel(), t.shape[0], t.shape[1], 2),
+                                                              "pto_gather_rows"))
+    odd, lines = best_us(calls)
+    assert odd <= 1.05 * lines, (odd, lines)
