@@ -69,14 +69,16 @@ __device__ inline uint32_t QuantFour(f32x4 x, uint8_t &scaleByte)
 
 // Four loads per lane (16384 x 8192: 109.4 us with eight, 108.2 with four) and the last, partial piece in the same launch
 // (333 x 4128: 7.2 -> 4.3 us; 4096 x 6144 21.7 -> 20.7).
-// STREAM: elements stored past the caches.  The usual next reader is a GEMM, which finds what is stored the ordinary way in the
-// memory-side cache (256 MB): 1000 x 4096 and the product with 6144 columns behind it 39.7 -> 34.4 us, 4096 x 4096 and 2048
-// columns 52.8 -> 48.1, 8192 x 8192 and 512 columns 99 -> 90; the quantiser alone within 3 % up to 64 Mi elements (1000 x 4096
-// 5.4 and 5.0 us, 8192 x 8192 53.7 and 52.0).  Above that its input and output no longer fit there together and the ordinary stores cost
-// the quantiser 6 % (16384 x 8192: 106 and 113 us).
+// How the elements are stored.  Past the caches they have to be read from memory by the GEMM that usually follows; the others it finds in the memory-side
+// cache (256 MB): 1000 x 4096 and the product with 6144 columns behind it 34.8 -> 31.2 us, 4096 x 6144 and 2048 columns 67.6 -> 60.0, 8192 x 8192 and 512
+// columns 99.8 -> 83.7.  Left in the L2 they are written back behind the last one, which costs larger sizes more than it saves; through the L2
+// to memory does not (past the caches / in the L2 / through: 2048 x 4096 6.18 / 6.07 / 6.09, 4096 x 4096 11.9 / 12.9 / 12.0, 4096 x 6144 18.3 / 19.9 / 17.8,
+// 8192 x 8192 52.5 / 52.9 / 50.3; inputs in no cache: 1000 x 4096 4.66 / 4.76 / 5.00, 4096 x 6144 21.1 / 20.7 / 20.4, 8192 x 8192 54.7 / 57.1 / 55.2).
+// Above 64 Mi elements input and output do not fit that cache together (12288 x 8192: 79.3 all three).
+enum QuantStore { kInL2, kThroughL2, kPastCaches };
+constexpr size_t kQuantThroughFrom = ((size_t)1 << 23) + 1, kQuantStreamFrom = ((size_t)1 << 26) + 1;
 // (n is a multiple of 32, so groups and lanes are whole; the last workgroup's steps past n load and store nothing)
-constexpr size_t kQuantStreamFrom = ((size_t)1 << 26) + 1;
-template <bool STREAM>
+template <QuantStore STORE>
 __global__ __launch_bounds__(kQuantThreads) void QuantMxFp8(uint8_t *q, uint8_t *e8m0, const float *src, size_t n, size_t firstTile)
 {
     const size_t base = (firstTile + blockIdx.x) * (size_t)kQuantTile + 4 * threadIdx.x;
@@ -95,8 +97,10 @@ __global__ __launch_bounds__(kQuantThreads) void QuantMxFp8(uint8_t *q, uint8_t 
         uint8_t scaleByte;
         const uint32_t four = QuantFour(x[i], scaleByte); // every lane takes part in the lane moves
         if (at < n) {
-            if constexpr (STREAM)
+            if constexpr (STORE == kPastCaches)
                 __builtin_nontemporal_store(four, reinterpret_cast<uint32_t *>(q + at));
+            else if constexpr (STORE == kThroughL2)
+                __hip_atomic_store(reinterpret_cast<uint32_t *>(q + at), four, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
             else
                 *reinterpret_cast<uint32_t *>(q + at) = four;
             if ((threadIdx.x & 7) == 0)
@@ -122,7 +126,9 @@ extern "C" int pto_quant_mxfp8_f32(void *stream, uint8_t *q, uint8_t *scale, con
     constexpr size_t kMaxBlocks = 1u << 30;
     for (size_t t0 = 0; t0 < tiles; t0 += kMaxBlocks) {
         const size_t nb = tiles - t0 < kMaxBlocks ? tiles - t0 : kMaxBlocks;
-        (n >= kQuantStreamFrom ? QuantMxFp8<true> : QuantMxFp8<false>)<<<dim3((unsigned)nb), dim3(kQuantThreads), 0, st>>>(q, scale, src, n, t0);
+        // (through: whole 64-byte pieces only)
+        const bool through = n >= kQuantThroughFrom && reinterpret_cast<uintptr_t>(q) % 64 == 0;
+        (n >= kQuantStreamFrom ? QuantMxFp8<kPastCaches> : through ? QuantMxFp8<kThroughL2> : QuantMxFp8<kInL2>)<<<dim3((unsigned)nb), dim3(kQuantThreads), 0, st>>>(q, scale, src, n, t0);
     }
     return pto_amd::check_launch();
 }

@@ -148,3 +148,18 @@ def test_quant_mxfp8_both_sides_of_the_streaming_size():
         out.append((q, s))
     for whole, more in zip(*out):
         assert torch.equal(whole, more[:rows]) and more[rows].any()
+
+
+@pytest.mark.parametrize("rows,shift", [(8192, 0), (8193, 0), (8193, 4), (9001, 32)])
+def test_quant_mxfp8_through_the_l2(rows, shift):
+    """More than 2^23 elements are stored through the L2 where the output begins at a 64-byte piece: the bytes of the same rows quantised in parts of 2^20
+    elements, and nothing around them."""
+    cols, lib, stream = 1024, capi.load(), torch.cuda.current_stream().cuda_stream
+    x = torch.randn((rows, cols), device="cuda:0", generator=torch.Generator("cuda:0").manual_seed(rows))
+    q, s = torch.full((rows * cols + 128,), 77, dtype=torch.uint8, device="cuda:0"), torch.zeros((rows, cols // 32), dtype=torch.uint8, device="cuda:0")
+    capi.check(lib.pto_quant_mxfp8_f32(stream, q.data_ptr() + shift, s.data_ptr(), x.data_ptr(), rows, cols), "pto_quant_mxfp8_f32")
+    part, scale = torch.zeros((rows, cols), dtype=torch.uint8, device="cuda:0"), torch.zeros_like(s)
+    for r in range(0, rows, 1024):
+        capi.check(lib.pto_quant_mxfp8_f32(stream, part[r:].data_ptr(), scale[r:].data_ptr(), x[r:].data_ptr(), min(1024, rows - r), cols), "pto_quant_mxfp8_f32")
+    assert torch.equal(q[shift:shift + rows * cols].view(rows, cols), part) and torch.equal(s, scale)
+    assert (q[:shift] == 77).all() and (q[shift + rows * cols:] == 77).all()
