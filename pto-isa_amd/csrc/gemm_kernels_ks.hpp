@@ -218,10 +218,11 @@ int launch_gemm_ks(hipStream_t st, float *c, const half *a, const half *b, int m
     const long long tiles = (long long)((m + BM - 1) / BM) * ((n + BN - 1) / BN);
     if (tiles > 0x7fffffffll)
         return PTO_ERR_UNSUPPORTED;
-    // (half pieces past the L2 cost no more than they save while C is small: 1000 x 3000 x 2048 18.4 -> 17.9 us, 1024 x 3064 x 1024 13.0 and 13.1,
-    // 1024 x 6136 x 1024 18.8 and 19.8; and operands and C together: 503 x 6088 x 3072, 52 MB, 25.0 -> 24.5, x 6016, 91 MB, 51.2 -> 54.0)
+    // (half pieces past the L2 pay while C is small and k short: 1000 x 3000 x 1024 12.5 -> 12.0 us, with a conversion of C behind it 19.5 -> 18.5;
+    // 503 x 6088 x 1024 12.0 -> 11.6, 19.8 -> 18.3.  With more to read before, the product gains little and the reader of C loses more: 1000 x 3000 x 1536 15.5 -> 14.3,
+    // 20.2 -> 20.9; x 2048 18.4 -> 18.3, 22.5 -> 23.6; 503 x 6088 x 3072 24.2 -> 24.1, 28.4 -> 29.7.  1024 x 6136 x 1024, 25 MB of C, 18.8 and 19.8)
     const uint64_t bytes = 4ull * m * n;
-    const int through = pto_amd::store_through(c, 4ull * n, bytes) || (bytes <= 12u << 20 && bytes + 2ull * ((uint64_t)m + n) * k <= 64u << 20 && (n * 4ull | (uintptr_t)c) % 32 == 0);
+    const int through = pto_amd::store_through(c, 4ull * n, bytes) || (bytes <= 12u << 20 && k <= 1280 && (n * 4ull | (uintptr_t)c) % 32 == 0);
     (k % 64 ? half64 : whole)<<<dim3((unsigned)tiles), dim3(512), lds, st>>>(c, a, b, m, n, k, through);
     return pto_amd::check_launch();
 }

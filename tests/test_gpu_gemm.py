@@ -243,3 +243,14 @@ def test_gemm_results_past_the_l2(m, n, k, shift):
     want = a.float() @ b.float().t()
     assert torch.equal(c[shift:shift + m * n].view(m, n), want)
     assert (c[:shift] == 7.0).all() and (c[shift + m * n:] == 7.0).all()
+
+
+@pytest.mark.parametrize("m,n,k", [(250, 520, 1280), (250, 520, 1408), (1000, 3000, 1280), (1000, 3000, 1408)])
+def test_gemm_half_pieces_and_k(m, n, k):
+    """Half 64-byte pieces of C on both sides of the longest k at which they go past the L2: whole numbers, exact."""
+    lib = capi.load()
+    g = torch.Generator(device="cuda:0").manual_seed(k)
+    a, b = (torch.randint(-4, 5, (r, k), generator=g, device="cuda:0").half() for r in (m, n))
+    c = torch.full((m * n + 64,), 7.0, device="cuda:0")
+    capi.check(lib.pto_gemm_f16f32(torch.cuda.current_stream().cuda_stream, c.data_ptr(), a.data_ptr(), b.data_ptr(), m, n, k), "pto_gemm_f16f32")
+    assert torch.equal(c[:m * n].view(m, n), a.float() @ b.float().t()) and (c[m * n:] == 7.0).all()
