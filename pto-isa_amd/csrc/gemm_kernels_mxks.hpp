@@ -331,7 +331,8 @@ __global__ __launch_bounds__(512, MIN_WAVES) AICORE
                     }
                 });
             } else {
-                constexpr int q = g * kKept; // half a block
+                static_assert(kKept == 2, "whole blocks, or half of the only one");
+                constexpr int q = g * kKept;
                 const Words4 x = eight(std::integral_constant<int, q>());
                 const int row = rowLane + (int)r32, col = colLane + 8 * (q + (int)h);
                 if (row < m && col < n)

@@ -68,3 +68,20 @@ __global__ void Eights(_Float16 *p, Words4 v)
                 break
             waited += int(w[1]) + 1 if w[0] == "s_nop" else 1
         assert waited >= 2, code[i:i + 4]
+
+
+def test_mx_tile_of_three_blocks_a_wave_is_refused(tmp_path):
+    """The bf16 way out of the k-split MX kernels stores whole blocks of a wave, or half of its only one: a shape with three is a compile error
+    (it would store a third of its columns, and at the wrong place)."""
+    build = importlib.util.module_from_spec(importlib.util.spec_from_file_location("pto_amd_build", os.path.join(os.path.dirname(capi.LIB_PATH), "build.py")))
+    build.__spec__.loader.exec_module(build)
+    for bn, fine in ((128, True), (192, False)):
+        source = tmp_path / ("shape%d.hip" % bn)
+        source.write_text("""#define PTO_WAVES_M 4
+#define PTO_WAVES_N 1
+#define PTO_MFMA_M 16
+#include "gemm_kernels_mxks.hpp"
+int Launch(void *c, const uint8_t *x) { return launch_gemm_mxks<0, 0, bfloat16_t, 64, %d, 3, 2>(nullptr, c, x, x, x, x, 64, 192, 512); }
+""" % bn)
+        r = subprocess.run([build.HIPCC] + build.FLAGS + ["--cuda-device-only", "-fsyntax-only", str(source)], capture_output=True, text=True)
+        assert (r.returncode == 0) == fine and fine == ("half of the only one" not in r.stderr), r.stderr
