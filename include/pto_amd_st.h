@@ -194,6 +194,9 @@ int pto_st_tmrgsort_lists_16(void *stream, void *out, uint32_t *executed, const 
 int pto_st_matmul_vec_operands_f16_64x64x128(void *stream, float *out, float *mid, const uint16_t *a, const uint16_t *b);
 /* TTRANS on fp32: out [128,64] = in [64,128] transposed. */
 int pto_st_ttrans_f32_64x128(void *stream, float *out, const float *in);
+/* The conversion of two floats to bf16 (what the MX GEMMs store) against the closed form, every 32-bit pattern in either half: out[0] += inputs
+ * whose bits differ, out[1] = one of them. */
+int pto_st_bf16_pairs(void *stream, uint32_t *out);
 /* TPREFETCH of an int32 [16,64] matrix into a tile, TPACK to int16 (out16) and on to int8 (out8): the low bits of every
  * element (npu/a5/TPack.hpp:21-72); print != 0: TPRINT of a [4,16] tile with a [3,10] valid region and of a [2,4] view of
  * the input, in the reference's format (npu/a2a3/TPrint.hpp:44-190), on the process's standard output. */

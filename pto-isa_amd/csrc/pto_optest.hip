@@ -703,6 +703,26 @@ __global__ __launch_bounds__(kBlockThreads) AICORE void PushPopKernel(__gm__ flo
     TSTORE(go, oAcc);
 }
 
+// ---- the conversion of two elements to bf16 against the closed form of one ----
+// Every 32-bit pattern goes through the lower half, and through the upper one (an odd factor permutes them).
+__global__ __launch_bounds__(kBlockThreads) AICORE void Bf16Pairs(__gm__ uint32_t *out)
+{
+    const uint32_t threads = gridDim.x * kBlockThreads, first = blockIdx.x * kBlockThreads + threadIdx.x;
+    uint32_t wrong = 0, input = 0;
+    for (uint64_t i = first; i < (uint64_t)1 << 32; i += threads) {
+        const uint32_t lo = (uint32_t)i, hi = lo * 0x9e3779b1u;
+        const float a = __builtin_bit_cast(float, lo), b = __builtin_bit_cast(float, hi);
+        const uint32_t pair = detail::f32x2_to_bf16_bits_rne(a, b);
+        const bool low = (uint16_t)pair != detail::f32_to_bf16_bits_rne(a), high = (uint16_t)(pair >> 16) != detail::f32_to_bf16_bits_rne(b);
+        wrong += low || high ? 1u : 0u;
+        input = low ? lo : high ? hi : input;
+    }
+    if (wrong != 0) {
+        atomicAdd(out, wrong);
+        out[1] = input;
+    }
+}
+
 } // namespace
 
 PTO_DEVICE_CODE_END
@@ -1530,6 +1550,13 @@ extern "C" int pto_st_ttrans_f32_64x128(void *stream, float *out, const float *i
 {
     PTO_ST_NONNULL(out, in);
     TransKernel<<<dim3(1), dim3(kBlockThreads), 0, static_cast<hipStream_t>(stream)>>>(out, in);
+    return pto_amd::check_launch();
+}
+
+extern "C" int pto_st_bf16_pairs(void *stream, uint32_t *out)
+{
+    PTO_ST_NONNULL(out);
+    Bf16Pairs<<<dim3(4096), dim3(kBlockThreads), 0, static_cast<hipStream_t>(stream)>>>(out);
     return pto_amd::check_launch();
 }
 

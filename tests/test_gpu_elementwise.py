@@ -39,6 +39,15 @@ def test_tcvt_bf16_boundaries_and_strided_sweep(oracle):
     assert np.array_equal(got[~nan], want[~nan])
 
 
+def test_bf16_of_two_floats_is_the_closed_form():
+    """The hardware conversion by which the MX GEMMs store bf16: the bits of the closed form (pinned above) for every float, ties, subnormals, the edge to
+    infinity, infinities and NaNs among them, in either half of the pair."""
+    out = torch.zeros(2, dtype=torch.int32, device="cuda:0")
+    capi.check(capi.load_st().pto_st_bf16_pairs(torch.cuda.current_stream().cuda_stream, out.data_ptr()), "pto_st_bf16_pairs")
+    wrong, one = out.cpu().numpy().view(np.uint32)
+    assert wrong == 0, hex(one)
+
+
 @pytest.mark.parametrize("n", [0, 1, 7, 8, 8191, 8192, 8193, 3 * 8192 + 5])
 def test_tcvt_ragged_sizes(oracle, n):
     from gpu_util import tcvt
