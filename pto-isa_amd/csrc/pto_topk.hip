@@ -411,9 +411,10 @@ __global__ __launch_bounds__(kTopkThreads, MODE == kSelect && E == 16 ? 4 : 1) v
                 least = low0 < low1 ? low0 : low1;
             }
             uint32_t t = ~WaveMax(~least);
-            // (groups more than wanted; with four waves and more than 64 groups of each, more than a sixteenth would come close to the longest list)
-            const int close = W == 4 && wanted > 64 ? wanted / 16 : wanted / 8;
-            const int loose = wanted > 64 ? (W == 1 || (W == 2 && wanted <= 96) ? 32 : close) : wanted / 2 + 4 < 16 ? wanted / 2 + 4 : 16;
+            // (groups more than wanted: as many as leave random rows' lists below 256 or 512, which are sorted in the same time; 64 x 4096, top 320 9.3 us, 15.4 where one
+            // row is past 512; 600 x 2048, top 160 8.2 and 9.1 past 256)
+            const int close = W == 4 && wanted > 64 ? wanted / 32 : wanted / 8;
+            const int loose = wanted <= 64 ? (wanted / 2 + 4 < 16 ? wanted / 2 + 4 : 16) : W == 1 ? 32 : W == 2 && wanted <= 96 ? (wanted <= 80 ? 12 : 32) : close;
             // (the first look is right above the smallest: the end already where most are equal.  Few distinct scores may have no place for a tight
             // threshold: from the eighth look on as many groups more will do as no longer a sort pays for; 4800 x 1024, top 40 of 60 distinct 10.2 -> 8.4 us)
             auto search = [&](auto groups, const uint32_t *max) __attribute__((always_inline)) {
@@ -710,15 +711,14 @@ extern "C" int pto_topk_f32(void *stream, float *out_score, uint32_t *out_index,
     const int most = 5 * 4 * pto_amd::compute_units() / rows; // waves per row for five on every SIMD
     // A threshold, then a sort of what reaches it (us, merges that keep topk / threshold):
     //   4096 columns:    1 row,  top   1 8.0 / 5.8    128 rows, top 50 10.2 / 6.5   1200 rows, top 300 31.7 / 22.6
-    //   2048 columns:    8 rows, top  10 6.0 / 5.3    900 rows, top 30 11.0 / 6.2   2400 rows, top 256 26.2 / 17.3; few rows and many keys: 8 rows, top 200 7.6 / 8.7
+    //   2048 columns:    8 rows, top  10 6.0 / 5.3    900 rows, top 30 11.0 / 6.2   2400 rows, top 256 26.2 / 17.3; few rows and many keys: 64 rows, top 140 7.6 / 8.4
     //   1024 columns:  600 rows, top 128 7.1 / 6.6   1500 rows, top 16  7.7 / 5.3   4800 rows, top 128 21.2 / 11.4; 128 rows, top 16 4.8 / 4.9, top 128 5.4 / 6.6, 700 rows, top 4 5.1 / 5.3
     //    512 columns: 4000 rows, top  16 7.9 / 6.1   8000 rows, top 60 16.6 / 12.6; 1000 rows, top 16 4.7 / 4.7, top 60 5.2 / 5.5
     // One wave per row of 1024 and two per row of 2048 where without the threshold there are four (1500 rows, top 16: 5.2 with one, 6.1 with four).
-    // (these with random scores.)  Near the line no kind of row measured is slower by more than 3 % than without, but for 8 x 2048, top 150, masked from the
-    // middle on 7.5 / 8.1.  600 x 1024, top 100: random 7.2 / 6.6, sixty distinct scores 7.2 / 6.6, all equal but 2 % 7.2 / 5.7; 8 x 2048, top 30, all
+    // (these with random scores.)  Near the line no kind of row measured is slower by more than 3 % than without.  600 x 1024, top 100: random 7.2 / 6.6, sixty distinct scores 7.2 / 6.6, all equal but 2 % 7.2 / 5.7; 8 x 2048, top 30, all
     // equal but 2 %: 6.4 / 6.6.  Just past 1024 and 2048 columns the waves' thresholds lie lower for the short rows (1600 x 2049, top 100: 37.3 / 20.3).
     const int padded = valid_cols <= 512 ? 512 : valid_cols <= 1024 ? 1024 : valid_cols <= 2048 ? 2048 : 4096;
-    if (valid_cols > 256 && topk <= padded / 8 && topk <= (valid_cols > 2048 || most < 10 ? 40 : 20) * kMostSelected) {
+    if (valid_cols > 256 && topk <= padded / 8 && topk <= (valid_cols > 2048 || most < 10 ? 320 : most < 20 ? 160 : 128)) {
 #define PTO_TOPK_SELECT(E, W) return launch_topk<E, W>(st, out_score, out_index, src, in_idx, rows, valid_cols, ld, topk, true);
         if (valid_cols > 2048)
             PTO_TOPK_SELECT(16, 4)

@@ -244,7 +244,7 @@ def test_topk_threshold_fails_next_to_a_long_list(oracle, rows, cols, topk):
 
 
 @pytest.mark.parametrize("rows,cols,topks", [(515, 1025, (20, 228, 244, 256)), (515, 1100, (37, 228, 256)), (517, 2048, (100, 256)), (130, 2049, (33, 256, 320)),
-                                             (130, 4096, (97, 320)), (900, 1024, (9, 60, 128)), (5200, 512, (16, 64))])
+                                             (130, 4096, (97, 320)), (900, 1024, (9, 60, 128)), (5200, 512, (16, 64)), (250, 1500, (128, 129)), (300, 1500, (160, 161))])
 def test_topk_threshold_and_the_columns(oracle, rows, cols, topks):
     """Rows whose level changes along the columns, which the waves of a row share out among them, next to random ones in the same workgroup, and rows of
     which far more keys equal the threshold than are wanted, in all blocks of 64 columns: those with the lowest columns, behind the larger ones, and
