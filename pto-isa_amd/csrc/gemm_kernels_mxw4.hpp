@@ -388,7 +388,7 @@ AICORE inline __attribute__((always_inline)) void MxW4TileCompute(__gm__ const u
 
 // This wave's accumulator blocks to C (row-major, n elements between rows; fp32, or bf16 rounded to nearest even).  bf16: a lane has
 // four columns of a row, 8 bytes; two blocks side by side change lanes so that it has eight of one of them, and a store
-// instruction writes 64 bytes of each of its sixteen rows, as with fp32 (and the hardware conversion: 6144^3 188 -> 179 us in fp8, 121 -> 112
+// instruction writes 64 bytes of each of its sixteen rows, as with fp32 (and the hardware conversion: 6144^3 182 -> 175 us in fp8, 121 -> 112
 // in fp4, 1000 x 6144 x 4096 in fp8 31.5 -> 28.3, of which 1.3 by storing past the L2).
 template <typename OutT, int BN>
 AICORE inline __attribute__((always_inline)) void MxW4StoreTile(OutT *out, int64_t n, int row0, int col0, int through)

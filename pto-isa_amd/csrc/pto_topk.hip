@@ -33,7 +33,7 @@
 //   indices); the rank of a column in that order then stands in the scores' keys for the column.  4800 x 1024 whole: 42 us (127
 //   with keys in the LDS and a pass over it per stage); 1000 x 256: 6.6 (15).
 // What bounds it: vector instructions, 2520 per row of 1024 (3850 in the integer network this replaced), behind a phase of
-// loads and before one of stores that all waves share: of 23.2 us (4800 x 1024, top 1000, 58 MB = 9 us at 6.5 TB/s) 10 are
+// loads and before one of stores that all waves share: of 21.9 us (4800 x 1024, top 1000, 58 MB = 9 us at 6.5 TB/s) 9 are
 // launch, loads and stores (five waves on a SIMD instead of four, at 96 registers of 106: 28.0 and 28.2 us on one card).  Persistent waves that load the next row while they sort one, and wave priorities that let
 // some run ahead, do not hide them (32 us and no change).
 #include <hip/hip_runtime.h>
@@ -248,8 +248,8 @@ constexpr int kWholeBits = 2;
 // one key per lane and four waves per row: for few rows of which more than 16 are wanted, where the whole sort is the shorter one
 template <int E, int W>
 constexpr bool kOnlyWhole = E == 1 && W == 4;
-// kCut: merges that keep what topk asks for; kSelect: by a threshold, kCut where that fails.  What bounds kSelect: 5.5 us of 8.3 (4800 x 1024, top 40) are
-// launch and the 20 MB of the rows; the rest is 480 vector and 270 scalar instructions a row (the whole network: 2520 vector ones).  Four places of the interval at a time instead
+// kCut: merges that keep what topk asks for; kSelect: by a threshold, kCut where that fails.  What bounds kSelect (4800 x 1024, top 40, 6.9 us):
+// the launch, the 20 MB of the rows (3.1 us at 6.5 TB/s), and 480 vector and 280 scalar instructions a row (the whole network: 2520 vector ones).  Four places of the interval at a time instead
 // of one took 2.2 us more (scalar instructions), positions in the list by ballots instead of one scan over the lanes 1.2.
 constexpr int kMostSelected = 8; // times 64 keys
 enum Mode { kCut, kWhole, kSelect };
