@@ -709,14 +709,14 @@ extern "C" int pto_topk_f32(void *stream, float *out_score, uint32_t *out_index,
     // up to 1706 rows (1700 rows with two 25.6, with four 24.5; 2000 rows 26.2, 26.9).  129 to 256 columns: four up to 365 rows where
     // more than 16 are wanted (one / four: 128 rows 3.6 / 3.3, 300 rows 3.6 / 3.4, 600 rows 3.7 / 3.7; top 7 of 128 rows 3.2 / 3.6).
     const int most = 5 * 4 * pto_amd::compute_units() / rows; // waves per row for five on every SIMD
-    // A threshold, then a sort of what reaches it (us, merges that keep topk / threshold):
-    //   4096 columns:    1 row,  top   1 8.0 / 5.8    128 rows, top 50 10.2 / 6.5   1200 rows, top 300 31.7 / 22.6
-    //   2048 columns:    8 rows, top  10 6.0 / 5.3    900 rows, top 30 11.0 / 6.2   2400 rows, top 256 26.2 / 17.3; few rows and many keys: 64 rows, top 140 7.6 / 8.4
-    //   1024 columns:  600 rows, top 128 7.1 / 6.6   1500 rows, top 16  7.7 / 5.3   4800 rows, top 128 21.2 / 11.4; 128 rows, top 16 4.8 / 4.9, top 128 5.4 / 6.6, 700 rows, top 4 5.1 / 5.3
-    //    512 columns: 4000 rows, top  16 7.9 / 6.1   8000 rows, top 60 16.6 / 12.6; 1000 rows, top 16 4.7 / 4.7, top 60 5.2 / 5.5
+    // A threshold, then a sort of what reaches it (us, merges that keep topk / threshold; random scores):
+    //   4096 columns:    1 row,  top   1 7.9 / 5.5    128 rows, top 50 10.4 / 6.6   1200 rows, top 300 31.9 / 18.8
+    //   2048 columns:    8 rows, top  10 6.1 / 5.4    900 rows, top 30 10.9 / 6.0   2400 rows, top 256 25.0 / 16.5; few rows and many keys: 64 rows, top 140 7.6 / 8.4
+    //   1024 columns:  600 rows, top 128 7.2 / 6.5   1500 rows, top 16  7.6 / 5.4   4800 rows, top 128 19.9 / 9.9; 128 rows, top 16 4.8 / 4.9, top 128 5.4 / 6.6, 700 rows, top 4 5.1 / 5.3
+    //    512 columns: 4000 rows, top  16 7.5 / 6.0   8000 rows, top 60 14.7 / 10.6; 1000 rows, top 16 4.7 / 4.7, top 60 5.2 / 5.5
     // One wave per row of 1024 and two per row of 2048 where without the threshold there are four (1500 rows, top 16: 5.2 with one, 6.1 with four).
-    // (these with random scores.)  Near the line no kind of row measured is slower by more than 3 % than without.  600 x 1024, top 100: random 7.2 / 6.6, sixty distinct scores 7.2 / 6.6, all equal but 2 % 7.2 / 5.7; 8 x 2048, top 30, all
-    // equal but 2 %: 6.4 / 6.6.  Just past 1024 and 2048 columns the waves' thresholds lie lower for the short rows (1600 x 2049, top 100: 37.3 / 20.3).
+    // Near the line no kind of row measured is slower by more than 3 % than without.  600 x 1024, top 100: random 7.2 / 6.6, sixty distinct scores 7.2 / 6.6, all
+    // equal but 2 % 7.2 / 5.7; 8 x 2048, top 30, all equal but 2 %: 6.4 / 6.6.  Just past 1024 and 2048 columns the waves' thresholds lie lower for the short rows (1600 x 2049, top 100: 37.3 / 20.3).
     const int padded = valid_cols <= 512 ? 512 : valid_cols <= 1024 ? 1024 : valid_cols <= 2048 ? 2048 : 4096;
     if (valid_cols > 256 && topk <= padded / 8 && topk <= (valid_cols > 2048 || most < 10 ? 320 : most < 20 ? 160 : 128)) {
 #define PTO_TOPK_SELECT(E, W) return launch_topk<E, W>(st, out_score, out_index, src, in_idx, rows, valid_cols, ld, topk, true);
