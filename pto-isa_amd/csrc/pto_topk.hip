@@ -29,13 +29,15 @@
 //   Where too many keys equal the threshold (masked rows), as many of them as are wanted are taken in the order of their columns; where that does
 //   not do either, or the indices do not increase, the row is sorted as before.  4800 x 1024, top 40 18.7 -> 6.9 us (all equal but 2 % 18.5 -> 7.9);
 //   600 x 2048, top 100 10.8 -> 7.1 (ascending 5.9, masked from the middle on 7.4); 600 x 4096, top 100 18.3 -> 7.9.
+// * Whole sorts of 257 columns and more (BucketSort): the keys are counted into buckets and put in place, two and more in a bucket by a few exchanges of
+//   neighbours; rows too uneven for that go through the network.  4800 x 1024, top 1000 21.2 -> 14.2 us, 1 x 4096 whole 12.5 -> 7.9, 2400 x 2048 26.6 -> 16.9.
 // * Any other index vector: the same network sorts the (index, column) pairs first, once per workgroup (the rows share their
 //   indices); the rank of a column in that order then stands in the scores' keys for the column.  4800 x 1024 whole: 42 us (127
 //   with keys in the LDS and a pass over it per stage); 1000 x 256: 6.6 (15).
-// What bounds it: vector instructions, 2520 per row of 1024 (3850 in the integer network this replaced), behind a phase of
-// loads and before one of stores that all waves share: of 21.9 us (4800 x 1024, top 1000, 58 MB = 9 us at 6.5 TB/s) 9 are
-// launch, loads and stores (five waves on a SIMD instead of four, at 96 registers of 106: 28.0 and 28.2 us on one card).  Persistent waves that load the next row while they sort one, and wave priorities that let
-// some run ahead, do not hide them (32 us and no change).
+// What bounds the network: vector instructions, 2520 per row of 1024 (3850 in the integer network this replaced), behind a phase of
+// loads and before one of stores that all waves share (five waves on a SIMD instead of four: no change; persistent waves that load the next row while they sort
+// one, and wave priorities that let some run ahead, do not hide them: 32 us and no change).  By buckets 4800 x 1024, top 1000 (58 MB = 9 us at 6.5 TB/s)
+// is bound by the launch, the loads and the stores, with some 800 vector and 110 LDS instructions a row between them.
 #include <hip/hip_runtime.h>
 
 #include "common.hpp"
@@ -253,6 +255,9 @@ constexpr bool kOnlyWhole = E == 1 && W == 4;
 // of one took 2.2 us more (scalar instructions), positions in the list by ballots instead of one scan over the lanes 1.2.
 constexpr int kMostSelected = 8; // times 64 keys
 enum Mode { kCut, kWhole, kSelect };
+// whole sorts by buckets first
+template <int E, int W>
+constexpr bool kBuckets = E >= 4 && E * W >= 8;
 // the largest value of the wave, the same in every lane's scalar registers; the sum up to and with this lane
 __device__ inline uint32_t WaveMax(uint32_t v)
 {
@@ -275,20 +280,315 @@ __device__ inline uint32_t WaveScan(uint32_t v)
     v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xc, 0xf, false);
     return v;
 }
+// the key of a score: its order, the column's bits (behind equal scores the lower column, with the larger ones, comes first)
+__device__ inline double TopkKey(uint32_t bits, uint32_t columnBits)
+{
+    const bool negZero = bits == kSign; // compares equal to +0: same key, remembered below the column bits
+    const uint32_t order = ScoreOrder(negZero ? 0u : bits);
+    return Key(__builtin_amdgcn_alignbit(0x3ffu, order, 12), (order << 20) | (columnBits + (negZero ? 1u : 0u)));
+}
+__device__ inline float Larger(float a, float b, float c)
+{
+    float r;
+    asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+    return r;
+}
+__device__ inline float Smaller(float a, float b, float c)
+{
+    float r;
+    asm("v_min3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+    return r;
+}
+// the largest and the smallest value of the wave, in every lane (quad_perm twice, row_half_mirror, row_mirror, row_bcast:15 and :31, of which the last lane has
+// both; the two chains side by side, each with the wait states that a lane move asks for)
+__device__ inline void WaveEnds(float &hi, float &lo)
+{
+#define PTO_TOPK_BOTH(move) "v_max_f32_dpp %0, %0, %0 " move "\n\tv_min_f32_dpp %1, %1, %1 " move "\n\ts_nop 0\n\t"
+    asm volatile("s_nop 1\n\t" PTO_TOPK_BOTH("quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf") PTO_TOPK_BOTH("quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf")
+                     PTO_TOPK_BOTH("row_half_mirror row_mask:0xf bank_mask:0xf") PTO_TOPK_BOTH("row_mirror row_mask:0xf bank_mask:0xf")
+                         PTO_TOPK_BOTH("row_bcast:15 row_mask:0xa bank_mask:0xf") PTO_TOPK_BOTH("row_bcast:31 row_mask:0xc bank_mask:0xf") "s_nop 0"
+                 : "+v"(hi), "+v"(lo));
+#undef PTO_TOPK_BOTH
+    hi = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, hi), 63));
+    lo = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, lo), 63));
+}
+
+// Sorting of the 64 E W keys of a row, descending, by counting: the scores are spread evenly over 2 N buckets between the row's largest
+// and its smallest one, the keys in each are counted, sums over the counts say where a bucket begins, every key goes to the next place of its
+// bucket in a list, and neighbours change places (odd and even pairs in turn) as often as the fullest bucket has keys (5 to 9 of 1024 random scores).
+// 2 N counters of 16 bits: with N of them buckets hold twice as many keys.  Which rows: any whose scores are finite and not crowded in a small part of
+// their range; the others (masked with infinities, nearly all equal, heavy tails) are found by a look at 64 scores that takes them 1 to 6 % of their time
+// (us, network / with the look before it / buckets of random scores: 4800 x 1024, top 1000 21.0 / 21.9 / 14.2; 9000 x 512 whole 16.7 / 17.8 / 11.3;
+// 1500 x 1000, top 900 10.1 / 10.2 / 7.8; 1600 x 2048 20.9 / 21.1 / 11.5; 1 x 4096 12.5 / 12.7 / 7.9).  Tried for them and slower than the network: 64 of the row's own scores,
+// sorted, as the limits of ranges that are spread evenly each (4800 x 1024 27 us).  512 columns in up to 731 rows stay with the network (4.2 us; by
+// buckets 4.5 in two waves a row, 4.5 in one), as do 256 and less.
+// bits[e]: the score in column i0 + 64 e; afterwards key e of the lane with number q = 64 (wave of the row) + lane is of rank q E + e.
+// mem: 8 N bytes for the row; across: four sets of a word per wave of the workgroup.
+// Is it so in every lane of the workgroup?  One barrier (__syncthreads_and: three, and an atomic).  votes: a word per wave, another set of them for the next vote
+__device__ inline bool Everyone(bool v, uint32_t *votes)
+{
+    votes[threadIdx.x / 64] = __builtin_amdgcn_ballot_w64(!v) == 0;
+    __syncthreads();
+    static_assert(kTopkWaves == 4, "four words");
+    return __builtin_amdgcn_readfirstlane((int)(votes[0] & votes[1] & votes[2] & votes[3])) != 0;
+}
+__device__ inline bool WholeWave(bool v) { return __builtin_amdgcn_ballot_w64(!v) == 0; }
+
+enum Counted { kSorted, kNothingDone, kLost }; // kNothingDone: scores too uneven, or some not finite; kLost: the same, and bits is gone
+template <int E, int W>
+struct BucketSort {
+    static constexpr int N = 64 * E * W, kLogN = __builtin_ctz(N);
+    static constexpr int kCrowd = 6;   // of 64 scores, in a 512th of the range: the fullest bucket would have some 24 keys
+    static constexpr int kSurely = 16; // keys in a bucket up to which all passes are made without a look whether they are needed
+    static constexpr int kMost = 32;   // and with one; more only where they are in order by themselves (equal ones)
+    double k[E];
+
+    static __device__ inline void Meet()
+    {
+        if constexpr (W > 1) {
+            __syncthreads();
+        } else {
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+        }
+    }
+    // where place p of the list (and word w of the counters, four at a time) stands, so that lanes E apart meet in no bank
+    static __device__ inline uint32_t Place(uint32_t p) { return p ^ ((p >> 5) & (uint32_t)(E - 1)); }
+    static __device__ inline uint32_t Word(uint32_t w) { return w ^ ((w >> 4) & (uint32_t)(E - 4)); }
+    // the neighbours' keys across the lanes' borders: the first key of the lane above, the last one of the lane below
+    __device__ inline void Neighbours(double &above, double &below, int waveOfRow, int lane, uint64_t *edges)
+    {
+        StageEdge();
+        above = Key((uint32_t)__builtin_amdgcn_update_dpp(0, (int)High(k[0]), 0x130, 0xf, 0xf, false), // wave_shl:1
+                    (uint32_t)__builtin_amdgcn_update_dpp(0, (int)Low(k[0]), 0x130, 0xf, 0xf, false));
+        below = Key((uint32_t)__builtin_amdgcn_update_dpp(0x40000000, (int)High(k[E - 1]), 0x138, 0xf, 0xf, false), // wave_shr:1
+                    (uint32_t)__builtin_amdgcn_update_dpp(0, (int)Low(k[E - 1]), 0x138, 0xf, 0xf, false));
+        if constexpr (W > 1) { // edges: the first and the last key of each wave of the row
+            if (lane == 0)
+                edges[2 * waveOfRow] = __builtin_bit_cast(uint64_t, k[0]);
+            if (lane == 63)
+                edges[2 * waveOfRow + 1] = __builtin_bit_cast(uint64_t, k[E - 1]);
+            __syncthreads();
+            if (lane == 63 && waveOfRow + 1 < W)
+                above = __builtin_bit_cast(double, edges[2 * (waveOfRow + 1)]);
+            if (lane == 0 && waveOfRow > 0)
+                below = __builtin_bit_cast(double, edges[2 * (waveOfRow - 1) + 1]);
+        }
+    }
+    static __device__ inline void Exchange(double &hi, double &lo)
+    {
+        const double a = Max(hi, lo), b = Min(hi, lo);
+        hi = a;
+        lo = b;
+    }
+
+    __device__ inline __attribute__((always_inline)) Counted Sort(const uint32_t (&bits)[E], uint32_t i0, int validCols, int waveOfRow, int lane, uint32_t *mem, uint32_t *across)
+    {
+        const uint32_t q = (uint32_t)(waveOfRow * 64 + lane), wave = threadIdx.x / 64;
+        // the range
+        auto score = [&](int e) { return __builtin_bit_cast(float, bits[e]); };
+        float top = score(0), low = score(0);
+#pragma unroll
+        for (int e = 0; e < E; e += 2) {
+            top = Larger(top, score(e), score(e + 1));
+            low = Smaller(low, score(e), score(e + 1));
+        }
+        WaveEnds(top, low);
+        float range = top - low;
+        // a look at 64 scores (two columns in turn of either half) of each wave before anything else is done: how many are near either of two of them
+        bool even = (range >= 1e-30f) & (range <= 1e37f);
+        {
+            uint32_t seen = bits[0], half = bits[E / 2];
+            asm("" : "+v"(half)); // (else the choice is made between their addresses, and bits put into memory)
+            seen = (lane & 1) ? half : seen;
+            if (validCols != N) // (what stands behind the last column is near nothing)
+                seen = i0 + ((lane & 1) ? 32u * E : 0u) < (uint32_t)validCols ? seen : 0x7fffffffu;
+#pragma unroll
+            for (int g = 0; g < 2; ++g) {
+                const float one = __builtin_bit_cast(float, __builtin_amdgcn_readlane((int)seen, g == 0 ? 9 : 38));
+                even &= __builtin_popcountll(__builtin_amdgcn_ballot_w64(__builtin_fabsf(__builtin_bit_cast(float, seen) - one) <= range * (1.0f / 1024.0f))) < kCrowd;
+            }
+            if (validCols != N) // (a wave that has nothing behind the last column)
+                even = even || (int)i0 - lane + 64 >= validCols;
+        }
+        if (W > 1 ? !Everyone(even, across) : !WholeWave(even))
+            return kNothingDone;
+        // counters of buckets w and N + w in word w; behind them W words for each of a few exchanges
+        uint32_t *const count = mem, *const each = mem + N;
+#pragma unroll
+        for (int c = 0; c < E / 4; ++c)
+            reinterpret_cast<uint4 *>(count)[(waveOfRow * (E / 4) + c) * 64 + lane] = make_uint4(0, 0, 0, 0);
+        if constexpr (W > 1) {
+            reinterpret_cast<float *>(each)[waveOfRow] = top;
+            reinterpret_cast<float *>(each)[W + waveOfRow] = low;
+        }
+        Meet();
+        if constexpr (W > 1) {
+#pragma unroll
+            for (int w = 0; w < W; ++w) {
+                top = __builtin_fmaxf(top, reinterpret_cast<const float *>(each)[w]);
+                low = __builtin_fminf(low, reinterpret_cast<const float *>(each)[W + w]);
+            }
+            range = top - low;
+        }
+        const float scale = (float)(2 * N - 1) * __builtin_amdgcn_rcpf(range);
+        auto isColumn = [&](int e) { return i0 + 64u * (uint32_t)e < (uint32_t)validCols; };
+        uint32_t at[E], one[E];
+        float odd = range <= 1e37f ? 0.0f : __builtin_nanf(""); // a NaN where a score is none
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+            // (both steps round larger and smaller scores the same way: no score passes another)
+            const uint32_t b = (uint32_t)((top - score(e)) * scale);
+            odd = __builtin_fmaf(score(e), 0.0f, odd);
+            one[e] = 1u << ((b >> (kLogN - 4)) & 16u);
+            at[e] = Word(b & (uint32_t)(N - 1));
+        }
+        if (validCols != N) {
+#pragma unroll
+            for (int e = 0; e < E; ++e) {
+                one[e] = isColumn(e) ? one[e] : 0u;
+                at[e] = isColumn(e) ? at[e] : q; // (many lanes at one counter would wait for each other)
+            }
+        }
+#pragma unroll
+        for (int e = 0; e < E; ++e)
+            __hip_atomic_fetch_add(count + at[e], one[e], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        Meet();
+        // where the buckets begin, both halves of a word at once (no sum is above 4096); the upper half behind all of the lower one
+        uint32_t full = 0; // keys in the fullest bucket
+        {
+            uint4 *const mine = reinterpret_cast<uint4 *>(count) + q * (E / 4);
+            auto chunk = [&](int j) { return Word(q * E + 4 * j) / 4 - q * (E / 4); };
+            uint32_t c[E], sum = 0;
+#pragma unroll
+            for (int j = 0; j < E / 4; ++j) {
+                const uint4 v = mine[chunk(j)];
+                c[4 * j] = v.x, c[4 * j + 1] = v.y, c[4 * j + 2] = v.z, c[4 * j + 3] = v.w;
+            }
+            typedef uint16_t Pair __attribute__((ext_vector_type(2)));
+#pragma unroll
+            for (int e = 0; e < E; ++e) {
+                sum += c[e];
+                full = __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(Pair, full), __builtin_bit_cast(Pair, c[e])));
+            }
+            full = (full >> 16) > (full & 0xffffu) ? full >> 16 : full & 0xffffu;
+            full = WaveMax(odd == odd ? full : 0xffffu); // (more than any has)
+            const uint32_t upTo = WaveScan(sum);
+            uint32_t all = (uint32_t)__builtin_amdgcn_readlane((int)upTo, 63), begin = upTo - sum;
+            if constexpr (W > 1) {
+                each[2 * W + waveOfRow] = all;
+                across[kTopkWaves + wave] = full;
+                __syncthreads();
+                all = 0;
+#pragma unroll
+                for (int w = 0; w < W; ++w) {
+                    const uint32_t n = each[2 * W + w];
+                    begin += w < waveOfRow ? n : 0u;
+                    all += n;
+                }
+#pragma unroll
+                for (int w = 0; w < kTopkWaves; ++w)
+                    full = across[kTopkWaves + w] > full ? across[kTopkWaves + w] : full;
+                full = (uint32_t)__builtin_amdgcn_readfirstlane((int)full);
+            }
+            if (full == 0xffffu)
+                return kNothingDone;
+            begin += all << 16;
+#pragma unroll
+            for (int e = 0; e < E; ++e) {
+                const uint32_t n = c[e];
+                c[e] = begin;
+                begin += n;
+            }
+#pragma unroll
+            for (int j = 0; j < E / 4; ++j)
+                mine[chunk(j)] = make_uint4(c[4 * j], c[4 * j + 1], c[4 * j + 2], c[4 * j + 3]);
+        }
+        Meet();
+        // every key to the next place of its bucket.  (Equal scores in many columns: wave after wave, so that they are not in disorder)
+        const int turns = W > 1 && full > (uint32_t)kSurely ? W : 1;
+        for (int turn = 0; turn < turns; ++turn) {
+            if (turns == 1 || turn == waveOfRow) {
+#pragma unroll
+                for (int e = 0; e < E; ++e)
+                    at[e] = __hip_atomic_fetch_add(count + at[e], one[e], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+            }
+            if (turns > 1)
+                __syncthreads();
+        }
+        const uint32_t columnBits = (4095u - i0) << 8;
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+            at[e] = __builtin_amdgcn_ubfe(at[e], one[e] >> 12, 16);
+            k[e] = TopkKey(bits[e], columnBits - (uint32_t)(e * 64 << 8));
+        }
+        if (validCols != N) { // (what stands behind the columns goes behind the keys)
+#pragma unroll
+            for (int e = 0; e < E; ++e)
+                if (!isColumn(e)) {
+                    at[e] = i0 + 64u * (uint32_t)e;
+                    k[e] = 1.0;
+                }
+        }
+        Meet(); // (the counters are no longer needed)
+        uint64_t *const list = reinterpret_cast<uint64_t *>(mem);
+#pragma unroll
+        for (int e = 0; e < E; ++e)
+            list[Place(at[e])] = __builtin_bit_cast(uint64_t, k[e]);
+        Meet();
+#pragma unroll
+        for (int e = 0; e < E; ++e)
+            k[e] = __builtin_bit_cast(double, list[Place(q * E + (uint32_t)e)]);
+        Meet();
+        const int passes = full <= (uint32_t)kMost ? (int)(full + 1u) / 2 : 1;
+        for (int pass = 0;; ++pass) { // (two places for the edges in turn, and two others for the look)
+            double above, below;
+            if (full <= (uint32_t)kSurely) {
+                if (pass == passes)
+                    return kSorted;
+            } else {
+                Neighbours(above, below, waveOfRow, lane, list + (pass & 1) * 16 + 8);
+                bool sorted = k[E - 1] >= above;
+#pragma unroll
+                for (int e = 1; e < E; ++e)
+                    sorted = sorted & (k[e - 1] >= k[e]);
+                if (W > 1 ? Everyone(sorted, across + (2 + (pass & 1)) * kTopkWaves) : WholeWave(sorted))
+                    return kSorted;
+                if (pass == passes)
+                    return kLost;
+            }
+#pragma unroll
+            for (int e = 0; e < E; e += 2)
+                Exchange(k[e], k[e + 1]);
+            Neighbours(above, below, waveOfRow, lane, list + (pass & 1) * 16);
+#pragma unroll
+            for (int e = 1; e + 1 < E; e += 2)
+                Exchange(k[e], k[e + 1]);
+            k[E - 1] = Max(k[E - 1], above);
+            k[0] = Min(k[0], below);
+        }
+    }
+};
 template <int E, int W, bool LOW_DPP, Mode MODE>
-__global__ __launch_bounds__(kTopkThreads, MODE == kSelect && E == 16 ? 4 : 1) void TopkRows(float *outScore, uint32_t *outIndex, const float *src, const uint32_t *inIdx,
+__global__ __launch_bounds__(kTopkThreads, MODE == kSelect && E == 16 ? 4 : MODE == kWhole && E == 16 && W == 1 ? 4 : 1) void TopkRows(float *outScore, uint32_t *outIndex, const float *src, const uint32_t *inIdx,
                                                          int rows, int validCols, int ld, int topk, int keepBits, int through)
 {
     constexpr int N = 64 * E * W, kRows = kTopkWaves / W, kBits = RowSort<E, W, LOW_DPP>::kLaneBits;
     constexpr int kStaged = 64 * E + 4 * E; // words of a wave's results, one of padding behind every 16
     constexpr int kStages = E <= 8 ? 2 : 1;  // scores and columns side by side, or one after the other (LDS for four workgroups more)
     // exchanges, then results (or, between two sorts, the ranks of the columns); behind them the columns in the order of their indices
-    constexpr size_t kExchange = W > 1 ? (size_t)kTopkWaves * E * 64 * 8 : 0, kStage = (size_t)kTopkWaves * kStaged * 4 * kStages;
+    // buckets: per row of one wave a piece of its own, in which its results are staged as well
+    constexpr bool kCount = MODE == kWhole && kBuckets<E, W>;
+    constexpr size_t kOwn = kCount && W == 1 && N * 8 > kStaged * 4 * kStages ? N * 8 : kStaged * 4 * kStages;
+    constexpr size_t kExchange = W > 1 ? (size_t)kTopkWaves * E * 64 * 8 : 0, kStage = (size_t)kTopkWaves * kOwn;
     constexpr size_t kSelected = MODE == kSelect ? 384 + (size_t)kRows * 68 * kMostSelected * 8 : 0, kSort = kExchange > kStage ? kExchange : kStage;
     constexpr size_t kWork = kSort > kSelected ? kSort : kSelected;
     static_assert(kWork >= (size_t)N * 2, "the ranks fit");
-    __shared__ __attribute__((aligned(16))) char lds[kWork + (size_t)N * 2];
-    uint16_t *rankOf = reinterpret_cast<uint16_t *>(lds), *columnOf = reinterpret_cast<uint16_t *>(lds + kWork);
+    // (behind the first wave's results where its piece has room: 32 KiB a workgroup are five workgroups a compute unit)
+    constexpr size_t kColumns = kOwn >= kStaged * 4 * kStages + (size_t)N * 2 ? (size_t)kStaged * 4 * kStages : kWork;
+    __shared__ __attribute__((aligned(16))) char lds[kColumns < kWork ? kWork : kWork + (size_t)N * 2];
+    [[maybe_unused]] __shared__ uint32_t across[kTopkWaves * 6];
+    uint16_t *rankOf = reinterpret_cast<uint16_t *>(lds), *columnOf = reinterpret_cast<uint16_t *>(lds + kColumns);
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / 64), lane = tid % 64;
     const int waveOfRow = wave % W, row0 = (int)blockIdx.x * kRows, row = row0 + wave / W < rows ? row0 + wave / W : rows - 1;
     // this lane's first column; then every kStep-th.  Where a threshold selects, the waves of a row take blocks of 64 columns in turn, so that each
@@ -319,7 +619,7 @@ __global__ __launch_bounds__(kTopkThreads, MODE == kSelect && E == 16 ? 4 : 1) v
     // are the indices first, first + 1, ... or at least increasing with the column?  (then the column decides among equal
     // scores, as the index would; the same answer in every wave of the workgroup.)  Where a threshold selects, the four waves look at
     // a quarter each
-    constexpr bool kQuarters = MODE == kSelect && W < 4;
+    constexpr bool kQuarters = (MODE == kSelect || kCount) && W < 4;
     constexpr int kIds = kQuarters ? E * W / 4 : E;
     constexpr uint32_t kIdStep = kQuarters ? 64 : kStep;
     uint32_t ids[kIds];
@@ -338,8 +638,8 @@ __global__ __launch_bounds__(kTopkThreads, MODE == kSelect && E == 16 ? 4 : 1) v
         const uint32_t at = id0 + e * kIdStep < (uint32_t)validCols ? id0 + e * kIdStep : (uint32_t)validCols - 1u;
         wrong |= (ids[e] - first) ^ at;
     }
-    auto everyone = [&](bool v) { return W > 1 || kQuarters ? __syncthreads_and(v) != 0 : __builtin_amdgcn_ballot_w64(!v) == 0; };
-    const bool consecutive = everyone(wrong == 0 && first <= 0xffffffffu - (uint32_t)validCols);
+    auto everyone = [&](bool v, int vote) { return W > 1 || kQuarters ? Everyone(v, across + vote * kTopkWaves) : WholeWave(v); };
+    const bool consecutive = everyone(wrong == 0 && first <= 0xffffffffu - (uint32_t)validCols, 4);
     bool increasing = consecutive;
     if (__builtin_expect(!consecutive, 0)) {
         bool ok = true;
@@ -348,20 +648,20 @@ __global__ __launch_bounds__(kTopkThreads, MODE == kSelect && E == 16 ? 4 : 1) v
             if (i + 1 < validCols)
                 ok = ok && inIdx[i] < inIdx[i + 1];
         }
-        increasing = everyone(ok);
+        increasing = everyone(ok, 5);
     }
     RowSort<E, W, LOW_DPP> s;
     s.q = (uint32_t)waveOfRow * 64u + LaneRank((uint32_t)lane);
     s.xchg = reinterpret_cast<uint64_t *>(lds);
     // the ranks of a wave go in order through its piece of LDS, so that its stores cover consecutive addresses
-    uint32_t *staged = reinterpret_cast<uint32_t *>(lds) + wave * (kStaged * kStages), *stagedColumn = staged + (kStages - 1) * kStaged;
-    const int firstRank = waveOfRow * 64 * E, laneRank = (int)LaneRank((uint32_t)lane) * E, count = topk - firstRank;
+    uint32_t *staged = reinterpret_cast<uint32_t *>(lds + wave * kOwn), *stagedColumn = staged + (kStages - 1) * kStaged;
+    const int firstRank = waveOfRow * 64 * E, count = topk - firstRank;
     auto ordered = [] { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); __builtin_amdgcn_wave_barrier(); };
     // lane by lane consecutive words, all read before the first is stored; through: past the L2 (launch_topk)
     constexpr bool kThrough = MODE != kCut || N > 512; // (below, topk is 64 at most: 1000 x 300, top 30 5.2 us with the branch, 5.1 without)
     constexpr int kStored = MODE == kWhole ? E : E * W > 8 ? E * W / 8 : 1; // times 64: of a row that is not sorted whole, an eighth and less
     constexpr auto stored = std::integral_constant<int, kStored>();
-    auto store = [&](auto keys, uint32_t *to, int n, auto &&word) __attribute__((always_inline)) {
+    auto store = [&](auto keys, uint32_t *to, int n, int lane, auto &&word) __attribute__((always_inline)) {
         uint32_t w[decltype(keys)::value];
 #pragma unroll
         for (int e = 0; e < decltype(keys)::value; ++e)
@@ -554,11 +854,11 @@ __global__ __launch_bounds__(kTopkThreads, MODE == kSelect && E == 16 ? 4 : 1) v
                         at[i] = 4095u - ((low >> 8) & 0xfffu);
                     }
                     ordered();
-                    store(keys, toScore, topk, [&](int i) { return score[i + i / 16]; });
+                    store(keys, toScore, topk, lane, [&](int i) { return score[i + i / 16]; });
                     if (consecutive)
-                        store(keys, toIndex, topk, [&](int i) { return first + at[i + i / 16]; });
+                        store(keys, toIndex, topk, lane, [&](int i) { return first + at[i + i / 16]; });
                     else
-                        store(keys, toIndex, topk, [&](int i) { return inIdx[i < topk ? at[i + i / 16] : 0u]; }); // (behind topk may stand a column that is none)
+                        store(keys, toIndex, topk, lane, [&](int i) { return inIdx[i < topk ? at[i + i / 16] : 0u]; }); // (behind topk may stand a column that is none)
                 };
                 if (total <= 64)
                     finish(std::integral_constant<int, 1>());
@@ -572,6 +872,60 @@ __global__ __launch_bounds__(kTopkThreads, MODE == kSelect && E == 16 ? 4 : 1) v
             }
             asm volatile("" : "+v"(i0)); // (nothing that depends on it is kept so far either)
             load(scores, bits);
+        }
+    }
+    // staging and stores of the sorted keys; rank: of the lane's first one
+    auto finish = [&](const double (&k)[E], int rank, int lane) __attribute__((always_inline)) {
+        if (W > 1)
+            __syncthreads(); // (the exchanges are over)
+        if (row0 + wave / W >= rows || count <= 0)
+            return;
+        uint32_t *toScore = reinterpret_cast<uint32_t *>(outScore) + (size_t)row * (size_t)topk + firstRank;
+        uint32_t *toIndex = outIndex + (size_t)row * (size_t)topk + firstRank;
+        uint32_t column[E];
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+            const uint32_t low = Low(k[e]), order = (High(k[e]) << 12) | (low >> 20);
+            column[e] = 4095u - ((low >> 8) & 0xfffu);
+            staged[rank + e + (rank + e) / 16] = (low & 1u) ? kSign : ScoreBits(order);
+            if (kStages == 2)
+                stagedColumn[rank + e + (rank + e) / 16] = column[e];
+        }
+        ordered();
+        store(stored, toScore, count, lane, [&](int i) { return staged[i + i / 16]; });
+        if (kStages == 1) {
+            ordered();
+#pragma unroll
+            for (int e = 0; e < E; ++e)
+                stagedColumn[rank + e + (rank + e) / 16] = column[e];
+            ordered();
+        }
+        if (__builtin_expect(!consecutive, 0)) { // (staged: the column, or its rank)
+#pragma unroll
+            for (int e = 0; e < kStored; ++e) {
+                const int i = e * 64 + lane;
+                if (i < count) {
+                    const uint32_t c = stagedColumn[i + i / 16];
+                    toIndex[i] = inIdx[increasing ? c : columnOf[c]];
+                }
+            }
+            return;
+        }
+        store(stored, toIndex, count, lane, [&](int i) { return first + stagedColumn[i + i / 16]; });
+    };
+    if constexpr (kCount) {
+        if (increasing) {
+            uint32_t column0 = i0;
+            int here = lane;
+            asm volatile("" : "+v"(column0), "+v"(here)); // (nothing of this is kept in registers for what comes behind)
+            BucketSort<E, W> b;
+            const Counted done = b.Sort(bits, column0, validCols, waveOfRow, here, reinterpret_cast<uint32_t *>(lds + (W == 1 ? wave * kOwn : (size_t)(wave / W) * N * 8)), across);
+            if (__builtin_expect(done == kSorted, 1)) {
+                finish(b.k, here * E, here);
+                return;
+            }
+            if (done == kLost)
+                load(scores, bits);
         }
     }
     const uint32_t columnBits = (4095u - i0) << 8;
@@ -604,11 +958,8 @@ __global__ __launch_bounds__(kTopkThreads, MODE == kSelect && E == 16 ? 4 : 1) v
     }
     s.form = 0;
 #pragma unroll
-    for (int e = 0; e < E; ++e) {
-        const bool negZero = bits[e] == kSign; // compares equal to +0: same key, remembered below the column bits
-        const uint32_t order = ScoreOrder(negZero ? 0u : bits[e]);
-        s.k[e] = Key(__builtin_amdgcn_alignbit(0x3ffu, order, 12), (order << 20) | (columnBits - (e * kStep << 8) + (negZero ? 1u : 0u)));
-    }
+    for (int e = 0; e < E; ++e)
+        s.k[e] = TopkKey(bits[e], columnBits - (e * kStep << 8));
     if (__builtin_expect(!increasing, 0)) {
         __syncthreads(); // the ranks are there
 #pragma unroll
@@ -623,43 +974,7 @@ __global__ __launch_bounds__(kTopkThreads, MODE == kSelect && E == 16 ? 4 : 1) v
                 s.k[e] = 1.0;
     }
     s.template Sort<MODE == kWhole ? kBits : kBits - kWholeBits - 1>(keepBits);
-
-    if (W > 1)
-        __syncthreads(); // (the exchanges are over)
-    if (row0 + wave / W >= rows || count <= 0)
-        return;
-    uint32_t *toScore = reinterpret_cast<uint32_t *>(outScore) + (size_t)row * (size_t)topk + firstRank;
-    uint32_t *toIndex = outIndex + (size_t)row * (size_t)topk + firstRank;
-    uint32_t column[E];
-#pragma unroll
-    for (int e = 0; e < E; ++e) {
-        const uint32_t low = Low(s.k[e]), order = (High(s.k[e]) << 12) | (low >> 20);
-        column[e] = 4095u - ((low >> 8) & 0xfffu);
-        staged[laneRank + e + (laneRank + e) / 16] = (low & 1u) ? kSign : ScoreBits(order);
-        if (kStages == 2)
-            stagedColumn[laneRank + e + (laneRank + e) / 16] = column[e];
-    }
-    ordered();
-    store(stored, toScore, count, [&](int i) { return staged[i + i / 16]; });
-    if (kStages == 1) {
-        ordered();
-#pragma unroll
-        for (int e = 0; e < E; ++e)
-            stagedColumn[laneRank + e + (laneRank + e) / 16] = column[e];
-        ordered();
-    }
-    if (__builtin_expect(!consecutive, 0)) { // (staged: the column, or its rank)
-#pragma unroll
-        for (int e = 0; e < kStored; ++e) {
-            const int i = e * 64 + lane;
-            if (i < count) {
-                const uint32_t c = stagedColumn[i + i / 16];
-                toIndex[i] = inIdx[increasing ? c : columnOf[c]];
-            }
-        }
-        return;
-    }
-    store(stored, toIndex, count, [&](int i) { return first + stagedColumn[i + i / 16]; });
+    finish(s.k, (int)LaneRank((uint32_t)lane) * E, lane);
 }
 
 template <int E, int W>

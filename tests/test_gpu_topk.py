@@ -261,3 +261,59 @@ def test_topk_threshold_and_the_columns(oracle, rows, cols, topks):
     idx = np.arange(cols, dtype=np.uint32)
     for k in topks:
         assert same(topk_gpu(src, idx, cols, k), oracle.topk_f32(src, idx, cols, k)), k
+
+
+@pytest.mark.parametrize("rows,cols", [(750, 512), (803, 257), (9, 1024), (12, 513), (900, 1024), (860, 700), (2563, 1024), (2565, 600), (5, 2048), (14, 1025), (1710, 2048), (1711, 1100),
+                                       (13, 4096), (14, 2049), (12, 3000)])
+def test_topk_by_buckets(rows, cols):
+    """Whole sorts (more than an eighth of the padded row) of every kind of row that buckets take, give up on at the look, after counting, or after a first exchange: even
+    scores; equal ones in numbers around the fullest bucket's limits (16, 32); ascending and descending; one far outlier; a cluster of distinct scores; infinities; NaNs of either
+    sign; zeros of either sign; ranges too small and too large to spread; a part of the columns at another level.  NaNs, which the
+    comparator leaves open, in the order of their bits as before."""
+    r = np.random.Generator(np.random.Philox(key=rows + cols))
+    src, c = r.standard_normal((rows, cols + 5)).astype(np.float32), np.arange(cols + 5, dtype=np.float32)
+    kinds = 12 if rows < 100 else 18
+    for kind in range(kinds):
+        row = src[kind::kinds]
+        if kind == 1:
+            row[:] = r.integers(0, max(1, cols // 16), row.shape)
+        elif kind == 2:
+            row[:] = r.integers(0, max(1, cols // 40), row.shape)
+        elif kind == 3:
+            row[:] = c
+        elif kind == 4:
+            row[:] = np.where(c == cols // 3, np.float32(1e6), row)
+        elif kind == 5:
+            row[:, cols // 2:cols // 2 + 40] = 0.25 + row[:, cols // 2:cols // 2 + 40] * np.float32(1e-5)
+        elif kind == 6:
+            row[:] = np.where(c == cols - 1, np.float32(np.inf), np.where(c == 7, np.float32(-np.inf), row))
+        elif kind == 7:
+            row[:] = np.where(c == cols - 2, np.uint32(0xffc00001).view(np.float32), np.where(c == 70, np.float32(np.nan), row))
+        elif kind == 8:
+            row[:] = np.where(row < 0.0, np.float32(-0.0), np.where(row < 0.3, np.float32(0.0), row))
+        elif kind == 9:
+            row[:] *= np.float32(1e-33)
+        elif kind == 10:
+            row[:] *= np.float32(3e37)
+        elif kind == 11:
+            row[:] = np.where(c >= cols * 3 // 4, row + 100, row)
+        elif kind == 12:
+            row[:] = -c
+        elif kind == 13:
+            row[:] = np.exp(row * 4)
+        elif kind == 14:
+            row[:] = np.where(c >= cols // 2, -np.inf, row)
+        elif kind == 15:
+            row[:] = np.where(r.random(row.shape) < 0.98, np.float32(1.5), row)
+        elif kind == 16:
+            row[:] = np.float32(-2.0)
+        elif kind == 17:
+            row[:] = np.round(row * 64) / 64
+    idx = np.arange(cols, dtype=np.uint32)
+    eighth = (1 << (cols - 1).bit_length()) // 8
+    bits = src[:, :cols].view(np.uint32)
+    plain = np.where(bits == 0x80000000, np.uint32(0), bits)
+    order = np.where(plain >> 31, ~plain, plain | np.uint32(0x80000000))
+    for ids, k in ((idx, cols), (idx, max(321, eighth + 1) if cols > 321 else cols), (idx * np.uint32(3) + np.uint32(5), cols - 1), (np.uint32(0xFFFFFFFF) - idx, cols)):
+        at = np.lexsort((np.broadcast_to(ids, order.shape), ~order))[:, :k]
+        assert same(topk_gpu(src, ids, cols, k), (np.take_along_axis(src, at, 1), ids[at])), (k, ids[:2])
