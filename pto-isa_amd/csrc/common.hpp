@@ -61,8 +61,8 @@ inline int allow_lds(K kernel, int bytes)
 // defined in pto_gemm_w4.hip: tiles on four wavefronts, K-steps of 64; shape 0 .. 2 = 256 rows x 256 / 192 / 128 columns,
 // 3 .. 5 = 192 rows x the same widths.  PTO_ERR_UNSUPPORTED unless m and n hold a tile, n % 4 == 0 and k % 128 == 0
 int gemm_f16f32_w4(hipStream_t st, float *c, const _Float16 *a, const _Float16 *b, int m, int n, int k, int shape);
-// defined in pto_gemm_ks.hip: tiles on eight wavefronts with k split over two groups of them; shape 0 .. 8 = 32 x 64, 64 x 64,
-// 64 x 96, 128 x 64, 128 x 96, 128 x 128, 192 x 128, 256 x 128, 192 x 192.  PTO_ERR_UNSUPPORTED unless n % 4 == 0 and k % 32 == 0
+// defined in pto_gemm_ks.hip: tiles on eight wavefronts with k split over two groups of them; shape 0 .. 9 = 32 x 64, 64 x 64,
+// 64 x 96, 128 x 64, 128 x 96, 128 x 128, 192 x 128, 256 x 128, 192 x 192, 32 x 32.  PTO_ERR_UNSUPPORTED unless n % 4 == 0 and k % 32 == 0
 int gemm_f16f32_ks(hipStream_t st, float *c, const _Float16 *a, const _Float16 *b, int m, int n, int k, int shape);
 // defined in pto_gemm_mxw4.hip (MXFP8 / MXFP4 on the four-wave engine: 256 x 192 or 256 x 128 tiles);
 // PTO_ERR_UNSUPPORTED unless m >= 256, n >= 128, n % 4 == 0, k % 512 == 0 (fp4, format 4: k % 1024 == 0)

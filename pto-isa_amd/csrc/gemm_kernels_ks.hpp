@@ -11,9 +11,11 @@
 // What bounds a step: the copies.  A compute unit takes in 53 bytes per clock of L2-resident lines (measured with all of
 // them loading), so the (BM + BN) 128 bytes of a 128 x 128 step are 620 clocks against 512 of its MFMAs; with one part
 // taken out a step of 0.46 us (1024 x 3072 x 8192) runs 0.43 without the fragment reads, 0.36 with copies alone and 0.33
-// with MFMAs alone.  The place of the copies in the step, raised wave priority and deeper rings changed nothing (1 %).
+// with MFMAs alone.  The place of the copies in the step, raised wave priority and deeper rings changed nothing (1 %; a 32 x 64 step, 12 KiB in
+// 0.13 us: rings of 6 to 13 stages 0 to 20 % slower, two steps from one barrier to the next 0 to 10 %).  So where units are idle the tile gets
+// smaller: 32 x 32, 0.09 us a step, on twice as many of them (512^3 3.78 -> 3.33 us, 256 x 256 x 6144 15.8 -> 11.5; four stages 14.8, five 12.0, eight 11.5).
 // (1000 x 3000 x 2048 on 128 x 96 tiles runs 0.4 us a step: 28 KiB of copies, from beyond the L2.)
-// Small tiles lose there what they win in compute units at work: 512^3 8.96 -> 3.9 us, 1000 x 3000 x 2048 21.1 -> 18.0,
+// Small tiles lose there what they win in compute units at work: 512^3 8.96 -> 3.3 us, 1000 x 3000 x 2048 21.1 -> 18.0,
 // 128 x 4096 x 4096 68 -> 12.  C past the L2 where that pays (store_through): 1000 x 3072 x 2048 18.5 -> 17.0.
 //
 // Rows past m and columns past n repeat the last one on the way in (their memory may not exist) and are not stored.
@@ -69,7 +71,7 @@ __global__ __launch_bounds__(512, MIN_WAVES) AICORE void GemmF16F32Ks(float *out
     constexpr int MB = BM / 32, NB = BN / 32;                  // 16 x 16 blocks of a wave
     constexpr int kInst = (BM + BN) / 8, kCopies = (kInst + 7) / 8; // copy instructions of 8 rows a step; per wave
     constexpr uint32_t kStage = (BM + BN) * 128, kRing = S * kStage;
-    static_assert(BM % 32 == 0 && BN % 32 == 0 && S >= 3 && (MB * NB) % 2 == 0, "tile shape");
+    static_assert(BM % 32 == 0 && BN % 32 == 0 && S >= 3 && ((MB * NB) % 2 == 0 || MB * NB == 1), "tile shape");
 
     int tm, tn;
     TileOfBlock<GROUP_M>((int)blockIdx.x, (m + BM - 1) / BM, (n + BN - 1) / BN, tm, tn);
@@ -173,7 +175,7 @@ __global__ __launch_bounds__(512, MIN_WAVES) AICORE void GemmF16F32Ks(float *out
     if (it < steps)
         step(std::integral_constant<int, 0>(), std::false_type(), it);
 
-    // Partial sums: each group keeps half of its wave's blocks, gives the other half to its partner (same rows and
+    // Partial sums: each group keeps half of its wave's blocks (of one block the second group keeps it), gives the other half to its partner (same rows and
     // columns, other k) and stores the sums of the half it keeps.
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); // the copies past the end
     __builtin_amdgcn_s_barrier();

@@ -50,7 +50,7 @@ namespace {
 // shape on average (21 % at worst) and 12 of the 2293 are over 2 % slower than with four-wave tiles (k a multiple of 128)
 // or blocks alone, the worst 7.6 % (with a fit to 330 problems that counted every one alike: 24 of 1893, and 12.4 %).  What the figures say: a
 // small tile's step is cheap and moves more bytes per flop (64 x 64: 0.2 us a step, 128 x 128: 0.45, the four-wave 256 x 192:
-// 1.1), so it wins while it puts more compute units to work -- 512^3 8.9 us on twelve 192 x 128 tiles, 4.0 on 32 x 64 ones;
+// 1.1), so it wins while it puts more compute units to work -- 512^3 8.9 us on twelve 192 x 128 tiles, 3.8 on 32 x 64 ones, 3.3 on 32 x 32;
 // 1024^3 13.7 and 6.8; 128 x 4096 x 4096 68 and 12; 768 x 768 x 6144 48 and 20 -- and the tiles of 192 and 256 rows win from
 // about one whole round of them on (2048^3 22.7 against 21.0 on 128 x 128, 4096^3 104 against 137 on 192 x 128).
 struct TileShape {
@@ -62,6 +62,9 @@ constexpr TileShape kShapes[] = {
     {TileShape::kW4, 0, 256, 256, 9.263, 7.420, 0.770, 1.429, 0.085, 0.610}, {TileShape::kW4, 1, 256, 192, 8.193, 6.015, 0.543, 1.115, 0.070, 0.533},
     {TileShape::kW4, 2, 256, 128, 6.567, 3.898, 0.379, 0.817, 0.083, 0.373}, {TileShape::kW4, 3, 192, 256, 7.814, 4.941, 0.581, 1.150, 0.084, 0.490},
     {TileShape::kW4, 4, 192, 192, 7.134, 4.643, 0.393, 0.916, 0.072, 0.451}, {TileShape::kW4, 5, 192, 128, 4.741, 1.197, 0.337, 0.658, 0.159, 0.242},
+    // 32 x 32, fitted to 400 problems of up to 900 such tiles: it is the shortest where they are one round, and by 8 to 29 % (512^3 3.78 -> 3.33 us, 512 x 512 x 2048
+    // 7.4 -> 6.0, 256 x 256 x 6144 15.8 -> 11.5, 300 x 700 x 1024 4.70 -> 4.14), and never where they are two (640 x 512 x 1024 4.8 / 5.4)
+    {TileShape::kKs, 9, 32, 32, 2.487, 0.411, 0.091, 0.076, 0.159, 0.017},
     {TileShape::kKs, 0, 32, 64, 2.670, 0.853, 0.135, 0.136, 0.178, 0.026},   {TileShape::kKs, 1, 64, 64, 2.822, 0.902, 0.152, 0.165, 0.175, 0.044},
     {TileShape::kKs, 2, 64, 96, 3.214, 0.965, 0.207, 0.240, 0.183, 0.052},   {TileShape::kKs, 3, 128, 64, 3.221, 0.868, 0.249, 0.258, 0.180, 0.080},
     {TileShape::kKs, 4, 128, 96, 4.595, 2.050, 0.258, 0.411, 0.162, 0.127},  {TileShape::kKs, 5, 128, 128, 5.026, 2.036, 0.293, 0.488, 0.140, 0.156},

@@ -17,6 +17,7 @@ int gemm_f16f32_ks(hipStream_t st, float *c, const _Float16 *a, const _Float16 *
     case 6: return launch_gemm_ks<192, 128, 4, 2>(st, c, a, b, m, n, k);
     case 7: return launch_gemm_ks<256, 128, 3, 2>(st, c, a, b, m, n, k);
     case 8: return launch_gemm_ks<192, 192, 3, 2>(st, c, a, b, m, n, k);
+    case 9: return launch_gemm_ks<32, 32, 6, 4>(st, c, a, b, m, n, k);
     default: return PTO_ERR_UNSUPPORTED;
     }
 }
@@ -26,7 +27,7 @@ int gemm_f16f32_ks(hipStream_t st, float *c, const _Float16 *a, const _Float16 *
 // tile shape by number, as above
 extern "C" int pto_gemm_f16f32_ks_variant(void *stream, float *c, const uint16_t *a, const uint16_t *b, int m, int n, int k, int variant)
 {
-    if (!c || !a || !b || m <= 0 || n <= 0 || k <= 0 || variant < 0 || variant > 8)
+    if (!c || !a || !b || m <= 0 || n <= 0 || k <= 0 || variant < 0 || variant > 9)
         return PTO_ERR_BAD_ARG;
     return pto_amd::gemm_f16f32_ks(static_cast<hipStream_t>(stream), c, reinterpret_cast<const _Float16 *>(a),
                                    reinterpret_cast<const _Float16 *>(b), m, n, k, variant);

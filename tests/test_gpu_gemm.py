@@ -254,3 +254,16 @@ def test_gemm_half_pieces_and_k(m, n, k):
     c = torch.full((m * n + 64,), 7.0, device="cuda:0")
     capi.check(lib.pto_gemm_f16f32(torch.cuda.current_stream().cuda_stream, c.data_ptr(), a.data_ptr(), b.data_ptr(), m, n, k), "pto_gemm_f16f32")
     assert torch.equal(c[:m * n].view(m, n), a.float() @ b.float().t()) and (c[m * n:] == 7.0).all()
+
+
+def test_gemm_32x32_tiles_exact():
+    """The tile of one block a wave, as the other shapes are tested; then the entry point on both sides of a whole round of such tiles, k of one step and of more and
+    fewer than the ring has stages."""
+    test_gemm_k_split_tile_shapes_exact(9, 32, 32)
+    lib = capi.load()
+    for m, n, k in ((512, 512, 128), (513, 512, 128), (512, 516, 256), (192, 128, 384), (250, 260, 512), (192, 1364, 640), (128, 256, 32), (128, 2048, 96)):
+        g = torch.Generator(device="cuda:0").manual_seed(m + n + k)
+        a, b = (torch.randint(-4, 5, (r, k), generator=g, device="cuda:0").half() for r in (m, n))
+        c = torch.full((m * n + 64,), 7.0, device="cuda:0")
+        capi.check(lib.pto_gemm_f16f32(torch.cuda.current_stream().cuda_stream, c.data_ptr(), a.data_ptr(), b.data_ptr(), m, n, k), "pto_gemm_f16f32")
+        assert torch.equal(c[:m * n].view(m, n), a.float() @ b.float().t()) and (c[m * n:] == 7.0).all(), (m, n, k)
