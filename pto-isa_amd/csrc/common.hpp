@@ -64,10 +64,13 @@ int gemm_f16f32_w4(hipStream_t st, float *c, const _Float16 *a, const _Float16 *
 // defined in pto_gemm_ks.hip: tiles on eight wavefronts with k split over two groups of them; shape 0 .. 9 = 32 x 64, 64 x 64,
 // 64 x 96, 128 x 64, 128 x 96, 128 x 128, 192 x 128, 256 x 128, 192 x 192, 32 x 32.  PTO_ERR_UNSUPPORTED unless n % 4 == 0 and k % 32 == 0
 int gemm_f16f32_ks(hipStream_t st, float *c, const _Float16 *a, const _Float16 *b, int m, int n, int k, int shape);
-// defined in pto_gemm_mxw4.hip (MXFP8 / MXFP4 on the four-wave engine: 256 x 192 or 256 x 128 tiles);
-// PTO_ERR_UNSUPPORTED unless m >= 256, n >= 128, n % 4 == 0, k % 512 == 0 (fp4, format 4: k % 1024 == 0)
+// defined in pto_gemm_mxw4.hip (MXFP8 / MXFP4 on the four-wave engine: 256 x 256, 256 x 192 or 256 x 128 tiles);
+// PTO_ERR_UNSUPPORTED unless m >= 256, n >= width, n % 4 == 0, k % 512 == 0 (fp4, format 4: k % 1024 == 0)
 int gemm_mx_w4(hipStream_t st, void *c, const uint8_t *a, const uint8_t *b, const uint8_t *sa, const uint8_t *sb, int m, int n, int k,
                   int format, int c_fp32, int width);
+// defined in pto_gemm_mxw4_256.hip: width 256 of the above
+int gemm_mx_w4_256(hipStream_t st, void *c, const uint8_t *a, const uint8_t *b, const uint8_t *sa, const uint8_t *sb, int m, int n, int k,
+                   int format, int c_fp32);
 // defined in pto_gemm_mxks.hip (MXFP8 / MXFP4 tiles on eight wavefronts with k split over two groups of them); shape 0 .. 5 =
 // 64 x 64, 64 x 128, 128 x 64, 128 x 128, 128 x 192, 192 x 128.  PTO_ERR_UNSUPPORTED unless n % 4 == 0 and k % 512 == 0
 int gemm_mx_ks(hipStream_t st, void *c, const uint8_t *a, const uint8_t *b, const uint8_t *sa, const uint8_t *sb, int m, int n, int k,

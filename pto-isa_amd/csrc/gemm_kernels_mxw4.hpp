@@ -1,4 +1,4 @@
-// MXFP8 GEMM tile of 256 x BN (BN = 192 or 128) on four wavefronts: the four-wave fp16 kernel of gemm_kernels_w4.hpp with
+// MXFP8 GEMM tile of 256 x BN (BN = 256, 192 or 128) on four wavefronts: the four-wave fp16 kernel of gemm_kernels_w4.hpp with
 // 8-bit operands.  A K-step is the same 128 bytes per operand row (128 k instead of 64), so copies, LDS images and fragment
 // reads are byte for byte those of the fp16 kernel; what differs:
 //   * one v_mfma_scale_f32_16x16x128_f8f6f4 (8 passes) per 16 x 16 block and step instead of two v_mfma_f32_16x16x32_f16
@@ -15,6 +15,11 @@
 //   * four B stages (96 + 64 KiB = the whole LDS at BN = 192), which makes the step's second barrier unnecessary: a
 //     stage is overwritten two steps after its last read, with the barrier of the step in between.
 // Steps come in groups of four (B stage, A slot and scale byte repeat): k % 512 == 0.
+// BN = 256: all 256 accumulation registers, a sixth fewer copies and a seventh fewer fragment reads per MFMA than at 192.  Three B stages fit, so a step has a
+// second barrier again, ahead of its first copy of B, and as three stages and eight (sixteen) steps of a scale period do not go together, they take
+// turns at run time.  Two sets of scale registers do not fit: rows are loaded over their own first three quarters when the last one has been moved
+// aside, and spread in place.  What the time goes into (2040 x 8100 x 8192 fp4 on 256 x 128 tiles, 72.8 us; one part taken out): copies 8.8, reads of B 5.3 and of
+// A 3.0, scales 3.9; with none of them 53.3, the MFMAs at the clock they hold.  With 256 x 256 tiles 66.0; fp8 121 -> 104.
 // MXFP4 (format 4, two e2m1 per byte): a K-step of 128 bytes is 256 k = two MFMAs (4 passes each, 16-byte operands: lane group
 // g holds bytes 16 g .. + 15 of the MFMA's 64) and eight scale blocks per row, so a scale register lasts two steps (the MFMA of
 // step j % 2 and half kk selects byte 2 (j % 2) + kk), the 64 scale bytes of a row eight steps, and two block rows / columns
@@ -159,7 +164,8 @@ AICORE inline __attribute__((always_inline)) void MxW4TileCompute(__gm__ const u
                                                                   __gm__ const uint8_t *scale0, __gm__ const uint8_t *scale1, int k,
                                                                   int row0, int col0)
 {
-    constexpr int NMB = 4, NNB = BN / 16, NBUF = 4, BSTAGES = 4, NA = 8, NCB = BN / 32, NCOPY = NA + NCB;
+    constexpr bool WIDE = BN == 256;
+    constexpr int NMB = 4, NNB = BN / 16, NBUF = 4, BSTAGES = WIDE ? 3 : 4, NA = 8, NCB = BN / 32, NCOPY = NA + NCB;
     using S = MxW4Sched<NNB, NCOPY>;
     constexpr bool FP4 = FMT_A == 4;
     static_assert((FMT_A == 4) == (FMT_B == 4), "fp4 with fp4");
@@ -219,6 +225,9 @@ AICORE inline __attribute__((always_inline)) void MxW4TileCompute(__gm__ const u
         return MxW4Load16(i < NMB ? saWave : sbPanel, voff);
     };
 
+    // WIDE: three B stages take turns at run time: of step it, of it + 1 and of the copies for it + 2
+    uint32_t bNow[2] = {bAddr[0][0], bAddr[1][0]}, bThen[2] = {bAddr[0][1], bAddr[1][1]};
+    uint32_t stageNow = 0, stageThen = kBBytes, stageCopy = 2 * kBBytes;
     uint32_t voffA[2], voffB;
     auto setLds = [&](uint32_t waveBase, auto immTag) __attribute__((always_inline)) {
         asm volatile("s_add_u32 m0, %0, %1" ::"s"(waveBase), "n"(decltype(immTag)::value) : "memory", "scc");
@@ -230,15 +239,22 @@ AICORE inline __attribute__((always_inline)) void MxW4TileCompute(__gm__ const u
         f16x8 h[2];
     };
     Pair aF[2][NMB], bF[NBUF];
-    uint32_t sc[kScales][4], scNext[kScales][4] = {}; // scales of the current kSuperSteps steps and of the next, a register per quarter
-    u32x4 raw[kScaleLoads];
+    // scales of the current kSuperSteps steps and of the next, a register per quarter.  WIDE: one set.  In the last quarter, which then stands apart
+    // (scLast), the rows' new ones are loaded over the others
+    uint32_t sc[kScales][4], scNext[WIDE ? 1 : kScales][4] = {};
+    u32x4 raw[kScaleLoads], rows[WIDE ? kScales : 1];
+    uint32_t scLast[WIDE ? kScales : 1];
+    constexpr int kLastQuarter = 3 * kGroupSteps;
     auto readA = [&](auto setTag, auto qTag) __attribute__((always_inline)) {
         constexpr int set = decltype(setTag)::value, q = decltype(qTag)::value, mb = q / 2, kk = q % 2;
         aF[set][mb].h[kk] = W4LdsRead16<mb * 2048>(aAddr[kk][set]);
     };
     auto readB = [&](auto stageTag, auto nbTag, auto kkTag) __attribute__((always_inline)) {
         constexpr int stage = decltype(stageTag)::value, nb = decltype(nbTag)::value, kk = decltype(kkTag)::value;
-        bF[nb % NBUF].h[kk] = W4LdsRead16<nb * 2048>(bAddr[kk][stage]);
+        if constexpr (WIDE)
+            bF[nb % NBUF].h[kk] = W4LdsRead16<nb * 2048>(stage == 0 ? bNow[kk] : bThen[kk]);
+        else
+            bF[nb % NBUF].h[kk] = W4LdsRead16<nb * 2048>(bAddr[kk][stage]);
     };
     auto operand = [](const Pair &p) {
         const u32x4 lo = __builtin_bit_cast(u32x4, p.h[0]), hi = __builtin_bit_cast(u32x4, p.h[1]);
@@ -272,7 +288,12 @@ AICORE inline __attribute__((always_inline)) void MxW4TileCompute(__gm__ const u
     W4For<0, kScales>([&](auto iTag) __attribute__((always_inline)) {
         constexpr int i = decltype(iTag)::value;
         MxW4Pin(first[i]); // (older than the copies waited for above)
-        MxW4ScaleSpread(first[i], sc[i]);
+        if constexpr (WIDE) {
+            rows[i] = first[i];
+            W4For<0, 4>([&](auto partTag) __attribute__((always_inline)) { MxW4ScaleSpreadPart<decltype(partTag)::value>(rows[i]); });
+        } else {
+            MxW4ScaleSpread(first[i], sc[i]);
+        }
     });
     __builtin_amdgcn_sched_barrier(0);
     W4For<0, NA>([&](auto qTag) __attribute__((always_inline)) { readA(integral_constant<int, 0>(), qTag); });
@@ -286,9 +307,10 @@ AICORE inline __attribute__((always_inline)) void MxW4TileCompute(__gm__ const u
     // those of B to the stage of step it - 2; scale rows kScaleLoads t .. of the next period are loaded at the start of the step
     // and spread over the lane groups behind its barrier.
     auto step = [&](auto tTag, int it, int super) __attribute__((always_inline)) {
-        constexpr int t = decltype(tTag)::value, j = t % 4, s = j, par = j % 2, sNext = (j + 1) % BSTAGES, sCopy = (j + 2) % BSTAGES;
+        constexpr int t = decltype(tTag)::value, j = t % 4, par = j % 2;
+        constexpr int s = WIDE ? 0 : j, sNext = WIDE ? 1 : (j + 1) % BSTAGES, sCopy = (j + 2) % BSTAGES;
         constexpr int quarter = t / kGroupSteps, jj = t % kGroupSteps, left = kScales - kScaleLoads * t;
-        constexpr int nLoads = left < 0 ? 0 : (left < kScaleLoads ? left : kScaleLoads);
+        constexpr int nLoads = WIDE ? 0 : left < 0 ? 0 : (left < kScaleLoads ? left : kScaleLoads);
         const uint32_t kOff = (uint32_t)clampStep(it + 2) * kStepBytes;
         const int nextSuper = super + 1 < supers ? super + 1 : supers - 1;
         W4For<0, S::kSlots>([&](auto idxTag) __attribute__((always_inline)) {
@@ -304,8 +326,31 @@ AICORE inline __attribute__((always_inline)) void MxW4TileCompute(__gm__ const u
                 voffA[1] = aCopyOff[1] + kOff;
                 voffB = bCopyOff + kOff;
             }
+            if constexpr (WIDE) {
+                // the last quarter's scales out of the way; the next rows loaded, a slot each; their parts from kSpread slots on, a slot each
+                constexpr int since = (t - kLastQuarter) * S::kSlots + idx;
+                if constexpr (t == kLastQuarter - 1 && idx < kScales)
+                    asm volatile("v_mov_b32 %0, %1" : "=v"(scLast[idx]) : "v"(rows[idx][3]));
+                if constexpr (since >= 0 && since < kScales)
+                    rows[since] = scaleLoad(integral_constant<int, since>(), nextSuper);
+                constexpr int kSpread = 2 * S::kSlots - 4 * kScales;
+                static_assert(kSpread >= kScales, "all loaded before the first is spread");
+                if constexpr (since == kSpread) // (the copies issued since the last of the loads may be under way)
+                    hw::wait_vm<S::copiesBefore(kSpread) - S::copiesBefore(kScales)>();
+                if constexpr (since >= kSpread && since < kSpread + 4 * kScales) {
+                    constexpr int row = (since - kSpread) / 4, part = (since - kSpread) % 4;
+                    if constexpr (part == 0)
+                        MxW4Pin(rows[row]);
+                    MxW4ScaleSpreadPart<part>(rows[row]);
+                }
+                if constexpr (idx == S::copySlot(NA) - 2) { // every wave has read all of the step before, whose B stage the copies go to
+                    __builtin_amdgcn_s_barrier();
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
             if constexpr (idx == S::kBarrier) {
                 // this wave's copies of the step before have landed (and this step's scale rows, which are older than its copies)
+                // (WIDE: the scale rows of a step, some of them behind its first copies, are older than its last ones as well)
                 hw::wait_vm<S::copiesBefore(S::kBarrier)>();
                 __builtin_amdgcn_s_barrier();
                 __builtin_amdgcn_sched_barrier(0);
@@ -331,7 +376,7 @@ AICORE inline __attribute__((always_inline)) void MxW4TileCompute(__gm__ const u
             }
             if constexpr (S::aReadAt(idx) >= 0) {
                 if constexpr (S::aReadAt(idx) == 0) // this wave's A copies of the step before have landed
-                    hw::wait_vm<NCB + nLoads + S::copiesBefore(idx)>();
+                    hw::wait_vm<NCB + nLoads + S::copiesBefore(idx) + (WIDE && t == kLastQuarter ? idx + 1 : 0)>();
                 readA(integral_constant<int, par ^ 1>(), integral_constant<int, S::aReadAt(idx)>());
             }
             if constexpr (S::copyAt(idx) >= 0) {
@@ -345,6 +390,8 @@ AICORE inline __attribute__((always_inline)) void MxW4TileCompute(__gm__ const u
                 constexpr int c = S::copyAt(idx + 1);
                 if constexpr (c < NA)
                     setLds(aLdsWave, integral_constant<int, par * kASlot + c * 1024>());
+                else if constexpr (WIDE)
+                    setLds(bLdsWave + stageCopy, integral_constant<int, (c - NA) * 4096>());
                 else
                     setLds(bLdsWave, integral_constant<int, sCopy * kBBytes + (c - NA) * 4096>());
             }
@@ -352,17 +399,38 @@ AICORE inline __attribute__((always_inline)) void MxW4TileCompute(__gm__ const u
                 constexpr int lo = 4 * (nb - PD) + 1;
                 asm volatile("s_waitcnt lgkmcnt(%0)" ::"n"(2 * (PD - 1) + 1 + (lo > 0 ? S::aReadsIn(lo, idx) : 0)) : "memory");
             }
+            auto scaleOf = [&](auto rowTag) __attribute__((always_inline)) {
+                constexpr int row = decltype(rowTag)::value;
+                if constexpr (!WIDE)
+                    return sc[row][quarter];
+                else if constexpr (quarter == 3)
+                    return scLast[row];
+                else
+                    return (uint32_t)rows[row][quarter];
+            };
             if constexpr (FP4) {
+                // (the second half right behind the first: with the halves of two blocks in turn 2 % slower)
                 MxW4MfmaFp4<mb * NNB + nb, 2 * jj>(__builtin_bit_cast(u32x4, bF[nb % NBUF].h[0]), __builtin_bit_cast(u32x4, aF[par][mb].h[0]),
-                                                   sc[NMB + nb][quarter], sc[mb][quarter]);
-                MxW4MfmaFp4<mb * NNB + nb, 2 * jj + 1>(__builtin_bit_cast(u32x4, bF[nb % NBUF].h[1]),
-                                                       __builtin_bit_cast(u32x4, aF[par][mb].h[1]), sc[NMB + nb][quarter], sc[mb][quarter]);
+                                                   scaleOf(integral_constant<int, NMB + nb>()), scaleOf(integral_constant<int, mb>()));
+                MxW4MfmaFp4<mb * NNB + nb, 2 * jj + 1>(__builtin_bit_cast(u32x4, bF[nb % NBUF].h[1]), __builtin_bit_cast(u32x4, aF[par][mb].h[1]),
+                                                       scaleOf(integral_constant<int, NMB + nb>()), scaleOf(integral_constant<int, mb>()));
             } else {
-                MxW4Mfma<mb * NNB + nb, jj, FMT_B, FMT_A>(operand(bF[nb % NBUF]), operand(aF[par][mb]), sc[NMB + nb][quarter],
-                                                          sc[mb][quarter]);
+                MxW4Mfma<mb * NNB + nb, jj, FMT_B, FMT_A>(operand(bF[nb % NBUF]), operand(aF[par][mb]), scaleOf(integral_constant<int, NMB + nb>()),
+                                                          scaleOf(integral_constant<int, mb>()));
             }
             __builtin_amdgcn_sched_barrier(0);
         });
+        if constexpr (WIDE) {
+            const uint32_t done = stageNow;
+            stageNow = stageThen;
+            stageThen = stageCopy;
+            stageCopy = done;
+#pragma unroll
+            for (int kk = 0; kk < 2; ++kk) {
+                bNow[kk] = bThen[kk];
+                bThen[kk] = bAddr[kk][0] + stageThen;
+            }
+        }
     };
     for (int super = 0; super < supers; ++super) {
         const int it0 = super * kSuperSteps;
@@ -375,11 +443,13 @@ AICORE inline __attribute__((always_inline)) void MxW4TileCompute(__gm__ const u
                 step(integral_constant<int, 4 * q + 3>(), it0 + 4 * q + 3, super);
             }
         });
+        if constexpr (!WIDE) {
 #pragma unroll
-        for (int i = 0; i < kScales; ++i)
+            for (int i = 0; i < kScales; ++i)
 #pragma unroll
-            for (int u = 0; u < 4; ++u)
-                sc[i][u] = scNext[i][u];
+                for (int u = 0; u < 4; ++u)
+                    sc[i][u] = scNext[i][u];
+        }
     }
     hw::wait_vm0(); // the copies issued past the end of K
     // the last MFMAs have written their accumulators
@@ -444,7 +514,7 @@ int launch_gemm_mxw4(hipStream_t st, void *c, const uint8_t *a, const uint8_t *b
     // (n % 4: four consecutive elements of a row are inside or outside together)
     if (m < 256 || n < BN || n % 4 || k % (FMT_A == 4 ? 1024 : 512) || k <= 0)
         return PTO_ERR_UNSUPPORTED;
-    constexpr int lds = 4 * 128 * BN + 4 * 2 * 64 * 128; // four B stages + two A slots per wave
+    constexpr int lds = (BN == 256 ? 3 : 4) * 128 * BN + 4 * 2 * 64 * 128; // four (three) B stages + two A slots per wave
     auto kernel = GemmMxW4<FMT_A, FMT_B, OutT, BN, 4>;
     static const int attr = pto_amd::allow_lds(kernel, lds);
     if (attr != PTO_OK)

@@ -347,7 +347,7 @@ int gemm_mx_dispatch(hipStream_t st, void *c, const uint8_t *a, const uint8_t *b
 } // namespace
 
 namespace {
-// Three kernels: 256 x 256 tiles on eight wavefronts (this file; quarter tiles in a last partial round), 256 x 192 and 256 x 128
+// Three kernels: 256 x 256 tiles on eight wavefronts (this file; quarter tiles in a last partial round), 256 x 256, 256 x 192 and 256 x 128
 // tiles on four (pto_gemm_mxw4.hip), and tiles of 64 .. 192 rows with k split over two groups of wavefronts
 // (pto_gemm_mxks.hip).  What a problem takes with one tile shape, in microseconds, launch included: tiles are dealt to the
 // compute units, `more` rounds beyond the first, `share` of the units busy in the last one, steps of 128 bytes,
@@ -355,19 +355,24 @@ namespace {
 // the 256 x 256 tiles take `ragged` longer a step and round where m or n is no multiple of 256 (the last tiles are moved back).
 // Least-squares fits to 1520 problems (256 x 256 x 512 .. 6144^3 ragged, .. 16384 x 8192 x 8192 in whole tiles, both results,
 // three operand sets in turn) in which those near a shape's best use count most (root mean square of the relative error there
-// 2 .. 5 %).  The k-split shapes are taken 2 %, the 256 x 256 tiles 3 % dearer than fitted (against moves on the noise of the
+// 2 .. 5 %).  The k-split shapes are taken 2 %, the 256 x 256 tiles of either kind 3 % dearer than fitted (against moves on the noise of the
 // fit); so chosen, a problem is 0.4 % (fp8) and 0.3 % (fp4) from its best shape on average, 12 % at worst, and 8 of the 1520
 // are over 2 % slower than on 256-row tiles alone, the worst 10.6 % (with a fit to ragged bf16 problems only: 16, and 24 %).
 // Against the 256-row tiles alone: 256 x 256 x 6144 fp8 34.0 -> 12.0 us, 512 x 512 x 2048 fp4 12.0 -> 4.9, 592 x 736 x 4096
 // 24.6 -> 9.8, 2048^3 17.3 -> 13.5, geometric mean of the problems 1.58 (fp8), 1.66 (fp4).  (128 x 192 with fp8 is the best
 // shape of 9 of 1002 problems, by up to 5 %: 1024 x 4608 x 1536.)
+// 256 x 256 tiles on four wavefronts: fitted to 440 problems of 150 to 1024 such tiles, and compared with the other shapes only where the last round is
+// 78 % full or more.  Taken for 133 of them, by 10 % on average (fp8, one of 0.980 the least gain) and 7 % (fp4, three 3 to 5 % slower):
+// 2040 x 8100 x 8192 fp8 121 -> 104 us, fp4 70.3 -> 66.0; 4096^3 62 -> 54 and 40.6 -> 36.6; 8192^3 492 -> 418 and 308 -> 256.  Below 78 % and k of 1024 and more they are 4 to 17 % slower.
 struct MxShape {
     enum Kernel { kBlock, kW4, kKs } kernel;
     int number, bm, bn;
     double fixed, perRound, step, stepRound, perMega, stepShare, perMegaF32;
 };
-constexpr MxShape kMxShapes[2][9] = {
+constexpr double kMxWideShare = 0.78;
+constexpr MxShape kMxShapes[2][10] = {
     {{MxShape::kBlock, 0, 256, 256, 6.233, 4.744, 0.882, 1.791, 0.025, 0.728, 0.076},
+     {MxShape::kW4, 0, 256, 256, 9.531, 8.670, 0.647, 1.435, 0.000, 0.784, 0.075},
      {MxShape::kW4, 0, 256, 192, 8.332, 5.596, 0.666, 1.163, 0.062, 0.369, 0.033},
      {MxShape::kW4, 0, 256, 128, 6.086, 2.935, 0.553, 0.842, 0.093, 0.144, 0.035},
      {MxShape::kKs, 0, 64, 64, 2.595, 0.634, 0.196, 0.185, 0.191, 0.051, 0.027},
@@ -377,6 +382,7 @@ constexpr MxShape kMxShapes[2][9] = {
      {MxShape::kKs, 4, 128, 192, 5.785, 2.957, 0.481, 0.728, 0.124, 0.168, 0.059},
      {MxShape::kKs, 5, 192, 128, 5.833, 2.802, 0.482, 0.730, 0.129, 0.170, 0.056}}, // fp8
     {{MxShape::kBlock, 0, 256, 256, 5.763, 3.741, 1.024, 2.102, 0.045, 0.821, 0.085},
+     {MxShape::kW4, 0, 256, 256, 9.012, 5.823, 0.809, 2.199, 0.000, 0.939, 0.076},
      {MxShape::kW4, 0, 256, 192, 8.060, 6.472, 0.880, 1.293, 0.066, 0.435, 0.026},
      {MxShape::kW4, 0, 256, 128, 6.084, 3.053, 0.645, 0.951, 0.098, 0.213, 0.036},
      {MxShape::kKs, 0, 64, 64, 2.952, 0.929, 0.213, 0.209, 0.125, 0.078, 0.033},
@@ -404,6 +410,9 @@ int gemm_mx_any(hipStream_t st, void *c, const uint8_t *a, const uint8_t *b, con
             continue;
         const long long tiles = (long long)((m + s.bm - 1) / s.bm) * ((n + s.bn - 1) / s.bn), rest = tiles % cus;
         double more = (double)((tiles - 1) / cus), share = (double)((tiles - 1) % cus + 1) / cus, extra = 0.0;
+        const bool wide = s.kernel == MxShape::kW4 && s.bn == 256;
+        if (wide && share < kMxWideShare)
+            continue;
         if (s.kernel == MxShape::kBlock && !(m % 256 == 0 && n % 256 == 0)) {
             extra = steps * kMxStepRagged[fp4] * (more + 1.0);
         } else if (s.kernel == MxShape::kBlock && rest > 0 && rest * 4 <= cus && tiles > cus) {
@@ -413,7 +422,7 @@ int gemm_mx_any(hipStream_t st, void *c, const uint8_t *a, const uint8_t *b, con
         }
         const double time = (s.fixed + s.perRound * more + steps * (s.step + s.stepRound * more + s.stepShare * share) +
                              (s.perMega + (c_fp32 ? s.perMegaF32 : 0.0)) * (4e-6 * m * n) + extra) *
-                            (s.kernel == MxShape::kW4 ? 1.0 : s.kernel == MxShape::kKs ? 1.02 : 1.03);
+                            (s.kernel == MxShape::kKs ? 1.02 : s.kernel == MxShape::kBlock || wide ? 1.03 : 1.0);
         if (best == nullptr || time < bestTime) {
             best = &s;
             bestTime = time;
@@ -451,8 +460,10 @@ extern "C" int pto_gemm_mxfp4(void *stream, void *c, const uint8_t *a, const uin
 extern "C" int pto_gemm_mxfp8_variant(void *stream, void *c, const uint8_t *a, const uint8_t *b, const uint8_t *scale_a,
                                       const uint8_t *scale_b, int m, int n, int k, int format, int c_fp32, int variant)
 {
-    if (!c || !a || !b || !scale_a || !scale_b || m <= 0 || n <= 0 || k <= 0 || variant < 0 || variant > 12)
+    if (!c || !a || !b || !scale_a || !scale_b || m <= 0 || n <= 0 || k <= 0 || variant < 0 || variant > 13)
         return PTO_ERR_BAD_ARG;
+    if (variant == 13) // 256 x 256 on four wavefronts
+        return pto_amd::gemm_mx_w4(static_cast<hipStream_t>(stream), c, a, b, scale_a, scale_b, m, n, k, format, c_fp32, 256);
     if (variant >= 7) // k split over two groups of wavefronts, shape by number
         return pto_amd::gemm_mx_ks(static_cast<hipStream_t>(stream), c, a, b, scale_a, scale_b, m, n, k, format, c_fp32, variant - 7);
     if (variant >= 5) // the four-wave engine: 5 = 256 x 192 tiles, 6 = 256 x 128

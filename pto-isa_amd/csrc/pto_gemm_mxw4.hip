@@ -6,10 +6,12 @@
 
 namespace pto_amd {
 // format: 0 = e4m3 x e4m3, 1 = e5m2 x e5m2, 2 = A e4m3 x B e5m2, 3 = A e5m2 x B e4m3, 4 = e2m1 x e2m1 (k then counts 4-bit
-// elements, two per byte); width: 192 or 128
+// elements, two per byte); width: 256, 192 or 128
 int gemm_mx_w4(hipStream_t st, void *c, const uint8_t *a, const uint8_t *b, const uint8_t *sa, const uint8_t *sb, int m, int n, int k,
                   int format, int c_fp32, int width)
 {
+    if (width == 256)
+        return gemm_mx_w4_256(st, c, a, b, sa, sb, m, n, k, format, c_fp32);
     if (format < 0 || format > 4 || (width != 192 && width != 128))
         return PTO_ERR_UNSUPPORTED;
 #define PTO_MXW4_CASE(FMT, FA, FB)                                                                                         \
