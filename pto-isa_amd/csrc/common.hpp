@@ -64,13 +64,33 @@ int gemm_f16f32_w4(hipStream_t st, float *c, const _Float16 *a, const _Float16 *
 // defined in pto_gemm_ks.hip: tiles on eight wavefronts with k split over two groups of them; shape 0 .. 9 = 32 x 64, 64 x 64,
 // 64 x 96, 128 x 64, 128 x 96, 128 x 128, 192 x 128, 256 x 128, 192 x 192, 32 x 32.  PTO_ERR_UNSUPPORTED unless n % 4 == 0 and k % 32 == 0
 int gemm_f16f32_ks(hipStream_t st, float *c, const _Float16 *a, const _Float16 *b, int m, int n, int k, int shape);
-// defined in pto_gemm_mxw4.hip (MXFP8 / MXFP4 on the four-wave engine: 256 x 256, 256 x 192 or 256 x 128 tiles);
+// defined in pto_gemm_mxw4_<width>.hip (MXFP8 / MXFP4 on the four-wave engine: tiles of 256 x width);
 // PTO_ERR_UNSUPPORTED unless m >= 256, n >= width, n % 4 == 0, k % 512 == 0 (fp4, format 4: k % 1024 == 0)
-int gemm_mx_w4(hipStream_t st, void *c, const uint8_t *a, const uint8_t *b, const uint8_t *sa, const uint8_t *sb, int m, int n, int k,
-                  int format, int c_fp32, int width);
-// defined in pto_gemm_mxw4_256.hip: width 256 of the above
+int gemm_mx_w4_96(hipStream_t st, void *c, const uint8_t *a, const uint8_t *b, const uint8_t *sa, const uint8_t *sb, int m, int n, int k,
+                  int format, int c_fp32);
+int gemm_mx_w4_128(hipStream_t st, void *c, const uint8_t *a, const uint8_t *b, const uint8_t *sa, const uint8_t *sb, int m, int n, int k,
+                   int format, int c_fp32);
+int gemm_mx_w4_160(hipStream_t st, void *c, const uint8_t *a, const uint8_t *b, const uint8_t *sa, const uint8_t *sb, int m, int n, int k,
+                   int format, int c_fp32);
+int gemm_mx_w4_192(hipStream_t st, void *c, const uint8_t *a, const uint8_t *b, const uint8_t *sa, const uint8_t *sb, int m, int n, int k,
+                   int format, int c_fp32);
+int gemm_mx_w4_224(hipStream_t st, void *c, const uint8_t *a, const uint8_t *b, const uint8_t *sa, const uint8_t *sb, int m, int n, int k,
+                   int format, int c_fp32);
 int gemm_mx_w4_256(hipStream_t st, void *c, const uint8_t *a, const uint8_t *b, const uint8_t *sa, const uint8_t *sb, int m, int n, int k,
                    int format, int c_fp32);
+inline int gemm_mx_w4(hipStream_t st, void *c, const uint8_t *a, const uint8_t *b, const uint8_t *sa, const uint8_t *sb, int m, int n, int k,
+                      int format, int c_fp32, int width)
+{
+    switch (width) {
+    case 96: return gemm_mx_w4_96(st, c, a, b, sa, sb, m, n, k, format, c_fp32);
+    case 128: return gemm_mx_w4_128(st, c, a, b, sa, sb, m, n, k, format, c_fp32);
+    case 160: return gemm_mx_w4_160(st, c, a, b, sa, sb, m, n, k, format, c_fp32);
+    case 192: return gemm_mx_w4_192(st, c, a, b, sa, sb, m, n, k, format, c_fp32);
+    case 224: return gemm_mx_w4_224(st, c, a, b, sa, sb, m, n, k, format, c_fp32);
+    case 256: return gemm_mx_w4_256(st, c, a, b, sa, sb, m, n, k, format, c_fp32);
+    default: return PTO_ERR_UNSUPPORTED;
+    }
+}
 // defined in pto_gemm_mxks.hip (MXFP8 / MXFP4 tiles on eight wavefronts with k split over two groups of them); shape 0 .. 5 =
 // 64 x 64, 64 x 128, 128 x 64, 128 x 128, 128 x 192, 192 x 128.  PTO_ERR_UNSUPPORTED unless n % 4 == 0 and k % 512 == 0
 int gemm_mx_ks(hipStream_t st, void *c, const uint8_t *a, const uint8_t *b, const uint8_t *sa, const uint8_t *sb, int m, int n, int k,

@@ -1,4 +1,4 @@
-// MXFP8 GEMM tile of 256 x BN (BN = 256, 192 or 128) on four wavefronts: the four-wave fp16 kernel of gemm_kernels_w4.hpp with
+// MXFP8 GEMM tile of 256 x BN (BN = 96, 128 .. 256 in steps of 32) on four wavefronts: the four-wave fp16 kernel of gemm_kernels_w4.hpp with
 // 8-bit operands.  A K-step is the same 128 bytes per operand row (128 k instead of 64), so copies, LDS images and fragment
 // reads are byte for byte those of the fp16 kernel; what differs:
 //   * one v_mfma_scale_f32_16x16x128_f8f6f4 (8 passes) per 16 x 16 block and step instead of two v_mfma_f32_16x16x32_f16
@@ -15,11 +15,12 @@
 //   * four B stages (96 + 64 KiB = the whole LDS at BN = 192), which makes the step's second barrier unnecessary: a
 //     stage is overwritten two steps after its last read, with the barrier of the step in between.
 // Steps come in groups of four (B stage, A slot and scale byte repeat): k % 512 == 0.
-// BN = 256: all 256 accumulation registers, a sixth fewer copies and a seventh fewer fragment reads per MFMA than at 192.  Three B stages fit, so a step has a
+// BN = 224 and 256: up to all 256 accumulation registers, a sixth fewer copies and a seventh fewer fragment reads per MFMA than at 192.  Three B stages fit, so a step has a
 // second barrier again, ahead of its first copy of B, and as three stages and eight (sixteen) steps of a scale period do not go together, they take
 // turns at run time.  Two sets of scale registers do not fit: rows are loaded over their own first three quarters when the last one has been moved
 // aside, and spread in place.  What the time goes into (2040 x 8100 x 8192 fp4 on 256 x 128 tiles, 72.8 us; one part taken out): copies 8.8, reads of B 5.3 and of
-// A 3.0, scales 3.9; with none of them 53.3, the MFMAs at the clock they hold.  With 256 x 256 tiles 66.0; fp8 121 -> 104.
+// A 3.0, scales 3.9; with none of them 53.3, the MFMAs at the clock they hold.  With 256 x 256 tiles 66.0; fp8 121 -> 104.  The widths between are for products whose rounds they fill:
+// 1000 x 6144 x 4096 fp8 on 256 x 96 tiles 27.6 -> 25.7 us, fp4 19.0 -> 17.4.
 // MXFP4 (format 4, two e2m1 per byte): a K-step of 128 bytes is 256 k = two MFMAs (4 passes each, 16-byte operands: lane group
 // g holds bytes 16 g .. + 15 of the MFMA's 64) and eight scale blocks per row, so a scale register lasts two steps (the MFMA of
 // step j % 2 and half kk selects byte 2 (j % 2) + kk), the 64 scale bytes of a row eight steps, and two block rows / columns
@@ -148,11 +149,12 @@ struct MxW4Sched {
             if (aReadSlot(q) <= aReadSlot(q - 1))
                 return false;
         for (int j = 1; j < NCOPY; ++j)
-            if (copySlot(j) <= copySlot(j - 1) + 1) // the LDS address of copy j is set one slot before it
+            if (copySlot(j) <= copySlot(j - 1)) // the LDS address of copy j is set one slot before it, behind a copy there
                 return false;
         return true;
     }
-    static_assert(aReadSlot(7) < kBarrier && copySlot(NCOPY - 1) < kSlots && copySlot(0) >= 2 && distinct(), "order of the step");
+    // (A is read ahead of the block column behind which the next step waits for nothing older)
+    static_assert(aReadSlot(7) < 4 * (NNB - 1) && copySlot(NCOPY - 1) < kSlots && copySlot(0) >= 2 && distinct(), "order of the step");
     static_assert(kBarrier + 8 < kSlots, "two scale rows are spread in the slots behind the barrier");
 };
 
@@ -164,7 +166,7 @@ AICORE inline __attribute__((always_inline)) void MxW4TileCompute(__gm__ const u
                                                                   __gm__ const uint8_t *scale0, __gm__ const uint8_t *scale1, int k,
                                                                   int row0, int col0)
 {
-    constexpr bool WIDE = BN == 256;
+    constexpr bool WIDE = BN > 192;
     constexpr int NMB = 4, NNB = BN / 16, NBUF = 4, BSTAGES = WIDE ? 3 : 4, NA = 8, NCB = BN / 32, NCOPY = NA + NCB;
     using S = MxW4Sched<NNB, NCOPY>;
     constexpr bool FP4 = FMT_A == 4;
@@ -249,13 +251,15 @@ AICORE inline __attribute__((always_inline)) void MxW4TileCompute(__gm__ const u
         constexpr int set = decltype(setTag)::value, q = decltype(qTag)::value, mb = q / 2, kk = q % 2;
         aF[set][mb].h[kk] = W4LdsRead16<mb * 2048>(aAddr[kk][set]);
     };
-    auto readB = [&](auto stageTag, auto nbTag, auto kkTag) __attribute__((always_inline)) {
-        constexpr int stage = decltype(stageTag)::value, nb = decltype(nbTag)::value, kk = decltype(kkTag)::value;
+    // (bufTag: the block column counted on through the steps, so that the buffers take turns whatever their number in a step)
+    auto readB = [&](auto stageTag, auto nbTag, auto kkTag, auto bufTag) __attribute__((always_inline)) {
+        constexpr int stage = decltype(stageTag)::value, nb = decltype(nbTag)::value, kk = decltype(kkTag)::value, buf = decltype(bufTag)::value % NBUF;
         if constexpr (WIDE)
-            bF[nb % NBUF].h[kk] = W4LdsRead16<nb * 2048>(stage == 0 ? bNow[kk] : bThen[kk]);
+            bF[buf].h[kk] = W4LdsRead16<nb * 2048>(stage == 0 ? bNow[kk] : bThen[kk]);
         else
-            bF[nb % NBUF].h[kk] = W4LdsRead16<nb * 2048>(bAddr[kk][stage]);
+            bF[buf].h[kk] = W4LdsRead16<nb * 2048>(bAddr[kk][stage]);
     };
+    static_assert(2 * NNB % NBUF == 0, "the same turn every second step");
     auto operand = [](const Pair &p) {
         const u32x4 lo = __builtin_bit_cast(u32x4, p.h[0]), hi = __builtin_bit_cast(u32x4, p.h[1]);
         return i32x8{(int)lo[0], (int)lo[1], (int)lo[2], (int)lo[3], (int)hi[0], (int)hi[1], (int)hi[2], (int)hi[3]};
@@ -299,7 +303,7 @@ AICORE inline __attribute__((always_inline)) void MxW4TileCompute(__gm__ const u
     W4For<0, NA>([&](auto qTag) __attribute__((always_inline)) { readA(integral_constant<int, 0>(), qTag); });
     W4For<0, 2 * PD>([&](auto fTag) __attribute__((always_inline)) {
         constexpr int f = decltype(fTag)::value;
-        readB(integral_constant<int, 0>(), integral_constant<int, f / 2>(), integral_constant<int, f % 2>());
+        readB(integral_constant<int, 0>(), integral_constant<int, f / 2>(), integral_constant<int, f % 2>(), integral_constant<int, f / 2>());
     });
 
     // ---- K-step `it`, number t = it % kSuperSteps of its scale period: B stage t % 4, A register set and LDS slot t % 2, scale
@@ -370,9 +374,9 @@ AICORE inline __attribute__((always_inline)) void MxW4TileCompute(__gm__ const u
             if constexpr (mb < 2) { // half mb of the B operand of block column nb + PD
                 constexpr int g = nb + PD;
                 if constexpr (g < NNB)
-                    readB(integral_constant<int, s>(), integral_constant<int, g>(), integral_constant<int, mb>());
+                    readB(integral_constant<int, s>(), integral_constant<int, g>(), integral_constant<int, mb>(), integral_constant<int, g + NNB * par>());
                 else
-                    readB(integral_constant<int, sNext>(), integral_constant<int, g - NNB>(), integral_constant<int, mb>());
+                    readB(integral_constant<int, sNext>(), integral_constant<int, g - NNB>(), integral_constant<int, mb>(), integral_constant<int, g + NNB * par>());
             }
             if constexpr (S::aReadAt(idx) >= 0) {
                 if constexpr (S::aReadAt(idx) == 0) // this wave's A copies of the step before have landed
@@ -410,12 +414,12 @@ AICORE inline __attribute__((always_inline)) void MxW4TileCompute(__gm__ const u
             };
             if constexpr (FP4) {
                 // (the second half right behind the first: with the halves of two blocks in turn 2 % slower)
-                MxW4MfmaFp4<mb * NNB + nb, 2 * jj>(__builtin_bit_cast(u32x4, bF[nb % NBUF].h[0]), __builtin_bit_cast(u32x4, aF[par][mb].h[0]),
+                MxW4MfmaFp4<mb * NNB + nb, 2 * jj>(__builtin_bit_cast(u32x4, bF[(nb + NNB * par) % NBUF].h[0]), __builtin_bit_cast(u32x4, aF[par][mb].h[0]),
                                                    scaleOf(integral_constant<int, NMB + nb>()), scaleOf(integral_constant<int, mb>()));
-                MxW4MfmaFp4<mb * NNB + nb, 2 * jj + 1>(__builtin_bit_cast(u32x4, bF[nb % NBUF].h[1]), __builtin_bit_cast(u32x4, aF[par][mb].h[1]),
+                MxW4MfmaFp4<mb * NNB + nb, 2 * jj + 1>(__builtin_bit_cast(u32x4, bF[(nb + NNB * par) % NBUF].h[1]), __builtin_bit_cast(u32x4, aF[par][mb].h[1]),
                                                        scaleOf(integral_constant<int, NMB + nb>()), scaleOf(integral_constant<int, mb>()));
             } else {
-                MxW4Mfma<mb * NNB + nb, jj, FMT_B, FMT_A>(operand(bF[nb % NBUF]), operand(aF[par][mb]), scaleOf(integral_constant<int, NMB + nb>()),
+                MxW4Mfma<mb * NNB + nb, jj, FMT_B, FMT_A>(operand(bF[(nb + NNB * par) % NBUF]), operand(aF[par][mb]), scaleOf(integral_constant<int, NMB + nb>()),
                                                           scaleOf(integral_constant<int, mb>()));
             }
             __builtin_amdgcn_sched_barrier(0);
@@ -514,7 +518,7 @@ int launch_gemm_mxw4(hipStream_t st, void *c, const uint8_t *a, const uint8_t *b
     // (n % 4: four consecutive elements of a row are inside or outside together)
     if (m < 256 || n < BN || n % 4 || k % (FMT_A == 4 ? 1024 : 512) || k <= 0)
         return PTO_ERR_UNSUPPORTED;
-    constexpr int lds = (BN == 256 ? 3 : 4) * 128 * BN + 4 * 2 * 64 * 128; // four (three) B stages + two A slots per wave
+    constexpr int lds = (BN > 192 ? 3 : 4) * 128 * BN + 4 * 2 * 64 * 128; // four (three) B stages + two A slots per wave
     auto kernel = GemmMxW4<FMT_A, FMT_B, OutT, BN, 4>;
     static const int attr = pto_amd::allow_lds(kernel, lds);
     if (attr != PTO_OK)
@@ -523,5 +527,23 @@ int launch_gemm_mxw4(hipStream_t st, void *c, const uint8_t *a, const uint8_t *b
     kernel<<<dim3((unsigned)tiles), dim3(kBlockThreads), lds, st>>>(reinterpret_cast<OutT *>(c), a, b, sa, sb, m, n, k,
                                                                pto_amd::store_through(c, sizeof(OutT) * (uint64_t)n, sizeof(OutT) * (uint64_t)m * n));
     return pto_amd::check_launch();
+}
+// format: 0 = e4m3 x e4m3, 1 = e5m2 x e5m2, 2 = A e4m3 x B e5m2, 3 = A e5m2 x B e4m3, 4 = e2m1 x e2m1 (k then counts 4-bit
+// elements, two per byte)
+template <int BN>
+int launch_gemm_mxw4_format(hipStream_t st, void *c, const uint8_t *a, const uint8_t *b, const uint8_t *sa, const uint8_t *sb, int m, int n, int k,
+                            int format, int c_fp32)
+{
+#define PTO_MXW4_CASE(FMT, FA, FB)                                                              \
+    if (format == FMT)                                                                         \
+        return c_fp32 ? launch_gemm_mxw4<FA, FB, float, BN>(st, c, a, b, sa, sb, m, n, k) :     \
+                        launch_gemm_mxw4<FA, FB, bfloat16_t, BN>(st, c, a, b, sa, sb, m, n, k);
+    PTO_MXW4_CASE(0, 0, 0)
+    PTO_MXW4_CASE(1, 1, 1)
+    PTO_MXW4_CASE(2, 0, 1)
+    PTO_MXW4_CASE(3, 1, 0)
+    PTO_MXW4_CASE(4, 4, 4)
+#undef PTO_MXW4_CASE
+    return PTO_ERR_UNSUPPORTED;
 }
 } // namespace

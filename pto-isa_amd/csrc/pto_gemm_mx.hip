@@ -347,8 +347,8 @@ int gemm_mx_dispatch(hipStream_t st, void *c, const uint8_t *a, const uint8_t *b
 } // namespace
 
 namespace {
-// Three kernels: 256 x 256 tiles on eight wavefronts (this file; quarter tiles in a last partial round), 256 x 256, 256 x 192 and 256 x 128
-// tiles on four (pto_gemm_mxw4.hip), and tiles of 64 .. 192 rows with k split over two groups of wavefronts
+// Three kernels: 256 x 256 tiles on eight wavefronts (this file; quarter tiles in a last partial round), tiles of 256 rows and 96 to 256
+// columns on four (pto_gemm_mxw4_*.hip), and tiles of 64 .. 192 rows with k split over two groups of wavefronts
 // (pto_gemm_mxks.hip).  What a problem takes with one tile shape, in microseconds, launch included: tiles are dealt to the
 // compute units, `more` rounds beyond the first, `share` of the units busy in the last one, steps of 128 bytes,
 //   time = fixed + per_round more + steps (step + step_round more + step_share share) + (per_mega + fp32 result: per_mega_f32) (4e-6 m n);
@@ -369,9 +369,14 @@ struct MxShape {
     int number, bm, bn;
     double fixed, perRound, step, stepRound, perMega, stepShare, perMegaF32;
 };
-constexpr double kMxWideShare = 0.78;
-constexpr MxShape kMxShapes[2][10] = {
-    {{MxShape::kBlock, 0, 256, 256, 6.233, 4.744, 0.882, 1.791, 0.025, 0.728, 0.076},
+// 256 x 96, 160 and 224: fitted to 300 problems of 0.7 million results and more each in fp8 and fp4, compared where the last round is 70 % full and taken 2 % dearer: for 61 of the
+// 300 by 7 % (fp8) and 53 by 9 % (fp4) on average, for one of either more than 2 % slower (5 and 7 %).  5632 x 1536 x 512 fp8 to fp32 on 256 x 160 tiles -16 %,
+// 3840 x 1536 x 1024 fp4 on 256 x 96 -15 %, 7424 x 3584 x 7168 fp8 on 256 x 224 -17 %.
+constexpr MxShape kMxShapes[2][13] = {
+    {{MxShape::kW4, 0, 256, 96, 4.642, 1.735, 0.532, 0.751, 0.065, 0.144, 0.101},
+     {MxShape::kW4, 0, 256, 160, 7.914, 5.683, 0.436, 0.980, 0.024, 0.535, 0.069},
+     {MxShape::kW4, 0, 256, 224, 8.683, 6.830, 0.837, 1.359, 0.000, 0.492, 0.075},
+     {MxShape::kBlock, 0, 256, 256, 6.233, 4.744, 0.882, 1.791, 0.025, 0.728, 0.076},
      {MxShape::kW4, 0, 256, 256, 9.531, 8.670, 0.647, 1.435, 0.000, 0.784, 0.075},
      {MxShape::kW4, 0, 256, 192, 8.332, 5.596, 0.666, 1.163, 0.062, 0.369, 0.033},
      {MxShape::kW4, 0, 256, 128, 6.086, 2.935, 0.553, 0.842, 0.093, 0.144, 0.035},
@@ -381,7 +386,10 @@ constexpr MxShape kMxShapes[2][10] = {
      {MxShape::kKs, 3, 128, 128, 4.635, 2.138, 0.354, 0.508, 0.146, 0.110, 0.048},
      {MxShape::kKs, 4, 128, 192, 5.785, 2.957, 0.481, 0.728, 0.124, 0.168, 0.059},
      {MxShape::kKs, 5, 192, 128, 5.833, 2.802, 0.482, 0.730, 0.129, 0.170, 0.056}}, // fp8
-    {{MxShape::kBlock, 0, 256, 256, 5.763, 3.741, 1.024, 2.102, 0.045, 0.821, 0.085},
+    {{MxShape::kW4, 0, 256, 96, 5.728, 3.703, 0.484, 0.757, 0.000, 0.394, 0.113},
+     {MxShape::kW4, 0, 256, 160, 8.388, 4.324, 0.510, 1.238, 0.000, 0.644, 0.094},
+     {MxShape::kW4, 0, 256, 224, 7.526, 7.963, 1.089, 1.412, 0.000, 0.701, 0.098},
+     {MxShape::kBlock, 0, 256, 256, 5.763, 3.741, 1.024, 2.102, 0.045, 0.821, 0.085},
      {MxShape::kW4, 0, 256, 256, 9.012, 5.823, 0.809, 2.199, 0.000, 0.939, 0.076},
      {MxShape::kW4, 0, 256, 192, 8.060, 6.472, 0.880, 1.293, 0.066, 0.435, 0.026},
      {MxShape::kW4, 0, 256, 128, 6.084, 3.053, 0.645, 0.951, 0.098, 0.213, 0.036},
@@ -410,8 +418,8 @@ int gemm_mx_any(hipStream_t st, void *c, const uint8_t *a, const uint8_t *b, con
             continue;
         const long long tiles = (long long)((m + s.bm - 1) / s.bm) * ((n + s.bn - 1) / s.bn), rest = tiles % cus;
         double more = (double)((tiles - 1) / cus), share = (double)((tiles - 1) % cus + 1) / cus, extra = 0.0;
-        const bool wide = s.kernel == MxShape::kW4 && s.bn == 256;
-        if (wide && share < kMxWideShare)
+        const bool wide = s.kernel == MxShape::kW4 && s.bn == 256, between = s.kernel == MxShape::kW4 && s.bn % 64 == 32;
+        if ((wide && share < 0.78) || (between && share < 0.70))
             continue;
         if (s.kernel == MxShape::kBlock && !(m % 256 == 0 && n % 256 == 0)) {
             extra = steps * kMxStepRagged[fp4] * (more + 1.0);
@@ -422,7 +430,7 @@ int gemm_mx_any(hipStream_t st, void *c, const uint8_t *a, const uint8_t *b, con
         }
         const double time = (s.fixed + s.perRound * more + steps * (s.step + s.stepRound * more + s.stepShare * share) +
                              (s.perMega + (c_fp32 ? s.perMegaF32 : 0.0)) * (4e-6 * m * n) + extra) *
-                            (s.kernel == MxShape::kKs ? 1.02 : s.kernel == MxShape::kBlock || wide ? 1.03 : 1.0);
+                            (s.kernel == MxShape::kKs || between ? 1.02 : s.kernel == MxShape::kBlock || wide ? 1.03 : 1.0);
         if (best == nullptr || time < bestTime) {
             best = &s;
             bestTime = time;
@@ -460,10 +468,11 @@ extern "C" int pto_gemm_mxfp4(void *stream, void *c, const uint8_t *a, const uin
 extern "C" int pto_gemm_mxfp8_variant(void *stream, void *c, const uint8_t *a, const uint8_t *b, const uint8_t *scale_a,
                                       const uint8_t *scale_b, int m, int n, int k, int format, int c_fp32, int variant)
 {
-    if (!c || !a || !b || !scale_a || !scale_b || m <= 0 || n <= 0 || k <= 0 || variant < 0 || variant > 13)
+    if (!c || !a || !b || !scale_a || !scale_b || m <= 0 || n <= 0 || k <= 0 || variant < 0 || variant > 16)
         return PTO_ERR_BAD_ARG;
-    if (variant == 13) // 256 x 256 on four wavefronts
-        return pto_amd::gemm_mx_w4(static_cast<hipStream_t>(stream), c, a, b, scale_a, scale_b, m, n, k, format, c_fp32, 256);
+    if (variant >= 13) // further widths on four wavefronts: 256, 96, 160, 224
+        return pto_amd::gemm_mx_w4(static_cast<hipStream_t>(stream), c, a, b, scale_a, scale_b, m, n, k, format, c_fp32,
+                                   variant == 13 ? 256 : variant == 14 ? 96 : variant == 15 ? 160 : 224);
     if (variant >= 7) // k split over two groups of wavefronts, shape by number
         return pto_amd::gemm_mx_ks(static_cast<hipStream_t>(stream), c, a, b, scale_a, scale_b, m, n, k, format, c_fp32, variant - 7);
     if (variant >= 5) // the four-wave engine: 5 = 256 x 192 tiles, 6 = 256 x 128

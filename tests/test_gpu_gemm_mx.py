@@ -412,8 +412,9 @@ def test_mx_gemm_results_in_pieces_of_64_bytes(variant, m, n, shift, c_fp32):
 
 @pytest.mark.parametrize("fmt,m,n,k", [(0, 256, 256, 512), (1, 260, 300, 2048), (2, 512, 256, 2560), (3, 256, 516, 4608), (4, 256, 256, 1024), (4, 300, 516, 2048), (4, 512, 256, 3072),
                                        (4, 257, 260, 5120)])
-def test_mx_gemm_256x256_on_four_wavefronts(oracle, fmt, m, n, k):
-    """One tile, tiles moved back in m and in n; less than a scale period (2048 k), whole ones and a part behind whole ones: every scale of either operand exactly, integer operands
+@pytest.mark.parametrize("variant", [13, 14, 15, 16])
+def test_mx_gemm_further_widths_on_four_wavefronts(oracle, variant, fmt, m, n, k):
+    """256 x 256, 96, 160 and 224.  One tile, tiles moved back in m and in n; less than a scale period (2048 k), whole ones and a part behind whole ones: every scale of either operand exactly, integer operands
     exactly, the generator's distribution to the GEMM tolerance, the bf16 result = RNE of the fp32 one."""
     fa, fb = {2: (0, 1), 3: (1, 0)}.get(fmt, (fmt, fmt))
     rng = np.random.default_rng(k)
@@ -421,22 +422,22 @@ def test_mx_gemm_256x256_on_four_wavefronts(oracle, fmt, m, n, k):
     width = k // 2 if fmt == 4 else k
     a, b = np.full((m, width), ones[fa], dtype=np.uint8), np.full((n, width), ones[fb], dtype=np.uint8)
     sa, sb = (rng.integers(125, 131, size=(r, k // 32)).astype(np.uint8) for r in (m, n))
-    rc, got = _mx_variant(a, b, sa, sb, fmt, 13)
-    capi.check(rc, "256 x 256 on four wavefronts")
+    rc, got = _mx_variant(a, b, sa, sb, fmt, variant)
+    capi.check(rc, "four-wave MX kernel")
     assert np.array_equal(got.astype(np.float64), 32.0 * (np.exp2(sa.astype(np.float64) - 127) @ np.exp2(sb.astype(np.float64) - 127).T))
     for dist in ("integer", "bytes"):
         (a, _, sa, sb), (_, b, _, _) = (datagen.mx_inputs(m, n, k, f, dist=dist) for f in (fa, fb))
-        rc, got = _mx_variant(a, b, sa, sb, fmt, 13)
+        rc, got = _mx_variant(a, b, sa, sb, fmt, variant)
         want = oracle.mx_gemm(a, b, sa, sb, fa, fb)
         assert rc == 0 and (np.array_equal(got, want) if dist == "integer" else np.all(np.isfinite(got)) and rel_err(got, want) <= TOL), dist
-        rc, got16 = _mx_variant(a, b, sa, sb, fmt, 13, c_fp32=False)
+        rc, got16 = _mx_variant(a, b, sa, sb, fmt, variant, c_fp32=False)
         assert rc == 0 and np.array_equal(got16, bf16_rne(got))
 
 
 @pytest.mark.parametrize("fmt", [1, 4])
-@pytest.mark.parametrize("m,n", [(2560, 5120), (2816, 4608), (2500, 5116)])
-def test_mx_gemm_on_both_sides_of_the_256x256_tiles(fmt, m, n):
-    """The entry point at 200 and 198 tiles of 256 x 256 of 256 compute units: integer operands, the result of the 256 x 128 tiles."""
+@pytest.mark.parametrize("m,n", [(2560, 5120), (2816, 4608), (2500, 5116), (1000, 6144), (3840, 1536), (2048, 5120), (3133, 3680), (1537, 3328)])
+def test_mx_gemm_whatever_tile_the_entry_point_takes(fmt, m, n):
+    """The entry point at 200 and 198 tiles of 256 x 256 of 256 compute units, and where other widths fill a round: integer operands, the result of the 256 x 128 tiles."""
     k = 1024
     a, b, sa, sb = datagen.mx_inputs(m, n, k, fmt, dist="integer") if fmt != 4 else datagen.mx_inputs(m, n, k, fmt)
     rc, got = _mx_variant(a, b, sa, sb, fmt, 4)
