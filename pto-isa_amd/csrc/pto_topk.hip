@@ -254,7 +254,7 @@ constexpr bool kOnlyWhole = E == 1 && W == 4;
 // the launch, the 20 MB of the rows (3.1 us at 6.5 TB/s), and 480 vector and 280 scalar instructions a row (the whole network: 2520 vector ones).  Four places of the interval at a time instead
 // of one took 2.2 us more (scalar instructions), positions in the list by ballots instead of one scan over the lanes 1.2.
 constexpr int kMostSelected = 8; // times 64 keys
-enum Mode { kCut, kWhole, kSelect };
+enum Mode { kCut, kWhole, kSelect, kCountedCut }; // (the last: by buckets, kCut where that fails)
 // whole sorts by buckets first
 template <int E, int W>
 constexpr bool kBuckets = E >= 4 && E * W >= 8;
@@ -578,7 +578,7 @@ __global__ __launch_bounds__(kTopkThreads, MODE == kSelect && E == 16 ? 4 : MODE
     constexpr int kStages = E <= 8 ? 2 : 1;  // scores and columns side by side, or one after the other (LDS for four workgroups more)
     // exchanges, then results (or, between two sorts, the ranks of the columns); behind them the columns in the order of their indices
     // buckets: per row of one wave a piece of its own, in which its results are staged as well
-    constexpr bool kCount = MODE == kWhole && kBuckets<E, W>;
+    constexpr bool kCount = (MODE == kWhole || MODE == kCountedCut) && kBuckets<E, W>;
     constexpr size_t kOwn = kCount && W == 1 && N * 8 > kStaged * 4 * kStages ? N * 8 : kStaged * 4 * kStages;
     constexpr size_t kExchange = W > 1 ? (size_t)kTopkWaves * E * 64 * 8 : 0, kStage = (size_t)kTopkWaves * kOwn;
     constexpr size_t kSelected = MODE == kSelect ? 384 + (size_t)kRows * 68 * kMostSelected * 8 : 0, kSort = kExchange > kStage ? kExchange : kStage;
@@ -989,7 +989,10 @@ int launch_topk(hipStream_t st, float *out_score, uint32_t *out_index, const flo
     // (LDS / DPP, whole sorts: 300 x 128 3.48 / 3.26 us, 300 x 256 4.53 / 4.28); with more the moves take issue slots (4800 x 128
     // 5.09 / 5.23).  8 and 16 keys per lane cover the latency either way and take DPP.
     const bool dpp = E >= 8 || (long long)rows * W <= 4 * 4 * pto_amd::compute_units();
-    constexpr Mode kFew = kOnlyWhole<E, W> ? kWhole : kCut;
+    // Past 1024 columns buckets instead of merges that keep topk, wherever no threshold is taken (us, merges / buckets, random scores; nearly all equal ones):
+    // 2048 columns, 16 rows, top 129 7.0 / 5.5; 7.0 / 7.35, 300 rows, top 256 8.5 / 6.2; 8.4 / 8.8; 4096 columns, 16 rows, top 321 11.4 / 7.5; 11.45 / 11.9,
+    // 1500 rows, top 512 34.3 / 19.5; 33.7 / 34.9.  1024 columns, 16 rows, top 64 4.6 / 4.4; 4.6 / 5.0: what it gives and what it takes are alike there
+    constexpr Mode kFew = kOnlyWhole<E, W> ? kWhole : W == 4 && E >= 8 ? kCountedCut : kCut;
     constexpr bool kDpp = E >= 8 || kOnlyWhole<E, W>; // (names the one form that there is)
     auto kernel = dpp ? (whole ? TopkRows<E, W, true, kWhole> : TopkRows<E, W, true, kFew>) :
                         (whole ? TopkRows<E, W, kDpp, kWhole> : TopkRows<E, W, kDpp, kFew>);

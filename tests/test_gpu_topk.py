@@ -266,7 +266,7 @@ def test_topk_threshold_and_the_columns(oracle, rows, cols, topks):
 @pytest.mark.parametrize("rows,cols", [(750, 512), (803, 257), (9, 1024), (12, 513), (900, 1024), (860, 700), (2563, 1024), (2565, 600), (5, 2048), (14, 1025), (1710, 2048), (1711, 1100),
                                        (13, 4096), (14, 2049), (12, 3000)])
 def test_topk_by_buckets(rows, cols):
-    """Whole sorts (more than an eighth of the padded row) of every kind of row that buckets take, give up on at the look, after counting, or after a first exchange: even
+    """Whole sorts (more than an eighth of the padded row), and an eighth where no threshold is taken, of every kind of row that buckets take, give up on at the look, after counting, or after a first exchange: even
     scores; equal ones in numbers around the fullest bucket's limits (16, 32); ascending and descending; one far outlier; a cluster of distinct scores; infinities; NaNs of either
     sign; zeros of either sign; ranges too small and too large to spread; a part of the columns at another level.  NaNs, which the
     comparator leaves open, in the order of their bits as before."""
@@ -314,6 +314,7 @@ def test_topk_by_buckets(rows, cols):
     bits = src[:, :cols].view(np.uint32)
     plain = np.where(bits == 0x80000000, np.uint32(0), bits)
     order = np.where(plain >> 31, ~plain, plain | np.uint32(0x80000000))
-    for ids, k in ((idx, cols), (idx, max(321, eighth + 1) if cols > 321 else cols), (idx * np.uint32(3) + np.uint32(5), cols - 1), (np.uint32(0xFFFFFFFF) - idx, cols)):
+    for ids, k in ((idx, cols), (idx, max(321, eighth + 1) if cols > 321 else cols), (idx * np.uint32(3) + np.uint32(5), cols - 1), (np.uint32(0xFFFFFFFF) - idx, cols),
+                   (idx, eighth), (idx * np.uint32(3) + np.uint32(5), eighth - 1), (np.uint32(0xFFFFFFFF) - idx, eighth)):
         at = np.lexsort((np.broadcast_to(ids, order.shape), ~order))[:, :k]
         assert same(topk_gpu(src, ids, cols, k), (np.take_along_axis(src, at, 1), ids[at])), (k, ids[:2])
