@@ -31,9 +31,10 @@
 //   600 x 2048, top 100 10.8 -> 7.1 (ascending 5.9, masked from the middle on 7.4); 600 x 4096, top 100 18.3 -> 7.9.
 // * Whole sorts of 257 columns and more (BucketSort): the keys are counted into buckets and put in place, two and more in a bucket by a few exchanges of
 //   neighbours; rows too uneven for that go through the network.  4800 x 1024, top 1000 21.2 -> 14.2 us, 1 x 4096 whole 12.5 -> 7.9, 2400 x 2048 26.6 -> 16.9.
-// * Any other index vector: the same network sorts the (index, column) pairs first, once per workgroup (the rows share their
-//   indices); the rank of a column in that order then stands in the scores' keys for the column.  4800 x 1024 whole: 42 us (127
-//   with keys in the LDS and a pass over it per stage); 1000 x 256: 6.6 (15).
+// * Any other index vector: the (index, column) pairs are sorted first, once per workgroup (the rows share their
+//   indices), by buckets where the indices are below 2^24 and the columns 257 to 2048, or by the network; the rank of a column in that order then stands in
+//   the scores' keys for the column.  4800 x 1024 whole: 30 us, 35 with indices of any size (both by the network 40, with keys in the LDS and a pass over it
+//   per stage 127); 1000 x 256: 6.6 (15).  Scores by buckets where a row is one wave's; with more waves they go through the network.
 // What bounds the network: vector instructions, 2520 per row of 1024 (3850 in the integer network this replaced), behind a phase of
 // loads and before one of stores that all waves share (five waves on a SIMD instead of four: no change; persistent waves that load the next row while they sort
 // one, and wave priorities that let some run ahead, do not hide them: 32 us and no change).  By buckets 4800 x 1024, top 1000 (58 MB = 9 us at 6.5 TB/s)
@@ -323,6 +324,7 @@ __device__ inline void WaveEnds(float &hi, float &lo)
 // sorted, as the limits of ranges that are spread evenly each (4800 x 1024 27 us).  512 columns in up to 731 rows stay with the network (4.2 us; by
 // buckets 4.5 in two waves a row, 4.5 in one), as do 256 and less.
 // bits[e]: the score in column i0 + 64 e; afterwards key e of the lane with number q = 64 (wave of the row) + lane is of rank q E + e.
+// RANKS: rankOf[column] decides among equal scores and is returned in the column's place.
 // mem: 8 N bytes for the row; across: four sets of a word per wave of the workgroup.
 // Is it so in every lane of the workgroup?  One barrier (__syncthreads_and: three, and an atomic).  votes: a word per wave, another set of them for the next vote
 __device__ inline bool Everyone(bool v, uint32_t *votes)
@@ -382,7 +384,8 @@ struct BucketSort {
         lo = b;
     }
 
-    __device__ inline __attribute__((always_inline)) Counted Sort(const uint32_t (&bits)[E], uint32_t i0, int validCols, int waveOfRow, int lane, uint32_t *mem, uint32_t *across)
+    template <bool RANKS = false>
+    __device__ inline __attribute__((always_inline)) Counted Sort(const uint32_t (&bits)[E], uint32_t i0, int validCols, int waveOfRow, int lane, uint32_t *mem, uint32_t *across, [[maybe_unused]] const uint16_t *rankOf = nullptr)
     {
         const uint32_t q = (uint32_t)(waveOfRow * 64 + lane), wave = threadIdx.x / 64;
         // the range
@@ -520,7 +523,7 @@ struct BucketSort {
 #pragma unroll
         for (int e = 0; e < E; ++e) {
             at[e] = __builtin_amdgcn_ubfe(at[e], one[e] >> 12, 16);
-            k[e] = TopkKey(bits[e], columnBits - (uint32_t)(e * 64 << 8));
+            k[e] = TopkKey(bits[e], RANKS ? (4095u - rankOf[i0 + 64u * (uint32_t)e]) << 8 : columnBits - (uint32_t)(e * 64 << 8));
         }
         if (validCols != N) { // (what stands behind the columns goes behind the keys)
 #pragma unroll
@@ -585,10 +588,12 @@ __global__ __launch_bounds__(kTopkThreads, MODE == kSelect && E == 16 ? 4 : MODE
     constexpr size_t kWork = kSort > kSelected ? kSort : kSelected;
     static_assert(kWork >= (size_t)N * 2, "the ranks fit");
     // (behind the first wave's results where its piece has room: 32 KiB a workgroup are five workgroups a compute unit)
-    constexpr size_t kColumns = kOwn >= kStaged * 4 * kStages + (size_t)N * 2 ? (size_t)kStaged * 4 * kStages : kWork;
-    __shared__ __attribute__((aligned(16))) char lds[kColumns < kWork ? kWork : kWork + (size_t)N * 2];
+    // (one wave per row and buckets: both tables of the columns' order behind everything, as the rows are still counted when they are read)
+    constexpr bool kApart = kCount && W == 1;
+    constexpr size_t kColumns = kApart ? kWork + (size_t)N * 2 : kOwn >= kStaged * 4 * kStages + (size_t)N * 2 ? (size_t)kStaged * 4 * kStages : kWork;
+    __shared__ __attribute__((aligned(16))) char lds[kColumns < kWork ? kWork : kColumns + (size_t)N * 2];
     [[maybe_unused]] __shared__ uint32_t across[kTopkWaves * 6];
-    uint16_t *rankOf = reinterpret_cast<uint16_t *>(lds), *columnOf = reinterpret_cast<uint16_t *>(lds + kColumns);
+    uint16_t *rankOf = reinterpret_cast<uint16_t *>(lds + (kApart ? kWork : 0)), *columnOf = reinterpret_cast<uint16_t *>(lds + kColumns);
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / 64), lane = tid % 64;
     const int waveOfRow = wave % W, row0 = (int)blockIdx.x * kRows, row = row0 + wave / W < rows ? row0 + wave / W : rows - 1;
     // this lane's first column; then every kStep-th.  Where a threshold selects, the waves of a row take blocks of 64 columns in turn, so that each
@@ -934,38 +939,91 @@ __global__ __launch_bounds__(kTopkThreads, MODE == kSelect && E == 16 ? 4 : MODE
             s.form = 0;
             uint32_t all[E];
             load(inIdx, all);
+            bool listed = false;
+            if constexpr (kCount && N < 4096) { // (4096 columns: scalar registers would be spilled)
+                // indices below 2^24 by buckets: as scores, exactly (2400 x 2048, top 2000 54.3 -> 43.7 us, 1000 x 1024, top 700 16.2 -> 13.9; 4800 x 1024
+                // whole 39.9 -> 35.0, and 30.0 with its scores by buckets as well; indices that this turns away 15.7 -> 15.8)
+                constexpr uint32_t kBelow = 1u << 24;
+                bool small = true;
 #pragma unroll
-            for (int e = 0; e < E; ++e) {
-                const uint32_t order = ~all[e];
-                s.k[e] = Key(__builtin_amdgcn_alignbit(0x3ffu, order, 12), (order << 20) | (columnBits - (e * kStep << 8)));
-                if (i0 + e * kStep >= (uint32_t)validCols)
-                    s.k[e] = 1.0;
+                for (int e = 0; e < E; ++e)
+                    small = small & (all[e] < kBelow);
+                if (W > 1 ? Everyone(small, across + 4 * kTopkWaves) : WholeWave(small)) {
+                    uint32_t as[E];
+#pragma unroll
+                    for (int e = 0; e < E; ++e)
+                        as[e] = __builtin_bit_cast(uint32_t, (float)(kBelow - 1u - all[e]));
+                    uint32_t column0 = i0;
+                    int here = lane;
+                    asm volatile("" : "+v"(column0), "+v"(here));
+                    BucketSort<E, W> b;
+                    listed = b.Sort(as, column0, validCols, waveOfRow, here, reinterpret_cast<uint32_t *>(lds + (W == 1 ? 0 : (size_t)(wave / W) * N * 8)), across) == kSorted;
+                    if (listed) {
+                        if (W > 1)
+                            __syncthreads(); // (neighbours have read each other's keys)
+#pragma unroll
+                        for (int e = 0; e < E; ++e) {
+                            const uint32_t rank = (uint32_t)((waveOfRow * 64 + here) * E + e), column = 4095u - ((Low(b.k[e]) >> 8) & 0xfffu);
+                            if (wave < W && rank < (uint32_t)validCols) {
+                                rankOf[column] = (uint16_t)rank;
+                                columnOf[rank] = (uint16_t)column;
+                            }
+                        }
+                    } else {
+                        load(inIdx, all);
+                    }
+                }
             }
-            s.template Sort<kBits>(kBits);
-            asm volatile("" : "+v"(i0), "+v"(s.q)); // (nothing that depends on them is kept in registers across the sort)
-            if (W > 1)
-                __syncthreads(); // (the exchanges are over)
+            if (!listed) {
 #pragma unroll
-            for (int e = 0; e < E; ++e) {
-                const uint32_t rank = s.q * E + e, column = 4095u - ((Low(s.k[e]) >> 8) & 0xfffu);
-                if (wave < W && rank < (uint32_t)validCols) {
-                    rankOf[column] = (uint16_t)rank;
-                    columnOf[rank] = (uint16_t)column;
+                for (int e = 0; e < E; ++e) {
+                    const uint32_t order = ~all[e];
+                    s.k[e] = Key(__builtin_amdgcn_alignbit(0x3ffu, order, 12), (order << 20) | (columnBits - (e * kStep << 8)));
+                    if (i0 + e * kStep >= (uint32_t)validCols)
+                        s.k[e] = 1.0;
+                }
+                s.template Sort<kBits>(kBits);
+                asm volatile("" : "+v"(i0), "+v"(s.q)); // (nothing that depends on them is kept in registers across the sort)
+                if (W > 1)
+                    __syncthreads(); // (the exchanges are over)
+#pragma unroll
+                for (int e = 0; e < E; ++e) {
+                    const uint32_t rank = s.q * E + e, column = 4095u - ((Low(s.k[e]) >> 8) & 0xfffu);
+                    if (wave < W && rank < (uint32_t)validCols) {
+                        rankOf[column] = (uint16_t)rank;
+                        columnOf[rank] = (uint16_t)column;
+                    }
                 }
             }
         }
         load(scores, bits);
+        if constexpr (kApart) {
+            __syncthreads(); // the ranks are there
+            uint32_t column0 = i0;
+            int here = lane;
+            asm volatile("" : "+v"(column0), "+v"(here));
+            BucketSort<E, W> b; // (9000 x 512, top 400 29.4 -> 22.7 us with this and the columns' order by buckets; 3000 x 777, top 700 25.6 -> 18.1)
+            const Counted done = b.template Sort<true>(bits, column0, validCols, 0, here, reinterpret_cast<uint32_t *>(lds + wave * kOwn), across, rankOf);
+            if (done == kSorted) {
+                finish(b.k, here * E, here);
+                return;
+            }
+            if (done == kLost)
+                load(scores, bits);
+        }
     }
     s.form = 0;
 #pragma unroll
     for (int e = 0; e < E; ++e)
         s.k[e] = TopkKey(bits[e], columnBits - (e * kStep << 8));
     if (__builtin_expect(!increasing, 0)) {
-        __syncthreads(); // the ranks are there
+        if (!kApart)
+            __syncthreads(); // the ranks are there
 #pragma unroll
         for (int e = 0; e < E; ++e)
             s.k[e] = Key(High(s.k[e]), (Low(s.k[e]) & 0xfff000ffu) | (4095u - rankOf[i0 + e * kStep]) << 8); // (past the row's end: overwritten below)
-        __syncthreads(); // and read, before their memory is used for something else
+        if (!kApart)
+            __syncthreads(); // and read, before their memory is used for something else
     }
     if (kClamp || validCols != N) {
 #pragma unroll
@@ -1020,11 +1078,13 @@ extern "C" int pto_topk_f32(void *stream, float *out_score, uint32_t *out_index,
     if (ld < valid_cols || topk > valid_cols || valid_cols > 4096)
         return PTO_ERR_UNSUPPORTED;
     hipStream_t st = static_cast<hipStream_t>(stream);
-    // Waves per row.  One wave per row does the least work, more put more of the chip to work on few rows (one / two / four waves,
-    // whole sorts: 1024 columns, 600 rows 9.8 / 8.8 / 7.7 us, 1000 rows 10.3 / 9.3 / 9.2, 2400 rows 17.5 / 16.2 / 17.9, 4800
-    // rows 25.3 / 26.9 / 28.8; 1000 rows top 256 8.7 / 8.1 / 8.2): on 256 units four up to 853 rows, two up to 2560.  512 columns:
-    // four up to 731 rows (600 rows 5.7 / 5.4 / 5.1, 853 rows 5.8 / 5.5 / 5.6, top 15 4.5 / 4.6 / 5.1), then one.  2048 columns: four
-    // up to 1706 rows (1700 rows with two 25.6, with four 24.5; 2000 rows 26.2, 26.9).  129 to 256 columns: four up to 365 rows where
+    // Waves per row.  One wave per row does the least work, more put more of the chip to work on few rows.  1024 columns, one / two / four waves,
+    // whole sorts, us, on 256 units (by buckets; the network): 300 rows 6.7 / 5.8 / 5.1; 600 rows 6.6 / 6.4 / 5.6; 9.8 / 8.8 / 7.7, 1000 rows 6.6 / 6.4 / 6.1;
+    // 10.3 / 9.3 / 9.2, 1500 rows 8.2 / 7.5 / 7.2, 2400 rows 9.7 / 9.2 / 10.2; 17.5 / 16.2 / 17.9, 4800 rows 25.3 / 26.9 / 28.8 (network): four up to 853 rows, two
+    // up to 2560 (1000 rows top 256 by the network 8.7 / 8.1 / 8.2).  512 columns: four waves and the network up to 731 rows (network: 600 rows 5.7 / 5.4 / 5.1,
+    // 853 rows 5.8 / 5.5 / 5.6, top 15 4.5 / 4.6 / 5.1; 300 rows network in four 4.1, buckets in one or two 4.5; 700 rows 4.6, 4.5 and 4.9), then one.
+    // 2048 columns: four up to 1706 rows (two / four, by buckets: 16 rows 7.9 / 5.6, 800 rows 9.8 / 8.6, 1600 rows 13.4 / 11.5, 2400 rows 17.2 / 17.2; network: 1700
+    // rows 25.6 / 24.5, 2000 rows 26.2 / 26.9).  129 to 256 columns: four up to 365 rows where
     // more than 16 are wanted (one / four: 128 rows 3.6 / 3.3, 300 rows 3.6 / 3.4, 600 rows 3.7 / 3.7; top 7 of 128 rows 3.2 / 3.6).
     const int most = 5 * 4 * pto_amd::compute_units() / rows; // waves per row for five on every SIMD
     // A threshold, then a sort of what reaches it (us, merges that keep topk / threshold; random scores):

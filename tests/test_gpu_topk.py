@@ -318,3 +318,24 @@ def test_topk_by_buckets(rows, cols):
                    (idx, eighth), (idx * np.uint32(3) + np.uint32(5), eighth - 1), (np.uint32(0xFFFFFFFF) - idx, eighth)):
         at = np.lexsort((np.broadcast_to(ids, order.shape), ~order))[:, :k]
         assert same(topk_gpu(src, ids, cols, k), (np.take_along_axis(src, at, 1), ids[at])), (k, ids[:2])
+
+
+@pytest.mark.parametrize("rows,cols", [(803, 257), (750, 512), (9, 1024), (12, 513), (900, 1024), (860, 700), (2563, 1024), (2565, 600), (5, 2048), (14, 1025), (1710, 2048), (1711, 1100),
+                                       (7, 4096)])
+def test_topk_any_index_order_by_buckets(rows, cols):
+    """Indices in any order whose order is found by buckets (below 2^24), or not (one at 2^24, all of them far apart, crowded, all equal but a few): equal
+    ones by column. Random scores, and every third row of few distinct ones with zeros of either sign, every fifth masked with infinities from the middle on."""
+    r = np.random.Generator(np.random.Philox(key=3 * rows + cols))
+    src, column = r.standard_normal((rows, cols)).astype(np.float32), np.arange(cols)
+    src[1::3] = np.where(r.random(src[1::3].shape) < 0.5, np.float32(-1.0), np.float32(1.0)) * r.integers(0, 9, src[1::3].shape).astype(np.float32)
+    src[4::5, cols // 2:] = -np.inf
+    shuffled = r.permutation(cols)
+    top = (1 << 24) - 1
+    kinds = (shuffled, top - shuffled, np.where(shuffled == 3, top + 1, shuffled), shuffled * ((1 << 32) // cols - 1), r.integers(0, cols // 2, cols),
+             np.where(shuffled < 5, shuffled, 77), np.where(shuffled == 0, top, shuffled % 40), 2 * shuffled + 1000 - 7 * (shuffled % 2))
+    score = -(src + np.float32(0.0))
+    for n, ids in enumerate(kinds):
+        ids = ids.astype(np.uint32)
+        k = cols if n % 2 else cols - cols // 4
+        order = np.lexsort((np.broadcast_to(column, src.shape), np.broadcast_to(ids, src.shape), score))[:, :k]
+        assert same(topk_gpu(src, ids, cols, k), (np.take_along_axis(src, order, 1), ids[order])), n
