@@ -574,7 +574,7 @@ struct BucketSort {
 };
 template <int E, int W, bool LOW_DPP, Mode MODE>
 __global__ __launch_bounds__(kTopkThreads, MODE == kSelect && E == 16 ? 4 : MODE == kWhole && E == 16 && W == 1 ? 4 : 1) void TopkRows(float *outScore, uint32_t *outIndex, const float *src, const uint32_t *inIdx,
-                                                         int rows, int validCols, int ld, int topk, int keepBits, int through)
+                                                         int rows, int validCols, int ld, int topk, int keepBits, int through, int buckets)
 {
     constexpr int N = 64 * E * W, kRows = kTopkWaves / W, kBits = RowSort<E, W, LOW_DPP>::kLaneBits;
     constexpr int kStaged = 64 * E + 4 * E; // words of a wave's results, one of padding behind every 16
@@ -919,7 +919,7 @@ __global__ __launch_bounds__(kTopkThreads, MODE == kSelect && E == 16 ? 4 : MODE
         store(stored, toIndex, count, lane, [&](int i) { return first + stagedColumn[i + i / 16]; });
     };
     if constexpr (kCount) {
-        if (increasing) {
+        if (increasing && buckets) {
             uint32_t column0 = i0;
             int here = lane;
             asm volatile("" : "+v"(column0), "+v"(here)); // (nothing of this is kept in registers for what comes behind)
@@ -1062,9 +1062,13 @@ int launch_topk(hipStream_t st, float *out_score, uint32_t *out_index, const flo
     // instruction's 256 bytes (8192 x 64, top 1 3.2 / 3.7, 131072 x 64, top 33 32.6 / 34.1), nor where they are much more than the L2s'
     // 32 MB, which then are written back while others sort (30000 x 2048, top 1500 261 / 268).
     const int through = topk >= 64 && 8ll * rows * topk <= 1ll << 26;
+    // Just past what a threshold is taken for, 257 to 320 of 1025 to 2048 columns, the network as before: 600 x 1025 random scores take 9.0 us by threshold for the
+    // top 256 and would take 7.7 by buckets for the top 257, but rows masked from the middle on 9.1 by threshold and 12.6 where buckets turn them away; both
+    // in one kernel, buckets ahead of the threshold, is 15 % faster with random rows, 5 to 20 % slower with masked and 50 % with sixty distinct scores
+    const int buckets = !(64 * E * W == 2048 && topk > 256 && topk <= 320);
     constexpr int kRows = kTopkWaves / W;
     kernel<<<dim3((unsigned)(((long long)rows + kRows - 1) / kRows)), dim3(kTopkThreads), 0, st>>>(out_score, out_index, src, in_idx, rows, valid_cols,
-                                                                                                   ld, topk, keepBits, through);
+                                                                                                   ld, topk, keepBits, through, buckets);
     return pto_amd::check_launch();
 }
 
