@@ -38,7 +38,8 @@
 // What bounds the network: vector instructions, 2520 per row of 1024 (3850 in the integer network this replaced), behind a phase of
 // loads and before one of stores that all waves share (five waves on a SIMD instead of four: no change; persistent waves that load the next row while they sort
 // one, and wave priorities that let some run ahead, do not hide them: 32 us and no change).  By buckets 4800 x 1024, top 1000 (58 MB = 9 us at 6.5 TB/s)
-// is bound by the launch, the loads and the stores, with some 800 vector and 110 LDS instructions a row between them.
+// is bound by the launch, the loads and the stores, with 1190 vector and 142 LDS instructions a row between them (SQ_INSTS_VALU, SQ_INSTS_LDS; the LDS is busy for 760 clocks a row,
+// 6 us in all, half of them where counters of one bank meet).
 #include <hip/hip_runtime.h>
 
 #include "common.hpp"
