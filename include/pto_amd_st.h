@@ -24,7 +24,8 @@ int pto_gemm_f16f32_ks_variant(void *stream, float *c, const uint16_t *a, const 
 /* MX GEMM: variant 0 .. 3: bit 0 = quarter tiles in the last round, bit 1 = the shallower copy pipeline (csrc/pto_gemm_mx.hip);
  * 4 = what the public entry points pick; 5, 6 = the four-wave kernel with 256 x 192, 256 x 128 tiles, 13 .. 16 = with 256 x 256, 96, 160 and 224
  * (csrc/pto_gemm_mxw4_*.hip);
- * 7 .. 12 = eight wavefronts, k split over two groups: 64 x 64, 64 x 128, 128 x 64, 128 x 128, 128 x 192, 192 x 128 tiles
+ * 7 .. 12 = eight wavefronts, k split over two groups: 64 x 64, 64 x 128, 128 x 64, 128 x 128, 128 x 192, 192 x 128 tiles, 17 and 18 = the
+ * same on two and four: 32 x 32, 32 x 64
  * (csrc/pto_gemm_mxks.hip) */
 int pto_gemm_mxfp8_variant(void *stream, void *c, const uint8_t *a, const uint8_t *b, const uint8_t *scale_a,
                            const uint8_t *scale_b, int m, int n, int k, int format, int c_fp32, int variant);

@@ -1,8 +1,12 @@
-// MXFP8 / MXFP4 GEMM tiles of 64 .. 192 rows for problems that the 256-row tiles of gemm_kernels_mxw4.hpp leave compute units
+// MXFP8 / MXFP4 GEMM tiles of 32 .. 192 rows for problems that the 256-row tiles of gemm_kernels_mxw4.hpp leave compute units
 // idle on: the kernel of gemm_kernels_ks.hpp (eight wavefronts in a 2 x 2 x 2 grid, rows x columns x k) on MX operands.  A
 // K-step is again 128 bytes of every row; group g multiplies bytes 64 g .. 64 g + 63 of them: one v_mfma_scale_f32_32x32x64
 // (fp8: 64 k, 16 passes) or two (fp4: 128 k, 8 passes each) per 32 x 32 block.  Copies, stages and the meeting of the two
 // partial sums are those of the fp16 kernel.
+//
+// 32 x 32 tiles are two wavefronts, one for each half of k, and 32 x 64 ones four: a unit's copies bound a step, so products of few tiles gain by
+// smaller ones on more units.  64 x 64 -> 32 x 32 (launched from a graph): 512^3 fp8 4.25 -> 3.58 us, fp4 4.09 -> 3.49; 256 x 256 x 6144 12.6 -> 9.6, 8.2 -> 6.4;
+// 64 x 64 -> 32 x 64: 256 x 1536 x 2048 5.80 -> 4.92, 5.26 -> 4.55.  Six and eight stages for them: 512 x 512 x 2048 fp8 4.51 -> 5.03 and 5.16, only from k = 4096 on up to 11 % faster.
 //
 // Scales.  32 bytes of a row's scales last P = 8 steps (fp8) or 4 (fp4); they come into one of two LDS buffers with one or two
 // copy instructions per wave and period (two lanes per row), a period ahead.  A lane's MFMA operand needs the scale of its own
@@ -50,26 +54,31 @@ constexpr int MxKsLdsBytes() // S stages of 128-byte rows, two buffers of 32 sca
     return stages > sums ? stages : sums;
 }
 
+// wavefronts of a tile: at most two by two of 32 rows and columns and more, times two groups of k
+constexpr int MxKsGrid(int extent) { return extent < 64 ? 1 : 2; }
+constexpr int MxKsWaves(int bm, int bn) { return 2 * MxKsGrid(bm) * MxKsGrid(bn); }
+
 // FMT: 0 = e4m3, 1 = e5m2, 4 = e2m1 (both operands then); ld = bytes of a row of A and B, ldScale = of their scales
 template <int FMT_A, int FMT_B, typename OutT, int BM, int BN, int S, int MIN_WAVES, int GROUP_M>
-__global__ __launch_bounds__(512, MIN_WAVES) AICORE
+__global__ __launch_bounds__(64 * MxKsWaves(BM, BN), MIN_WAVES) AICORE
     void GemmMxKs(__gm__ OutT *out, __gm__ const uint8_t *src0, __gm__ const uint8_t *src1, __gm__ const uint8_t *scale0,
                   __gm__ const uint8_t *scale1, int m, int n, uint32_t ld, uint32_t ldScale, int through)
 {
     constexpr bool FP4 = FMT_A == 4;
     static_assert((FMT_A == 4) == (FMT_B == 4), "fp4 with fp4");
-    constexpr int MB = BM / 64, NB = BN / 64;                       // 32 x 32 blocks of a wave
-    constexpr int kInst = (BM + BN) / 8, kCopies = (kInst + 7) / 8; // copy instructions of 8 rows a step; per wave
-    constexpr int kScaleInst = (BM + BN) / 32, kScaleCopies = (kScaleInst + 7) / 8; // of 32 rows' scales a period; per wave
+    constexpr int WM = MxKsGrid(BM), WN = MxKsGrid(BN), kWaves = MxKsWaves(BM, BN);
+    constexpr int MB = BM / WM / 32, NB = BN / WN / 32;                           // 32 x 32 blocks of a wave
+    constexpr int kInst = (BM + BN) / 8, kCopies = (kInst + kWaves - 1) / kWaves; // copy instructions of 8 rows a step; per wave
+    constexpr int kScaleInst = (BM + BN) / 32, kScaleCopies = (kScaleInst + kWaves - 1) / kWaves; // of 32 rows' scales a period; per wave
     constexpr int kStepScales = FP4 ? 8 : 4, P = 32 / kStepScales;  // scale bytes of a row and step; steps of a period
     constexpr uint32_t kStage = (BM + BN) * 128, kRing = S * kStage, kScaleBuf = (BM + BN) * 32;
     // (S <= P: the wait for step it + P at the top of step it + P - 1 then covers the scales issued in step it)
-    static_assert(BM % 64 == 0 && BN % 64 == 0 && S >= 3 && S <= P, "tile shape");
+    static_assert(BM % (32 * WM) == 0 && BN % (32 * WN) == 0 && S >= 3 && S <= P, "tile shape");
 
     int tm, tn;
     TileOfBlock<GROUP_M>((int)blockIdx.x, (m + BM - 1) / BM, (n + BN - 1) / BN, tm, tn);
     const int row0 = tm * BM, col0 = tn * BN;
-    const int wave = hw::wave(), group = wave >> 2, wm = (wave >> 1) & 1, wn = wave & 1;
+    const int wave = hw::wave(), group = wave / (WM * WN), wm = wave / WN % WM, wn = wave % WN;
     const uint32_t lane = (uint32_t)hw::lane();
     const uint32_t ldsBase = (uint32_t)(uintptr_t)hw::lds_base();
     const int steps = (int)(ld / 128); // a multiple of Q
@@ -79,7 +88,7 @@ __global__ __launch_bounds__(512, MIN_WAVES) AICORE
     uint32_t off[kCopies], lds[kCopies];
 #pragma unroll
     for (int j = 0; j < kCopies; ++j) {
-        const int i = 8 * j + wave < kInst ? 8 * j + wave : kInst - 1;
+        const int i = kWaves * j + wave < kInst ? kWaves * j + wave : kInst - 1;
         const bool isA = i < BM / 8;
         const int first = isA ? row0 + 8 * i : col0 + 8 * (i - BM / 8), last = (isA ? m : n) - 1;
         const int row = first + (int)(lane / 8) < last ? first + (int)(lane / 8) : last;
@@ -100,7 +109,7 @@ __global__ __launch_bounds__(512, MIN_WAVES) AICORE
     const uint32_t scaleChunk = ((lane % 2) ^ (lane / 16 % 2)) * 16u;
 #pragma unroll
     for (int j = 0; j < kScaleCopies; ++j) {
-        const int i = (8 * j + wave) % kScaleInst;
+        const int i = (kWaves * j + wave) % kScaleInst;
         const bool isA = i < BM / 32;
         const int first = isA ? row0 + 32 * i : col0 + 32 * (i - BM / 32), last = (isA ? m : n) - 1;
         const int row = first + (int)(lane / 2) < last ? first + (int)(lane / 2) : last;
@@ -126,8 +135,8 @@ __global__ __launch_bounds__(512, MIN_WAVES) AICORE
     for (int q = 0; q < 2; ++q) {
         const uint32_t chunk = (uint32_t)group * 4u + (FP4 ? 2u * h + (uint32_t)q : h + 2u * (uint32_t)q);
         const uint32_t fragOff = r32 * 128u + ((chunk ^ ((r32 / 2) % 8)) * 16u);
-        aAddr[q] = ldsBase + (uint32_t)(wm * (BM / 2)) * 128u + fragOff;
-        bAddr[q] = ldsBase + (uint32_t)(BM + wn * (BN / 2)) * 128u + fragOff;
+        aAddr[q] = ldsBase + (uint32_t)(wm * (BM / WM)) * 128u + fragOff;
+        bAddr[q] = ldsBase + (uint32_t)(BM + wn * (BN / WN)) * 128u + fragOff;
     }
     // The 16 scale bytes of a row that last Q steps (4 of fp8, 2 of fp4) come into registers with one read per block; those of
     // step t among them are bytes 4 t + 2 group + h (fp8), 8 t + 4 group + 2 h and the next (fp4).
@@ -152,7 +161,7 @@ __global__ __launch_bounds__(512, MIN_WAVES) AICORE
     };
     auto readScales = [&](int it) __attribute__((always_inline)) { // of steps it .. it + Q - 1
         const uint32_t addr = (scaleLane ^ (uint32_t)((it / Q % 2) * 16)) + ldsBase + kRing + (uint32_t)((it / P) & 1) * kScaleBuf;
-        const uint32_t saAddr = addr + (uint32_t)(wm * (BM / 2)) * 32u, sbAddr = addr + (uint32_t)(BM + wn * (BN / 2)) * 32u;
+        const uint32_t saAddr = addr + (uint32_t)(wm * (BM / WM)) * 32u, sbAddr = addr + (uint32_t)(BM + wn * (BN / WN)) * 32u;
         StaticFor<0, NB>([&](auto i) __attribute__((always_inline)) { scales[MB + decltype(i)::value] = KsLdsRead16<decltype(i)::value * 1024>(sbAddr); });
         StaticFor<0, MB>([&](auto i) __attribute__((always_inline)) { scales[decltype(i)::value] = KsLdsRead16<decltype(i)::value * 1024>(saAddr); });
     };
@@ -245,7 +254,7 @@ __global__ __launch_bounds__(512, MIN_WAVES) AICORE
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
     char *sums = hw::lds_base();
-    const int pair = wave & 3;
+    const int pair = wave % (WM * WN);
     constexpr int kQuads = MB * NB * 4, kKept = kQuads / 2;
     auto quad = [&](auto qTag) __attribute__((always_inline)) {
         constexpr int idx = decltype(qTag)::value / 4, r = 4 * (decltype(qTag)::value % 4);
@@ -266,7 +275,7 @@ __global__ __launch_bounds__(512, MIN_WAVES) AICORE
     };
     // Two quads side by side change lanes: then a store instruction writes 64 bytes of fp32 of each of 16 rows, or 32 of bf16 (eight columns
     // a lane) of 32 rows, and with the block's other two quads 64 of bf16 of 16 rows.
-    const int rowLane = row0 + wm * (BM / 2), colLane = col0 + wn * (BN / 2);
+    const int rowLane = row0 + wm * (BM / WM), colLane = col0 + wn * (BN / WN);
     auto words = [](const ks_f32x4 &v) __attribute__((always_inline)) { return __builtin_bit_cast(Words4, v); };
     StaticFor<0, 2>([&](auto gTag) __attribute__((always_inline)) {
         constexpr int g = decltype(gTag)::value;
@@ -360,7 +369,7 @@ int launch_gemm_mxks(hipStream_t st, void *c, const uint8_t *a, const uint8_t *b
     const long long tiles = (long long)((m + BM - 1) / BM) * ((n + BN - 1) / BN);
     if (tiles > 0x7fffffffll)
         return PTO_ERR_UNSUPPORTED;
-    kernel<<<dim3((unsigned)tiles), dim3(512), lds, st>>>(reinterpret_cast<OutT *>(c), a, b, sa, sb, m, n, (uint32_t)(FMT_A == 4 ? k / 2 : k),
+    kernel<<<dim3((unsigned)tiles), dim3(64 * MxKsWaves(BM, BN)), lds, st>>>(reinterpret_cast<OutT *>(c), a, b, sa, sb, m, n, (uint32_t)(FMT_A == 4 ? k / 2 : k),
                                                           (uint32_t)(k / 32), pto_amd::store_through(c, sizeof(OutT) * (uint64_t)n, sizeof(OutT) * (uint64_t)m * n));
     return pto_amd::check_launch();
 }

@@ -348,7 +348,7 @@ int gemm_mx_dispatch(hipStream_t st, void *c, const uint8_t *a, const uint8_t *b
 
 namespace {
 // Three kernels: 256 x 256 tiles on eight wavefronts (this file; quarter tiles in a last partial round), tiles of 256 rows and 96 to 256
-// columns on four (pto_gemm_mxw4_*.hip), and tiles of 64 .. 192 rows with k split over two groups of wavefronts
+// columns on four (pto_gemm_mxw4_*.hip), and tiles of 32 .. 192 rows with k split over two groups of wavefronts
 // (pto_gemm_mxks.hip).  What a problem takes with one tile shape, in microseconds, launch included: tiles are dealt to the
 // compute units, `more` rounds beyond the first, `share` of the units busy in the last one, steps of 128 bytes,
 //   time = fixed + per_round more + steps (step + step_round more + step_share share) + (per_mega + fp32 result: per_mega_f32) (4e-6 m n);
@@ -372,7 +372,10 @@ struct MxShape {
 // 256 x 96, 160 and 224: fitted to 300 problems of 0.7 million results and more each in fp8 and fp4, compared where the last round is 70 % full and taken 2 % dearer: for 61 of the
 // 300 by 7 % (fp8) and 53 by 9 % (fp4) on average, for one of either more than 2 % slower (5 and 7 %).  5632 x 1536 x 512 fp8 to fp32 on 256 x 160 tiles -16 %,
 // 3840 x 1536 x 1024 fp4 on 256 x 96 -15 %, 7424 x 3584 x 7168 fp8 on 256 x 224 -17 %.
-constexpr MxShape kMxShapes[2][13] = {
+// 32 x 32 and 32 x 64 with k split: fitted to 249 problems of up to 1.3 million results each in fp8 and fp4, both results (256 x 256 x 512 .. 1400 x 1000 x 7168), taken 3 % dearer and up to the
+// five rounds of that fit: for 303 of 498 by 17 % (fp8) and 255 by 15 % (fp4) on average, for one 3 % slower (512 x 1024 x 2048 fp8).  512^3 fp8 4.25 -> 3.58 us, 256 x 256 x 6144
+// 12.6 -> 9.6, 256 x 1536 x 2048 5.8 -> 4.9; fp4 4.1 -> 3.5, 8.2 -> 6.4, 5.3 -> 4.6; past their two rounds the larger ones are faster (1024^3 fp8 64 x 64 5.1, 32 x 64 5.8, 32 x 32 6.4).
+constexpr MxShape kMxShapes[2][15] = {
     {{MxShape::kW4, 0, 256, 96, 4.642, 1.735, 0.532, 0.751, 0.065, 0.144, 0.101},
      {MxShape::kW4, 0, 256, 160, 7.914, 5.683, 0.436, 0.980, 0.024, 0.535, 0.069},
      {MxShape::kW4, 0, 256, 224, 8.683, 6.830, 0.837, 1.359, 0.000, 0.492, 0.075},
@@ -385,7 +388,9 @@ constexpr MxShape kMxShapes[2][13] = {
      {MxShape::kKs, 2, 128, 64, 3.318, 1.545, 0.284, 0.315, 0.201, 0.039, 0.036},
      {MxShape::kKs, 3, 128, 128, 4.635, 2.138, 0.354, 0.508, 0.146, 0.110, 0.048},
      {MxShape::kKs, 4, 128, 192, 5.785, 2.957, 0.481, 0.728, 0.124, 0.168, 0.059},
-     {MxShape::kKs, 5, 192, 128, 5.833, 2.802, 0.482, 0.730, 0.129, 0.170, 0.056}}, // fp8
+     {MxShape::kKs, 5, 192, 128, 5.833, 2.802, 0.482, 0.730, 0.129, 0.170, 0.056},
+     {MxShape::kKs, 6, 32, 32, 2.750, 0.419, 0.117, 0.066, 0.000, 0.032, 0.081},
+     {MxShape::kKs, 7, 32, 64, 2.922, 0.785, 0.120, 0.124, 0.000, 0.082, 0.086}}, // fp8
     {{MxShape::kW4, 0, 256, 96, 5.728, 3.703, 0.484, 0.757, 0.000, 0.394, 0.113},
      {MxShape::kW4, 0, 256, 160, 8.388, 4.324, 0.510, 1.238, 0.000, 0.644, 0.094},
      {MxShape::kW4, 0, 256, 224, 7.526, 7.963, 1.089, 1.412, 0.000, 0.701, 0.098},
@@ -398,7 +403,9 @@ constexpr MxShape kMxShapes[2][13] = {
      {MxShape::kKs, 2, 128, 64, 3.647, 2.183, 0.294, 0.356, 0.147, 0.100, 0.038},
      {MxShape::kKs, 3, 128, 128, 4.723, 2.682, 0.406, 0.591, 0.136, 0.166, 0.045},
      {MxShape::kKs, 4, 128, 192, 5.718, 3.475, 0.547, 0.827, 0.125, 0.234, 0.054},
-     {MxShape::kKs, 5, 192, 128, 5.765, 3.304, 0.543, 0.883, 0.122, 0.257, 0.056}}, // fp4
+     {MxShape::kKs, 5, 192, 128, 5.765, 3.304, 0.543, 0.883, 0.122, 0.257, 0.056},
+     {MxShape::kKs, 6, 32, 32, 3.162, 0.265, 0.121, 0.075, 0.000, 0.035, 0.076},
+     {MxShape::kKs, 7, 32, 64, 3.255, 0.578, 0.136, 0.119, 0.000, 0.073, 0.101}}, // fp4
 };
 // fp8, fp4: the round of 128 x 128 quarter tiles, fixed and a step; `ragged`
 constexpr double kMxQuarter[2] = {0.000, 4.513}, kMxStepQuarter[2] = {0.830, 0.753}, kMxStepRagged[2] = {0.080, 0.125};
@@ -418,8 +425,8 @@ int gemm_mx_any(hipStream_t st, void *c, const uint8_t *a, const uint8_t *b, con
             continue;
         const long long tiles = (long long)((m + s.bm - 1) / s.bm) * ((n + s.bn - 1) / s.bn), rest = tiles % cus;
         double more = (double)((tiles - 1) / cus), share = (double)((tiles - 1) % cus + 1) / cus, extra = 0.0;
-        const bool wide = s.kernel == MxShape::kW4 && s.bn == 256, between = s.kernel == MxShape::kW4 && s.bn % 64 == 32;
-        if ((wide && share < 0.78) || (between && share < 0.70))
+        const bool wide = s.kernel == MxShape::kW4 && s.bn == 256, between = s.kernel == MxShape::kW4 && s.bn % 64 == 32, small = s.bm == 32;
+        if ((wide && share < 0.78) || (between && share < 0.70) || (small && more > 4.0))
             continue;
         if (s.kernel == MxShape::kBlock && !(m % 256 == 0 && n % 256 == 0)) {
             extra = steps * kMxStepRagged[fp4] * (more + 1.0);
@@ -430,7 +437,7 @@ int gemm_mx_any(hipStream_t st, void *c, const uint8_t *a, const uint8_t *b, con
         }
         const double time = (s.fixed + s.perRound * more + steps * (s.step + s.stepRound * more + s.stepShare * share) +
                              (s.perMega + (c_fp32 ? s.perMegaF32 : 0.0)) * (4e-6 * m * n) + extra) *
-                            (s.kernel == MxShape::kKs || between ? 1.02 : s.kernel == MxShape::kBlock || wide ? 1.03 : 1.0);
+                            (s.kernel == MxShape::kBlock || wide || small ? 1.03 : s.kernel == MxShape::kKs || between ? 1.02 : 1.0);
         if (best == nullptr || time < bestTime) {
             best = &s;
             bestTime = time;
@@ -468,8 +475,10 @@ extern "C" int pto_gemm_mxfp4(void *stream, void *c, const uint8_t *a, const uin
 extern "C" int pto_gemm_mxfp8_variant(void *stream, void *c, const uint8_t *a, const uint8_t *b, const uint8_t *scale_a,
                                       const uint8_t *scale_b, int m, int n, int k, int format, int c_fp32, int variant)
 {
-    if (!c || !a || !b || !scale_a || !scale_b || m <= 0 || n <= 0 || k <= 0 || variant < 0 || variant > 16)
+    if (!c || !a || !b || !scale_a || !scale_b || m <= 0 || n <= 0 || k <= 0 || variant < 0 || variant > 18)
         return PTO_ERR_BAD_ARG;
+    if (variant >= 17) // 32 x 32 and 32 x 64 with k split
+        return pto_amd::gemm_mx_ks(static_cast<hipStream_t>(stream), c, a, b, scale_a, scale_b, m, n, k, format, c_fp32, variant - 11);
     if (variant >= 13) // further widths on four wavefronts: 256, 96, 160, 224
         return pto_amd::gemm_mx_w4(static_cast<hipStream_t>(stream), c, a, b, scale_a, scale_b, m, n, k, format, c_fp32,
                                    variant == 13 ? 256 : variant == 14 ? 96 : variant == 15 ? 160 : 224);

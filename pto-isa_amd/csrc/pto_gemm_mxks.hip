@@ -1,4 +1,4 @@
-// The 64- to 192-row MXFP8 / MXFP4 GEMM tiles with k split over two groups of wavefronts (gemm_kernels_mxks.hpp).
+// The 32- to 192-row MXFP8 / MXFP4 GEMM tiles with k split over two groups of wavefronts (gemm_kernels_mxks.hpp).
 #define PTO_WAVES_M 4
 #define PTO_WAVES_N 1
 #define PTO_MFMA_M 16
@@ -15,6 +15,8 @@ int launch_shape(hipStream_t st, void *c, const uint8_t *a, const uint8_t *b, co
     case 3: return launch_gemm_mxks<FMT_A, FMT_B, OutT, 128, 128, 4, 2>(st, c, a, b, sa, sb, m, n, k);
     case 4: return launch_gemm_mxks<FMT_A, FMT_B, OutT, 128, 192, 3, 2>(st, c, a, b, sa, sb, m, n, k);
     case 5: return launch_gemm_mxks<FMT_A, FMT_B, OutT, 192, 128, 3, 2>(st, c, a, b, sa, sb, m, n, k);
+    case 6: return launch_gemm_mxks<FMT_A, FMT_B, OutT, 32, 32, 4, 2>(st, c, a, b, sa, sb, m, n, k);
+    case 7: return launch_gemm_mxks<FMT_A, FMT_B, OutT, 32, 64, 4, 2>(st, c, a, b, sa, sb, m, n, k);
     default: return PTO_ERR_UNSUPPORTED;
     }
 }

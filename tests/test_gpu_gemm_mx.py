@@ -443,3 +443,37 @@ def test_mx_gemm_whatever_tile_the_entry_point_takes(fmt, m, n):
     rc, got = _mx_variant(a, b, sa, sb, fmt, 4)
     rc6, want = _mx_variant(a, b, sa, sb, fmt, 6)
     assert rc == 0 and rc6 == 0 and np.array_equal(got, want)
+
+
+@pytest.mark.parametrize("fmt,m,n,k", [(0, 32, 32, 512), (1, 260, 300, 2048), (2, 257, 96, 1536), (3, 33, 516, 4608), (4, 32, 64, 512), (4, 300, 516, 1024), (4, 31, 100, 1536),
+                                       (4, 257, 260, 5120)])
+@pytest.mark.parametrize("variant", [17, 18])
+def test_mx_gemm_tiles_of_32_rows(oracle, variant, fmt, m, n, k):
+    """32 x 32 and 32 x 64 tiles with k split.  One tile, less than one, rows and columns past the edge; less than a scale period (1024 k of fp8, 1024 of fp4), whole ones and a part: every scale of
+    either operand exactly, integer operands exactly, the generator's distribution to the GEMM tolerance, the bf16 result = RNE of the fp32 one."""
+    fa, fb = {2: (0, 1), 3: (1, 0)}.get(fmt, (fmt, fmt))
+    rng = np.random.default_rng(k + m)
+    ones = {0: 0x38, 1: 0x3C, 4: 0x22}
+    width = k // 2 if fmt == 4 else k
+    a, b = np.full((m, width), ones[fa], dtype=np.uint8), np.full((n, width), ones[fb], dtype=np.uint8)
+    sa, sb = (rng.integers(125, 131, size=(r, k // 32)).astype(np.uint8) for r in (m, n))
+    rc, got = _mx_variant(a, b, sa, sb, fmt, variant)
+    capi.check(rc, "k-split MX kernel")
+    assert np.array_equal(got.astype(np.float64), 32.0 * (np.exp2(sa.astype(np.float64) - 127) @ np.exp2(sb.astype(np.float64) - 127).T))
+    for dist in ("integer", "bytes"):
+        (a, _, sa, sb), (_, b, _, _) = (datagen.mx_inputs(m, n, k, f, dist=dist) for f in (fa, fb))
+        rc, got = _mx_variant(a, b, sa, sb, fmt, variant)
+        want = oracle.mx_gemm(a, b, sa, sb, fa, fb)
+        assert rc == 0 and (np.array_equal(got, want) if dist == "integer" else np.all(np.isfinite(got)) and rel_err(got, want) <= TOL), dist
+        rc, got16 = _mx_variant(a, b, sa, sb, fmt, variant, c_fp32=False)
+        assert rc == 0 and np.array_equal(got16, bf16_rne(got))
+
+
+@pytest.mark.parametrize("fmt", [0, 4])
+@pytest.mark.parametrize("m,n,k", [(256, 256, 512), (512, 512, 2048), (256, 1536, 2048), (700, 700, 1536), (333, 260, 6144)])
+def test_mx_gemm_few_tiles_through_the_entry_point(fmt, m, n, k):
+    """Where 32-row tiles are taken, or nearly: integer operands, the result of the 64 x 64 tiles."""
+    a, b, sa, sb = datagen.mx_inputs(m, n, k, fmt, dist="integer") if fmt != 4 else datagen.mx_inputs(m, n, k, fmt)
+    rc, got = _mx_variant(a, b, sa, sb, fmt, 4)
+    rc7, want = _mx_variant(a, b, sa, sb, fmt, 7)
+    assert rc == 0 and rc7 == 0 and np.array_equal(got, want)
