@@ -319,9 +319,11 @@ __device__ inline void WaveEnds(float &hi, float &lo)
 // and its smallest one, the keys in each are counted, sums over the counts say where a bucket begins, every key goes to the next place of its
 // bucket in a list, and neighbours change places (odd and even pairs in turn) as often as the fullest bucket has keys (5 to 9 of 1024 random scores).
 // 2 N counters of 16 bits: with N of them buckets hold twice as many keys.  Which rows: any whose scores are finite and not crowded in a small part of
-// their range; the others (masked with infinities, nearly all equal, heavy tails) are found by a look at 64 scores that takes them 1 to 6 % of their time
-// (us, network / with the look before it / buckets of random scores: 4800 x 1024, top 1000 21.0 / 21.9 / 14.2; 9000 x 512 whole 16.7 / 17.8 / 11.3;
-// 1500 x 1000, top 900 10.1 / 10.2 / 7.8; 1600 x 2048 20.9 / 21.1 / 11.5; 1 x 4096 12.5 / 12.7 / 7.9).  Tried for them and slower than the network: 64 of the row's own scores,
+// their range; the others go through the network, found by a look at 64 scores of each wave before anything is counted (masked with infinities, half zeros, squares,
+// exponentials), or by the count before anything is scattered (forty close scores among spread ones, a twentieth equal).  Microseconds, network / turned away by the look /
+// by the count / buckets of normal scores: 4800 x 1024, top 1000 21.5 / 22.7 / 25.3 / 15.6; 2400 x 1024 14.2 / 14.5 / 16.3 / 9.9; 600 x 1024 7.4 / 7.8 / 8.8 / 5.9; 1600 x 2048
+// 21.5 / 22.0 / 24.4 / 12.2; 9000 x 512 17.5 / 18.7 / 21.0 / 12.1; 1200 x 4096 34.0 / 35.8 / 39.9 / 20.0; 16 x 4096 13.1 / 13.7 / 16.3 / 8.6 (a count that is found wanting only
+// behind the scatter and a pass took 1.25 to 1.4 times the network's, up to 1.8 where the look saw less).  Tried for them and slower than the network: 64 of the row's own scores,
 // sorted, as the limits of ranges that are spread evenly each (4800 x 1024 27 us).  512 columns in up to 731 rows stay with the network (4.2 us; by
 // buckets 4.5 in two waves a row, 4.5 in one), as do 256 and less.
 // bits[e]: the score in column i0 + 64 e; afterwards key e of the lane with number q = 64 (wave of the row) + lane is of rank q E + e.
@@ -341,9 +343,8 @@ enum Counted { kSorted, kNothingDone, kLost }; // kNothingDone: scores too uneve
 template <int E, int W>
 struct BucketSort {
     static constexpr int N = 64 * E * W, kLogN = __builtin_ctz(N);
-    static constexpr int kCrowd = 6;   // of 64 scores, in a 512th of the range: the fullest bucket would have some 24 keys
-    static constexpr int kSurely = 16; // keys in a bucket up to which all passes are made without a look whether they are needed
-    static constexpr int kMost = 32;   // and with one; more only where they are in order by themselves (equal ones)
+    static constexpr int kCrowd = 10; // of 64 scores, in a 128th of the range
+    static constexpr int kSurely = 16, kMost = E == 4 ? 16 : E == 8 ? 24 : 48; // keys in a bucket: up to kMost by neighbours; more than kSurely may be equal ones
     double k[E];
 
     static __device__ inline void Meet()
@@ -358,6 +359,24 @@ struct BucketSort {
     // where place p of the list (and word w of the counters, four at a time) stands, so that lanes E apart meet in no bank
     static __device__ inline uint32_t Place(uint32_t p) { return p ^ ((p >> 5) & (uint32_t)(E - 1)); }
     static __device__ inline uint32_t Word(uint32_t w) { return w ^ ((w >> 4) & (uint32_t)(E - 4)); }
+    // how many scores are equal to the one 64 columns on, in the row (more than one wave to it: in all rows of the workgroup)
+    static __device__ inline int Equal(const uint32_t (&bits)[E], uint32_t i0, int validCols, [[maybe_unused]] uint32_t *counts)
+    {
+        int n = 0;
+#pragma unroll
+        for (int e = 1; e < E; ++e)
+            n += __builtin_popcountll(__builtin_amdgcn_ballot_w64(bits[e - 1] == bits[e] && i0 + 64u * (uint32_t)e < (uint32_t)validCols));
+        if constexpr (W > 1) {
+            counts[threadIdx.x / 64] = (uint32_t)n;
+            __syncthreads();
+            n = 0;
+#pragma unroll
+            for (int w = 0; w < kTopkWaves; ++w)
+                n += (int)counts[w];
+            n = __builtin_amdgcn_readfirstlane(n);
+        }
+        return n;
+    }
     // the neighbours' keys across the lanes' borders: the first key of the lane above, the last one of the lane below
     __device__ inline void Neighbours(double &above, double &below, int waveOfRow, int lane, uint64_t *edges)
     {
@@ -399,19 +418,23 @@ struct BucketSort {
         }
         WaveEnds(top, low);
         float range = top - low;
-        // a look at 64 scores (two columns in turn of either half) of each wave before anything else is done: how many are near either of two of them
+        // a look at 64 scores of each wave (four columns in turn, a quarter of its columns apart) before anything else is done: how many are near the ends of the
+        // range, or near either of two of them
         bool even = (range >= 1e-30f) & (range <= 1e37f);
         {
-            uint32_t seen = bits[0], half = bits[E / 2];
-            asm("" : "+v"(half)); // (else the choice is made between their addresses, and bits put into memory)
-            seen = (lane & 1) ? half : seen;
+            uint32_t second = bits[E / 4], fourth = bits[3 * E / 4];
+            asm("" : "+v"(second), "+v"(fourth)); // (else the choice is made between their addresses, and bits put into memory)
+            uint32_t seen = (lane & 1) ? second : bits[0], further = (lane & 1) ? fourth : bits[E / 2];
+            asm("" : "+v"(further));
+            seen = (lane & 2) ? further : seen;
             if (validCols != N) // (what stands behind the last column is near nothing)
-                seen = i0 + ((lane & 1) ? 32u * E : 0u) < (uint32_t)validCols ? seen : 0x7fffffffu;
+                seen = i0 + 16u * E * ((uint32_t)lane & 3u) < (uint32_t)validCols ? seen : 0x7fffffffu;
+            const float x = __builtin_bit_cast(float, seen);
+            auto few = [&](float distance, float within) __attribute__((always_inline)) { return __builtin_popcountll(__builtin_amdgcn_ballot_w64(distance <= range * within)) < kCrowd; };
+            even &= few(top - x, 1.0f / 128.0f) & few(x - low, 1.0f / 128.0f);
 #pragma unroll
-            for (int g = 0; g < 2; ++g) {
-                const float one = __builtin_bit_cast(float, __builtin_amdgcn_readlane((int)seen, g == 0 ? 9 : 38));
-                even &= __builtin_popcountll(__builtin_amdgcn_ballot_w64(__builtin_fabsf(__builtin_bit_cast(float, seen) - one) <= range * (1.0f / 1024.0f))) < kCrowd;
-            }
+            for (int g = 0; g < 2; ++g)
+                even &= few(__builtin_fabsf(x - __builtin_bit_cast(float, __builtin_amdgcn_readlane((int)seen, g == 0 ? 9 : 38))), 1.0f / 256.0f);
             if (validCols != N) // (a wave that has nothing behind the last column)
                 even = even || (int)i0 - lane + 64 >= validCols;
         }
@@ -508,9 +531,19 @@ struct BucketSort {
             for (int j = 0; j < E / 4; ++j)
                 mine[chunk(j)] = make_uint4(c[4 * j], c[4 * j + 1], c[4 * j + 2], c[4 * j + 3]);
         }
+        // Many keys in a bucket: few distinct scores, whose equal ones will stand in order by themselves, or too many to be exchanged.  D scores alike in number
+        // bring some N / D pairs of equal ones 64 columns apart, most of what the fullest bucket has keys; a part f of the row that is equal, with other
+        // scores among it in the bucket, f times that bucket's; distinct ones none.  (64, and a sixth: where keys and pairs are few and vary by chance)
+        bool equal = false;
+        if (full > (uint32_t)kSurely) {
+            const int same = Equal(bits, i0, validCols, across + 2 * kTopkWaves) / (W > 1 ? kTopkWaves / W : 1);
+            equal = 6 * same >= (int)full && 3 * same + 64 >= 2 * (int)full;
+            if (!equal && full > (uint32_t)kMost)
+                return kNothingDone;
+        }
         Meet();
         // every key to the next place of its bucket.  (Equal scores in many columns: wave after wave, so that they are not in disorder)
-        const int turns = W > 1 && full > (uint32_t)kSurely ? W : 1;
+        const int turns = W > 1 && equal ? W : 1;
         for (int turn = 0; turn < turns; ++turn) {
             if (turns == 1 || turn == waveOfRow) {
 #pragma unroll
@@ -544,23 +577,9 @@ struct BucketSort {
         for (int e = 0; e < E; ++e)
             k[e] = __builtin_bit_cast(double, list[Place(q * E + (uint32_t)e)]);
         Meet();
-        const int passes = full <= (uint32_t)kMost ? (int)(full + 1u) / 2 : 1;
-        for (int pass = 0;; ++pass) { // (two places for the edges in turn, and two others for the look)
-            double above, below;
-            if (full <= (uint32_t)kSurely) {
-                if (pass == passes)
-                    return kSorted;
-            } else {
-                Neighbours(above, below, waveOfRow, lane, list + (pass & 1) * 16 + 8);
-                bool sorted = k[E - 1] >= above;
-#pragma unroll
-                for (int e = 1; e < E; ++e)
-                    sorted = sorted & (k[e - 1] >= k[e]);
-                if (W > 1 ? Everyone(sorted, across + (2 + (pass & 1)) * kTopkWaves) : WholeWave(sorted))
-                    return kSorted;
-                if (pass == passes)
-                    return kLost;
-            }
+        double above, below;
+        const int passes = equal ? 0 : (int)(full + 1u) / 2;
+        for (int pass = 0; pass < passes; ++pass) { // (two places for the edges in turn)
 #pragma unroll
             for (int e = 0; e < E; e += 2)
                 Exchange(k[e], k[e + 1]);
@@ -571,6 +590,16 @@ struct BucketSort {
             k[E - 1] = Max(k[E - 1], above);
             k[0] = Min(k[0], below);
         }
+        if (equal) {
+            Neighbours(above, below, waveOfRow, lane, list);
+            bool sorted = k[E - 1] >= above;
+#pragma unroll
+            for (int e = 1; e < E; ++e)
+                sorted = sorted & (k[e - 1] >= k[e]);
+            if (W > 1 ? !Everyone(sorted, across + 3 * kTopkWaves) : !WholeWave(sorted))
+                return kLost;
+        }
+        return kSorted;
     }
 };
 template <int E, int W, bool LOW_DPP, Mode MODE>
