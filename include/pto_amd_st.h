@@ -21,6 +21,9 @@ int pto_gemm_f16f32_variant(void *stream, float *c, const uint16_t *a, const uin
 int pto_gemm_f16f32_w4_variant(void *stream, float *c, const uint16_t *a, const uint16_t *b, int m, int n, int k, int variant);
 /* eight wavefronts, k split over two groups: tile shapes by number (csrc/pto_gemm_ks.hip) */
 int pto_gemm_f16f32_ks_variant(void *stream, float *c, const uint16_t *a, const uint16_t *b, int m, int n, int k, int variant);
+/* the entry point's choice for `units` compute units, without a launch: the shape's place in the list of csrc/pto_gemm.hip; expected[17], or null: the time
+ * of each of them, an infinity where it does not take the problem */
+int pto_gemm_f16f32_choice(int m, int n, int k, int units, double *expected);
 /* MX GEMM: variant 0 .. 3: bit 0 = quarter tiles in the last round, bit 1 = the shallower copy pipeline (csrc/pto_gemm_mx.hip);
  * 4 = what the public entry points pick; 5, 6 = the four-wave kernel with 256 x 192, 256 x 128 tiles, 13 .. 16 = with 256 x 256, 96, 160 and 224
  * (csrc/pto_gemm_mxw4_*.hip);

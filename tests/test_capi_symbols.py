@@ -42,3 +42,21 @@ def test_argument_validation_needs_no_gpu():
     assert lib.pto_tcvt_f32_f16(0, 0, 0, 0, capi.CAST_RINT) == capi.OK          # empty input: nothing to do
     assert lib.pto_gather_rows(0, 0, 0, 0, 0, 0, 0, 2) == capi.OK
     assert lib.pto_version().startswith(b"pto-amd")
+
+
+def test_gemm_choice_of_a_shape():
+    """The shape that the fp16 product takes is the one of the shortest expected time, whatever is left out on the way to it; few tiles: 32 x 32 ones."""
+    import ctypes
+    import random
+    lib, rng, times = capi.load_st(), random.Random(5), (ctypes.c_double * 17)()
+    for _ in range(4000):
+        m, n, k = (rng.randint(1, 24 if rng.random() < 0.7 else 80) * step for step in (128, 256, 32))
+        if rng.random() < 0.5:  # any rows and columns from 192 and 128 on
+            m, n, k = m + rng.randint(64, 191), n - 4 * rng.randint(0, 31), (k + 127) // 128 * 128
+        units = rng.choice((64, 256, 304))
+        shape = lib.pto_gemm_f16f32_choice(m, n, k, units, times)
+        assert 0 <= shape < 17 and times[shape] == min(times), (m, n, k, units)
+        assert shape == lib.pto_gemm_f16f32_choice(m, n, k, units, None)
+    for m, n, k in ((512, 512, 512), (192, 128, 128), (256, 256, 6144)):
+        assert lib.pto_gemm_f16f32_choice(m, n, k, 256, None) == 0
+    assert lib.pto_gemm_f16f32_choice(191, 128, 128, 256, None) == capi.ERR_UNSUPPORTED
