@@ -32,6 +32,9 @@ int pto_gemm_f16f32_choice(int m, int n, int k, int units, double *expected);
  * (csrc/pto_gemm_mxks.hip) */
 int pto_gemm_mxfp8_variant(void *stream, void *c, const uint8_t *a, const uint8_t *b, const uint8_t *scale_a,
                            const uint8_t *scale_b, int m, int n, int k, int format, int c_fp32, int variant);
+/* the entry points' choice for `units` compute units, without a launch: a variant as above; expected[19], or null: the time of each variant, an infinity where
+ * it does not take the problem or is not one that the entry points choose */
+int pto_gemm_mx_choice(int m, int n, int k, int format, int c_fp32, int units, double *expected);
 /* flash attention: workgroup size, occupancy, queries per wave and MFMA shape by number (csrc/pto_fa.hip: 1 / 2 / 5 = four
  * waves at 1 / 2 / 3 workgroups per compute unit, 6 = key tiles of 32, 8 = 64 queries per wave, 10 / 20 / 21 = eight waves on
  * 32 x 32 x 16 / 16 x 16 x 32 MFMAs / the latter with fp32 output); causal != 0: the diagonal ends in the last key */

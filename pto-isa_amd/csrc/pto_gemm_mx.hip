@@ -375,59 +375,63 @@ struct MxShape {
 // 32 x 32 and 32 x 64 with k split: fitted to 249 problems of up to 1.3 million results each in fp8 and fp4, both results (256 x 256 x 512 .. 1400 x 1000 x 7168), taken 3 % dearer and up to the
 // five rounds of that fit: for 303 of 498 by 17 % (fp8) and 255 by 15 % (fp4) on average, for one 3 % slower (512 x 1024 x 2048 fp8).  512^3 fp8 4.25 -> 3.58 us, 256 x 256 x 6144
 // 12.6 -> 9.6, 256 x 1536 x 2048 5.8 -> 4.9; fp4 4.1 -> 3.5, 8.2 -> 6.4, 5.3 -> 4.6; past their two rounds the larger ones are faster (1024^3 fp8 64 x 64 5.1, 32 x 64 5.8, 32 x 32 6.4).
-constexpr MxShape kMxShapes[2][15] = {
-    {{MxShape::kW4, 0, 256, 96, 4.642, 1.735, 0.532, 0.751, 0.065, 0.144, 0.101},
-     {MxShape::kW4, 0, 256, 160, 7.914, 5.683, 0.436, 0.980, 0.024, 0.535, 0.069},
-     {MxShape::kW4, 0, 256, 224, 8.683, 6.830, 0.837, 1.359, 0.000, 0.492, 0.075},
-     {MxShape::kBlock, 0, 256, 256, 6.233, 4.744, 0.882, 1.791, 0.025, 0.728, 0.076},
-     {MxShape::kW4, 0, 256, 256, 9.531, 8.670, 0.647, 1.435, 0.000, 0.784, 0.075},
-     {MxShape::kW4, 0, 256, 192, 8.332, 5.596, 0.666, 1.163, 0.062, 0.369, 0.033},
-     {MxShape::kW4, 0, 256, 128, 6.086, 2.935, 0.553, 0.842, 0.093, 0.144, 0.035},
+constexpr int kMxShapeCount = 15;
+constexpr MxShape kMxShapes[2][kMxShapeCount] = {
+    {{MxShape::kKs, 6, 32, 32, 2.750, 0.419, 0.117, 0.066, 0.000, 0.032, 0.081},
+     {MxShape::kKs, 7, 32, 64, 2.922, 0.785, 0.120, 0.124, 0.000, 0.082, 0.086},
      {MxShape::kKs, 0, 64, 64, 2.595, 0.634, 0.196, 0.185, 0.191, 0.051, 0.027},
      {MxShape::kKs, 1, 64, 128, 3.318, 1.592, 0.277, 0.320, 0.188, 0.054, 0.039},
      {MxShape::kKs, 2, 128, 64, 3.318, 1.545, 0.284, 0.315, 0.201, 0.039, 0.036},
      {MxShape::kKs, 3, 128, 128, 4.635, 2.138, 0.354, 0.508, 0.146, 0.110, 0.048},
      {MxShape::kKs, 4, 128, 192, 5.785, 2.957, 0.481, 0.728, 0.124, 0.168, 0.059},
      {MxShape::kKs, 5, 192, 128, 5.833, 2.802, 0.482, 0.730, 0.129, 0.170, 0.056},
-     {MxShape::kKs, 6, 32, 32, 2.750, 0.419, 0.117, 0.066, 0.000, 0.032, 0.081},
-     {MxShape::kKs, 7, 32, 64, 2.922, 0.785, 0.120, 0.124, 0.000, 0.082, 0.086}}, // fp8
-    {{MxShape::kW4, 0, 256, 96, 5.728, 3.703, 0.484, 0.757, 0.000, 0.394, 0.113},
-     {MxShape::kW4, 0, 256, 160, 8.388, 4.324, 0.510, 1.238, 0.000, 0.644, 0.094},
-     {MxShape::kW4, 0, 256, 224, 7.526, 7.963, 1.089, 1.412, 0.000, 0.701, 0.098},
-     {MxShape::kBlock, 0, 256, 256, 5.763, 3.741, 1.024, 2.102, 0.045, 0.821, 0.085},
-     {MxShape::kW4, 0, 256, 256, 9.012, 5.823, 0.809, 2.199, 0.000, 0.939, 0.076},
-     {MxShape::kW4, 0, 256, 192, 8.060, 6.472, 0.880, 1.293, 0.066, 0.435, 0.026},
-     {MxShape::kW4, 0, 256, 128, 6.084, 3.053, 0.645, 0.951, 0.098, 0.213, 0.036},
+     {MxShape::kW4, 0, 256, 96, 4.642, 1.735, 0.532, 0.751, 0.065, 0.144, 0.101},
+     {MxShape::kW4, 0, 256, 160, 7.914, 5.683, 0.436, 0.980, 0.024, 0.535, 0.069},
+     {MxShape::kW4, 0, 256, 224, 8.683, 6.830, 0.837, 1.359, 0.000, 0.492, 0.075},
+     {MxShape::kBlock, 0, 256, 256, 6.233, 4.744, 0.882, 1.791, 0.025, 0.728, 0.076},
+     {MxShape::kW4, 0, 256, 256, 9.531, 8.670, 0.647, 1.435, 0.000, 0.784, 0.075},
+     {MxShape::kW4, 0, 256, 192, 8.332, 5.596, 0.666, 1.163, 0.062, 0.369, 0.033},
+     {MxShape::kW4, 0, 256, 128, 6.086, 2.935, 0.553, 0.842, 0.093, 0.144, 0.035}}, // fp8
+    {{MxShape::kKs, 6, 32, 32, 3.162, 0.265, 0.121, 0.075, 0.000, 0.035, 0.076},
+     {MxShape::kKs, 7, 32, 64, 3.255, 0.578, 0.136, 0.119, 0.000, 0.073, 0.101},
      {MxShape::kKs, 0, 64, 64, 2.952, 0.929, 0.213, 0.209, 0.125, 0.078, 0.033},
      {MxShape::kKs, 1, 64, 128, 3.633, 2.235, 0.289, 0.363, 0.135, 0.113, 0.039},
      {MxShape::kKs, 2, 128, 64, 3.647, 2.183, 0.294, 0.356, 0.147, 0.100, 0.038},
      {MxShape::kKs, 3, 128, 128, 4.723, 2.682, 0.406, 0.591, 0.136, 0.166, 0.045},
      {MxShape::kKs, 4, 128, 192, 5.718, 3.475, 0.547, 0.827, 0.125, 0.234, 0.054},
      {MxShape::kKs, 5, 192, 128, 5.765, 3.304, 0.543, 0.883, 0.122, 0.257, 0.056},
-     {MxShape::kKs, 6, 32, 32, 3.162, 0.265, 0.121, 0.075, 0.000, 0.035, 0.076},
-     {MxShape::kKs, 7, 32, 64, 3.255, 0.578, 0.136, 0.119, 0.000, 0.073, 0.101}}, // fp4
+     {MxShape::kW4, 0, 256, 96, 5.728, 3.703, 0.484, 0.757, 0.000, 0.394, 0.113},
+     {MxShape::kW4, 0, 256, 160, 8.388, 4.324, 0.510, 1.238, 0.000, 0.644, 0.094},
+     {MxShape::kW4, 0, 256, 224, 7.526, 7.963, 1.089, 1.412, 0.000, 0.701, 0.098},
+     {MxShape::kBlock, 0, 256, 256, 5.763, 3.741, 1.024, 2.102, 0.045, 0.821, 0.085},
+     {MxShape::kW4, 0, 256, 256, 9.012, 5.823, 0.809, 2.199, 0.000, 0.939, 0.076},
+     {MxShape::kW4, 0, 256, 192, 8.060, 6.472, 0.880, 1.293, 0.066, 0.435, 0.026},
+     {MxShape::kW4, 0, 256, 128, 6.084, 3.053, 0.645, 0.951, 0.098, 0.213, 0.036}}, // fp4
 };
 // fp8, fp4: the round of 128 x 128 quarter tiles, fixed and a step; `ragged`
 constexpr double kMxQuarter[2] = {0.000, 4.513}, kMxStepQuarter[2] = {0.830, 0.753}, kMxStepRagged[2] = {0.080, 0.125};
 
-int gemm_mx_any(hipStream_t st, void *c, const uint8_t *a, const uint8_t *b, const uint8_t *sa, const uint8_t *sb, int m, int n, int k,
-                int format, int c_fp32)
-{
-    const bool fp4 = format == 4;
-    const bool block = m >= 256 && n >= 256 && k % 512 == 0, w4 = m >= 256 && n >= 128 && n % 4 == 0 && k % (fp4 ? 1024 : 512) == 0;
-    if (!block && !w4)
-        return PTO_ERR_UNSUPPORTED;
-    const int cus = pto_amd::compute_units(), steps = k / (fp4 ? 256 : 128);
-    const MxShape *best = nullptr;
-    double bestTime = 0.0;
-    for (const MxShape &s : kMxShapes[fp4]) {
-        if ((s.kernel == MxShape::kBlock && !block) || (s.kernel == MxShape::kW4 && (!w4 || n < s.bn)) || (s.kernel == MxShape::kKs && n % 4))
-            continue;
+// Which shape; as pto_gemm.hip chooses, small tiles first and shapes passed over that could not win in one round of full speed
+struct MxChoice {
+    int m, n, k, cus;
+    bool fp4, c_fp32;
+    bool block = m >= 256 && n >= 256 && k % 512 == 0, w4 = m >= 256 && n >= 128 && n % 4 == 0 && k % (fp4 ? 1024 : 512) == 0;
+    double steps = k / (fp4 ? 256 : 128), mega = 4e-6 * m * n;
+    static bool Wide(const MxShape &s) { return s.kernel == MxShape::kW4 && s.bn == 256; }
+    static bool Between(const MxShape &s) { return s.kernel == MxShape::kW4 && s.bn % 64 == 32; }
+    bool Any() const { return block || w4; }
+    bool Takes(const MxShape &s) const { return s.kernel == MxShape::kBlock ? block : s.kernel == MxShape::kW4 ? w4 && n >= s.bn : n % 4 == 0; }
+    static double Factor(const MxShape &s)
+    {
+        return s.kernel == MxShape::kBlock || Wide(s) || s.bm == 32 ? 1.03 : s.kernel == MxShape::kKs || Between(s) ? 1.02 : 1.0;
+    }
+    double AtLeast(const MxShape &s) const { return (s.fixed + steps * s.step) * Factor(s); } // (no figure of a shape is negative)
+    double Time(const MxShape &s) const
+    {
         const long long tiles = (long long)((m + s.bm - 1) / s.bm) * ((n + s.bn - 1) / s.bn), rest = tiles % cus;
         double more = (double)((tiles - 1) / cus), share = (double)((tiles - 1) % cus + 1) / cus, extra = 0.0;
-        const bool wide = s.kernel == MxShape::kW4 && s.bn == 256, between = s.kernel == MxShape::kW4 && s.bn % 64 == 32, small = s.bm == 32;
-        if ((wide && share < 0.78) || (between && share < 0.70) || (small && more > 4.0))
-            continue;
+        if ((Wide(s) && share < 0.78) || (Between(s) && share < 0.70) || (s.bm == 32 && more > 4.0))
+            return __builtin_inf();
         if (s.kernel == MxShape::kBlock && !(m % 256 == 0 && n % 256 == 0)) {
             extra = steps * kMxStepRagged[fp4] * (more + 1.0);
         } else if (s.kernel == MxShape::kBlock && rest > 0 && rest * 4 <= cus && tiles > cus) {
@@ -435,17 +439,36 @@ int gemm_mx_any(hipStream_t st, void *c, const uint8_t *a, const uint8_t *b, con
             share = 1.0;
             extra = kMxQuarter[fp4] + steps * kMxStepQuarter[fp4];
         }
-        const double time = (s.fixed + s.perRound * more + steps * (s.step + s.stepRound * more + s.stepShare * share) +
-                             (s.perMega + (c_fp32 ? s.perMegaF32 : 0.0)) * (4e-6 * m * n) + extra) *
-                            (s.kernel == MxShape::kBlock || wide || small ? 1.03 : s.kernel == MxShape::kKs || between ? 1.02 : 1.0);
-        if (best == nullptr || time < bestTime) {
-            best = &s;
-            bestTime = time;
-        }
+        return (s.fixed + s.perRound * more + steps * (s.step + s.stepRound * more + s.stepShare * share) + (s.perMega + (c_fp32 ? s.perMegaF32 : 0.0)) * mega + extra) *
+               Factor(s);
     }
-    switch (best->kernel) {
-    case MxShape::kW4: return pto_amd::gemm_mx_w4(st, c, a, b, sa, sb, m, n, k, format, c_fp32, best->bn);
-    case MxShape::kKs: return pto_amd::gemm_mx_ks(st, c, a, b, sa, sb, m, n, k, format, c_fp32, best->number);
+    const MxShape &Best() const
+    {
+        const MxShape *best = nullptr;
+        double bestTime = __builtin_inf();
+        for (const MxShape &s : kMxShapes[fp4]) {
+            if (!Takes(s) || AtLeast(s) >= bestTime)
+                continue;
+            const double time = Time(s);
+            if (time < bestTime) {
+                best = &s;
+                bestTime = time;
+            }
+        }
+        return *best; // (Any(): the 256 x 256 tiles of eight wavefronts, or those of 128 columns of four, take it)
+    }
+};
+
+int gemm_mx_any(hipStream_t st, void *c, const uint8_t *a, const uint8_t *b, const uint8_t *sa, const uint8_t *sb, int m, int n, int k,
+                int format, int c_fp32)
+{
+    const MxChoice choice{m, n, k, pto_amd::compute_units(), format == 4, c_fp32 != 0};
+    if (!choice.Any())
+        return PTO_ERR_UNSUPPORTED;
+    const MxShape &best = choice.Best();
+    switch (best.kernel) {
+    case MxShape::kW4: return pto_amd::gemm_mx_w4(st, c, a, b, sa, sb, m, n, k, format, c_fp32, best.bn);
+    case MxShape::kKs: return pto_amd::gemm_mx_ks(st, c, a, b, sa, sb, m, n, k, format, c_fp32, best.number);
     default: return gemm_mx_dispatch(st, c, a, b, sa, sb, m, n, k, format, c_fp32, 1);
     }
 }
@@ -470,6 +493,30 @@ extern "C" int pto_gemm_mxfp4(void *stream, void *c, const uint8_t *a, const uin
 }
 
 #if defined(PTO_ST_HOOKS)
+// The choice among the shapes without a launch (needs no device): the variant, as below (1: the 256 x 256 tiles of eight wavefronts), that the entry points take
+// on `units` compute units; expected: the time of each variant, an infinity where it is none of them or does not take the problem
+extern "C" int pto_gemm_mx_choice(int m, int n, int k, int format, int c_fp32, int units, double *expected)
+{
+    if (m <= 0 || n <= 0 || k <= 0 || units <= 0)
+        return PTO_ERR_BAD_ARG;
+    const MxChoice choice{m, n, k, units, format == 4, c_fp32 != 0};
+    if (!choice.Any())
+        return PTO_ERR_UNSUPPORTED;
+    auto variant = [](const MxShape &s) {
+        if (s.kernel == MxShape::kKs)
+            return s.number + (s.number < 6 ? 7 : 11);
+        return s.kernel == MxShape::kBlock ? 1 : s.bn == 192 ? 5 : s.bn == 128 ? 6 : s.bn == 256 ? 13 : s.bn == 96 ? 14 : s.bn == 160 ? 15 : 16;
+    };
+    if (expected != nullptr) {
+        for (int v = 0; v < 19; ++v)
+            expected[v] = __builtin_inf();
+        for (const MxShape &s : kMxShapes[choice.fp4])
+            if (choice.Takes(s))
+                expected[variant(s)] = choice.Time(s);
+    }
+    return variant(choice.Best());
+}
+
 // Tuning hook (not part of the public header): variant bit 0 = quarter tiles in the last round, bit 1 = the shallower copy
 // pipeline; format 0 / 1 = fp8 e4m3 / e5m2, 4 = fp4 e2m1.
 extern "C" int pto_gemm_mxfp8_variant(void *stream, void *c, const uint8_t *a, const uint8_t *b, const uint8_t *scale_a,

@@ -60,3 +60,21 @@ def test_gemm_choice_of_a_shape():
     for m, n, k in ((512, 512, 512), (192, 128, 128), (256, 256, 6144)):
         assert lib.pto_gemm_f16f32_choice(m, n, k, 256, None) == 0
     assert lib.pto_gemm_f16f32_choice(191, 128, 128, 256, None) == capi.ERR_UNSUPPORTED
+
+
+def test_mx_gemm_choice_of_a_shape():
+    """As above: the shortest expected time of all variants, whatever is left out on the way to it."""
+    import ctypes
+    import random
+    lib, rng, times = capi.load_st(), random.Random(7), (ctypes.c_double * 19)()
+    seen = set()
+    for _ in range(6000):
+        top = rng.choice((1000, 6000, 12000))
+        m, n, k = rng.randint(256, top), rng.randint(64, top // 4) * 4 + rng.choice((0, 0, 0, 1)), 1024 * rng.randint(1, 8)
+        fmt, fp32, units = rng.choice((0, 4)), rng.randint(0, 1), rng.choice((64, 256, 304))
+        variant = lib.pto_gemm_mx_choice(m, n, k, fmt, fp32, units, times)
+        assert 0 <= variant < 19 and times[variant] == min(times) < float("inf"), (m, n, k, fmt, fp32, units)
+        assert variant == lib.pto_gemm_mx_choice(m, n, k, fmt, fp32, units, None)
+        seen.add((fmt, variant))
+    assert seen >= {(fmt, variant) for fmt in (0, 4) for variant in (1, 5, 6, 7, 8, 10, 13, 14, 15, 16, 17, 18)}, seen
+    assert lib.pto_gemm_mx_choice(255, 256, 1024, 0, 1, 256, None) == capi.ERR_UNSUPPORTED

@@ -434,11 +434,14 @@ def test_mx_gemm_further_widths_on_four_wavefronts(oracle, variant, fmt, m, n, k
         assert rc == 0 and np.array_equal(got16, bf16_rne(got))
 
 
-@pytest.mark.parametrize("fmt", [1, 4])
-@pytest.mark.parametrize("m,n", [(2560, 5120), (2816, 4608), (2500, 5116), (1000, 6144), (3840, 1536), (2048, 5120), (3133, 3680), (1537, 3328)])
-def test_mx_gemm_whatever_tile_the_entry_point_takes(fmt, m, n):
-    """The entry point at 200 and 198 tiles of 256 x 256 of 256 compute units, and where other widths fill a round: integer operands, the result of the 256 x 128 tiles."""
-    k = 1024
+@pytest.mark.parametrize("fmt,m,n,k,variant", [(1, 2560, 5120, 1024, 16), (1, 2816, 4608, 1024, 16), (1, 2500, 5116, 1024, 16), (1, 1000, 6144, 1024, 14), (1, 3840, 1536, 1024, 14),
+                                               (1, 2048, 5120, 1024, 15), (1, 3133, 3680, 1024, 16), (1, 1537, 3328, 1024, 14), (1, 2368, 5632, 1024, 13),
+                                               (4, 2560, 5120, 1024, 13), (4, 2816, 4608, 1024, 1), (4, 2500, 5116, 1024, 13), (4, 1000, 6144, 1024, 14), (4, 3840, 1536, 1024, 14),
+                                               (4, 2048, 5120, 1024, 5), (4, 3133, 3680, 1024, 16), (4, 1537, 3328, 1024, 14), (4, 2048, 5120, 3072, 15)])
+def test_mx_gemm_whatever_tile_the_entry_point_takes(fmt, m, n, k, variant):
+    """The entry point where its choice on 256 compute units is `variant`, each width on four wavefronts (13 .. 16: 256, 96, 160, 224 columns) in either format; fp4 at 200 and 198 tiles of
+    256 x 256, either side of the line from which they are taken on four wavefronts: integer operands, the result of the 256 x 128 tiles."""
+    assert capi.load_st().pto_gemm_mx_choice(m, n, k, fmt, 1, 256, None) == variant
     a, b, sa, sb = datagen.mx_inputs(m, n, k, fmt, dist="integer") if fmt != 4 else datagen.mx_inputs(m, n, k, fmt)
     rc, got = _mx_variant(a, b, sa, sb, fmt, 4)
     rc6, want = _mx_variant(a, b, sa, sb, fmt, 6)
@@ -469,11 +472,14 @@ def test_mx_gemm_tiles_of_32_rows(oracle, variant, fmt, m, n, k):
         assert rc == 0 and np.array_equal(got16, bf16_rne(got))
 
 
-@pytest.mark.parametrize("fmt", [0, 4])
-@pytest.mark.parametrize("m,n,k", [(256, 256, 512), (512, 512, 2048), (256, 1536, 2048), (700, 700, 1536), (333, 260, 6144)])
-def test_mx_gemm_few_tiles_through_the_entry_point(fmt, m, n, k):
-    """Where 32-row tiles are taken, or nearly: integer operands, the result of the 64 x 64 tiles."""
+@pytest.mark.parametrize("fmt,m,n,k,variant", [(0, 256, 256, 512, 17), (0, 512, 512, 2048, 17), (0, 256, 1536, 2048, 18), (0, 700, 700, 1536, 18), (0, 333, 260, 6144, 17),
+                                               (4, 256, 256, 512, 7), (4, 256, 256, 1024, 17), (4, 512, 512, 2048, 17), (4, 256, 1536, 2048, 18), (4, 700, 700, 1536, 18), (4, 333, 260, 6144, 17)])
+def test_mx_gemm_few_tiles_through_the_entry_point(fmt, m, n, k, variant):
+    """Where the choice is 32-row tiles (17, 18), or the 64 x 64 ones (7) just short of them: integer operands, the result of the 64 x 64 tiles, and of 64 x 128 ones."""
+    assert capi.load_st().pto_gemm_mx_choice(m, n, k, fmt, 1, 256, None) == variant
     a, b, sa, sb = datagen.mx_inputs(m, n, k, fmt, dist="integer") if fmt != 4 else datagen.mx_inputs(m, n, k, fmt)
     rc, got = _mx_variant(a, b, sa, sb, fmt, 4)
-    rc7, want = _mx_variant(a, b, sa, sb, fmt, 7)
-    assert rc == 0 and rc7 == 0 and np.array_equal(got, want)
+    assert rc == 0
+    for other in (7, 8):
+        rc, want = _mx_variant(a, b, sa, sb, fmt, other)
+        assert rc == 0 and np.array_equal(got, want), other
