@@ -534,8 +534,11 @@ struct BucketSort {
         // Many keys in a bucket: few distinct scores, whose equal ones will stand in order by themselves, or too many to be exchanged.  D scores alike in number
         // bring some N / D pairs of equal ones 64 columns apart, most of what the fullest bucket has keys; a part f of the row that is equal, with other
         // scores among it in the bucket, f times that bucket's; distinct ones none.  (64, and a sixth: where keys and pairs are few and vary by chance)
+        // By rank equal ones are in no order.
         bool equal = false;
-        if (full > (uint32_t)kSurely) {
+        if (full > (uint32_t)(RANKS ? kMost : kSurely)) {
+            if (RANKS)
+                return kNothingDone;
             const int same = Equal(bits, i0, validCols, across + 2 * kTopkWaves) / (W > 1 ? kTopkWaves / W : 1);
             equal = 6 * same >= (int)full && 3 * same + 64 >= 2 * (int)full;
             if (!equal && full > (uint32_t)kMost)
