@@ -345,6 +345,7 @@ struct BucketSort {
     static constexpr int N = 64 * E * W, kLogN = __builtin_ctz(N);
     static constexpr int kCrowd = 10; // of 64 scores, in a 128th of the range
     static constexpr int kSurely = 16, kMost = E == 4 ? 16 : E == 8 ? 24 : 48; // keys in a bucket: up to kMost by neighbours; more than kSurely may be equal ones
+    static constexpr int kTries = 4; // passes where more than kMost are taken for equal ones
     double k[E];
 
     static __device__ inline void Meet()
@@ -359,13 +360,16 @@ struct BucketSort {
     // where place p of the list (and word w of the counters, four at a time) stands, so that lanes E apart meet in no bank
     static __device__ inline uint32_t Place(uint32_t p) { return p ^ ((p >> 5) & (uint32_t)(E - 1)); }
     static __device__ inline uint32_t Word(uint32_t w) { return w ^ ((w >> 4) & (uint32_t)(E - 4)); }
-    // how many scores are equal to the one 64 columns on, in the row (more than one wave to it: in all rows of the workgroup)
+    // how many scores are equal to the one 64 or 128 columns before, in the row (more than one wave to it: in all rows of the workgroup)
     static __device__ inline int Equal(const uint32_t (&bits)[E], uint32_t i0, int validCols, [[maybe_unused]] uint32_t *counts)
     {
-        int n = 0;
+        asm volatile("" : "+v"(i0)); // (no mask of the columns is kept in registers for this)
+        uint32_t mine = 0;
 #pragma unroll
         for (int e = 1; e < E; ++e)
-            n += __builtin_popcountll(__builtin_amdgcn_ballot_w64(bits[e - 1] == bits[e] && i0 + 64u * (uint32_t)e < (uint32_t)validCols));
+            if (i0 + 64u * (uint32_t)e < (uint32_t)validCols)
+                mine += (uint32_t)(bits[e] == bits[e - 1]) + (e > 1 ? (uint32_t)(bits[e] == bits[e > 1 ? e - 2 : 0]) : 0u);
+        int n = __builtin_amdgcn_readlane((int)WaveScan(mine), 63);
         if constexpr (W > 1) {
             counts[threadIdx.x / 64] = (uint32_t)n;
             __syncthreads();
@@ -531,16 +535,16 @@ struct BucketSort {
             for (int j = 0; j < E / 4; ++j)
                 mine[chunk(j)] = make_uint4(c[4 * j], c[4 * j + 1], c[4 * j + 2], c[4 * j + 3]);
         }
-        // Many keys in a bucket: few distinct scores, whose equal ones will stand in order by themselves, or too many to be exchanged.  D scores alike in number
-        // bring some N / D pairs of equal ones 64 columns apart, most of what the fullest bucket has keys; a part f of the row that is equal, with other
-        // scores among it in the bucket, f times that bucket's; distinct ones none.  (64, and a sixth: where keys and pairs are few and vary by chance)
+        // Many keys in a bucket: mostly few distinct scores, whose equal ones will stand in order by themselves, or too many to be exchanged.  D scores alike in
+        // number bring some 2 N / D pairs of equal ones 64 and 128 columns apart, most of what the fullest bucket has keys; a part f of the row that is equal, with
+        // other scores among it in the bucket, 2 f times that bucket's; distinct ones none.  (128, and a third: where keys and pairs are few and vary by chance)
         // By rank equal ones are in no order.
         bool equal = false;
         if (full > (uint32_t)(RANKS ? kMost : kSurely)) {
             if (RANKS)
                 return kNothingDone;
             const int same = Equal(bits, i0, validCols, across + 2 * kTopkWaves) / (W > 1 ? kTopkWaves / W : 1);
-            equal = 6 * same >= (int)full && 3 * same + 64 >= 2 * (int)full;
+            equal = 3 * same >= (int)full && 3 * same + 128 >= 4 * (int)full;
             if (!equal && full > (uint32_t)kMost)
                 return kNothingDone;
         }
@@ -580,12 +584,29 @@ struct BucketSort {
         for (int e = 0; e < E; ++e)
             k[e] = __builtin_bit_cast(double, list[Place(q * E + (uint32_t)e)]);
         Meet();
-        double above, below;
-        const int passes = equal ? 0 : (int)(full + 1u) / 2;
-        for (int pass = 0; pass < passes; ++pass) { // (two places for the edges in turn)
+        // As many passes as the fullest bucket can need; with equal scores, which can need none, a look before each whether all is in order (bfloat16 scores: equal ones in
+        // the fullest buckets, a few distinct ones in others)
+        const bool enough = full <= (uint32_t)kMost;
+        const int passes = enough ? (int)(full + 1u) / 2 : kTries;
+        for (int pass = 0;; ++pass) { // (two places for the edges in turn, and two others for the look)
+            if (pass == passes && enough)
+                return kSorted;
+            if (__builtin_expect(equal, 0)) {
+                double above, below;
+                Neighbours(above, below, waveOfRow, lane, list + (pass & 1) * 16 + 8);
+                bool sorted = k[E - 1] >= above;
+#pragma unroll
+                for (int e = 1; e < E; ++e)
+                    sorted = sorted & (k[e - 1] >= k[e]);
+                if (W > 1 ? Everyone(sorted, across + (2 + (pass & 1)) * kTopkWaves) : WholeWave(sorted))
+                    return kSorted;
+                if (pass == passes)
+                    return kLost;
+            }
 #pragma unroll
             for (int e = 0; e < E; e += 2)
                 Exchange(k[e], k[e + 1]);
+            double above, below;
             Neighbours(above, below, waveOfRow, lane, list + (pass & 1) * 16);
 #pragma unroll
             for (int e = 1; e + 1 < E; e += 2)
@@ -593,20 +614,12 @@ struct BucketSort {
             k[E - 1] = Max(k[E - 1], above);
             k[0] = Min(k[0], below);
         }
-        if (equal) {
-            Neighbours(above, below, waveOfRow, lane, list);
-            bool sorted = k[E - 1] >= above;
-#pragma unroll
-            for (int e = 1; e < E; ++e)
-                sorted = sorted & (k[e - 1] >= k[e]);
-            if (W > 1 ? !Everyone(sorted, across + 3 * kTopkWaves) : !WholeWave(sorted))
-                return kLost;
-        }
-        return kSorted;
     }
 };
+// waves on a SIMD at the least: of what few registers more or less decide (1600 x 2048 with five instead of seven 11.8 -> 12.9 us)
+constexpr int Resident(int e, int w, Mode mode) { return mode == kSelect ? (e == 16 ? 4 : 1) : mode == kCut ? 1 : e == 16 && w <= 2 ? 4 : e == 8 && w >= 2 ? 7 : 1; }
 template <int E, int W, bool LOW_DPP, Mode MODE>
-__global__ __launch_bounds__(kTopkThreads, MODE == kSelect && E == 16 ? 4 : MODE == kWhole && E == 16 && W == 1 ? 4 : 1) void TopkRows(float *outScore, uint32_t *outIndex, const float *src, const uint32_t *inIdx,
+__global__ __launch_bounds__(kTopkThreads, Resident(E, W, MODE)) void TopkRows(float *outScore, uint32_t *outIndex, const float *src, const uint32_t *inIdx,
                                                          int rows, int validCols, int ld, int topk, int keepBits, int through, int buckets)
 {
     constexpr int N = 64 * E * W, kRows = kTopkWaves / W, kBits = RowSort<E, W, LOW_DPP>::kLaneBits;

@@ -126,6 +126,23 @@ def test_topk_of_few_distinct_scores_in_any_index_order(rows, cols):
     assert few <= 1.03 * masked, (few, masked)
 
 
+@pytest.mark.parametrize("rows,cols,kind", [(16, 4096, "bfloat16"), (1200, 4096, "bfloat16"), (2000, 777, "sixty")])
+def test_topk_of_rows_with_equal_scores(rows, cols, kind):
+    """Scores on a grid, with equal ones in the fullest buckets and a few distinct ones in others: sorted by buckets, not given up on because a first look behind the scatter does
+    not find them in order (0.7 to 0.8 of the time of masked rows, which the network sorts; given up on 0.9 to 1.25 of it)."""
+    lib = capi.load()
+    stream = torch.cuda.current_stream().cuda_stream
+    random, column = torch.randn((rows, cols), device="cuda:0"), torch.arange(cols, device="cuda:0")
+    score, index = torch.empty((rows, cols), device="cuda:0"), torch.empty((rows, cols), dtype=torch.int32, device="cuda:0")
+    ids = column.to(torch.int32)
+
+    def call(src):
+        return lambda: capi.check(lib.pto_topk_f32(stream, score.data_ptr(), index.data_ptr(), src.data_ptr(), ids.data_ptr(), rows, cols, cols, cols), "pto_topk_f32")
+    grid = random.bfloat16().float() if kind == "bfloat16" else torch.randint(0, 60, (rows, cols), device="cuda:0").float()
+    equal, masked = best_us([call(grid), call(random.masked_fill(column > cols // 2, -torch.inf))])
+    assert equal <= 0.83 * masked, (equal, masked)
+
+
 def test_gather_of_odd_rows_against_whole_lines():
     """A table that an XCD's L2 holds is read whole whatever its rows: 592 bytes to a row no slower than 512 (8 to 15 % slower when cut into slices)."""
     lib = capi.load()

@@ -323,12 +323,12 @@ def test_topk_by_buckets(rows, cols):
 @pytest.mark.parametrize("rows,cols", [(748, 512), (741, 300), (36, 1024), (37, 600), (888, 1000), (2592, 1024), (2571, 700), (40, 2048), (19, 1300), (1716, 1500), (38, 4096), (21, 2500)])
 def test_topk_of_crowded_scores(rows, cols):
     """Rows around every limit of the sort by buckets: clusters of 14 to 60 distinct scores closer than a bucket (16, 24 and 48 are exchanged by neighbours), few
-    distinct scores (whose equal ones stand in order), a part of the row equal with other scores among it, squares and others that crowd at an end of their range."""
+    distinct scores (whose equal ones stand in order), a part of the row equal with other scores among it, squares and others that crowd at an end of their range, bfloat16 scores."""
     r = np.random.Generator(np.random.Philox(key=7 * rows + cols))
     src = r.random((rows, cols), dtype=np.float32)
     normal = r.standard_normal((rows, cols)).astype(np.float32)
     for row in range(rows):
-        kind = row % 19
+        kind = row % 20
         if kind < 10:
             n = (14, 15, 16, 17, 22, 23, 24, 25, 46, 60)[kind]
             src[row, r.permutation(cols)[:n]] = np.float32(0.5) + np.arange(n, dtype=np.float32) * np.float32(6e-8)
@@ -336,8 +336,10 @@ def test_topk_of_crowded_scores(rows, cols):
             src[row] = r.integers(0, (11, 30, 70, 190)[kind - 10], cols)
         elif kind < 17:
             src[row] = np.where(r.random(cols) < (0.05, 0.25, 0.6)[kind - 14], np.float32(0.3), normal[row])
-        else:
+        elif kind < 19:
             src[row] = normal[row] ** 2 if kind == 17 else 1 / (1 + np.exp(-6 * normal[row]))
+        else:
+            src[row] = (normal[row].view(np.uint32) & np.uint32(0xFFFF0000)).view(np.float32)
     idx = np.arange(cols, dtype=np.uint32)
     for ids, k in ((idx, cols), (r.permutation(cols).astype(np.uint32), cols - cols // 3)):
         at = np.lexsort((np.broadcast_to(ids, src.shape), -src))[:, :k]
