@@ -635,11 +635,11 @@ __global__ __launch_bounds__(kTopkThreads, Resident(E, W, MODE)) void TopkRows(f
     constexpr size_t kSelected = MODE == kSelect ? 384 + (size_t)kRows * 68 * kMostSelected * 8 : 0, kSort = kExchange > kStage ? kExchange : kStage;
     constexpr size_t kWork = kSort > kSelected ? kSort : kSelected;
     static_assert(kWork >= (size_t)N * 2, "the ranks fit");
-    // (behind the first wave's results where its piece has room: 32 KiB a workgroup are five workgroups a compute unit)
-    // (one wave per row and buckets: both tables of the columns' order behind everything, as the rows are still counted when they are read)
+    // (one wave per row and buckets: both tables of the columns' order behind everything, as the rows are still counted when they are read; 16 keys a lane: 36 KiB a
+    // workgroup, four to a compute unit, as their registers allow)
     constexpr bool kApart = kCount && W == 1;
-    constexpr size_t kColumns = kApart ? kWork + (size_t)N * 2 : kOwn >= kStaged * 4 * kStages + (size_t)N * 2 ? (size_t)kStaged * 4 * kStages : kWork;
-    __shared__ __attribute__((aligned(16))) char lds[kColumns < kWork ? kWork : kColumns + (size_t)N * 2];
+    constexpr size_t kColumns = kApart ? kWork + (size_t)N * 2 : kWork;
+    __shared__ __attribute__((aligned(16))) char lds[kColumns + (size_t)N * 2];
     [[maybe_unused]] __shared__ uint32_t across[kTopkWaves * 6];
     uint16_t *rankOf = reinterpret_cast<uint16_t *>(lds + (kApart ? kWork : 0)), *columnOf = reinterpret_cast<uint16_t *>(lds + kColumns);
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / 64), lane = tid % 64;
