@@ -1098,7 +1098,9 @@ int launch_topk(hipStream_t st, float *out_score, uint32_t *out_index, const flo
     // Past 1024 columns buckets instead of merges that keep topk, wherever no threshold is taken (us, merges / buckets, random scores; nearly all equal ones):
     // 2048 columns, 16 rows, top 129 7.0 / 5.5; 7.0 / 7.35, 300 rows, top 256 8.5 / 6.2; 8.4 / 8.8; 4096 columns, 16 rows, top 321 11.4 / 7.5; 11.45 / 11.9,
     // 1500 rows, top 512 34.3 / 19.5; 33.7 / 34.9.  1024 columns, 16 rows, top 64 4.6 / 4.4; 4.6 / 5.0: what it gives and what it takes are alike there
-    constexpr Mode kFew = kOnlyWhole<E, W> ? kWhole : W == 4 && E >= 8 ? kCountedCut : kCut;
+    // (16 keys a lane with up to two waves, eight with two: the dispatch has taken a threshold for every such topk, and no other kernel is built)
+    constexpr bool kThresholdBefore = (E == 16 && W <= 2) || (E == 8 && W == 2);
+    constexpr Mode kFew = kOnlyWhole<E, W> || kThresholdBefore ? kWhole : W == 4 && E >= 8 ? kCountedCut : kCut;
     constexpr bool kDpp = E >= 8 || kOnlyWhole<E, W>; // (names the one form that there is)
     auto kernel = dpp ? (whole ? TopkRows<E, W, true, kWhole> : TopkRows<E, W, true, kFew>) :
                         (whole ? TopkRows<E, W, kDpp, kWhole> : TopkRows<E, W, kDpp, kFew>);
