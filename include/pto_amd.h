@@ -57,7 +57,7 @@ int pto_last_hip_error(void);
 /* C[m,n] fp32 row-major = A[m,k] fp16 row-major x B, where B is stored [n,k] fp16 (a column-major
  * k x n operand), fp32 accumulation.  Accepted extents: m % 128 == 0, n % 256 == 0, k % 32 == 0 (multiples of the
  * 128 x 256 block of the reference kernel), or any m >= 192 and n >= 128 with n % 4 == 0 and k % 128 == 0.  Anything else:
- * PTO_ERR_UNSUPPORTED.  Tiles of 32 x 64 to 256 x 256, chosen by the extents; the sums are added in their order. */
+ * PTO_ERR_UNSUPPORTED.  Tiles of 32 x 32 to 256 x 256, chosen by the extents; the sums are added in their order. */
 int pto_gemm_f16f32(void *stream, float *c, const uint16_t *a, const uint16_t *b, int m, int n, int k);
 
 /* MXFP8 GEMM: C[m,n] row-major = (A .* 2^(scale_a - 127)) x (B .* 2^(scale_b - 127)) with fp32 accumulation.

@@ -91,8 +91,9 @@ inline int gemm_mx_w4(hipStream_t st, void *c, const uint8_t *a, const uint8_t *
     default: return PTO_ERR_UNSUPPORTED;
     }
 }
-// defined in pto_gemm_mxks.hip (MXFP8 / MXFP4 tiles on eight wavefronts with k split over two groups of them); shape 0 .. 5 =
-// 64 x 64, 64 x 128, 128 x 64, 128 x 128, 128 x 192, 192 x 128.  PTO_ERR_UNSUPPORTED unless n % 4 == 0 and k % 512 == 0
+// defined in pto_gemm_mxks.hip (MXFP8 / MXFP4 tiles with k split over two groups of wavefronts); shape 0 .. 5 = 64 x 64, 64 x 128,
+// 128 x 64, 128 x 128, 128 x 192, 192 x 128 on eight wavefronts, 6 = 32 x 32 on two, 7 = 32 x 64 on four.  PTO_ERR_UNSUPPORTED unless
+// n % 4 == 0 and k % 512 == 0
 int gemm_mx_ks(hipStream_t st, void *c, const uint8_t *a, const uint8_t *b, const uint8_t *sa, const uint8_t *sb, int m, int n, int k,
                int format, int c_fp32, int shape);
 // defined in pto_fa_w8.hip (head_dim 128, workgroups of eight wavefronts = 256 queries, two groups of four waves in

@@ -13,9 +13,9 @@
 // taken out a step of 0.46 us (1024 x 3072 x 8192) runs 0.43 without the fragment reads, 0.36 with copies alone and 0.33
 // with MFMAs alone.  The place of the copies in the step, raised wave priority and deeper rings changed nothing (1 %; a 32 x 64 step, 12 KiB in
 // 0.13 us: rings of 6 to 13 stages 0 to 20 % slower, two steps from one barrier to the next 0 to 10 %).  So where units are idle the tile gets
-// smaller: 32 x 32, 0.09 us a step, on twice as many of them (512^3 3.78 -> 3.33 us, 256 x 256 x 6144 15.8 -> 11.5; four stages 14.8, five 12.0, eight 11.5).
+// smaller: 32 x 32, 0.09 us a step, on twice as many of them (from a graph 512^3 3.76 -> 3.29 us, called one by one 3.87 -> 3.67 or what the host takes; 256 x 256 x 6144 15.8 -> 11.5; four stages 14.8, five 12.0, eight 11.5).
 // (1000 x 3000 x 2048 on 128 x 96 tiles runs 0.4 us a step: 28 KiB of copies, from beyond the L2.)
-// Small tiles lose there what they win in compute units at work: 512^3 8.96 -> 3.3 us, 1000 x 3000 x 2048 21.1 -> 18.0,
+// Small tiles lose there what they win in compute units at work: 512^3 8.96 -> 3.3 us (from a graph), 1000 x 3000 x 2048 21.1 -> 18.0,
 // 128 x 4096 x 4096 68 -> 12.  C past the L2 where that pays (store_through): 1000 x 3072 x 2048 18.5 -> 17.0.
 //
 // Rows past m and columns past n repeat the last one on the way in (their memory may not exist) and are not stored.

@@ -5,8 +5,9 @@
 // partial sums are those of the fp16 kernel.
 //
 // 32 x 32 tiles are two wavefronts, one for each half of k, and 32 x 64 ones four: a unit's copies bound a step, so products of few tiles gain by
-// smaller ones on more units.  64 x 64 -> 32 x 32 (launched from a graph): 512^3 fp8 4.25 -> 3.58 us, fp4 4.09 -> 3.49; 256 x 256 x 6144 12.6 -> 9.6, 8.2 -> 6.4;
-// 64 x 64 -> 32 x 64: 256 x 1536 x 2048 5.80 -> 4.92, 5.26 -> 4.55.  Six and eight stages for them: 512 x 512 x 2048 fp8 4.51 -> 5.03 and 5.16, only from k = 4096 on up to 11 % faster.
+// smaller ones on more units.  To bf16, launched from a graph, the same operands each time; thirty sets of them in turn: 64 x 64 -> 32 x 32, 512^3 fp8 3.60 -> 2.86 us; 4.0 -> 3.2,
+// fp4 3.40 -> 2.78; 3.6 -> 2.95, 256 x 256 x 6144 8.8 -> 6.3; 13.0 -> 9.3, fp4 7.5 -> 5.7; 9.0 -> 6.6; 64 x 64 -> 32 x 64, 256 x 1536 x 2048 5.1 -> 4.2; 6.4 -> 5.5, fp4
+// 4.6 -> 3.9; 5.3 -> 4.4.  (Called one by one 512^3 takes 4.1 on either: the host.)  Six and eight stages for them: 512 x 512 x 2048 fp8 4.51 -> 5.03 and 5.16, only from k = 4096 on up to 11 % faster.
 //
 // Scales.  32 bytes of a row's scales last P = 8 steps (fp8) or 4 (fp4); they come into one of two LDS buffers with one or two
 // copy instructions per wave and period (two lanes per row), a period ahead.  A lane's MFMA operand needs the scale of its own
@@ -17,8 +18,8 @@
 //
 // What bounds a step: the copies, as in the fp16 kernel.  One 64 x 64 tile takes 0.16 us a step, 64 x 128 0.24, 128 x 128 0.37,
 // 128 x 192 0.52: 79 to 102 bytes per ns and compute unit, where its MFMAs take 0.05, 0.11, 0.21, 0.32.
-// 512 x 512 x 512 fp8 9.1 -> 3.6 us, 256 x 256 x 6144 34.0 -> 11.9, 2048^3 17.3 -> 12.8; 3072^3 stays on 256 x 192 tiles (31
-// against 40).
+// fp8 to fp32, the same operands each time, 256 x 128 tiles on four wavefronts / the best of these: 512^3 9.4 / 2.9 us, 256 x 256 x 6144 29.8 / 6.3,
+// 2048^3 15.1 / 11.7 (128 x 128); 3072^3 stays on 256 x 192 tiles (31 against 40).
 //
 // The way out: bf16 by the hardware conversion (the integer form was 7 instructions an element), 16 bytes a lane, 64 bytes of a row to a
 // store instruction, past the L2 where that pays (store_through): 2048 x 2048 x 1024 to bf16 11.1 -> 8.6 us in fp8, 9.1 -> 6.7 in

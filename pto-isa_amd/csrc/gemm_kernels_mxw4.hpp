@@ -15,7 +15,7 @@
 //   * four B stages (96 + 64 KiB = the whole LDS at BN = 192), which makes the step's second barrier unnecessary: a
 //     stage is overwritten two steps after its last read, with the barrier of the step in between.
 // Steps come in groups of four (B stage, A slot and scale byte repeat): k % 512 == 0.
-// BN = 224 and 256: up to all 256 accumulation registers, a sixth fewer copies and a seventh fewer fragment reads per MFMA than at 192.  Three B stages fit, so a step has a
+// BN = 224 and 256: up to all 256 accumulation registers, a seventh fewer copies and a sixteenth fewer fragment reads per MFMA at 256 than at 192.  Three B stages fit, so a step has a
 // second barrier again, ahead of its first copy of B, and as three stages and eight (sixteen) steps of a scale period do not go together, they take
 // turns at run time.  Two sets of scale registers do not fit: rows are loaded over their own first three quarters when the last one has been moved
 // aside, and spread in place.  What the time goes into (2040 x 8100 x 8192 fp4 on 256 x 128 tiles, 72.8 us; one part taken out): copies 8.8, reads of B 5.3 and of
@@ -310,6 +310,8 @@ AICORE inline __attribute__((always_inline)) void MxW4TileCompute(__gm__ const u
     // register t / kGroupSteps, byte t % kGroupSteps (fp4: two bytes).  The copies of A of step it + 2 go to this step's A slot,
     // those of B to the stage of step it - 2; scale rows kScaleLoads t .. of the next period are loaded at the start of the step
     // and spread over the lane groups behind its barrier.
+    // WIDE: three B stages in turn (stageNow, stageThen, stageCopy), the copies of B of step it + 2 to the stage of step it - 1, behind a barrier of their
+    // own; all scale rows of the next period are loaded and spread in the last quarter of a period, over the three quarters that are used up.
     auto step = [&](auto tTag, int it, int super) __attribute__((always_inline)) {
         constexpr int t = decltype(tTag)::value, j = t % 4, par = j % 2;
         constexpr int s = WIDE ? 0 : j, sNext = WIDE ? 1 : (j + 1) % BSTAGES, sCopy = (j + 2) % BSTAGES;

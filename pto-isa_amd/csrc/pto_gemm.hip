@@ -60,7 +60,7 @@ struct TileShape {
 };
 // (small tiles first: for a small problem, whose call the host bounds, the choice is then the first shape's time and lower bounds of the others)
 constexpr TileShape kShapes[] = {
-    // 32 x 32, fitted to 400 problems of up to 900 such tiles: it is the shortest where they are one round, and by 8 to 29 % (from a graph 512^3 3.78 -> 3.33 us,
+    // 32 x 32, fitted to 400 problems of up to 900 such tiles: it is the shortest where they are one round, and by 8 to 29 % (from a graph 512^3 3.76 -> 3.29 us,
     // 512 x 512 x 2048 7.4 -> 6.0, 256 x 256 x 6144 15.8 -> 11.5, 300 x 700 x 1024 4.70 -> 4.14), and never where they are two (640 x 512 x 1024 4.8 / 5.4)
     {TileShape::kKs, 9, 32, 32, 2.487, 0.411, 0.091, 0.076, 0.159, 0.017},
     {TileShape::kKs, 0, 32, 64, 2.670, 0.853, 0.135, 0.136, 0.178, 0.026},   {TileShape::kKs, 1, 64, 64, 2.822, 0.902, 0.152, 0.165, 0.175, 0.044},

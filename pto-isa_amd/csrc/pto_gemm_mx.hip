@@ -373,8 +373,8 @@ struct MxShape {
 // 300 by 7 % (fp8) and 53 by 9 % (fp4) on average, for one of either more than 2 % slower (5 and 7 %).  5632 x 1536 x 512 fp8 to fp32 on 256 x 160 tiles -16 %,
 // 3840 x 1536 x 1024 fp4 on 256 x 96 -15 %, 7424 x 3584 x 7168 fp8 on 256 x 224 -17 %.
 // 32 x 32 and 32 x 64 with k split: fitted to 249 problems of up to 1.3 million results each in fp8 and fp4, both results (256 x 256 x 512 .. 1400 x 1000 x 7168), taken 3 % dearer and up to the
-// five rounds of that fit: for 303 of 498 by 17 % (fp8) and 255 by 15 % (fp4) on average, for one 3 % slower (512 x 1024 x 2048 fp8).  512^3 fp8 4.25 -> 3.58 us, 256 x 256 x 6144
-// 12.6 -> 9.6, 256 x 1536 x 2048 5.8 -> 4.9; fp4 4.1 -> 3.5, 8.2 -> 6.4, 5.3 -> 4.6; past their two rounds the larger ones are faster (1024^3 fp8 64 x 64 5.1, 32 x 64 5.8, 32 x 32 6.4).
+// five rounds of that fit: for 303 of 498 by 17 % (fp8) and 255 by 15 % (fp4) on average, for one 3 % slower (512 x 1024 x 2048 fp8; operands in turn, from
+// graphs: times at gemm_kernels_mxks.hpp); past their two rounds the larger ones are faster (1024^3 fp8 64 x 64 5.1, 32 x 64 5.8, 32 x 32 6.4).
 constexpr int kMxShapeCount = 15;
 constexpr MxShape kMxShapes[2][kMxShapeCount] = {
     {{MxShape::kKs, 6, 32, 32, 2.750, 0.419, 0.117, 0.066, 0.000, 0.032, 0.081},

@@ -38,7 +38,7 @@
 // What bounds the network: vector instructions, 2520 per row of 1024 (3850 in the integer network this replaced), behind a phase of
 // loads and before one of stores that all waves share (five waves on a SIMD instead of four: no change; persistent waves that load the next row while they sort
 // one, and wave priorities that let some run ahead, do not hide them: 32 us and no change).  By buckets 4800 x 1024, top 1000 (58 MB = 9 us at 6.5 TB/s)
-// is bound by the launch, the loads and the stores, with 1190 vector and 142 LDS instructions a row between them (SQ_INSTS_VALU, SQ_INSTS_LDS; the LDS is busy for 760 clocks a row,
+// is bound by the launch, the loads and the stores, with 1210 vector and 142 LDS instructions a row between them (SQ_INSTS_VALU, SQ_INSTS_LDS; the LDS is busy for 760 clocks a row,
 // 6 us in all, half of them where counters of one bank meet).
 #include <hip/hip_runtime.h>
 
@@ -319,12 +319,14 @@ __device__ inline void WaveEnds(float &hi, float &lo)
 // and its smallest one, the keys in each are counted, sums over the counts say where a bucket begins, every key goes to the next place of its
 // bucket in a list, and neighbours change places (odd and even pairs in turn) as often as the fullest bucket has keys (5 to 9 of 1024 random scores).
 // 2 N counters of 16 bits: with N of them buckets hold twice as many keys.  Which rows: any whose scores are finite and not crowded in a small part of
-// their range; the others go through the network, found by a look at 64 scores of each wave before anything is counted (masked with infinities, half zeros, squares,
-// exponentials), or by the count before anything is scattered (forty close scores among spread ones, a twentieth equal).  Microseconds, network / turned away by the look /
-// by the count / buckets of normal scores: 4800 x 1024, top 1000 21.5 / 22.7 / 25.3 / 15.6; 2400 x 1024 14.2 / 14.5 / 16.3 / 9.9; 600 x 1024 7.4 / 7.8 / 8.8 / 5.9; 1600 x 2048
-// 21.5 / 22.0 / 24.4 / 12.2; 9000 x 512 17.5 / 18.7 / 21.0 / 12.1; 1200 x 4096 34.0 / 35.8 / 39.9 / 20.0; 16 x 4096 13.1 / 13.7 / 16.3 / 8.6 (a count that is found wanting only
-// behind the scatter and a pass took 1.25 to 1.4 times the network's, up to 1.8 where the look saw less).  Tried for them and slower than the network: 64 of the row's own scores,
-// sorted, as the limits of ranges that are spread evenly each (4800 x 1024 27 us).  512 columns in up to 731 rows stay with the network (4.2 us; by
+// their range; the others go through the network, found by a look at 64 scores of each wave before anything is counted (masked with infinities, half zeros, most squares,
+// wide exponentials), or by the count before anything is scattered (forty close scores among spread ones, a twentieth equal).  Microseconds, whole rows, network alone / turned away by
+// the look / by the count / buckets of normal scores: 4800 x 1024 21.1 / 22.1 / 24.9 / 14.7; 2400 x 1024 13.9 / 14.1 / 16.1 / 9.8; 600 x 1024 7.5 / 7.6 / 8.6 / 5.6; 100 x 1024 5.4 / 5.5 /
+// 6.4 / 4.8; 1600 x 2048 21.2 / 21.5 / 24.2 / 12.0; 300 x 2048 9.6 / 10.0 / 11.8 / 6.8; 9000 x 512 16.9 / 18.2 / 20.7 / 11.8; 1200 x 4096 33.5 / 35.2 / 39.0 / 19.7; 16 x 4096 13.5 /
+// 14.0 / 15.8 / 8.7 (a count that is found wanting only behind the scatter and a pass took 1.25 to 1.4 times the network's, up to 1.8 where the look saw less).  Equal scores:
+// bfloat16 ones 1200 x 4096 23.3, 16 x 4096 10.8; sixty distinct ones 4800 x 1024 15.3, 2000 x 777 9.1 (network 12.4).  Tried for uneven rows and slower than the network: 64 of the
+// row's own scores, sorted, as the limits of ranges that are spread evenly each (4800 x 1024 27 us); tried for masked ones: infinities and equal scores among the 64 told from the others before
+// the range is (masked 22.2 -> 21.5, normal 14.75 -> 15.0).  512 columns in up to 731 rows stay with the network (4.2 us; by
 // buckets 4.5 in two waves a row, 4.5 in one), as do 256 and less.
 // bits[e]: the score in column i0 + 64 e; afterwards key e of the lane with number q = 64 (wave of the row) + lane is of rank q E + e.
 // RANKS: rankOf[column] decides among equal scores and is returned in the column's place.
@@ -1112,9 +1114,11 @@ int launch_topk(hipStream_t st, float *out_score, uint32_t *out_index, const flo
     // instruction's 256 bytes (8192 x 64, top 1 3.2 / 3.7, 131072 x 64, top 33 32.6 / 34.1), nor where they are much more than the L2s'
     // 32 MB, which then are written back while others sort (30000 x 2048, top 1500 261 / 268).
     const int through = topk >= 64 && 8ll * rows * topk <= 1ll << 26;
-    // Just past what a threshold is taken for, 257 to 320 of 1025 to 2048 columns, the network as before: 600 x 1025 random scores take 9.0 us by threshold for the
-    // top 256 and would take 7.7 by buckets for the top 257, but rows masked from the middle on 9.1 by threshold and 12.6 where buckets turn them away; both
-    // in one kernel, buckets ahead of the threshold, is 15 % faster with random rows, 5 to 20 % slower with masked and 50 % with sixty distinct scores
+    // Just past what a threshold is taken for, 257 to 320 of 1025 to 2048 columns, the network: by buckets random rows would be faster than the top 256 of them are by threshold, and few of
+    // many are not to take longer than more (past 2048 columns they do, by a fifth: 64 x 4096, top 320 9.0, top 321 7.5).  What it costs (us, random; masked from the middle on):
+    // 600 x 1025, top 256 by threshold 8.8; 8.4, top 257 by the network 11.6; 11.5, by buckets 7.4; 11.9; 1600 x 2048 11.3; 11.0, 19.4; 19.3, 10.9; 20.3.  Buckets for the top 256 too
+    // would slow masked rows by 40 to 85 % (below, at the threshold); both in one kernel, buckets ahead of the threshold, is 15 % faster with random rows, 5 to 20 % slower with
+    // masked and 50 % with sixty distinct scores
     const int buckets = !(64 * E * W == 2048 && topk > 256 && topk <= 320);
     constexpr int kRows = kTopkWaves / W;
     kernel<<<dim3((unsigned)(((long long)rows + kRows - 1) / kRows)), dim3(kTopkThreads), 0, st>>>(out_score, out_index, src, in_idx, rows, valid_cols,
@@ -1147,8 +1151,12 @@ extern "C" int pto_topk_f32(void *stream, float *out_score, uint32_t *out_index,
     //   1024 columns:  600 rows, top 128 7.2 / 6.5   1500 rows, top 16  7.6 / 5.4   4800 rows, top 128 19.9 / 9.9; 128 rows, top 16 4.8 / 4.9, top 128 5.4 / 6.6, 700 rows, top 4 5.1 / 5.3
     //    512 columns: 4000 rows, top  16 7.5 / 6.0   8000 rows, top 60 14.7 / 10.6; 1000 rows, top 16 4.7 / 4.7, top 60 5.2 / 5.5
     // One wave per row of 1024 and two per row of 2048 where without the threshold there are four (1500 rows, top 16: 5.2 with one, 6.1 with four).
-    // Near the line no kind of row measured is slower by more than 3 % than without.  600 x 1024, top 100: random 7.2 / 6.6, sixty distinct scores 7.2 / 6.6, all
-    // equal but 2 % 7.2 / 5.7; 8 x 2048, top 30, all equal but 2 %: 6.4 / 6.6.  Just past 1024 and 2048 columns the waves' thresholds lie lower for the short rows (1600 x 2049, top 100: 37.3 / 20.3).
+    // Near the line no kind of row measured is slower by more than 3 % than by merges.  600 x 1024, top 100: random 7.2 / 6.6, sixty distinct scores 7.2 / 6.6, all
+    // equal but 2 % 7.2 / 5.7; 8 x 2048, top 30, all equal but 2 %: 6.4 / 6.6.  Buckets (keeping topk) in its place would be faster near its upper end with random rows, and slower
+    // with masked ones, which they turn away.  Threshold / buckets, us, random; masked from the middle on: 600 x 1024, top 60 5.2 / 5.2; 5.5 / 7.0, top 128 6.2 / 5.2; 6.0 / 7.2, 4800 x 1024,
+    // top 128 9.8 / 11.9; 9.4 / 19.3; 600 x 2048, top 100 6.8 / 7.2; 7.1 / 10.5, top 160 7.7 / 7.3; 7.3 / 11.0, top 256 8.9 / 7.3; 8.6 / 11.1, 1600 x 2048, top 256 11.3 / 10.4; 11.0 / 19.6;
+    // 16 x 4096, top 320 9.1 / 7.4; 8.9 / 12.4, 300 x 4096, top 256 8.4 / 9.2; 8.7 / 14.8, 1200 x 4096, top 312 18.2 / 17.2; 17.6 / 30.7 (at top 320 one random
+    // row in some hundreds has more than 512 keys at its threshold and goes to the network: 22.9).  Just past 1024 and 2048 columns the waves' thresholds lie lower for the short rows (1600 x 2049, top 100: 37.3 / 20.3).
     const int padded = valid_cols <= 512 ? 512 : valid_cols <= 1024 ? 1024 : valid_cols <= 2048 ? 2048 : 4096;
     if (valid_cols > 256 && topk <= padded / 8 && topk <= (valid_cols > 2048 || most < 10 ? 320 : most < 20 ? 160 : 128)) {
 #define PTO_TOPK_SELECT(E, W) return launch_topk<E, W>(st, out_score, out_index, src, in_idx, rows, valid_cols, ld, topk, true);

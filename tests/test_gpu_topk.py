@@ -267,7 +267,7 @@ def test_topk_threshold_and_the_columns(oracle, rows, cols, topks):
                                        (13, 4096), (14, 2049), (12, 3000)])
 def test_topk_by_buckets(rows, cols):
     """Whole sorts (more than an eighth of the padded row), and an eighth where no threshold is taken, of every kind of row that buckets take, give up on at the look, after counting, or after a first exchange: even
-    scores; equal ones in numbers around the fullest bucket's limits (16, 32); ascending and descending; one far outlier; a cluster of distinct scores; infinities; NaNs of either
+    scores; equal ones in numbers around the fullest bucket's limits (16, 24, 48); ascending and descending; one far outlier; a cluster of distinct scores; infinities; NaNs of either
     sign; zeros of either sign; ranges too small and too large to spread; a part of the columns at another level.  NaNs, which the
     comparator leaves open, in the order of their bits as before."""
     r = np.random.Generator(np.random.Philox(key=rows + cols))
